@@ -98,7 +98,7 @@ def prepare(case, seed):
     dtype, d, n = DTYPES[c["dtype"]], _channels(c), _coefs(c)
     if c["op"] == "stream":
         walks = dict(c, length=24, points=False)
-        sigs = [P.sig(_paths(walks, gen), c["degree"]) for _ in range(2)]
+        sigs = [_rows(_signature(_paths(walks, gen), c["degree"])).to(dtype) for _ in range(2)]
         state = {"sig": sigs[0].requires_grad_(True), "block": sigs[1].requires_grad_(True),
                  "increment": (torch.randn((c["batch"], d), generator=gen, device="cuda", dtype=dtype) * 0.2).requires_grad_(True)}
     else:
@@ -175,3 +175,198 @@ def tolerance(case):
     rel, most = _SINGLE[case["op"]]
     unit = 1.0 if case["dtype"] == "f32" else 2.0 ** -29        # double precision: by the ratio of the two roundings
     return {"rel": rel * unit, "max": most * unit}
+
+
+# ---- the same in 64 bits, with plain torch ----
+# A signature is a list of its levels, level k of shape (rows, d ** k); the leading 1 is left out.
+
+def _augmented(path, time_aug, lead_lag):
+    if lead_lag:        # lag and lead channels, the lead moves first
+        twice = path.repeat_interleave(2, 1)
+        path = torch.cat((twice[:, :-1], twice[:, 1:]), 2)
+    if time_aug:
+        time = torch.linspace(0.0, 1.0, path.shape[1], dtype=path.dtype, device=path.device)
+        path = torch.cat((path, time.expand(path.shape[0], -1).unsqueeze(2)), 2)
+    return path
+
+
+def _outer(a, b):
+    return (a.unsqueeze(2) * b.unsqueeze(1)).reshape(a.shape[0], -1)
+
+
+def _times(a, b, unit=1.0):
+    """Truncated tensor product; with unit 0 of the two without their leading 1."""
+    out = []
+    for t in range(len(a)):
+        v = (a[t] + b[t]) if unit else torch.zeros_like(a[t])
+        for k in range(t):
+            v = v + _outer(a[k], b[t - 1 - k])
+        out.append(v)
+    return out
+
+
+def _extended(levels, z):
+    """levels times exp(z), by Horner's rule."""
+    out = list(levels)
+    for t in range(len(levels), 0, -1):
+        v = z / t
+        for k in range(1, t):
+            v = _outer(levels[k - 1] + v, z / (t - k))
+        out[t - 1] = levels[t - 1] + v
+    return out
+
+
+def _rows(levels):
+    return torch.cat(levels, 1)
+
+
+def _pieces(z, degree):
+    """Increments (rows, steps, d) cut in time into pieces that are swept beside each other: (rows * pieces, steps, d)."""
+    rows, steps, d = z.shape
+    size = 8.0 * rows * sum(d ** k for k in range(1, degree + 1))
+    pieces = 1
+    while pieces < 64 and steps >= 32 * pieces and size * 2 * pieces <= 3e7:
+        pieces *= 2
+    each = -(-steps // pieces)
+    z = torch.nn.functional.pad(z, (0, 0, 0, pieces * each - steps))
+    return z.reshape(rows * pieces, each, d), pieces
+
+
+def _joined(levels, pieces):
+    while pieces > 1:
+        halves = [v.reshape(-1, 2, v.shape[1]) for v in levels]
+        levels, pieces = _times([v[:, 0] for v in halves], [v[:, 1] for v in halves]), pieces // 2
+    return levels
+
+
+def _signature(path, degree, time_aug=False, lead_lag=False, grad_of=None):
+    """Levels of the signature, or with grad_of(levels) -> scalar: (levels, gradient with respect to the path)."""
+    path = path.detach().double()
+    if grad_of is not None:
+        path.requires_grad_(True)
+    with torch.set_grad_enabled(grad_of is not None):
+        points = _augmented(path, time_aug, lead_lag)
+        cut, pieces = _pieces(points[:, 1:] - points[:, :-1], degree)
+    z, d = cut.detach(), cut.shape[2]
+    state = [torch.zeros((z.shape[0], d ** k), dtype=torch.float64, device=z.device) for k in range(1, degree + 1)]
+    stride = max(1, math.isqrt(z.shape[1]))
+    kept = []               # the state before every `stride` steps, from which the gradient sweeps them again
+    for s in range(z.shape[1]):
+        if grad_of is not None and s % stride == 0:
+            kept.append(state)
+        state = _extended(state, z[:, s])
+    if grad_of is None:
+        return _joined(state, pieces)
+    ends = [v.requires_grad_(True) for v in state]
+    with torch.enable_grad():
+        whole = _joined(ends, pieces)
+        back = torch.autograd.grad(grad_of(whole), ends)
+    dz = torch.zeros_like(z)
+    for n in range(len(kept) - 1, -1, -1):
+        part = z[:, n * stride:(n + 1) * stride].clone().requires_grad_(True)
+        first = [v.detach().requires_grad_(True) for v in kept.pop()]
+        with torch.enable_grad():
+            v = first
+            for s in range(part.shape[1]):
+                v = _extended(v, part[:, s])
+        got = torch.autograd.grad(v, [part, *first], back)
+        dz[:, n * stride:(n + 1) * stride] = got[0]
+        back = got[1:]
+    return [v.detach() for v in whole], torch.autograd.grad(cut, path, dz)[0]
+
+
+def _logarithm(levels):
+    out, power = list(levels), levels
+    for k in range(2, len(levels) + 1):
+        power = _times(power, levels, 0.0)
+        out = [a + b * ((-1) ** (k + 1) / k) for a, b in zip(out, power)]
+    return out
+
+
+def _lyndon_words(d, degree):
+    """By length, then in alphabetical order (Duval's successor rule)."""
+    found, w = [[] for _ in range(degree)], [-1]
+    while w:
+        w[-1] += 1
+        found[len(w) - 1].append(tuple(w))
+        w = [w[i % len(w)] for i in range(degree)]
+        while w and w[-1] == d - 1:
+            w.pop()
+    return found
+
+
+def _index(word, d):
+    n = 0
+    for letter in word:
+        n = n * d + letter
+    return n
+
+
+def _coordinates(d, degree, method):
+    """Functions of the levels of a tensor logarithm: its coefficients at the Lyndon words, or its coordinates in the basis
+    of their brackets [u, v], v the longest proper suffix that is a Lyndon word."""
+    found, brackets, parts = _lyndon_words(d, degree), {}, []
+    for words in found:
+        at = torch.tensor([_index(w, d) for w in words], device="cuda")
+        matrix = None
+        if method == 2:
+            matrix = torch.eye(len(words), dtype=torch.float64)
+            position = {w: i for i, w in enumerate(words)}
+            for j, w in enumerate(words):
+                if len(w) == 1:
+                    brackets[w] = {w: 1.0}
+                    continue
+                cut = next(i for i in range(1, len(w)) if w[i:] in brackets)
+                terms = {}
+                for a, x in brackets[w[:cut]].items():
+                    for b, y in brackets[w[cut:]].items():
+                        terms[a + b] = terms.get(a + b, 0.0) + x * y
+                        terms[b + a] = terms.get(b + a, 0.0) - x * y
+                brackets[w] = terms
+                for a, x in terms.items():
+                    if a in position:
+                        matrix[position[a], j] = x
+            matrix = matrix.cuda()
+        parts.append((at, matrix))
+
+    def read(levels):
+        out = []
+        for v, (at, matrix) in zip(levels, parts):
+            v = v[:, at]
+            out.append(v if matrix is None else torch.linalg.solve_triangular(matrix, v.T, upper=False).T)
+        return _rows(out)
+    return read
+
+
+def exact(case, seed):
+    c, degree, d = case, case["degree"], _channels(case)
+    steps = (2 * c["length"] - 1) if c["lead_lag"] else c["length"]
+    # sweeps in launches: the forward sweep, and for the gradient a second one and the way back of each
+    launches = degree * (degree + 1) * 1.5 * (1 if c["op"] == "sig" else 5)
+    if c["op"] != "stream" and steps * launches * 6e-6 > 18 and c["batch"] * _coefs(c) > 50000:
+        return None
+    if c["op"] == "logsig" and c["method"] == 2 and sum(map(len, _lyndon_words(d, degree))) > 6000:
+        return None
+    state = prepare(case, seed)
+    rows = max(1, int(1e9 // (8 * _coefs(c) * (1 if c["op"] == "sig" else degree))))     # paths at a time
+    read = _coordinates(d, degree, c["method"]) if c["op"] == "logsig" else None
+    out = []
+    for n in range(0, c["batch"], rows):
+        part = slice(n, n + rows)
+        if c["op"] == "stream":
+            x, z, y = (state[k].detach()[part].double().requires_grad_(True) for k in ("sig", "increment", "block"))
+            with torch.enable_grad():
+                levels = [v.split([d ** k for k in range(1, degree + 1)], 1) for v in (x, y)]
+                whole = _rows(_times(_extended(levels[0], z), levels[1]))
+            out.append([whole.detach(), *torch.autograd.grad(whole, (x, z, y), state["grad"][part].double())])
+            continue
+        path, options = state["path"][part], (degree, c["time_aug"], c["lead_lag"])
+        if c["op"] == "sig":
+            out.append([_rows(_signature(path, *options))])
+            continue
+        grad = state["grad"][part].double()
+        last = (lambda v: read(_logarithm(v))) if read else _rows
+        levels, dpath = _signature(path, *options, grad_of=lambda v: (last(v) * grad).sum())
+        out.append([last(levels), dpath])
+    out = [torch.cat(v) for v in zip(*out)]
+    return out[0] if c["op"] == "sig" else out
