@@ -534,7 +534,10 @@ static bool want_degree3_gemm(uint64_t d_aug, uint64_t degree, uint64_t L, uint6
     if (L > kDeg3BufBytes / (d_aug * d_aug * (f64 ? 8 : 4))) return false;
     if (g_force_degree3 >= 0) return g_force_degree3 != 0;
     const uint64_t waves = ((d_aug + kWave - 1) / kWave) * ((d_aug + kDeg3RowsPerThread - 1) / kDeg3RowsPerThread) * batch;
-    const uint64_t from = backward ? (f64 ? 36u : 65u) : 112u;      // forward: 1.3x at 128 channels, slower at 80
+    // forward: 1.3x at 128 channels, slower at 80; in single precision the matrix form of the by-row sweep needs no rows
+    // buffer and takes half the time (200 paths of 256 steps, 112 channels 4.4 -> 2.2 ms, 128: 5.4 -> 2.3)
+    if (!backward && !f64) return false;
+    const uint64_t from = backward ? (f64 ? 36u : 65u) : 112u;
     return d_aug >= from && waves >= 1024;
 }
 
@@ -811,11 +814,18 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
         // segment: segments start on even steps
         const bool sparse_ll = lead_lag && g_lead_lag_sparse != 0;
         // many channels without a compiled instance: the by-row sweep, whole paths only (its launches fill the chip).
-        // Measured against the general run-time kernels (16 / 32 letters per lane) at 33 .. 96 channels, degrees 4 to 6:
-        // double precision 1.0-1.46x faster; single precision 0.95-1.2x where 32 does not divide the channel count,
-        // 0.72-0.89x where it does (the 32-letter kernel then has no partly empty group and feeds from two buffers).
-        const bool rows_win = sizeof(T) == 8 || s.d_aug % 32 != 0;
-        const bool by_rows = e->D <= 0 && rows_win && g_rows_forward != 0 && g_force_tail == 0 &&
+        // Double precision, against the general run-time kernels (16 / 32 letters per lane) at 33 .. 96 channels, degrees 4
+        // to 6: 1.0-1.46x faster.  Single precision runs on the matrix units, bit for bit the same: always faster than the
+        // run-time kernels (16 paths of 200 steps, 64 channels, degree 4: 2.60 -> 1.27 ms; 5 x 64, 70: 0.89 -> 0.48; 2 x 50,
+        // 33, degree 5: 0.69 -> 0.43), and than a compiled instance where its tiles of 32 x 32 are filled well enough
+        // (256 x 256, 64 channels, degree 3: 0.94 -> 0.39; 300 x 200, 96: 2.05 -> 1.39; 8 x 100, 48, degree 4: 0.28 -> 0.22;
+        // but 64 x 200, 40, degree 4, 39 % filled: 1.20 -> 1.83) by launches that need no time split (4 x 500, 48, degree 3,
+        // split: 0.080, whole: 0.103).
+        const uint64_t tile = (s.d_aug + 31) / 32 * 32, groups = (s.d_aug + kWave - 1) / kWave;
+        const bool rows_beat_instance = sizeof(T) == 4 && !lead_lag && 16 * s.d_aug * s.d_aug >= 9 * tile * tile &&
+                                        (degree >= 4 || batch * s.d_aug * groups * groups >= uint64_t(simd_count()));
+        const bool rows_win = e->D <= 0 || rows_beat_instance;
+        const bool by_rows = rows_win && g_rows_forward != 0 && g_force_tail == 0 &&
                              rows_bwd_supported(sizeof(T), s.d_aug, degree) && rows_bwd_fits(sizeof(T), s.d_aug, degree, batch);
         int nseg = by_rows ? 1 : g_force_segments > 0
                              ? int(std::min<uint64_t>(uint64_t(g_force_segments), s.L))
@@ -866,7 +876,7 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
         const std::string shown = by_rows ? std::string(sizeof(T) == 8 ? "rows_fwd_f64_n" : "rows_fwd_f32_n") + std::to_string(degree)
                                   : use_ll ? std::string(e->name) + "_ll" : std::string(e->name);
         MainKernelTimer timer(stream, shown.c_str());
-        if (by_rows) SIG_HIP(launch_rows_fwd<T>(p, int(degree)));
+        if (by_rows) SIG_HIP(sizeof(T) == 4 ? launch_rows_fwd_mfma(p, int(degree)) : launch_rows_fwd_f64(p, int(degree)));
         else SIG_HIP(use_ll ? e->fwd_lead_lag(p) : e->fwd(p));
         timer.stop(/*defer=*/true);
         if (nseg > 1) {
@@ -1177,7 +1187,10 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
         // (also where an instance would lose: measured at 48 .. 128 channels, degrees 3 and 4, the by-row sweep runs
         // 1.1-4x faster than compiled single-precision instances and 1-12x faster than double-precision ones; the
         // instance table leaves these backward shapes out)
-        const bool rows_win = e->D <= 0 || s.d_aug >= 48;
+        // (single precision up to 256 channels runs on the matrix units, and wins at degree 3 from 33 channels on: 64 paths
+        // of 200 steps, 40 channels 0.328 -> 0.234 ms, 16 x 200, 36: 0.340 -> 0.121; at degree 4 and 40 channels its tiles
+        // are 39 % filled: 4.6 -> 6.0; fewer waves are left to the time splits)
+        const bool rows_win = e->D <= 0 || s.d_aug >= 48 || (sizeof(T) == 4 && degree == 3 && !lead_lag && 2 * batch * s.d_aug >= uint64_t(simd_count()));
         const bool by_rows = !arena && rows_win && g_rows_backward != 0 && g_force_tail == 0 &&
                              rows_bwd_supported(sizeof(T), s.d_aug, degree) && rows_bwd_fits(sizeof(T), s.d_aug, degree, batch);
         int nseg = (arena || by_rows || !ef || degree > uint64_t(kCombMaxLevels)) ? 1
@@ -1229,6 +1242,14 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
             p.inc = inc;
         }
         p.dzinc = dzinc;
+        // single precision on the matrix units: the increment gradient is summed in double precision
+        double* wide_dz = nullptr;
+        if (by_rows && sizeof(T) == 4 && rows_bwd_mfma_supported(s.d_aug)) {
+            wide_dz = static_cast<double*>(buffer(6, checked_mul(dz_elems, sizeof(double), "increments")));
+            hipLaunchKernelGGL((zero_kernel<double>), dim3(grid_for(dz_elems)), dim3(kBlock), 0, stream, wide_dz, int64_t(dz_elems));
+            SIG_HIP(hipGetLastError());
+            p.dzinc = wide_dz;
+        }
         if (nseg > 1) {
             // (path, segment) rows, scalar-free: segment signatures, their running products from the left (the state
             // at each segment's end), from the right (what follows each segment), and the adjoints of the states
@@ -1287,11 +1308,14 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
         MainKernelTimer timer(stream, shown.c_str(), !arena);
         if (turn) turn->dirty[mine] = dz_bytes;        // from here on the accumulator holds sums
         if (by_rows) {
-            SIG_HIP(launch_rows_bwd<T>(p, int(degree)));
+            if (wide_dz) SIG_HIP(launch_rows_bwd_mfma(p, int(degree)));
+            else SIG_HIP(launch_rows_bwd<T>(p, int(degree)));
         } else {
             SIG_HIP(use_ll ? e->bwd_lead_lag(p) : e->bwd(p));
         }
         timer.stop();
+        if constexpr (sizeof(T) == 4)
+            if (wide_dz) SIG_HIP(launch_narrow(wide_dz, dzinc, int64_t(dz_elems), stream));
         if (turn) {
             // the same launch clears what the other accumulator still holds: it is the next call's
             const int other = 1 - mine;

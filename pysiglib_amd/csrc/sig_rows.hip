@@ -27,6 +27,7 @@
 #include <hip/hip_runtime.h>
 
 #include "sig_rows.h"
+#include "sig_rows_lanes.h"
 #include "sig_launch.h"
 
 namespace sigamd {
@@ -36,56 +37,6 @@ constexpr int kRowLettersOf = sizeof(T) == 8 ? 32 : 64;
 constexpr int kRowsMinDim = 33;         // below, the compiled table or the other run-time kernels are faster
 constexpr int kRowsMinDegree = 3;
 constexpr int kRowsMaxDegree = 8;
-
-template <int CTRL>
-__device__ __forceinline__ float dpp_moved(float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
-}
-template <int CTRL>
-__device__ __forceinline__ double dpp_moved(double v)
-{
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
-    return __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ float lane_value(float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); }
-__device__ __forceinline__ double lane_value(double v, int l)
-{
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l), __builtin_amdgcn_readlane(__double2loint(v), l));
-}
-// every lane receives the sum over its row of 16 lanes
-template <typename T>
-__device__ __forceinline__ T row_sum_rows(T v)
-{
-    v += dpp_moved<0xB1>(v);        // quad_perm [1, 0, 3, 2]
-    v += dpp_moved<0x4E>(v);        // quad_perm [2, 3, 0, 1]
-    v += dpp_moved<0x141>(v);       // row_half_mirror
-    v += dpp_moved<0x140>(v);       // row_mirror
-    return v;
-}
-// sum over the 64 lanes, valid in every lane
-template <typename T>
-__device__ __forceinline__ T wave_sum_rows(T v)
-{
-    v = row_sum_rows(v);
-    return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
-}
-// lanes 0-31: lo[lane] + lo[lane + 32];  lanes 32-63: hi[lane - 32] + hi[lane]
-__device__ __forceinline__ float half_sums(float lo, float hi)
-{
-    const auto r = __builtin_amdgcn_permlane32_swap(unsigned(__float_as_int(lo)), unsigned(__float_as_int(hi)), false, false);
-    return __int_as_float(int(r[0])) + __int_as_float(int(r[1]));
-}
-__device__ __forceinline__ double half_sums(double lo, double hi) { return pair_sum32(lo, hi); }
-// the sums of two values over the 64 lanes for the price of one and a half: the half-waves first exchange halves
-template <typename T>
-__device__ __forceinline__ void wave_sum_two(T a, T b, T& sum_a, T& sum_b)
-{
-    const T v = row_sum_rows(half_sums(a, b));
-    sum_a = lane_value(v, 0) + lane_value(v, 16);
-    sum_b = lane_value(v, 32) + lane_value(v, 48);
-}
 
 // Waves per block; a block fills a CU.  Degrees 3 and 4 fit 168 vector registers (three waves per SIMD: 7.0 ms against 7.7 ms
 // for 16 paths of 200 steps, 64 channels, degree 4); the longer chains above need more and run two waves per SIMD (a
@@ -365,7 +316,7 @@ __global__ __launch_bounds__((kRowsWavesOf<T, N> * kWave)) void rows_bwd_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Forward sweep in the same tiling (arithmetic: siglib/cpsig/cp_signature.h:464-499): a lane owns the prefix
+// Forward sweep in double precision in the same tiling (arithmetic: siglib/cpsig/cp_signature.h:464-499): a lane owns the prefix
 // (r, 64 blk + lane), its chain, and the KB top-level coefficients (prefix, letter) of the wave's letter tile.  Per step
 // the top level costs one multiply-add per coefficient, S_N[p, a] += U[p] * z[a], with z[a] wave-uniform from scalar
 // loads; the chain work of a lane is shared by 64 (32) of them instead of the 16 or 32 of the general run-time kernels.
@@ -512,24 +463,18 @@ hipError_t launch_rows_fwd_n(const FwdParams& p)
     return hipGetLastError();
 }
 
-template <typename T>
-hipError_t launch_rows_fwd(const FwdParams& p, int degree)
+hipError_t launch_rows_fwd_f64(const FwdParams& p, int degree)
 {
     if (p.nseg != 1 || p.from_points || p.d < kRowsMinDim || p.d > kRowsMaxDim) return hipErrorInvalidConfiguration;
     switch (degree) {
-        case 3: return launch_rows_fwd_n<T, 3>(p);
-        case 4: return launch_rows_fwd_n<T, 4>(p);
-        case 5: return launch_rows_fwd_n<T, 5>(p);
-        case 6: return launch_rows_fwd_n<T, 6>(p);
-        case 7: return launch_rows_fwd_n<T, 7>(p);
-        case 8:
-            if constexpr (sizeof(T) == 4) return launch_rows_fwd_n<T, 8>(p);
-            return hipErrorInvalidConfiguration;
+        case 3: return launch_rows_fwd_n<double, 3>(p);
+        case 4: return launch_rows_fwd_n<double, 4>(p);
+        case 5: return launch_rows_fwd_n<double, 5>(p);
+        case 6: return launch_rows_fwd_n<double, 6>(p);
+        case 7: return launch_rows_fwd_n<double, 7>(p);
         default: return hipErrorInvalidConfiguration;
     }
 }
-template hipError_t launch_rows_fwd<float>(const FwdParams&, int);
-template hipError_t launch_rows_fwd<double>(const FwdParams&, int);
 
 template <typename T, int N>
 hipError_t launch_rows(const BwdParams& p)
@@ -566,7 +511,7 @@ bool rows_bwd_fits(size_t elem_bytes, uint64_t d, uint64_t degree, uint64_t batc
         per_path *= d;
         if (per_path > (unsigned __int128)kMaxGridX * 8) return false;
     }
-    const unsigned __int128 blocks = (per_path + 7) / 8 * batch;      // at the smaller of the two block sizes
+    const unsigned __int128 blocks = (per_path + 3) / 4 * batch;      // at the smallest of the block sizes
     return blocks >= 1 && blocks <= (unsigned __int128)kMaxGridX;
 }
 

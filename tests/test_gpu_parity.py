@@ -753,6 +753,34 @@ def test_by_row_reverse_sweep(P, oracle, shape, aug, scalar_term):
         assert bwd_rel_err(other, want) <= TOL[dtype], (dtype, bwd_rel_err(other, want))
 
 
+@pytest.mark.parametrize("shape,aug,scalar_term", [
+    ((40, 2, 33, 3), {}, False), ((33, 17, 47, 3), {}, True),       # one step; a whole chunk of sixteen reverse steps, prefixes and letters in part
+    ((22, 18, 48, 3), {}, False), ((2, 18, 63, 3), {}, False),      # one step beyond it, odd and even numbers of steps
+    ((16, 33, 64, 3), {}, True), ((2, 35, 65, 3), {}, False),       # two chunks; a second tile of a single prefix and letter
+    ((2, 3, 96, 3), dict(time_aug=True), False),                    # 97 channels: three of four groups of 32 and one more
+    ((1, 20, 256, 3), {}, False), ((1, 20, 257, 3), {}, True),      # either side of the reverse sweep's limit
+    ((1, 19, 48, 4), {}, False), ((1, 18, 65, 4), {}, True),
+])
+def test_by_row_sweeps_on_the_matrix_units(P, oracle, shape, aug, scalar_term):
+    """Single precision, at the edges of the tiles (64 prefixes x 64 letters, groups of 32) and of the chunks of steps,
+    against the oracle on the same inputs in double precision.  Rounding: the result is a sum over at most (steps x d^2)
+    products that themselves carry a few units of 6e-8; 1e-5 of a level (path) holds it with room."""
+    b, length, d, deg = shape
+    rng = np.random.default_rng(b * 100000 + length * 1000 + d * 10 + deg)
+    x = (np.cumsum(rng.standard_normal((b, length, d)), axis=1) / np.sqrt(d * length)).astype(np.float32)
+    d_aug = d + (1 if aug.get("time_aug") else 0)
+    off = 1 if scalar_term else 0
+    ref = oracle.signature(x.astype(np.float64), deg, scalar_term=scalar_term, n_jobs=-1, **aug)
+    g = rng.standard_normal(ref.shape).astype(np.float32)
+    fwd = P.sig(dev(x), deg, scalar_term=scalar_term, **aug)
+    assert level_rel_err(fwd.cpu().numpy()[:, off:], ref[:, off:], d_aug, deg) <= 1e-5
+    if scalar_term:
+        np.testing.assert_array_equal(fwd.cpu().numpy()[:, 0], 1.0)
+    want = oracle.sig_backprop(x.astype(np.float64), ref, g.astype(np.float64), deg, n_jobs=-1, **aug)
+    got = P.sig_backprop(dev(x), fwd, dev(g), deg, **aug).cpu().numpy()
+    assert bwd_rel_err(got, want) <= 1e-5
+
+
 @pytest.mark.parametrize("shape", [(3, 9, 2, 5), (2, 7, 2, 9), (5, 12, 2, 12), (2, 6, 3, 4), (3, 10, 3, 7), (2, 9, 3, 10),
                                    (4, 8, 4, 3), (2, 11, 4, 6), (70, 5, 2, 6), (1, 300, 3, 5)])
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
