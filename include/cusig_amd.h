@@ -267,15 +267,17 @@ CUSIG_AMD_API void cusig_amd_set_point_fed(int on) CUSIG_AMD_NOEXCEPT;
 CUSIG_AMD_API void cusig_amd_set_lead_lag_sparse(int on) CUSIG_AMD_NOEXCEPT;
 /* Tuning hook: number of time segments the backward sweep splits every path into (0 = automatic, 1 = never). */
 CUSIG_AMD_API void cusig_amd_force_bwd_segments(int segments) CUSIG_AMD_NOEXCEPT;
-/* Test hook: 1 (default) lets single-precision backward sweeps of 33 and more augmented channels at degrees 3 .. 8 that
- * the compiled instance table does not cover run the by-row reverse sweep (a wave holds its tile of top-level adjoints
- * both by prefix and by letter, so no per-step reduction across lanes is left); 0 sends them to the general run-time
- * kernels. */
-CUSIG_AMD_API void cusig_amd_set_rows_backward(int on) CUSIG_AMD_NOEXCEPT;
-/* Test hook: the same switch for the forward sweep of such shapes (33 and more channels without a compiled instance,
- * degrees 3 .. 8): 1 (default) runs the by-row forward sweep (64 or 32 top-level letters per lane), 0 the general
- * run-time kernels. */
-CUSIG_AMD_API void cusig_amd_set_rows_forward(int on) CUSIG_AMD_NOEXCEPT;
+/* Whether the last signature / sig_backprop sweep of this thread was a by-row sweep on the matrix units (single precision,
+ * 33 and more channels): 1 or 0.  Such sweeps carry the same cusig_amd_last_kernel_name as the form without them. */
+CUSIG_AMD_API int cusig_amd_last_sweep_on_matrix_units(void) CUSIG_AMD_NOEXCEPT;
+/* Test hook: the by-row reverse sweep of 33 and more augmented channels at degrees 3 and up (a wave holds its tile of
+ * top-level adjoints both by prefix and by letter): 0 never, 1 (default) where it is expected to be the fastest form,
+ * 2 wherever it applies, 3 the same with single precision kept off the matrix units.  (Degree 3 as matrix products has a
+ * hook of its own, cusig_amd_force_degree3, and goes first.) */
+CUSIG_AMD_API void cusig_amd_set_rows_backward(int mode) CUSIG_AMD_NOEXCEPT;
+/* Test hook: the same switch for the forward sweep of such shapes: 0 never, 1 (default) where it is expected to be the
+ * fastest form, 2 wherever it applies. */
+CUSIG_AMD_API void cusig_amd_set_rows_forward(int mode) CUSIG_AMD_NOEXCEPT;
 /* Tuning hook: how increments reach the waves: -1 automatic, 0 scalar loads, 1 LDS-staged where compiled. */
 CUSIG_AMD_API void cusig_amd_force_staged(int mode) CUSIG_AMD_NOEXCEPT;
 /* Test hook: nonzero makes the coefficient-per-thread kernels use their 64-bit index arithmetic (otherwise only

@@ -435,8 +435,11 @@ static int choose_segments(int64_t waves, int64_t L, int waves_per_simd, uint64_
 // with the remaining segments.  That costs a segmented forward sweep, two chains of Chen products and one product
 // adjoint, all over (path, segment) rows.
 static Hook g_force_bwd_segments{0};   // tuning hook (0 = automatic)
-static Hook g_rows_forward{1};         // test hook: the same for the forward sweep
-static Hook g_rows_backward{1};        // test hook: 0 = shapes beyond the table never take the by-row reverse sweep (sig_rows.hip)
+// test hooks, the by-row sweeps of many channels: 0 never, 1 by the rules below, 2 wherever they apply; backward also 3,
+// wherever they apply, single precision in the form without matrix units
+static Hook g_rows_forward{1};
+static Hook g_rows_backward{1};
+static thread_local int tl_matrix_form = 0;     // whether the last sweep on this thread was a by-row sweep on the matrix units
 
 // g pieces are chosen by the same kind of model as for the forward sweep (fullest SIMD, `pair_rate`, lane_step(g) =
 // seconds per step of a lone wave).  The extra work is larger here: the segmented forward sweep (a third of the
@@ -682,6 +685,7 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
     // everything below runs under the workspace mutex: one flag serves all callers
     std::lock_guard<std::mutex> lk(g_ws_mutex);
     tl_sig_nonfinite = -1;
+    tl_matrix_form = 0;
     int* flag = nullptr;
     if (!g_stream_ordered) {
         flag = nonfinite_flag();
@@ -825,7 +829,8 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
         const bool rows_beat_instance = sizeof(T) == 4 && !lead_lag && 16 * s.d_aug * s.d_aug >= 9 * tile * tile &&
                                         (degree >= 4 || batch * s.d_aug * groups * groups >= uint64_t(simd_count()));
         const bool rows_win = e->D <= 0 || rows_beat_instance;
-        const bool by_rows = rows_win && g_rows_forward != 0 && g_force_tail == 0 &&
+        const int rows_mode = g_rows_forward;
+        const bool by_rows = (rows_mode >= 2 || (rows_mode == 1 && rows_win)) && g_force_tail == 0 &&
                              rows_bwd_supported(sizeof(T), s.d_aug, degree) && rows_bwd_fits(sizeof(T), s.d_aug, degree, batch);
         int nseg = by_rows ? 1 : g_force_segments > 0
                              ? int(std::min<uint64_t>(uint64_t(g_force_segments), s.L))
@@ -876,6 +881,7 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
         const std::string shown = by_rows ? std::string(sizeof(T) == 8 ? "rows_fwd_f64_n" : "rows_fwd_f32_n") + std::to_string(degree)
                                   : use_ll ? std::string(e->name) + "_ll" : std::string(e->name);
         MainKernelTimer timer(stream, shown.c_str());
+        tl_matrix_form = by_rows && sizeof(T) == 4;
         if (by_rows) SIG_HIP(sizeof(T) == 4 ? launch_rows_fwd_mfma(p, int(degree)) : launch_rows_fwd_f64(p, int(degree)));
         else SIG_HIP(use_ll ? e->fwd_lead_lag(p) : e->fwd(p));
         timer.stop(/*defer=*/true);
@@ -992,6 +998,7 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
     auto finish = [&] { if (!arena) exit_sync(stream); };
     std::unique_lock<std::mutex> lk(g_ws_mutex, std::defer_lock);
     auto lock_pool = [&] { if (!arena && !lk.owns_lock()) lk.lock(); };
+    tl_matrix_form = 0;
     Degree3Buffers<T> d3;
     if (!arena && s.len_aug > 1 && want_degree3_gemm(s.d_aug, degree, s.L, batch, sizeof(T) == 8, true)) {
         lock_pool();
@@ -1191,7 +1198,8 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
         // of 200 steps, 40 channels 0.328 -> 0.234 ms, 16 x 200, 36: 0.340 -> 0.121; at degree 4 and 40 channels its tiles
         // are 39 % filled: 4.6 -> 6.0; fewer waves are left to the time splits)
         const bool rows_win = e->D <= 0 || s.d_aug >= 48 || (sizeof(T) == 4 && degree == 3 && !lead_lag && 2 * batch * s.d_aug >= uint64_t(simd_count()));
-        const bool by_rows = !arena && rows_win && g_rows_backward != 0 && g_force_tail == 0 &&
+        const int rows_mode = g_rows_backward;
+        const bool by_rows = !arena && (rows_mode >= 2 || (rows_mode == 1 && rows_win)) && g_force_tail == 0 &&
                              rows_bwd_supported(sizeof(T), s.d_aug, degree) && rows_bwd_fits(sizeof(T), s.d_aug, degree, batch);
         int nseg = (arena || by_rows || !ef || degree > uint64_t(kCombMaxLevels)) ? 1
                    : g_force_bwd_segments > 0 ? int(std::min<uint64_t>(uint64_t(g_force_bwd_segments), s.L))
@@ -1244,7 +1252,7 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
         p.dzinc = dzinc;
         // single precision on the matrix units: the increment gradient is summed in double precision
         double* wide_dz = nullptr;
-        if (by_rows && sizeof(T) == 4 && rows_bwd_mfma_supported(s.d_aug)) {
+        if (by_rows && sizeof(T) == 4 && rows_mode != 3 && rows_bwd_mfma_supported(s.d_aug)) {
             wide_dz = static_cast<double*>(buffer(6, checked_mul(dz_elems, sizeof(double), "increments")));
             hipLaunchKernelGGL((zero_kernel<double>), dim3(grid_for(dz_elems)), dim3(kBlock), 0, stream, wide_dz, int64_t(dz_elems));
             SIG_HIP(hipGetLastError());
@@ -1307,6 +1315,7 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
                                   : use_ll ? std::string(e->name) + "_ll" : std::string(e->name);
         MainKernelTimer timer(stream, shown.c_str(), !arena);
         if (turn) turn->dirty[mine] = dz_bytes;        // from here on the accumulator holds sums
+        tl_matrix_form = wide_dz != nullptr;
         if (by_rows) {
             if (wide_dz) SIG_HIP(launch_rows_bwd_mfma(p, int(degree)));
             else SIG_HIP(launch_rows_bwd<T>(p, int(degree)));
@@ -1500,8 +1509,9 @@ CUSIG_AMD_API void cusig_amd_set_lead_lag_sparse(int on) noexcept { if (g_test_h
 
 CUSIG_AMD_API void cusig_amd_force_bwd_segments(int segments) noexcept { if (g_test_hooks) g_force_bwd_segments = segments; }
 
-CUSIG_AMD_API void cusig_amd_set_rows_backward(int on) noexcept { if (g_test_hooks) g_rows_backward = on; }
-CUSIG_AMD_API void cusig_amd_set_rows_forward(int on) noexcept { if (g_test_hooks) g_rows_forward = on; }
+CUSIG_AMD_API int cusig_amd_last_sweep_on_matrix_units(void) noexcept { return tl_matrix_form; }
+CUSIG_AMD_API void cusig_amd_set_rows_backward(int mode) noexcept { if (g_test_hooks) g_rows_backward = mode; }
+CUSIG_AMD_API void cusig_amd_set_rows_forward(int mode) noexcept { if (g_test_hooks) g_rows_forward = mode; }
 
 CUSIG_AMD_API void cusig_amd_force_staged(int mode) noexcept { if (g_test_hooks) g_force_staged = mode; }
 

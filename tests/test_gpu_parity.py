@@ -732,6 +732,7 @@ def test_by_row_reverse_sweep(P, oracle, shape, aug, scalar_term):
             compiled = (deg == 3 and d_aug <= 128) or (deg == 4 and d_aug <= 48)
             if not compiled and (dtype == np.float64 or d_aug % 32):
                 assert name == "rows_fwd_%s_n%d" % ("f32" if dtype == np.float32 else "f64", deg), name
+            assert compiled or name.startswith("rows_fwd_"), name
             assert L.CUSIG.cusig_amd_last_sig_nonfinite() == 0
             if scalar_term:
                 np.testing.assert_array_equal(fwd[:, 0], 1.0)
@@ -753,6 +754,33 @@ def test_by_row_reverse_sweep(P, oracle, shape, aug, scalar_term):
         assert bwd_rel_err(other, want) <= TOL[dtype], (dtype, bwd_rel_err(other, want))
 
 
+@pytest.fixture
+def by_rows():
+    """The by-row sweeps wherever they apply, whatever the rules of the dispatch say; by_rows(forward, backward) picks
+    other forms (0 never, 1 the rules, 2 wherever they apply, backward 3: off the matrix units)."""
+    import ctypes
+    from pysiglib_amd import _loader as L
+    for name in ("cusig_amd_set_rows_forward", "cusig_amd_set_rows_backward", "cusig_amd_force_degree3"):
+        getattr(L.CUSIG, name).argtypes = (ctypes.c_int,)
+        getattr(L.CUSIG, name).restype = None
+    L.CUSIG.cusig_amd_last_sweep_on_matrix_units.restype = ctypes.c_int
+    L.CUSIG.cusig_amd_last_kernel_name.restype = ctypes.c_char_p
+
+    def choose(forward, backward):
+        L.CUSIG.cusig_amd_set_rows_forward(forward)
+        L.CUSIG.cusig_amd_set_rows_backward(backward)
+
+    choose.last_on_matrix_units = L.CUSIG.cusig_amd_last_sweep_on_matrix_units
+    choose.last_name = lambda: L.CUSIG.cusig_amd_last_kernel_name().decode()
+    L.CUSIG.cusig_amd_set_profiling(1)
+    L.CUSIG.cusig_amd_force_degree3(0)
+    choose(2, 2)
+    yield choose
+    choose(1, 1)
+    L.CUSIG.cusig_amd_force_degree3(-1)
+    L.CUSIG.cusig_amd_set_profiling(0)
+
+
 @pytest.mark.parametrize("shape,aug,scalar_term", [
     ((40, 2, 33, 3), {}, False), ((33, 17, 47, 3), {}, True),       # one step; a whole chunk of sixteen reverse steps, prefixes and letters in part
     ((22, 18, 48, 3), {}, False), ((2, 18, 63, 3), {}, False),      # one step beyond it, odd and even numbers of steps
@@ -760,25 +788,88 @@ def test_by_row_reverse_sweep(P, oracle, shape, aug, scalar_term):
     ((2, 3, 96, 3), dict(time_aug=True), False),                    # 97 channels: three of four groups of 32 and one more
     ((1, 20, 256, 3), {}, False), ((1, 20, 257, 3), {}, True),      # either side of the reverse sweep's limit
     ((1, 19, 48, 4), {}, False), ((1, 18, 65, 4), {}, True),
+    ((3, 2, 64, 3), {}, True), ((1, 2, 64, 4), {}, False), ((1, 3, 49, 4), {}, False),     # one step, two
+    ((2, 9, 18, 3), dict(lead_lag=True), False), ((1, 4, 33, 5), {}, True),                # 36 channels; chains of four letters
 ])
-def test_by_row_sweeps_on_the_matrix_units(P, oracle, shape, aug, scalar_term):
+def test_by_row_sweeps_on_the_matrix_units(P, oracle, by_rows, shape, aug, scalar_term):
     """Single precision, at the edges of the tiles (64 prefixes x 64 letters, groups of 32) and of the chunks of steps,
     against the oracle on the same inputs in double precision.  Rounding: the result is a sum over at most (steps x d^2)
     products that themselves carry a few units of 6e-8; 1e-5 of a level (path) holds it with room."""
     b, length, d, deg = shape
     rng = np.random.default_rng(b * 100000 + length * 1000 + d * 10 + deg)
     x = (np.cumsum(rng.standard_normal((b, length, d)), axis=1) / np.sqrt(d * length)).astype(np.float32)
-    d_aug = d + (1 if aug.get("time_aug") else 0)
+    d_aug = (2 * d if aug.get("lead_lag") else d) + (1 if aug.get("time_aug") else 0)
     off = 1 if scalar_term else 0
     ref = oracle.signature(x.astype(np.float64), deg, scalar_term=scalar_term, n_jobs=-1, **aug)
     g = rng.standard_normal(ref.shape).astype(np.float32)
     fwd = P.sig(dev(x), deg, scalar_term=scalar_term, **aug)
+    assert by_rows.last_name() == "rows_fwd_f32_n%d" % deg and by_rows.last_on_matrix_units() == 1
     assert level_rel_err(fwd.cpu().numpy()[:, off:], ref[:, off:], d_aug, deg) <= 1e-5
     if scalar_term:
         np.testing.assert_array_equal(fwd.cpu().numpy()[:, 0], 1.0)
     want = oracle.sig_backprop(x.astype(np.float64), ref, g.astype(np.float64), deg, n_jobs=-1, **aug)
     got = P.sig_backprop(dev(x), fwd, dev(g), deg, **aug).cpu().numpy()
+    assert by_rows.last_name() == "rows_bwd_f32_n%d" % deg
+    assert by_rows.last_on_matrix_units() == (1 if d_aug <= 256 else 0)
     assert bwd_rel_err(got, want) <= 1e-5
+
+
+@pytest.mark.parametrize("shape,aug,scalar_term", [
+    ((1, 5, 64, 4), {}, False), ((2, 6, 49, 4), {}, True), ((2, 5, 70, 4), {}, False),
+    ((2, 4, 52, 4), dict(time_aug=True), False), ((1, 4, 130, 3), {}, True),
+])
+def test_by_row_reverse_sweep_without_matrix_units(P, oracle, by_rows, shape, aug, scalar_term):
+    """The single-precision form that serves what the matrix form does not (more than 256 channels), at sizes that the
+    oracle can check."""
+    b, length, d, deg = shape
+    rng = np.random.default_rng(b * 100000 + length * 1000 + d * 10 + deg)
+    x = (np.cumsum(rng.standard_normal((b, length, d)), axis=1) / np.sqrt(d * length)).astype(np.float32)
+    ref = oracle.signature(x.astype(np.float64), deg, scalar_term=scalar_term, n_jobs=-1, **aug)
+    g = rng.standard_normal(ref.shape).astype(np.float32)
+    want = oracle.sig_backprop(x.astype(np.float64), ref, g.astype(np.float64), deg, n_jobs=-1, **aug)
+    by_rows(2, 3)
+    got = P.sig_backprop(dev(x), dev(ref.astype(np.float32)), dev(g), deg, **aug).cpu().numpy()
+    assert by_rows.last_name() == "rows_bwd_f32_n%d" % deg and by_rows.last_on_matrix_units() == 0
+    assert bwd_rel_err(got, want) <= 1e-5
+
+
+@pytest.mark.parametrize("shape", [(2, 10, 48, 3), (3, 11, 64, 3), (2, 12, 33, 4), (1, 4, 33, 6)])
+def test_by_row_sweeps_beside_the_run_time_kernels(P, by_rows, shape):
+    """The matrix form of the forward sweep rounds like the run-time-dimension kernels, bit for bit (at degree 6 too, whose
+    chains run level by level), and reports overflow like a scan of its result; the reverse sweep agrees to rounding."""
+    import ctypes
+    from pysiglib_amd import _loader as L
+    L.CUSIG.cusig_amd_ignore_instance_table.argtypes = (ctypes.c_int,)
+    b, length, d, deg = shape
+    torch.manual_seed(d + deg)
+    x = torch.randn((b, length, d), device=DEV).cumsum(1) / np.sqrt(d * length)
+    try:
+        L.CUSIG.cusig_amd_ignore_instance_table(1)
+        fwd = P.sig(x, deg)
+        assert by_rows.last_on_matrix_units() == 1 and L.CUSIG.cusig_amd_last_sig_nonfinite() == 0
+        g = torch.randn_like(fwd)
+        back = P.sig_backprop(x, fwd, g, deg)
+        assert by_rows.last_on_matrix_units() == 1
+        by_rows(0, 0)
+        assert torch.equal(fwd, P.sig(x, deg))
+        other = P.sig_backprop(x, fwd, g, deg)
+        assert not by_rows.last_name().startswith("rows_") and by_rows.last_on_matrix_units() == 0
+    finally:
+        L.CUSIG.cusig_amd_ignore_instance_table(0)
+    # both sides round to 6e-8 of terms that are summed over the d^(deg-1) prefixes, the run-time kernels with atomics
+    assert bwd_rel_err(back.cpu().numpy(), other.cpu().numpy()) <= TOL[np.float32]
+    by_rows(2, 2)
+    if deg <= 4:
+        for kind in ("overflow", "nan"):
+            bad = x.clone()
+            if kind == "overflow":
+                bad[b - 1] *= 1e30
+            else:
+                bad[0, length - 1, d - 1] = float("nan")
+            with pytest.warns(RuntimeWarning):
+                out = P.sig(bad, deg)
+            assert by_rows.last_on_matrix_units() == 1
+            assert L.CUSIG.cusig_amd_last_sig_nonfinite() == 1 and not bool(torch.isfinite(out).all())
 
 
 @pytest.mark.parametrize("shape", [(3, 9, 2, 5), (2, 7, 2, 9), (5, 12, 2, 12), (2, 6, 3, 4), (3, 10, 3, 7), (2, 9, 3, 10),
