@@ -611,17 +611,17 @@ static Shape make_shape(uint64_t dimension, uint64_t length, uint64_t degree, bo
     return s;
 }
 
-template <typename T>
+template <typename T, typename Z = T>
 static void compute_increments(const T* path, T* inc, uint64_t batch, uint64_t dimension, uint64_t length,
                                bool time_aug, bool lead_lag, T end_time, const Shape& s, hipStream_t stream,
-                               T* zero_out = nullptr, uint64_t zero_count = 0)
+                               Z* zero_out = nullptr, uint64_t zero_count = 0)
 {
     const T time_step = s.len_aug > 1 ? end_time / T(s.len_aug - 1) : T(0);
     (void)zero_count;       // always the whole increment gradient of the batch: batch * L * d elements
     const uint64_t per = (s.L + 2) * s.d_aug;
     launch_indexed(per, (per + 1) / 2, batch, [&](auto ix, dim3 grid) {
         using I = decltype(ix);
-        hipLaunchKernelGGL((increments_kernel<T, I>), grid, dim3(kBlock), 0, stream, path, inc, int64_t(batch), int64_t(length),
+        hipLaunchKernelGGL((increments_kernel<T, I, Z>), grid, dim3(kBlock), 0, stream, path, inc, int64_t(batch), int64_t(length),
                            int(dimension), int(time_aug), int(lead_lag), time_step, zero_out, DivBy<I>(s.d_aug));
     });
     SIG_HIP(hipGetLastError());
@@ -936,24 +936,24 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
 // backward  (siglib/cpsig/cp_signature.h:909-1019, siglib/cusig/cu_signature.cu:3417-3488)
 // ---------------------------------------------------------------------------
 // increment gradient -> raw path gradient; plain paths with a channel count that allows it take 16 bytes per lane
-template <typename T>
-static void launch_path_grad(const T* dzinc, T* out, uint64_t batch, uint64_t length, uint64_t dimension, bool time_aug,
-                             bool lead_lag, hipStream_t stream, T* clear = nullptr, uint64_t clear_count = 0)
+template <typename T, typename Z = T>
+static void launch_path_grad(const Z* dzinc, T* out, uint64_t batch, uint64_t length, uint64_t dimension, bool time_aug,
+                             bool lead_lag, hipStream_t stream, Z* clear = nullptr, uint64_t clear_count = 0)
 {
     constexpr int V = int(16 / sizeof(T));
     if (!time_aug && !lead_lag && dimension % V == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
-        reinterpret_cast<uintptr_t>(dzinc) % 16 == 0) {
+        reinterpret_cast<uintptr_t>(dzinc) % sizeof(VecOf<Z, V>) == 0) {
         const uint64_t per = length * (dimension / V);
         launch_indexed(per, per, batch, [&](auto ix, dim3 grid) {
             using I = decltype(ix);
-            hipLaunchKernelGGL((path_grad_vec_kernel<T, I, V>), grid, dim3(kBlock), 0, stream, dzinc, out, int64_t(batch),
+            hipLaunchKernelGGL((path_grad_vec_kernel<T, Z, I, V>), grid, dim3(kBlock), 0, stream, dzinc, out, int64_t(batch),
                                int64_t(length), DivBy<I>(dimension / V), clear, int64_t(clear_count));
         });
         return;
     }
     launch_indexed(length * dimension, (length * dimension + 1) / 2, batch, [&](auto ix, dim3 grid) {
         using I = decltype(ix);
-        hipLaunchKernelGGL((path_grad_kernel<T, I>), grid, dim3(kBlock), 0, stream, dzinc, out, int64_t(batch),
+        hipLaunchKernelGGL((path_grad_kernel<T, Z, I>), grid, dim3(kBlock), 0, stream, dzinc, out, int64_t(batch),
                            int64_t(length), int(time_aug), int(lead_lag), DivBy<I>(dimension), clear, int64_t(clear_count));
     });
 }
@@ -1224,8 +1224,12 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
         const KernelEntry* e_run = pick_variant(true, e, total_waves(geom, int64_t(batch) * nseg), sparse_ll);
         const bool point_fed = !arena && !by_rows && nseg == 1 && e_run->staged && !time_aug && !lead_lag && e_run->D > 0 &&
                                e_run->D <= kPointFedMaxDim && g_point_fed != 0;
+        // single precision on the matrix units: the increment gradient is summed in double precision, and rounded where the
+        // path gradient is formed from it
+        const bool on_matrix_units = by_rows && sizeof(T) == 4 && rows_mode != 3 && rows_bwd_mfma_supported(s.d_aug);
         T* inc = nullptr;
         T* dzinc = nullptr;
+        double* wide_dz = nullptr;
         DzPair* turn = nullptr;
         int mine = 0;
         if (point_fed) {
@@ -1244,20 +1248,17 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
             p.from_points = 1;
         } else {
             inc = static_cast<T*>(buffer(0, checked_mul(inc_elems + 2 * pad, sizeof(T), "increments"))) + pad;
-            dzinc = static_cast<T*>(buffer(1, dz_bytes));
             // one launch writes the increments and clears the increment-gradient accumulator (dz_elems <= increment elements)
-            compute_increments(path, inc, batch, dimension, length, time_aug, lead_lag, end_time, s, stream, dzinc, dz_elems);
+            if (on_matrix_units) {
+                wide_dz = static_cast<double*>(buffer(1, checked_mul(dz_elems, sizeof(double), "increments")));
+                compute_increments(path, inc, batch, dimension, length, time_aug, lead_lag, end_time, s, stream, wide_dz, dz_elems);
+            } else {
+                dzinc = static_cast<T*>(buffer(1, dz_bytes));
+                compute_increments(path, inc, batch, dimension, length, time_aug, lead_lag, end_time, s, stream, dzinc, dz_elems);
+            }
             p.inc = inc;
         }
-        p.dzinc = dzinc;
-        // single precision on the matrix units: the increment gradient is summed in double precision
-        double* wide_dz = nullptr;
-        if (by_rows && sizeof(T) == 4 && rows_mode != 3 && rows_bwd_mfma_supported(s.d_aug)) {
-            wide_dz = static_cast<double*>(buffer(6, checked_mul(dz_elems, sizeof(double), "increments")));
-            hipLaunchKernelGGL((zero_kernel<double>), dim3(grid_for(dz_elems)), dim3(kBlock), 0, stream, wide_dz, int64_t(dz_elems));
-            SIG_HIP(hipGetLastError());
-            p.dzinc = wide_dz;
-        }
+        p.dzinc = wide_dz ? static_cast<void*>(wide_dz) : dzinc;
         if (nseg > 1) {
             // (path, segment) rows, scalar-free: segment signatures, their running products from the left (the state
             // at each segment's end), from the right (what follows each segment), and the adjoints of the states
@@ -1315,16 +1316,14 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
                                   : use_ll ? std::string(e->name) + "_ll" : std::string(e->name);
         MainKernelTimer timer(stream, shown.c_str(), !arena);
         if (turn) turn->dirty[mine] = dz_bytes;        // from here on the accumulator holds sums
-        tl_matrix_form = wide_dz != nullptr;
+        tl_matrix_form = on_matrix_units;
         if (by_rows) {
-            if (wide_dz) SIG_HIP(launch_rows_bwd_mfma(p, int(degree)));
+            if (on_matrix_units) SIG_HIP(launch_rows_bwd_mfma(p, int(degree)));
             else SIG_HIP(launch_rows_bwd<T>(p, int(degree)));
         } else {
             SIG_HIP(use_ll ? e->bwd_lead_lag(p) : e->bwd(p));
         }
         timer.stop();
-        if constexpr (sizeof(T) == 4)
-            if (wide_dz) SIG_HIP(launch_narrow(wide_dz, dzinc, int64_t(dz_elems), stream));
         if (turn) {
             // the same launch clears what the other accumulator still holds: it is the next call's
             const int other = 1 - mine;
@@ -1334,6 +1333,9 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
             SIG_HIP(hipGetLastError());
             turn->dirty[other] = 0;
             turn->next = other;
+        } else if (wide_dz) {
+            launch_path_grad<T>(wide_dz, out, batch, length, dimension, time_aug, lead_lag, stream);
+            SIG_HIP(hipGetLastError());
         } else {
             launch_path_grad<T>(dzinc, out, batch, length, dimension, time_aug, lead_lag, stream);
             SIG_HIP(hipGetLastError());

@@ -1026,10 +1026,11 @@ void launch_indexed(uint64_t max_index, uint64_t per_item, uint64_t batch, F&& f
 // (siglib/cpsig/cp_path.h:46-62,262-279; siglib/cusig/cu_signature.cu:146-166).
 // Grid: x over the (L + 2) * d elements of one path, y over the paths; the only division is by d.
 // ---------------------------------------------------------------------------
-template <typename T, typename I>
+// Z: element type of the increment gradient, T or (some single-precision sweeps) double.
+template <typename T, typename I, typename Z>
 __global__ __launch_bounds__(kBlock) void increments_kernel(
     const T* __restrict__ path, T* __restrict__ inc, int64_t batch, int64_t len_raw, int d_raw,
-    int time_aug, int lead_lag, T time_step, T* __restrict__ zero_out, DivBy<I> dv)
+    int time_aug, int lead_lag, T time_step, Z* __restrict__ zero_out, DivBy<I> dv)
 {
     // zero_out (optional): the increment gradient [batch][L][d], cleared in the same launch; the backward
     // accumulates into it with atomics.
@@ -1042,7 +1043,7 @@ __global__ __launch_bounds__(kBlock) void increments_kernel(
     for (int64_t b = blockIdx.y; b < batch; b += gridDim.y) {
         const T* x = path + b * len_raw * d_raw;
         T* o = inc + b * int64_t(per);
-        T* zo = zero_out ? zero_out + b * int64_t(L) * int64_t(d) : nullptr;
+        Z* zo = zero_out ? zero_out + b * int64_t(L) * int64_t(d) : nullptr;
         for (I e = I(blockIdx.x) * kBlock + threadIdx.x; e < per; e += I(gridDim.x) * kBlock) {
             const I row = dv.quot(e);
             const I c = e - row * d;
@@ -1064,7 +1065,7 @@ __global__ __launch_bounds__(kBlock) void increments_kernel(
                 }
             }
             o[e] = v;
-            if (zo && e < L * d) zo[e] = T(0);
+            if (zo && e < L * d) zo[e] = Z(0);
         }
     }
 }
@@ -1079,6 +1080,7 @@ __global__ __launch_bounds__(kBlock) void increments_kernel(
 // `clear` (optional): clear_count elements of another buffer are set to zero by the same launch: the increment-gradient
 // accumulator the NEXT backward call will add into (the two accumulators of a device take turns, so a call whose
 // sweep forms its own increments needs no launch that clears one).
+// Z: element type of the increment gradient, T or double; a point's two terms meet in it and are rounded to T once.
 template <typename T>
 __device__ __forceinline__ void clear_range(T* __restrict__ clear, int64_t count)
 {
@@ -1088,10 +1090,10 @@ __device__ __forceinline__ void clear_range(T* __restrict__ clear, int64_t count
 }
 
 // Grid: x over the len_raw * d_raw elements of one path's gradient, y over the paths; the only division is by d_raw.
-template <typename T, typename I>
+template <typename T, typename Z, typename I>
 __global__ __launch_bounds__(kBlock) void path_grad_kernel(
-    const T* __restrict__ dzinc, T* __restrict__ out, int64_t batch, int64_t len_raw, int time_aug, int lead_lag,
-    DivBy<I> dv, T* __restrict__ clear, int64_t clear_count)
+    const Z* __restrict__ dzinc, T* __restrict__ out, int64_t batch, int64_t len_raw, int time_aug, int lead_lag,
+    DivBy<I> dv, Z* __restrict__ clear, int64_t clear_count)
 {
     clear_range(clear, clear_count);
     const I d_raw = I(dv.d);
@@ -1099,12 +1101,12 @@ __global__ __launch_bounds__(kBlock) void path_grad_kernel(
     const int64_t L = (lead_lag ? 2 * len_raw - 1 : len_raw) - 1;
     const I per = I(len_raw) * d_raw;
     for (int64_t b = blockIdx.y; b < batch; b += gridDim.y) {
-        const T* g = dzinc + b * L * int64_t(d);
+        const Z* g = dzinc + b * L * int64_t(d);
         T* o = out + b * int64_t(per);
         for (I e = I(blockIdx.x) * kBlock + threadIdx.x; e < per; e += I(gridDim.x) * kBlock) {
             const int64_t i = int64_t(dv.quot(e));
             const int64_t c = int64_t(e) - i * int64_t(d_raw);
-            T v = T(0);
+            Z v = Z(0);
             if (!lead_lag) {
                 if (i > 0) v += g[(i - 1) * d + c];
                 if (i < len_raw - 1) v -= g[i * d + c];
@@ -1112,7 +1114,7 @@ __global__ __launch_bounds__(kBlock) void path_grad_kernel(
                 if (i > 0) v += g[(2 * (i - 1)) * d + d_raw + c] + g[(2 * (i - 1) + 1) * d + c];
                 if (i < len_raw - 1) v -= g[(2 * i) * d + d_raw + c] + g[(2 * i + 1) * d + c];
             }
-            o[e] = v;
+            o[e] = T(v);
         }
     }
 }
@@ -1124,34 +1126,38 @@ template <typename T, int V>
 struct alignas(V * sizeof(T)) VecOf {
     T v[V];
 };
-template <typename T, typename I, int V>
+template <typename T, typename Z, typename I, int V>
 __global__ __launch_bounds__(kBlock) void path_grad_vec_kernel(
-    const T* __restrict__ dzinc, T* __restrict__ out, int64_t batch, int64_t len_raw, DivBy<I> dv,
-    T* __restrict__ clear, int64_t clear_count)
+    const Z* __restrict__ dzinc, T* __restrict__ out, int64_t batch, int64_t len_raw, DivBy<I> dv,
+    Z* __restrict__ clear, int64_t clear_count)
 {
     clear_range(clear, clear_count);
     using Vec = VecOf<T, V>;
+    using Acc = VecOf<Z, V>;
     const I dvec = I(dv.d);
     const I per = I(len_raw) * dvec;
     for (int64_t b = blockIdx.y; b < batch; b += gridDim.y) {
-        const Vec* g = reinterpret_cast<const Vec*>(dzinc) + b * (len_raw - 1) * int64_t(dvec);
+        const Acc* g = reinterpret_cast<const Acc*>(dzinc) + b * (len_raw - 1) * int64_t(dvec);
         Vec* o = reinterpret_cast<Vec*>(out) + b * int64_t(per);
         for (I e = I(blockIdx.x) * kBlock + threadIdx.x; e < per; e += I(gridDim.x) * kBlock) {
             const int64_t i = int64_t(dv.quot(e));
-            Vec r;
+            Acc r;
 #pragma unroll
-            for (int k = 0; k < V; ++k) r.v[k] = T(0);
+            for (int k = 0; k < V; ++k) r.v[k] = Z(0);
             if (i > 0) {
-                const Vec a = g[int64_t(e) - dvec];
+                const Acc a = g[int64_t(e) - dvec];
 #pragma unroll
                 for (int k = 0; k < V; ++k) r.v[k] += a.v[k];
             }
             if (i < len_raw - 1) {
-                const Vec a = g[e];
+                const Acc a = g[e];
 #pragma unroll
                 for (int k = 0; k < V; ++k) r.v[k] -= a.v[k];
             }
-            o[e] = r;
+            Vec v;
+#pragma unroll
+            for (int k = 0; k < V; ++k) v.v[k] = T(r.v[k]);
+            o[e] = v;
         }
     }
 }

@@ -21,7 +21,6 @@ hipError_t launch_rows_fwd_f64(const FwdParams& p, int degree);
 // single precision on the matrix units (sig_rows_mfma.hip)
 bool rows_bwd_mfma_supported(uint64_t d);
 hipError_t launch_rows_bwd_mfma(const BwdParams& p, int degree);      // p.dzinc: double, zeroed
-hipError_t launch_narrow(const double* in, float* out, int64_t n, hipStream_t stream);
 hipError_t launch_rows_fwd_mfma(const FwdParams& p, int degree);
 
 }  // namespace sigamd

@@ -11,8 +11,6 @@
 // multiply-adds: the forward sweep agrees with the vector kernels bit for bit.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
-
 #include "sig_rows.h"
 #include "sig_rows_lanes.h"
 #include "sig_launch.h"
@@ -435,18 +433,6 @@ __global__ __launch_bounds__((kMxWaves * kWave), 2) void rows_bwd_mfma_kernel(
         }
         __syncthreads();
     }
-}
-
-__global__ __launch_bounds__(kBlock) void narrow_kernel(const double* __restrict__ in, float* __restrict__ out, int64_t n)
-{
-    for (int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x; i < n; i += int64_t(gridDim.x) * kBlock) out[i] = float(in[i]);
-}
-
-hipError_t launch_narrow(const double* in, float* out, int64_t n, hipStream_t stream)
-{
-    const int64_t blocks = std::min<int64_t>((n + kBlock - 1) / kBlock, 8192);
-    hipLaunchKernelGGL(narrow_kernel, dim3(unsigned(blocks)), dim3(kBlock), 0, stream, in, out, n);
-    return hipGetLastError();
 }
 
 template <int N>

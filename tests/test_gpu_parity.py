@@ -833,6 +833,28 @@ def test_by_row_reverse_sweep_without_matrix_units(P, oracle, by_rows, shape, au
     assert bwd_rel_err(got, want) <= 1e-5
 
 
+@pytest.mark.parametrize("aug", [{}, dict(time_aug=True), dict(lead_lag=True)])
+def test_by_row_reverse_sweep_workspace(P, oracle, by_rows, aug):
+    """On the matrix units the increment gradient is held once, in double precision: the workspaces of a call are that and
+    the single-precision increments, each an eighth larger than asked for."""
+    from pysiglib_amd import _loader as L
+    import ctypes
+    L.CUSIG.cusig_amd_workspace_bytes.restype = ctypes.c_uint64
+    b, length, d, deg = 4, 300, 34, 3
+    rng = np.random.default_rng(34)
+    x = (np.cumsum(rng.standard_normal((b, length, d)), axis=1) / np.sqrt(d * length)).astype(np.float32)
+    ref = oracle.signature(x.astype(np.float64), deg, n_jobs=-1, **aug)
+    g = rng.standard_normal(ref.shape).astype(np.float32)
+    want = oracle.sig_backprop(x.astype(np.float64), ref, g.astype(np.float64), deg, n_jobs=-1, **aug)
+    L.CUSIG.cusig_shutdown()                    # the pool only grows
+    got = P.sig_backprop(dev(x), dev(ref.astype(np.float32)), dev(g), deg, **aug).cpu().numpy()
+    assert by_rows.last_on_matrix_units() == 1
+    steps, d_aug = ((2 * length - 2) if "lead_lag" in aug else length - 1), (2 * d if "lead_lag" in aug else d + len(aug))
+    asked = 4 * (b * (steps + 2) + 36) * d_aug + 8 * b * steps * d_aug
+    assert asked <= L.CUSIG.cusig_amd_workspace_bytes() <= asked + asked // 8 + 1024
+    assert bwd_rel_err(got, want) <= 1e-5
+
+
 @pytest.mark.parametrize("shape", [(2, 10, 48, 3), (3, 11, 64, 3), (2, 12, 33, 4), (1, 4, 33, 6)])
 def test_by_row_sweeps_beside_the_run_time_kernels(P, by_rows, shape):
     """The matrix form of the forward sweep rounds like the run-time-dimension kernels, bit for bit (at degree 6 too, whose
