@@ -833,6 +833,20 @@ def test_by_row_reverse_sweep_without_matrix_units(P, oracle, by_rows, shape, au
     assert bwd_rel_err(got, want) <= 1e-5
 
 
+@pytest.mark.parametrize("shape,aug", [((4, 33, 60, 3), {}), ((2, 12, 64, 3), {}), ((20, 20, 27, 3), dict(time_aug=True))])
+def test_lead_lag_paths_of_many_channels(P, oracle, by_rows, shape, aug):
+    """Lead-lag paths of 55 to 128 augmented channels at degree 3, in single precision: no compiled instance skips their
+    still letters, the matrix form of the by-row sweep serves them by the rules of the dispatch."""
+    b, length, d, deg = shape
+    rng = np.random.default_rng(b * 1000 + d)
+    x = (np.cumsum(rng.standard_normal((b, length, d)), axis=1) / np.sqrt(d * length)).astype(np.float32)
+    ref = oracle.signature(x.astype(np.float64), deg, n_jobs=-1, lead_lag=True, **aug)
+    by_rows(1, 1)
+    got = P.sig(dev(x), deg, lead_lag=True, **aug).cpu().numpy()
+    assert by_rows.last_on_matrix_units() == 1, by_rows.last_name()
+    assert level_rel_err(got, ref, 2 * d + len(aug), deg) <= 1e-5
+
+
 @pytest.mark.parametrize("aug", [{}, dict(time_aug=True), dict(lead_lag=True)])
 def test_by_row_reverse_sweep_workspace(P, oracle, by_rows, aug):
     """On the matrix units the increment gradient is held once, in double precision: the workspaces of a call are that and
