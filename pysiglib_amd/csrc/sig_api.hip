@@ -11,6 +11,7 @@
 #include <algorithm>
 #include <atomic>
 #include <charconv>
+#include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <map>
@@ -396,38 +397,54 @@ static int simd_count()
 // and 2.2 signature sets of traffic per piece at 4 TB/s (measured: d = 12, degree 4, 48 paths of 300 steps: whole
 // 92 us, 2 pieces 77, 3: 76, 4: 94, 6: 101 us).  Pieces keep at least 48 steps and 256 MB of segment signatures at most, and a
 // split must promise 7 % (batch 128, length 1024, d = 5, degree 7, f32: 0.587 -> 0.523 ms with three pieces).
+struct SplitPlan {
+    int pieces;
+    double seconds;     // what the model expects the call to take
+    double folds;       // the part of it that putting the pieces together takes
+};
+
+// Waves of an instance that fit a SIMD, a property of the compiled kernel: asked for once (the query takes 5 us, an eighth of a
+// short call: 86 paths of 2 steps, 48 channels, degree 3).  Called under the workspace mutex.
+static int resident_waves(const KernelEntry* e)
+{
+    static std::map<const KernelEntry*, int> known;
+    auto it = known.find(e);
+    if (it == known.end()) it = known.emplace(e, e->waves_per_simd()).first;
+    return it->second;
+}
+
 template <typename LaneStep>
-static int choose_segments(int64_t waves, int64_t L, int waves_per_simd, uint64_t sig_bytes_all_paths, LaneStep&& lane_step,
+static SplitPlan choose_segments(int64_t waves, int64_t L, int waves_per_simd, uint64_t sig_bytes_all_paths, LaneStep&& lane_step,
                            bool f64)
 {
     const int64_t simds = simd_count();
-    if (waves <= 0 || sig_bytes_all_paths == 0) return 1;
+    if (waves <= 0 || sig_bytes_all_paths == 0) return {1, 0.0, 0.0};
     const int occ = std::max(1, waves_per_simd);
-    if (waves > 4 * simds * occ) return 1;
     const double pair_rate = f64 ? 1.2 : 1.35;
+    auto folds = [&](int g) {
+        int launches = 0;
+        for (int m = g; m > 1; m = (m + 1) / 2) ++launches;
+        return g > 1 ? 8e-6 + 10e-6 * launches + 2.2 * g * double(sig_bytes_all_paths) / 4e12 : 0.0;
+    };
     auto estimate = [&](int g) {
         const int64_t fullest = (waves * g + simds - 1) / simds;          // waves of the fullest SIMD
         const int64_t rounds = fullest / occ, rest = fullest % occ;
         double steps = double(rounds) * occ / (occ > 1 ? pair_rate : 1.0);
         if (rest) steps += double(rest) / (rest > 1 ? pair_rate : 1.0);
-        double t = double((L + g - 1) / g) * lane_step(g) * steps;
-        if (g > 1) {
-            int launches = 0;
-            for (int m = g; m > 1; m = (m + 1) / 2) ++launches;
-            t += 8e-6 + 10e-6 * launches + 2.2 * g * double(sig_bytes_all_paths) / 4e12;
-        }
-        return t;
+        return double((L + g - 1) / g) * lane_step(g) * steps + folds(g);
     };
     int best = 1;
     double best_t = estimate(1);
     const double whole = best_t;
+    if (waves > 4 * simds * occ) return {1, whole, 0.0};
     // (one very long path of few channels: hundreds of pieces, each further doubling one more 10 us fold)
     for (int g : {2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 48, 64, 96, 128, 192, 256, 384, 512, 768, 1024}) {
         if (L / g < 48 || uint64_t(g) * sig_bytes_all_paths > (uint64_t(256) << 20)) break;
         const double t = estimate(g);
         if (t < best_t) { best = g; best_t = t; }
     }
-    return best_t < 0.93 * whole ? best : 1;
+    if (best_t < 0.93 * whole) return {best, best_t, folds(best)};
+    return {1, whole, 0.0};
 }
 
 // The backward sweep can be cut in time as well: the state at the end of segment g is the Chen product of the
@@ -448,13 +465,12 @@ static thread_local int tl_matrix_form = 0;     // whether the last sweep on thi
 // byte of segment signatures (48 paths of 300 steps, d = 12, degree 4, f64: whole 0.225 ms, 2 pieces 0.270,
 // 8: 0.578, 64: 4.65 ms; 8 paths of 4000 steps, d = 6, degree 4, f32: whole 3.42 ms, 32 pieces 0.249 ms).
 template <typename LaneStep>
-static int choose_bwd_segments(int64_t waves, int64_t L, int waves_per_simd, uint64_t sig_bytes_all_paths, LaneStep&& lane_step,
+static SplitPlan choose_bwd_segments(int64_t waves, int64_t L, int waves_per_simd, uint64_t sig_bytes_all_paths, LaneStep&& lane_step,
                                bool f64)
 {
     const int64_t simds = simd_count();
-    if (waves <= 0 || sig_bytes_all_paths == 0) return 1;
+    if (waves <= 0 || sig_bytes_all_paths == 0) return {1, 0.0, 0.0};
     const int occ = std::max(1, waves_per_simd);
-    if (waves > 2 * simds * occ) return 1;
     const double pair_rate = f64 ? 1.2 : 1.35;
     auto estimate = [&](int g) {
         const int64_t fullest = (waves * g + simds - 1) / simds;
@@ -473,12 +489,14 @@ static int choose_bwd_segments(int64_t waves, int64_t L, int waves_per_simd, uin
     int best = 1;
     double best_t = estimate(1);
     const double whole = best_t;
+    if (waves > 2 * simds * occ) return {1, whole, 0.0};
     for (int g : {2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128, 192, 256, 384, 512}) {
         if (L / g < 32 || uint64_t(g) * sig_bytes_all_paths > (uint64_t(64) << 20)) break;
         const double t = estimate(g);
         if (t < best_t) { best = g; best_t = t; }
     }
-    return best_t < 0.93 * whole ? best : 1;
+    if (best_t < 0.93 * whole) return {best, best_t, 0.0};
+    return {1, whole, 0.0};
 }
 
 // With at most two waves per SIMD the LDS-staged twin (all-VGPR FMAs, HBM latency hidden by a chunk of
@@ -511,6 +529,36 @@ static const KernelEntry* pick_variant(bool backward, const KernelEntry* base, i
     if (!want) return base;
     const KernelEntry* twin = staged_twin(backward, base);
     return twin ? twin : base;
+}
+
+// The by-row forward sweep in single precision against a compiled instance of the same shape, at degree 3: both are
+// estimated, the path length included, since only the instance's paths can be cut in time.  Seconds beside what the calls
+// have in common.
+// By rows: a wave alone on its SIMD takes 148 ns a step (long paths of 48 .. 128 channels, degree 3: 139-152), a full SIMD
+// 37 ns a wave and step plus 11.2 ns per product of 32 x 32 (8 waves per SIMD: 82 ns measured at 64 and 97 channels, 62 at
+// 72 and 96, whose tiles are partly empty).
+static double rows_fwd_seconds(uint64_t d, uint64_t batch, uint64_t L)
+{
+    const double tiles = double((d + kWave - 1) / kWave), halves = double((d + 31) / 32);
+    const double waves = double(batch) * double(d) * tiles * tiles;
+    const double per_wave = 37e-9 + 11.2e-9 * halves * halves / (tiles * tiles);
+    return double(L) * std::max(148e-9, per_wave * std::ceil(waves / double(simd_count())));
+}
+// The instance: `run` is the kernel that would be launched.  Scalar-fed sweeps of many channels wait for their loads: 170 ns a
+// step and 1.8 ns per instruction and wave of a SIMD (80 channels, 2.7 / 10.2 waves per SIMD: 288 / 589 ns), 1.3 times as
+// long where an odd channel count leaves the rows unaligned.  LDS-fed ones follow the model of choose_segments at two
+// subtree levels, at one they take 1.7 times as long (49 channels, 21 paths of 8000 steps: 0.94 / 1.74 ms).
+// Fitted to 17 channel counts of 48 .. 128 at 0.1 .. 8 waves per SIMD and 8 .. 8000 steps; time-split estimates scatter by
+// an eighth and are taken down by it, so that the instance keeps what it may win.  Paths of 8000 steps, degree 3, instance
+// in pieces / by rows: 4 x 72 channels 0.58 / 1.13 ms, 22 x 48: 1.13 / 1.40, 13 x 80: 2.1 / 2.4; 22 x 96: 6.1 / 4.1,
+// 19 x 112: 14.9 / 5.5.
+static double instance_fwd_seconds(const KernelEntry* run, const SplitPlan& plan, int64_t waves, uint64_t d, uint64_t L)
+{
+    if (run->staged) return (run->tail > 1 ? 1.0 : 1.7) * plan.seconds;
+    const double per_simd = double(waves) * plan.pieces / double(simd_count());
+    const double step = (170e-9 + 1.8e-9 * lane_step_cost(int(d), run->N, run->tail, run->k) * per_simd) * (d % 2 ? 1.3 : 1.0);
+    const double t = std::ceil(double(L) / plan.pieces) * step + plan.folds;
+    return plan.pieces > 1 ? 0.88 * t : t;
 }
 
 // ---------------------------------------------------------------------------
@@ -817,33 +865,40 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
         // lead-lag sweeps that skip the letters a step cannot move take the step's parity from its position in the
         // segment: segments start on even steps
         const bool sparse_ll = lead_lag && g_lead_lag_sparse != 0;
-        // many channels without a compiled instance: the by-row sweep, whole paths only (its launches fill the chip).
-        // Double precision, against the general run-time kernels (16 / 32 letters per lane) at 33 .. 96 channels, degrees 4
-        // to 6: 1.0-1.46x faster.  Single precision runs on the matrix units, bit for bit the same: always faster than the
-        // run-time kernels (16 paths of 200 steps, 64 channels, degree 4: 2.60 -> 1.27 ms; 5 x 64, 70: 0.89 -> 0.48; 2 x 50,
-        // 33, degree 5: 0.69 -> 0.43), and than a compiled instance where its tiles of 32 x 32 are filled well enough
-        // (256 x 256, 64 channels, degree 3: 0.94 -> 0.39; 300 x 200, 96: 2.05 -> 1.39; 8 x 100, 48, degree 4: 0.28 -> 0.22;
-        // but 64 x 200, 40, degree 4, 39 % filled: 1.20 -> 1.83) by launches that need no time split (4 x 500, 48, degree 3,
-        // split: 0.080, whole: 0.103).  Lead-lag paths of that many channels have no instance that skips the letters a step
-        // cannot move (those end at 40), so the same holds for them (degree 3, 200 paths of 129 points, 60 channels, 120
-        // augmented: 8.72 -> 2.11 ms, 4.42 as library products; 100 x 129 x 64: 2.90 -> 1.14, 2.41).
-        const uint64_t tile = (s.d_aug + 31) / 32 * 32, groups = (s.d_aug + kWave - 1) / kWave;
-        const bool rows_beat_instance = sizeof(T) == 4 && 16 * s.d_aug * s.d_aug >= 9 * tile * tile &&
-                                        (degree >= 4 || batch * s.d_aug * groups * groups >= uint64_t(simd_count()));
-        const bool rows_win = e->D <= 0 || rows_beat_instance;
+        // many channels: the by-row sweep, whole paths only.  Without a compiled instance always: in double precision
+        // 1.0-1.46x faster than the general run-time kernels (16 / 32 letters per lane) at 33 .. 96 channels, degrees 4 to 6;
+        // in single precision, on the matrix units and bit for bit the same (16 paths of 200 steps, 64 channels, degree 4:
+        // 2.60 -> 1.27 ms; 5 x 64, 70: 0.89 -> 0.48; 2 x 50, 33, degree 5: 0.69 -> 0.43).  In place of an instance in single
+        // precision, where its tiles of 32 x 32 are filled well enough (256 x 256, 64 channels, degree 3: 0.94 -> 0.39 ms;
+        // 300 x 200, 96: 2.05 -> 1.39; 8 x 100, 48, degree 4: 0.28 -> 0.22; but 64 x 200, 40, degree 4, 39 % filled:
+        // 1.20 -> 1.83) and, at degree 3, the estimates say so (at degree 4 it won at every size tried: one path of 8000 steps,
+        // 48 channels 2.40 -> 2.11, two 4.37 -> 3.48).  Lead-lag paths of that many channels have no instance that skips the
+        // letters a step cannot move (those end at 40), so the same holds for them (degree 3, 200 paths of 129 points, 60
+        // channels, 120 augmented: 8.72 -> 2.11 ms, 4.42 as library products; 100 x 129 x 64: 2.90 -> 1.14, 2.41).
+        const int64_t instance_waves = total_waves(geom, int64_t(batch));
+        auto split = [&]() -> SplitPlan {
+            if (g_force_segments > 0) return {int(std::min<uint64_t>(uint64_t(g_force_segments), s.L)), 0.0, 0.0};
+            return choose_segments(instance_waves, int64_t(s.L), resident_waves(e), batch * (s.full_len - 1) * sizeof(T),
+                                   [&](int g) {
+                                       const double c = lane_step_cost(int(s.d_aug), e->N, e->tail, e->k) * 2.4e-9;
+                                       const bool ring = pick_variant(false, e, instance_waves * g, sparse_ll)->staged;
+                                       return ring ? c : std::max(c, 240e-9);
+                                   },
+                                   sizeof(T) == 8);
+        };
+        const uint64_t tile = (s.d_aug + 31) / 32 * 32;
         const int rows_mode = g_rows_forward;
-        const bool by_rows = (rows_mode >= 2 || (rows_mode == 1 && rows_win)) && g_force_tail == 0 &&
-                             rows_bwd_supported(sizeof(T), s.d_aug, degree) && rows_bwd_fits(sizeof(T), s.d_aug, degree, batch);
-        int nseg = by_rows ? 1 : g_force_segments > 0
-                             ? int(std::min<uint64_t>(uint64_t(g_force_segments), s.L))
-                             : choose_segments(total_waves(geom, int64_t(batch)), int64_t(s.L), e->waves_per_simd(),
-                                               batch * (s.full_len - 1) * sizeof(T),
-                                               [&](int g) {
-                                                   const double c = lane_step_cost(int(s.d_aug), e->N, e->tail, e->k) * 2.4e-9;
-                                                   const bool ring = pick_variant(false, e, total_waves(geom, int64_t(batch)) * g, sparse_ll)->staged;
-                                                   return ring ? c : std::max(c, 240e-9);
-                                               },
-                                               sizeof(T) == 8);
+        bool by_rows = rows_mode != 0 && g_force_tail == 0 && rows_bwd_supported(sizeof(T), s.d_aug, degree) &&
+                       rows_bwd_fits(sizeof(T), s.d_aug, degree, batch);
+        if (rows_mode == 1 && e->D > 0) by_rows = by_rows && sizeof(T) == 4 && g_force_segments == 0 && 16 * s.d_aug * s.d_aug >= 9 * tile * tile;
+        SplitPlan plan{1, 0.0, 0.0};
+        const bool compare = by_rows && rows_mode == 1 && e->D > 0 && degree == 3;
+        if (!by_rows || compare) plan = split();
+        if (compare) {
+            const KernelEntry* run = pick_variant(false, e, instance_waves * plan.pieces, sparse_ll);
+            by_rows = rows_fwd_seconds(s.d_aug, batch, s.L) < instance_fwd_seconds(run, plan, instance_waves, s.d_aug, s.L);
+        }
+        int nseg = by_rows ? 1 : plan.pieces;
         const uint64_t n_coef = s.full_len - 1;
         FwdParams p;
         p.batch = int64_t(batch) * nseg; p.L = int64_t(s.L); p.d = int(s.d_aug); p.stream = stream;
@@ -1206,7 +1261,7 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
         int nseg = (arena || by_rows || !ef || degree > uint64_t(kCombMaxLevels)) ? 1
                    : g_force_bwd_segments > 0 ? int(std::min<uint64_t>(uint64_t(g_force_bwd_segments), s.L))
                                               : choose_bwd_segments(
-                                                    total_waves(geom, int64_t(batch)), int64_t(s.L), e->waves_per_simd(),
+                                                    total_waves(geom, int64_t(batch)), int64_t(s.L), resident_waves(e),
                                                     batch * n_coef * sizeof(T),
                                                     [&](int g) {
                                                         // a backward step issues about 3.2 times the forward's instructions
@@ -1214,7 +1269,7 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
                                                         const bool ring = pick_variant(true, e, total_waves(geom, int64_t(batch)) * g, sparse_ll)->staged;
                                                         return ring ? c : std::max(c, 700e-9);
                                                     },
-                                                    sizeof(T) == 8);
+                                                    sizeof(T) == 8).pieces;
         int64_t lseg = int64_t(s.L);
         if (nseg > 1) {
             lseg = (int64_t(s.L) + nseg - 1) / nseg;

@@ -847,6 +847,34 @@ def test_lead_lag_paths_of_many_channels(P, oracle, by_rows, shape, aug):
     assert level_rel_err(got, ref, 2 * d + len(aug), deg) <= 1e-5
 
 
+@pytest.mark.parametrize("shape,whole", [((4, 8001, 72, 3), False), ((22, 8001, 48, 3), False), ((2, 4001, 96, 3), False),
+                                         ((4, 201, 72, 3), True), ((11, 201, 96, 3), True), ((1, 400, 48, 4), True)])
+def test_long_paths_of_many_channels_are_cut_in_time(P, by_rows, shape, whole):
+    """Single precision, shapes that a compiled instance and the by-row sweep both serve: few long paths are left to the
+    instance, whose paths can be cut in time; pieces asked for by the hook are made.  Either way the other form agrees."""
+    import ctypes
+    from pysiglib_amd import _loader as L
+    b, length, d, deg = shape
+    torch.manual_seed(d)
+    x = torch.randn((b, length, d), device=DEV).cumsum(1) / np.sqrt(d * length)
+    by_rows(1, 1)
+    got = P.sig(x, deg)
+    assert by_rows.last_on_matrix_units() == int(whole), by_rows.last_name()
+    assert (L.CUSIG.cusig_amd_last_segments() == 1) == whole
+    by_rows(0 if whole else 2, 1)
+    other = P.sig(x, deg)
+    assert by_rows.last_on_matrix_units() == 1 - int(whole)
+    # rounding: either form adds `length` steps of 6e-8, in another order
+    assert level_rel_err(got.cpu().numpy(), other.cpu().numpy(), d, deg) <= TOL[np.float32]
+    by_rows(1, 1)
+    try:
+        L.CUSIG.cusig_amd_force_segments(3)
+        P.sig(x, deg)
+        assert L.CUSIG.cusig_amd_last_segments() == 3
+    finally:
+        L.CUSIG.cusig_amd_force_segments(0)
+
+
 @pytest.mark.parametrize("aug", [{}, dict(time_aug=True), dict(lead_lag=True)])
 def test_by_row_reverse_sweep_workspace(P, oracle, by_rows, aug):
     """On the matrix units the increment gradient is held once, in double precision: the workspaces of a call are that and
