@@ -561,6 +561,28 @@ static double instance_fwd_seconds(const KernelEntry* run, const SplitPlan& plan
     return plan.pieces > 1 ? 0.88 * t : t;
 }
 
+// The same choice for the backward of 33 .. 47 channels, degree 3.  By rows, a step takes 355 ns while no CU holds more than
+// one block of four waves and 488 ns with two, which is all it can hold (33 .. 47 channels, 2000 and 8000 steps: 353-368 and
+// 477-499 ns; 2.07 rounds of blocks 1.32 us, 2.2 rounds 1.46).  Up to sixteen steps cost alike; from 39 channels on the
+// instances start so much slower that eight are counted (9 points: 118 x 35 channels 56 / 68 us, 96 x 43: 84 / 69).
+static double rows_bwd_seconds(uint64_t d, uint64_t batch, uint64_t L)
+{
+    const uint64_t cus = uint64_t(simd_count()) / 4, blocks = batch * ((d + 3) / 4);
+    const uint64_t rounds = blocks / (2 * cus), rest = blocks % (2 * cus);
+    const double last = rest == 0 ? 0.0 : (rounds == 0 ? rest <= cus : rest <= 48) ? 355e-9 : 488e-9;
+    const uint64_t least = d < 39 ? 16 : 8;
+    return double((L + least - 1) / least * least) * (488e-9 * double(rounds) + last);
+}
+// The instances take longer than the model of choose_bwd_segments has it: whole paths 1.6 times (1.5-1.9 at 33 .. 47
+// channels), fewer than eight pieces 1.05 times (1.03-1.2), from 39 channels on 1.35 times (1.25-1.5); of more pieces, few
+// paths' way to fill the chip, it is 0.85 at the least.  Paths of 8000 steps,
+// instance in pieces / by rows: 16 x 33 channels 1.34 / 2.86 ms, 63 x 33: 4.38 / 7.99, 26 x 40: 2.93 / 3.83; 44 x 47,
+// whole: 12.1 / 6.9.
+static double instance_bwd_seconds(const SplitPlan& plan, uint64_t d)
+{
+    return plan.seconds * (plan.pieces == 1 ? 1.6 : plan.pieces >= 8 ? 0.85 : d < 39 ? 1.05 : 1.35);
+}
+
 // ---------------------------------------------------------------------------
 // degree 2 in closed form (matrix cores): taken for paths of many channels, where no specialised sweep exists
 // ---------------------------------------------------------------------------
@@ -1250,26 +1272,32 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
         // many channels beyond the compiled table: the by-row sweep, whole paths only (its launches fill the chip)
         // (also where an instance would lose: measured at 48 .. 128 channels, degrees 3 and 4, the by-row sweep runs
         // 1.1-4x faster than compiled single-precision instances and 1-12x faster than double-precision ones; the
-        // instance table leaves these backward shapes out)
-        // (single precision up to 256 channels runs on the matrix units, and wins at degree 3 from 33 channels on: 64 paths
-        // of 200 steps, 40 channels 0.328 -> 0.234 ms, 16 x 200, 36: 0.340 -> 0.121; at degree 4 and 40 channels its tiles
-        // are 39 % filled: 4.6 -> 6.0; fewer waves are left to the time splits)
-        const bool rows_win = e->D <= 0 || s.d_aug >= 48 || (sizeof(T) == 4 && degree == 3 && !lead_lag && 2 * batch * s.d_aug >= uint64_t(simd_count()));
+        // instance table leaves these backward shapes out).  Below 48 channels an instance exists up to degree 4; at degree 3
+        // the matrix form of single precision competes with it, the estimates decide (64 paths of 200 steps, 40 channels
+        // 0.328 -> 0.234 ms, 16 x 200, 36: 0.340 -> 0.121); at degree 4 and 40 channels its tiles are 39 % filled: 4.6 -> 6.0
+        // ms.  Lead-lag paths are left to the instances that skip their still letters.
+        const int64_t instance_waves = total_waves(geom, int64_t(batch));
+        auto split = [&]() -> SplitPlan {
+            if (arena || !ef || degree > uint64_t(kCombMaxLevels)) return {1, 0.0, 0.0};
+            if (g_force_bwd_segments > 0) return {int(std::min<uint64_t>(uint64_t(g_force_bwd_segments), s.L)), 0.0, 0.0};
+            return choose_bwd_segments(instance_waves, int64_t(s.L), resident_waves(e), batch * n_coef * sizeof(T),
+                                       [&](int g) {
+                                           // a backward step issues about 3.2 times the forward's instructions
+                                           const double c = lane_step_cost(int(s.d_aug), e->N, e->tail, e->k) * 7.7e-9;
+                                           const bool ring = pick_variant(true, e, instance_waves * g, sparse_ll)->staged;
+                                           return ring ? c : std::max(c, 700e-9);
+                                       },
+                                       sizeof(T) == 8);
+        };
         const int rows_mode = g_rows_backward;
-        const bool by_rows = !arena && (rows_mode >= 2 || (rows_mode == 1 && rows_win)) && g_force_tail == 0 &&
-                             rows_bwd_supported(sizeof(T), s.d_aug, degree) && rows_bwd_fits(sizeof(T), s.d_aug, degree, batch);
-        int nseg = (arena || by_rows || !ef || degree > uint64_t(kCombMaxLevels)) ? 1
-                   : g_force_bwd_segments > 0 ? int(std::min<uint64_t>(uint64_t(g_force_bwd_segments), s.L))
-                                              : choose_bwd_segments(
-                                                    total_waves(geom, int64_t(batch)), int64_t(s.L), resident_waves(e),
-                                                    batch * n_coef * sizeof(T),
-                                                    [&](int g) {
-                                                        // a backward step issues about 3.2 times the forward's instructions
-                                                        const double c = lane_step_cost(int(s.d_aug), e->N, e->tail, e->k) * 7.7e-9;
-                                                        const bool ring = pick_variant(true, e, total_waves(geom, int64_t(batch)) * g, sparse_ll)->staged;
-                                                        return ring ? c : std::max(c, 700e-9);
-                                                    },
-                                                    sizeof(T) == 8).pieces;
+        bool by_rows = !arena && rows_mode != 0 && g_force_tail == 0 && rows_bwd_supported(sizeof(T), s.d_aug, degree) &&
+                       rows_bwd_fits(sizeof(T), s.d_aug, degree, batch);
+        const bool compare = by_rows && rows_mode == 1 && e->D > 0 && s.d_aug < 48;
+        if (compare) by_rows = sizeof(T) == 4 && degree == 3 && !lead_lag && g_force_bwd_segments == 0;
+        SplitPlan plan{1, 0.0, 0.0};
+        if (!by_rows || compare) plan = split();
+        if (compare && by_rows) by_rows = rows_bwd_seconds(s.d_aug, batch, s.L) < instance_bwd_seconds(plan, s.d_aug);
+        int nseg = by_rows ? 1 : plan.pieces;
         int64_t lseg = int64_t(s.L);
         if (nseg > 1) {
             lseg = (int64_t(s.L) + nseg - 1) / nseg;

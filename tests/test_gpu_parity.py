@@ -875,6 +875,36 @@ def test_long_paths_of_many_channels_are_cut_in_time(P, by_rows, shape, whole):
         L.CUSIG.cusig_amd_force_segments(0)
 
 
+@pytest.mark.parametrize("shape,rows", [((16, 8001, 33, 3), False), ((63, 2001, 33, 3), False), ((52, 3, 40, 3), False),
+                                        ((16, 201, 36, 3), True), ((44, 2001, 47, 3), True), ((40, 65, 46, 3), True)])
+def test_long_backward_of_33_to_47_channels(P, by_rows, shape, rows):
+    """Single precision, degree 3: long paths that an instance finishes sooner in pieces, and very short ones, are left to it;
+    pieces asked for by the hook are made.  Either way the other form agrees."""
+    import ctypes
+    from pysiglib_amd import _loader as L
+    L.CUSIG.cusig_amd_force_bwd_segments.argtypes = (ctypes.c_int,)
+    b, length, d, deg = shape
+    torch.manual_seed(d)
+    x = torch.randn((b, length, d), device=DEV).cumsum(1) / np.sqrt(d * length)
+    s = P.sig(x, deg)
+    g = torch.randn_like(s)
+    by_rows(1, 1)
+    got = P.sig_backprop(x, s, g, deg)
+    assert by_rows.last_on_matrix_units() == int(rows), by_rows.last_name()
+    by_rows(1, 0 if rows else 2)
+    other = P.sig_backprop(x, s, g, deg)
+    assert by_rows.last_on_matrix_units() == 1 - int(rows)
+    # rounding: a path's gradient sums over d^2 prefixes and either form recovers the states over `length` steps
+    assert bwd_rel_err(got.cpu().numpy(), other.cpu().numpy()) <= TOL[np.float32]
+    by_rows(1, 1)
+    try:
+        L.CUSIG.cusig_amd_force_bwd_segments(2)
+        P.sig_backprop(x, s, g, deg)
+        assert by_rows.last_on_matrix_units() == 0
+    finally:
+        L.CUSIG.cusig_amd_force_bwd_segments(0)
+
+
 @pytest.mark.parametrize("aug", [{}, dict(time_aug=True), dict(lead_lag=True)])
 def test_by_row_reverse_sweep_workspace(P, oracle, by_rows, aug):
     """On the matrix units the increment gradient is held once, in double precision: the workspaces of a call are that and
