@@ -583,6 +583,20 @@ static double instance_bwd_seconds(const SplitPlan& plan, uint64_t d)
     return plan.seconds * (plan.pieces == 1 ? 1.6 : plan.pieces >= 8 ? 0.85 : d < 39 ? 1.05 : 1.35);
 }
 
+// The by-row reverse sweep in single precision on the matrix units or off them.  The matrix form works on sixteen steps at a
+// time and its smaller blocks add three times as many pieces to the gradient rows, which shows on paths of a few steps whose
+// tiles of 64 x 64 are partly empty (8 paths of 3 / 9 / 12 steps, 65 channels, a quarter filled, degree 4: off / on
+// 0.84 / 1.15, 1.24 / 1.33, 1.40 / 1.38 ms; 32 x 1, 65, degree 3: 74 / 87 us; 8 x 1 / 4, 72, a third filled: 1.23 / 1.32,
+// 1.42 / 1.34 ms; 1 x 1 / 4, 48, 56 %: 60 / 66, 64 / 67 us; 1 x 2 / 4 / 8, 33, degree 5: 278 / 314, 310 / 315, 393 / 320).  Full tiles win from one step on (8 x 1, 64, degree 4: 441 / 389 us),
+// and so do launches of up to two waves per SIMD at degree 3 (4 x 1, 96: 55 / 53 us).
+static bool rows_bwd_mfma_wins(uint64_t d, uint64_t degree, uint64_t batch, uint64_t L)
+{
+    const uint64_t groups = (d + kWave - 1) / kWave, tile = groups * kWave;
+    if (L >= 12 || 16 * d * d >= 14 * tile * tile) return true;
+    if (L >= 4 && (groups == 1 || 16 * d * d >= 5 * tile * tile)) return true;
+    return degree == 3 && batch * d * groups * groups <= 2 * uint64_t(simd_count());
+}
+
 // ---------------------------------------------------------------------------
 // degree 2 in closed form (matrix cores): taken for paths of many channels, where no specialised sweep exists
 // ---------------------------------------------------------------------------
@@ -1311,7 +1325,8 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
                                e_run->D <= kPointFedMaxDim && g_point_fed != 0;
         // single precision on the matrix units: the increment gradient is summed in double precision, and rounded where the
         // path gradient is formed from it
-        const bool on_matrix_units = by_rows && sizeof(T) == 4 && rows_mode != 3 && rows_bwd_mfma_supported(s.d_aug);
+        const bool on_matrix_units = by_rows && sizeof(T) == 4 && rows_mode != 3 && rows_bwd_mfma_supported(s.d_aug) &&
+                                     (rows_mode == 2 || rows_bwd_mfma_wins(s.d_aug, degree, batch, s.L));
         T* inc = nullptr;
         T* dzinc = nullptr;
         double* wide_dz = nullptr;

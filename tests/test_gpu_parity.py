@@ -905,6 +905,23 @@ def test_long_backward_of_33_to_47_channels(P, by_rows, shape, rows):
         L.CUSIG.cusig_amd_force_bwd_segments(0)
 
 
+@pytest.mark.parametrize("shape,matrix", [((2, 4, 65, 4), False), ((2, 13, 65, 4), True), ((32, 2, 72, 3), False),
+                                          ((2, 5, 72, 4), True), ((1, 2, 64, 4), True), ((4, 2, 96, 3), True)])
+def test_backward_of_short_paths_by_row(P, oracle, by_rows, shape, matrix):
+    """Single precision: few steps of partly empty tiles are left to the form of the by-row reverse sweep without matrix
+    units."""
+    b, length, d, deg = shape
+    rng = np.random.default_rng(b * 100000 + length * 1000 + d * 10 + deg)
+    x = (np.cumsum(rng.standard_normal((b, length, d)), axis=1) / np.sqrt(d * length)).astype(np.float32)
+    ref = oracle.signature(x.astype(np.float64), deg, n_jobs=-1)
+    g = rng.standard_normal(ref.shape).astype(np.float32)
+    want = oracle.sig_backprop(x.astype(np.float64), ref, g.astype(np.float64), deg, n_jobs=-1)
+    by_rows(1, 1)
+    got = P.sig_backprop(dev(x), dev(ref.astype(np.float32)), dev(g), deg).cpu().numpy()
+    assert by_rows.last_name() == "rows_bwd_f32_n%d" % deg and by_rows.last_on_matrix_units() == int(matrix)
+    assert bwd_rel_err(got, want) <= 1e-5
+
+
 @pytest.mark.parametrize("aug", [{}, dict(time_aug=True), dict(lead_lag=True)])
 def test_by_row_reverse_sweep_workspace(P, oracle, by_rows, aug):
     """On the matrix units the increment gradient is held once, in double precision: the workspaces of a call are that and
