@@ -292,7 +292,9 @@ __global__ __launch_bounds__((kMxWaves * kWave), 2) void rows_bwd_mfma_kernel(
         }
     }
 
-    extern __shared__ float mx_lds[];
+    extern __shared__ f32x4 mx_lds_raw[];               // read four words at a time: aligned by its type
+    static_assert(kMxStride % 4 == 0 && kMxWaveWords % 4 == 0, "a step's words start on 16 bytes");
+    T* mx_lds = reinterpret_cast<T*>(mx_lds_raw);
     __shared__ int wave_a0[W], wave_l0[W];
     T* mine = mx_lds + wib * kMxWaveWords;              // [step][kMxStride]: red, then U, then the by-letter sums
     T* mine_c = mine + kMxSteps * kMxStride;            // pieces of the last prefix letter
