@@ -270,7 +270,7 @@ CUSIG_AMD_API void cusig_amd_force_bwd_segments(int segments) CUSIG_AMD_NOEXCEPT
 /* Whether the last signature / sig_backprop sweep of this thread was a by-row sweep on the matrix units (single precision,
  * 33 and more channels): 1 or 0.  Such sweeps carry the same cusig_amd_last_kernel_name as the form without them. */
 CUSIG_AMD_API int cusig_amd_last_sweep_on_matrix_units(void) CUSIG_AMD_NOEXCEPT;
-/* Test hook: the by-row reverse sweep of 33 and more augmented channels at degrees 3 and up (a wave holds its tile of
+/* Test hook: the by-row reverse sweep of 33 and more augmented channels at degrees 3 .. 6 (a wave holds its tile of
  * top-level adjoints both by prefix and by letter): 0 never, 1 (default) where it is expected to be the fastest form,
  * 2 wherever it applies, 3 the same with single precision kept off the matrix units.  (Degree 3 as matrix products has a
  * hook of its own, cusig_amd_force_degree3, and goes first.) */
@@ -298,9 +298,9 @@ CUSIG_AMD_API void cusig_amd_set_chen_low_levels(int enabled) CUSIG_AMD_NOEXCEPT
 CUSIG_AMD_API void cusig_amd_set_stream_ordered(int enabled) CUSIG_AMD_NOEXCEPT;
 /* Tuning hook: the closed-form degree-2 kernels (matrix cores): -1 automatic, 0 never, 1 whenever the degree is 2. */
 CUSIG_AMD_API void cusig_amd_force_degree2(int mode) CUSIG_AMD_NOEXCEPT;
-/* Tuning hook: degree 3 as rocBLAS matrix products around a scan kernel (backward: two products, forward: one):
- * -1 automatic (backward from 48 channels in float32 and 36 in float64, forward from 112, given enough paths to fill
- * the chip, a librocblas that can be opened and a device that can hold the extra rows buffer of up to 1 GiB; otherwise
+/* Tuning hook: degree 3 as rocBLAS matrix products around a scan kernel (backward: two products; forward, double precision
+ * only: one): -1 automatic (backward from 65 channels in float32 and 36 in float64, forward from 112, given enough paths to
+ * fill the chip, a librocblas that can be opened and a device that can hold the extra rows buffer of up to 1 GiB; otherwise
  * the sweeps serve the shape), 0 never, 1 whenever the degree is 3 and one path's rows fit the buffer. */
 CUSIG_AMD_API void cusig_amd_force_degree3(int mode) CUSIG_AMD_NOEXCEPT;
 /* Test hook: 1 routes every sweep of 2, 3 or 4 augmented channels that the run-time-degree kernels can serve

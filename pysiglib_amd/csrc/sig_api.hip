@@ -609,21 +609,23 @@ static Hook g_force_degree3{-1};    // tuning hook: -1 automatic, 0 never, 1 whe
 // rows buffer [paths of a chunk][L][d^2] of the degree-3 matrix form: paths are taken in chunks that fit this many bytes
 constexpr uint64_t kDeg3BufBytes = uint64_t(1) << 30;
 
-// degree 3 as library matrix products around a scan (sig_degree3.h): two products backward, one forward.  Measured at
-// batch 512 (256 at 128 channels), length 256, backward, against the by-row reverse sweep (which needs neither the
-// library nor the rows buffer): float32 48 channels 2.96 / 2.80 ms, 64: 4.23 / 4.27, 80: 9.3 / 19.4, 128: 9.2 / 15.6;
-// float64 64 channels 6.8 / 9.8, 80: 14.6 / 35.5, 128: 27.0 / 40.8 (below 48 channels the compiled float64 instances:
-// 1.3x from 36).  The scan needs a wave per SIMD to be worth it (a wave: 8 rows x 64 columns of one path's level 2).
+// degree 3 as library matrix products around a scan (sig_degree3.h): two products backward, in double precision also one
+// forward (1.3x at 128 channels, slower at 80; in single precision the by-row sweep on the matrix units takes half the
+// products' time: 200 paths of 256 steps, 112 channels 4.4 / 2.2 ms, 128: 5.4 / 2.3).  Backward, library / by rows (which
+// needs neither the library nor the rows buffer), whole calls at batch 512, length 257 (256 paths from 97 channels on):
+// float32 48 channels 3.04 / 1.68 ms, 64: 3.74 / 2.31, 65: 7.00 / 9.49, 80: 8.64 / 11.7, 96: 9.07 / 14.4, 97: 6.07 / 7.25,
+// 128: 9.14 / 9.87; float64 64: 6.84 / 9.77, 80: 13.4 / 34.9, 128: 25.7 / 40.8 (below 48 channels the compiled float64
+// instances: 1.3x from 36).  The scan needs a wave per SIMD to be worth it (a wave: 8 rows x 64 columns of one path's
+// level 2).  In float32 that line still gives the library what the by-row sweep does sooner: 96 paths of 128 channels
+// 4.23 / 3.75, and short paths (32 x 16 steps, 128 channels 1.15 / 0.24; 128 x 64, 80: 1.05 / 0.93).
 static bool want_degree3_gemm(uint64_t d_aug, uint64_t degree, uint64_t L, uint64_t batch, bool f64, bool backward)
 {
     if (degree != 3 || d_aug < 2 || d_aug > uint64_t(kDeg3MaxDim) || L > 0x7fffffff) return false;
     // one path's rows must fit the buffer (longer paths stay with the sweeps, which need B * L * d elements)
     if (L > kDeg3BufBytes / (d_aug * d_aug * (f64 ? 8 : 4))) return false;
+    if (!backward && !f64) return false;
     if (g_force_degree3 >= 0) return g_force_degree3 != 0;
     const uint64_t waves = ((d_aug + kWave - 1) / kWave) * ((d_aug + kDeg3RowsPerThread - 1) / kDeg3RowsPerThread) * batch;
-    // forward: 1.3x at 128 channels, slower at 80; in single precision the matrix form of the by-row sweep needs no rows
-    // buffer and takes half the time (200 paths of 256 steps, 112 channels 4.4 -> 2.2 ms, 128: 5.4 -> 2.3)
-    if (!backward && !f64) return false;
     const uint64_t from = backward ? (f64 ? 36u : 65u) : 112u;
     return d_aug >= from && waves >= 1024;
 }
@@ -797,30 +799,32 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
                            path, out, int64_t(batch), int64_t(length), int(dimension), int(time_aug),
                            int(lead_lag), time_step, sc, flag);
     } else if (d3.ok) {
-        const int d = int(s.d_aug);
-        const int64_t L = int64_t(s.L);
-        const uint64_t chunk = d3.chunk;
-        T* inc = d3.inc;
-        T* rows = d3.rows;
-        compute_increments(path, inc, batch, dimension, length, time_aug, lead_lag, end_time, s, stream);
-        RocBlas::Handle h = d3.handle;
-        tl_last_segments = 1;
-        MainKernelTimer timer(stream, sizeof(T) == 8 ? "degree3_fwd_gemm_f64" : "degree3_fwd_gemm_f32");
-        const int64_t dd = int64_t(d) * d;
-        const int groups = (d + kDeg3RowsPerThread - 1) / kDeg3RowsPerThread;
-        for (uint64_t first = 0; first < batch; first += chunk) {
-            const int nb = int(std::min<uint64_t>(chunk, batch - first));
-            const dim3 sgrid(unsigned((d + kWave - 1) / kWave), unsigned(nb), unsigned((groups + kWavesPerBlock - 1) / kWavesPerBlock));
-            hipLaunchKernelGGL((degree3_fwd_scan_kernel<T>), sgrid, dim3(kBlock), 0, stream, (const T*)inc, rows, out, L, d,
-                               int64_t(s.stride), sc, int64_t(first));
-            // level 3 (row-major d^2 x d) = V^T Z; column-major: [d x d^2] = Z^T (stored: d x L) * (V^T stored: d^2 x L)^T
-            gemm_col_major<T>(h, false, true, d, int(dd), int(L), inc + (first * (s.L + 2) + 1) * s.d_aug, d, (L + 2) * d,
-                              (const T*)rows, int(dd), L * dd, T(0), out + first * s.stride + sc + d + dd, d, int64_t(s.stride), nb);
+        if constexpr (sizeof(T) == 8) {      // single precision: the by-row sweep on the matrix units
+            const int d = int(s.d_aug);
+            const int64_t L = int64_t(s.L);
+            const uint64_t chunk = d3.chunk;
+            T* inc = d3.inc;
+            T* rows = d3.rows;
+            compute_increments(path, inc, batch, dimension, length, time_aug, lead_lag, end_time, s, stream);
+            RocBlas::Handle h = d3.handle;
+            tl_last_segments = 1;
+            MainKernelTimer timer(stream, "degree3_fwd_gemm_f64");
+            const int64_t dd = int64_t(d) * d;
+            const int groups = (d + kDeg3RowsPerThread - 1) / kDeg3RowsPerThread;
+            for (uint64_t first = 0; first < batch; first += chunk) {
+                const int nb = int(std::min<uint64_t>(chunk, batch - first));
+                const dim3 sgrid(unsigned((d + kWave - 1) / kWave), unsigned(nb), unsigned((groups + kWavesPerBlock - 1) / kWavesPerBlock));
+                hipLaunchKernelGGL((degree3_fwd_scan_kernel<T>), sgrid, dim3(kBlock), 0, stream, (const T*)inc, rows, out, L, d,
+                                   int64_t(s.stride), sc, int64_t(first));
+                // level 3 (row-major d^2 x d) = V^T Z; column-major: [d x d^2] = Z^T (stored: d x L) * (V^T stored: d^2 x L)^T
+                gemm_col_major<T>(h, false, true, d, int(dd), int(L), inc + (first * (s.L + 2) + 1) * s.d_aug, d, (L + 2) * d,
+                                  (const T*)rows, int(dd), L * dd, T(0), out + first * s.stride + sc + d + dd, d, int64_t(s.stride), nb);
+            }
+            timer.stop();
+            if (flag)
+                hipLaunchKernelGGL((finite_rows_kernel<T>), dim3(grid_for(batch * s.stride)), dim3(kBlock), 0, stream, out,
+                                   int64_t(batch * s.stride), flag);
         }
-        timer.stop();
-        if (flag)
-            hipLaunchKernelGGL((finite_rows_kernel<T>), dim3(grid_for(batch * s.stride)), dim3(kBlock), 0, stream, out,
-                               int64_t(batch * s.stride), flag);
     } else if (use_degree2(false, s.d_aug, degree, batch)) {
         const int d = int(s.d_aug);
         const int tiles = (d + 15) / 16, col_groups = (tiles + kDeg2Cols - 1) / kDeg2Cols;
@@ -924,8 +928,8 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
         };
         const uint64_t tile = (s.d_aug + 31) / 32 * 32;
         const int rows_mode = g_rows_forward;
-        bool by_rows = rows_mode != 0 && g_force_tail == 0 && rows_bwd_supported(sizeof(T), s.d_aug, degree) &&
-                       rows_bwd_fits(sizeof(T), s.d_aug, degree, batch);
+        bool by_rows = rows_mode != 0 && g_force_tail == 0 && rows_fwd_supported(sizeof(T), s.d_aug, degree) &&
+                       rows_fits(sizeof(T), s.d_aug, degree, batch);
         if (rows_mode == 1 && e->D > 0) by_rows = by_rows && sizeof(T) == 4 && g_force_segments == 0 && 16 * s.d_aug * s.d_aug >= 9 * tile * tile;
         SplitPlan plan{1, 0.0, 0.0};
         const bool compare = by_rows && rows_mode == 1 && e->D > 0 && degree == 3;
@@ -1305,7 +1309,7 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
         };
         const int rows_mode = g_rows_backward;
         bool by_rows = !arena && rows_mode != 0 && g_force_tail == 0 && rows_bwd_supported(sizeof(T), s.d_aug, degree) &&
-                       rows_bwd_fits(sizeof(T), s.d_aug, degree, batch);
+                       rows_fits(sizeof(T), s.d_aug, degree, batch);
         const bool compare = by_rows && rows_mode == 1 && e->D > 0 && s.d_aug < 48;
         if (compare) by_rows = sizeof(T) == 4 && degree == 3 && !lead_lag && g_force_bwd_segments == 0;
         SplitPlan plan{1, 0.0, 0.0};

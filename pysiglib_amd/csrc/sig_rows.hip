@@ -1,4 +1,4 @@
-// Reverse signature sweep for paths of many channels (33 and more) at degrees 3 .. 8, where the compiled instance table
+// Reverse signature sweep for paths of many channels (33 and more) at degrees 3 .. 6, where the compiled instance table
 // has no faster kernel.
 //
 // Arithmetic: siglib/cpsig/cp_signature.h:1137-1187 (per step: un-multiply the state by exp(-z), pull the adjoint back
@@ -36,11 +36,14 @@ template <typename T>
 constexpr int kRowLettersOf = sizeof(T) == 8 ? 32 : 64;
 constexpr int kRowsMinDim = 33;         // below, the compiled table or the other run-time kernels are faster
 constexpr int kRowsMinDegree = 3;
-constexpr int kRowsMaxDegree = 8;
+// One signature of 33 channels takes 170 GB at degree 7 in single precision, 341 GB in double: no card holds what the
+// degrees beyond would read and write (backward: the signature and its gradient).
+constexpr int kRowsMaxDegreeBwd = 6;
 
-// Waves per block; a block fills a CU.  Degrees 3 and 4 fit 168 vector registers (three waves per SIMD: 7.0 ms against 7.7 ms
-// for 16 paths of 200 steps, 64 channels, degree 4); the longer chains above need more and run two waves per SIMD (a
-// third would spill: degree 5 9.4 -> 10.7 ms); double precision always runs two.
+// Waves per block; a block fills a CU.  In single precision degrees 3 and 4 fit 168 vector registers (three waves per SIMD:
+// 7.0 ms against 7.7 ms for 16 paths of 200 steps, 64 channels, degree 4); the longer chains above need more and run two
+// waves per SIMD (a third would spill: degree 5 9.4 -> 10.7 ms); double precision always runs two.  Single precision comes
+// here with more than 256 channels and with paths of a few steps, the rest runs on the matrix units.
 template <typename T, int N>
 constexpr int kRowsWavesOf = (N <= 4 && sizeof(T) == 4) ? 12 : 8;
 constexpr int kRowsMaxWaves = 12;
@@ -319,15 +322,16 @@ __global__ __launch_bounds__((kRowsWavesOf<T, N> * kWave)) void rows_bwd_kernel(
 // Forward sweep in double precision in the same tiling (arithmetic: siglib/cpsig/cp_signature.h:464-499): a lane owns the prefix
 // (r, 64 blk + lane), its chain, and the KB top-level coefficients (prefix, letter) of the wave's letter tile.  Per step
 // the top level costs one multiply-add per coefficient, S_N[p, a] += U[p] * z[a], with z[a] wave-uniform from scalar
-// loads; the chain work of a lane is shared by 64 (32) of them instead of the 16 or 32 of the general run-time kernels.
+// loads; the chain work of a lane is shared by 32 of them instead of the 16 of the general run-time kernels.
 // The letters are held in two halves: the next step's half is requested as soon as this step is done with it, so a
 // row never sits in the scalar registers twice.
 // ---------------------------------------------------------------------------
-template <typename T, int N>
+template <int N>
 __global__ __launch_bounds__(kBlock) void rows_fwd_kernel(
-    const T* __restrict__ inc, T* __restrict__ out, int64_t batch, int64_t L, int d, int64_t out_stride, int scalar,
+    const double* __restrict__ inc, double* __restrict__ out, int64_t batch, int64_t L, int d, int64_t out_stride, int scalar,
     int64_t rows /* d^(N-2) */, int nblk, int nga, int* __restrict__ nonfinite)
 {
+    using T = double;
     constexpr int KB = kRowLettersOf<T>;
     constexpr int HB = KB / 2;
     using Tr = Tree<T, -1, N, 1, 1>;
@@ -449,17 +453,17 @@ __global__ __launch_bounds__(kBlock) void rows_fwd_kernel(
     if (nonfinite && !(chk == T(0))) *nonfinite = 1;
 }
 
-template <typename T, int N>
-hipError_t launch_rows_fwd_n(const FwdParams& p)
+template <int N>
+static hipError_t launch_rows_fwd_n(const FwdParams& p)
 {
-    const int nblk = (p.d + kWave - 1) / kWave, nga = (p.d + kRowLettersOf<T> - 1) / kRowLettersOf<T>;
+    const int nblk = (p.d + kWave - 1) / kWave, nga = (p.d + kRowLettersOf<double> - 1) / kRowLettersOf<double>;
     int64_t rows = 1;
     for (int i = 0; i < N - 2; ++i) rows *= p.d;
     const int64_t waves = p.batch * rows * nblk * nga;
     const int64_t blocks = (waves + kWavesPerBlock - 1) / kWavesPerBlock;
     if (blocks < 1 || blocks > kMaxGridX) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL((rows_fwd_kernel<T, N>), dim3(unsigned(blocks)), dim3(kBlock), 0, p.stream, static_cast<const T*>(p.inc),
-                       static_cast<T*>(p.out), p.batch, p.L, p.d, p.out_stride, p.scalar, rows, nblk, nga, p.nonfinite);
+    hipLaunchKernelGGL((rows_fwd_kernel<N>), dim3(unsigned(blocks)), dim3(kBlock), 0, p.stream, static_cast<const double*>(p.inc),
+                       static_cast<double*>(p.out), p.batch, p.L, p.d, p.out_stride, p.scalar, rows, nblk, nga, p.nonfinite);
     return hipGetLastError();
 }
 
@@ -467,11 +471,10 @@ hipError_t launch_rows_fwd_f64(const FwdParams& p, int degree)
 {
     if (p.nseg != 1 || p.from_points || p.d < kRowsMinDim || p.d > kRowsMaxDim) return hipErrorInvalidConfiguration;
     switch (degree) {
-        case 3: return launch_rows_fwd_n<double, 3>(p);
-        case 4: return launch_rows_fwd_n<double, 4>(p);
-        case 5: return launch_rows_fwd_n<double, 5>(p);
-        case 6: return launch_rows_fwd_n<double, 6>(p);
-        case 7: return launch_rows_fwd_n<double, 7>(p);
+        case 3: return launch_rows_fwd_n<3>(p);
+        case 4: return launch_rows_fwd_n<4>(p);
+        case 5: return launch_rows_fwd_n<5>(p);
+        case 6: return launch_rows_fwd_n<6>(p);
         default: return hipErrorInvalidConfiguration;
     }
 }
@@ -496,14 +499,22 @@ hipError_t launch_rows(const BwdParams& p)
     return hipGetLastError();
 }
 
-bool rows_bwd_supported(size_t elem_bytes, uint64_t d, uint64_t degree)
+static bool rows_dim(size_t elem_bytes, uint64_t d)
 {
-    if (elem_bytes == 8 && degree > 7) return false;     // (its 56 chain values per lane no longer fit the registers)
-    return (elem_bytes == 4 || elem_bytes == 8) && d >= uint64_t(kRowsMinDim) && d <= uint64_t(kRowsMaxDim) && degree >= uint64_t(kRowsMinDegree) &&
-           degree <= uint64_t(kRowsMaxDegree);
+    return (elem_bytes == 4 || elem_bytes == 8) && d >= uint64_t(kRowsMinDim) && d <= uint64_t(kRowsMaxDim);
 }
 
-bool rows_bwd_fits(size_t elem_bytes, uint64_t d, uint64_t degree, uint64_t batch)
+bool rows_bwd_supported(size_t elem_bytes, uint64_t d, uint64_t degree)
+{
+    return rows_dim(elem_bytes, d) && degree >= uint64_t(kRowsMinDegree) && degree <= uint64_t(kRowsMaxDegreeBwd);
+}
+
+bool rows_fwd_supported(size_t elem_bytes, uint64_t d, uint64_t degree)
+{
+    return rows_dim(elem_bytes, d) && degree >= uint64_t(kRowsMinDegree) && degree <= (elem_bytes == 8 ? 6u : 7u);
+}
+
+bool rows_fits(size_t elem_bytes, uint64_t d, uint64_t degree, uint64_t batch)
 {
     const uint64_t nblk = (d + kWave - 1) / kWave, nga = elem_bytes == 8 ? (d + 31) / 32 : nblk;
     unsigned __int128 per_path = (unsigned __int128)nblk * nga;
@@ -524,10 +535,6 @@ hipError_t launch_rows_bwd(const BwdParams& p, int degree)
         case 4: return launch_rows<T, 4>(p);
         case 5: return launch_rows<T, 5>(p);
         case 6: return launch_rows<T, 6>(p);
-        case 7: return launch_rows<T, 7>(p);
-        case 8:
-            if constexpr (sizeof(T) == 4) return launch_rows<T, 8>(p);
-            return hipErrorInvalidConfiguration;
         default: return hipErrorInvalidConfiguration;
     }
 }

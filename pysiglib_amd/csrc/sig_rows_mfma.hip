@@ -1,4 +1,5 @@
-// Single-precision sweeps for paths of many channels (33 and more) at degrees 3 .. 8 on the matrix units.
+// Single-precision sweeps for paths of many channels (33 and more) on the matrix units, forward at degrees 3 .. 7, backward
+// at degrees 3 .. 6.
 //
 // Arithmetic: siglib/cpsig/cp_signature.h:464-499 (forward) and :1137-1187 (reverse).  The lower levels run as in
 // sig_rows.hip (a lane owns a word prefix of N - 1 letters and its chain); what bounds these sweeps is the top level, one
@@ -461,7 +462,6 @@ hipError_t launch_rows_fwd_mfma(const FwdParams& p, int degree)
         case 5: return launch_fwd_n<5>(p);
         case 6: return launch_fwd_n<6>(p);
         case 7: return launch_fwd_n<7>(p);
-        case 8: return launch_fwd_n<8>(p);
         default: return hipErrorInvalidConfiguration;
     }
 }
@@ -495,8 +495,6 @@ hipError_t launch_rows_bwd_mfma(const BwdParams& p, int degree)
         case 4: return launch_bwd_n<4>(p);
         case 5: return launch_bwd_n<5>(p);
         case 6: return launch_bwd_n<6>(p);
-        case 7: return launch_bwd_n<7>(p);
-        case 8: return launch_bwd_n<8>(p);
         default: return hipErrorInvalidConfiguration;
     }
 }
