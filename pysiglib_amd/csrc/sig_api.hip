@@ -586,15 +586,18 @@ static double instance_bwd_seconds(const SplitPlan& plan, uint64_t d)
 // The by-row reverse sweep in single precision on the matrix units or off them.  The matrix form works on sixteen steps at a
 // time and its smaller blocks add three times as many pieces to the gradient rows, which shows on paths of a few steps whose
 // tiles of 64 x 64 are partly empty (8 paths of 3 / 9 / 12 steps, 65 channels, a quarter filled, degree 4: off / on
-// 0.84 / 1.15, 1.24 / 1.33, 1.40 / 1.38 ms; 32 x 1, 65, degree 3: 74 / 87 us; 8 x 1 / 4, 72, a third filled: 1.23 / 1.32,
-// 1.42 / 1.34 ms; 1 x 1 / 4, 48, 56 %: 60 / 66, 64 / 67 us; 1 x 2 / 4 / 8, 33, degree 5: 278 / 314, 310 / 315, 393 / 320).  Full tiles win from one step on (8 x 1, 64, degree 4: 441 / 389 us),
-// and so do launches of up to two waves per SIMD at degree 3 (4 x 1, 96: 55 / 53 us).
+// 0.84 / 1.15, 1.24 / 1.33, 1.40 / 1.38 ms; 32 x 1, 65, degree 3: 76 / 87 us; 8 x 1 / 4, 72, a third filled: 1.24 / 1.32,
+// 1.43 / 1.34 ms; 1 x 2 / 4 / 8, 33, degree 5: 278 / 314, 310 / 315, 393 / 320 us).  Tiles filled to nine sixteenths win from
+// one step on where several waves share a SIMD (8 x 1, 49, degree 4: 187 / 166 us; 1 x 2, 96: 397 / 377; but 1 x 1, 48:
+// 60 / 66), full tiles always (8 x 1, 64: 441 / 389 us), and so do launches of up to two waves per SIMD at degree 3
+// (4 x 1, 96: 55 / 53 us).
 static bool rows_bwd_mfma_wins(uint64_t d, uint64_t degree, uint64_t batch, uint64_t L)
 {
-    const uint64_t groups = (d + kWave - 1) / kWave, tile = groups * kWave;
-    if (L >= 12 || 16 * d * d >= 14 * tile * tile) return true;
+    const uint64_t groups = (d + kWave - 1) / kWave, tile = groups * kWave, simds = uint64_t(simd_count());
+    const double waves = double(batch) * std::pow(double(d), double(degree) - 2) * double(groups * groups);
+    if (L >= 12 || 16 * d * d >= (waves >= 4.0 * double(simds) ? 9 : 14) * tile * tile) return true;
     if (L >= 4 && (groups == 1 || 16 * d * d >= 5 * tile * tile)) return true;
-    return degree == 3 && batch * d * groups * groups <= 2 * uint64_t(simd_count());
+    return degree == 3 && waves <= 2.0 * double(simds);
 }
 
 // ---------------------------------------------------------------------------
@@ -1327,8 +1330,9 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
         const KernelEntry* e_run = pick_variant(true, e, total_waves(geom, int64_t(batch) * nseg), sparse_ll);
         const bool point_fed = !arena && !by_rows && nseg == 1 && e_run->staged && !time_aug && !lead_lag && e_run->D > 0 &&
                                e_run->D <= kPointFedMaxDim && g_point_fed != 0;
-        // single precision on the matrix units: the increment gradient is summed in double precision, and rounded where the
-        // path gradient is formed from it
+        // by rows in single precision: the increment gradient is summed in double precision, and rounded where the path
+        // gradient is formed from it
+        const bool wide = by_rows && sizeof(T) == 4;
         const bool on_matrix_units = by_rows && sizeof(T) == 4 && rows_mode != 3 && rows_bwd_mfma_supported(s.d_aug) &&
                                      (rows_mode == 2 || rows_bwd_mfma_wins(s.d_aug, degree, batch, s.L));
         T* inc = nullptr;
@@ -1353,7 +1357,7 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
         } else {
             inc = static_cast<T*>(buffer(0, checked_mul(inc_elems + 2 * pad, sizeof(T), "increments"))) + pad;
             // one launch writes the increments and clears the increment-gradient accumulator (dz_elems <= increment elements)
-            if (on_matrix_units) {
+            if (wide) {
                 wide_dz = static_cast<double*>(buffer(1, checked_mul(dz_elems, sizeof(double), "increments")));
                 compute_increments(path, inc, batch, dimension, length, time_aug, lead_lag, end_time, s, stream, wide_dz, dz_elems);
             } else {

@@ -906,7 +906,7 @@ def test_long_backward_of_33_to_47_channels(P, by_rows, shape, rows):
 
 
 @pytest.mark.parametrize("shape,matrix", [((2, 4, 65, 4), False), ((2, 13, 65, 4), True), ((32, 2, 72, 3), False),
-                                          ((2, 5, 72, 4), True), ((1, 2, 64, 4), True), ((4, 2, 96, 3), True)])
+                                          ((2, 5, 72, 4), True), ((1, 2, 64, 4), True), ((4, 2, 96, 3), True), ((2, 4, 300, 3), False)])
 def test_backward_of_short_paths_by_row(P, oracle, by_rows, shape, matrix):
     """Single precision: few steps of partly empty tiles are left to the form of the by-row reverse sweep without matrix
     units."""
@@ -919,7 +919,9 @@ def test_backward_of_short_paths_by_row(P, oracle, by_rows, shape, matrix):
     by_rows(1, 1)
     got = P.sig_backprop(dev(x), dev(ref.astype(np.float32)), dev(g), deg).cpu().numpy()
     assert by_rows.last_name() == "rows_bwd_f32_n%d" % deg and by_rows.last_on_matrix_units() == int(matrix)
-    assert bwd_rel_err(got, want) <= 1e-5
+    # either form sums a gradient row in double precision: what is left is the rounding of the terms, a few 6e-8 each over
+    # the steps that recover the states (0.8e-7 .. 3e-7 measured; 1e-6 and more with single-precision rows)
+    assert np.linalg.norm(got - want) <= 6e-7 * np.linalg.norm(want)
 
 
 @pytest.mark.parametrize("aug", [{}, dict(time_aug=True), dict(lead_lag=True)])
