@@ -586,17 +586,18 @@ static double instance_bwd_seconds(const SplitPlan& plan, uint64_t d)
 // The by-row reverse sweep in single precision on the matrix units or off them.  The matrix form works on sixteen steps at a
 // time and its smaller blocks add three times as many pieces to the gradient rows, which shows on paths of a few steps whose
 // tiles of 64 x 64 are partly empty (8 paths of 3 / 9 / 12 steps, 65 channels, a quarter filled, degree 4: off / on
-// 0.84 / 1.15, 1.24 / 1.33, 1.40 / 1.38 ms; 32 x 1, 65, degree 3: 76 / 87 us; 8 x 1 / 4, 72, a third filled: 1.24 / 1.32,
-// 1.43 / 1.34 ms; 1 x 2 / 4 / 8, 33, degree 5: 278 / 314, 310 / 315, 393 / 320 us).  Tiles filled to nine sixteenths win from
-// one step on where several waves share a SIMD (8 x 1, 49, degree 4: 187 / 166 us; 1 x 2, 96: 397 / 377; but 1 x 1, 48:
-// 60 / 66), full tiles always (8 x 1, 64: 441 / 389 us), and so do launches of up to two waves per SIMD at degree 3
-// (4 x 1, 96: 55 / 53 us).
+// 0.84 / 1.15, 1.24 / 1.33, 1.40 / 1.38 ms; 32 x 1 / 10, 65, degree 3: 76 / 87, 111 / 97 us; 8 x 1 / 4, 72, a third filled,
+// degree 4: 1.24 / 1.32, 1.43 / 1.34 ms; 1 x 2 / 4 / 8, 33, degree 5: 278 / 314, 310 / 315, 393 / 320 us).  Tiles filled to
+// nine sixteenths win from one step on where several waves share a SIMD (8 x 1, 49, degree 4: 187 / 166 us; 1 x 2, 96:
+// 397 / 377; but 1 x 1, 48: 60 / 66) and at degree 3 (1 x 1, 200: 100 / 79 us), full tiles always (8 x 1, 64, degree 4:
+// 441 / 389 us), and so do launches of up to two waves per SIMD at degree 3 (4 x 1, 96: 55 / 53 us).
 static bool rows_bwd_mfma_wins(uint64_t d, uint64_t degree, uint64_t batch, uint64_t L)
 {
     const uint64_t groups = (d + kWave - 1) / kWave, tile = groups * kWave, simds = uint64_t(simd_count());
     const double waves = double(batch) * std::pow(double(d), double(degree) - 2) * double(groups * groups);
-    if (L >= 12 || 16 * d * d >= (waves >= 4.0 * double(simds) ? 9 : 14) * tile * tile) return true;
-    if (L >= 4 && (groups == 1 || 16 * d * d >= 5 * tile * tile)) return true;
+    const bool shared = degree == 3 || waves >= 4.0 * double(simds);
+    if (L >= (degree == 3 ? 6u : 12u) || 16 * d * d >= (shared ? 9 : 14) * tile * tile) return true;
+    if (L >= 3 && (groups == 1 || 16 * d * d >= 5 * tile * tile)) return true;
     return degree == 3 && waves <= 2.0 * double(simds);
 }
 
