@@ -21,6 +21,7 @@
 #include "sig_chen_adjoint.h"
 #include "sig_host.h"
 #include "sig_kernels.h"
+#include "sig_log_rows.h"
 #include "sig_lyndon.h"
 
 namespace sigamd {
@@ -205,19 +206,20 @@ static DeviceLyndon find_lyndon(uint64_t dimension, uint64_t degree, int method)
 }
 
 // out[b][i] = x[b][index[i]] (method 1) plus sum_k val[k] * x[b][col_pos[k]] over the row's entries (method 2;
-// col_pos[k] = index[col[k]], resolved when the tables are prepared)
+// col_pos[k] = index[col[k]], resolved when the tables are prepared).  Null index: x holds the listed coefficients alone, one
+// after the other, and col[k] is read
 template <typename T>
 __global__ __launch_bounds__(kBlock) void lyndon_compress_kernel(
     const T* __restrict__ expanded, T* __restrict__ out, int64_t batch, int64_t count, int64_t stride, int off,
     const uint64_t* __restrict__ index, const uint64_t* __restrict__ row_ptr, const uint64_t* __restrict__ col_pos,
-    const int32_t* __restrict__ val)
+    const uint32_t* __restrict__ col, const int32_t* __restrict__ val)
 {
     for (int64_t b = blockIdx.y; b < batch; b += gridDim.y) {
         const T* x = expanded + b * stride + off;
         for (int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x; i < count; i += int64_t(gridDim.x) * kBlock) {
-            T acc = x[index[i]];
+            T acc = x[index ? index[i] : uint64_t(i)];
             if (row_ptr)
-                for (uint64_t k = row_ptr[i]; k < row_ptr[i + 1]; ++k) acc = fmadd(T(val[k]), x[col_pos[k]], acc);
+                for (uint64_t k = row_ptr[i]; k < row_ptr[i + 1]; ++k) acc = fmadd(T(val[k]), x[index ? col_pos[k] : col[k]], acc);
             out[b * count + i] = acc;
         }
     }
@@ -241,6 +243,8 @@ __global__ __launch_bounds__(kBlock) void lyndon_expand_kernel(
         }
     }
 }
+
+extern std::atomic<int> g_chen_adjoint_mode;      // test hook (defined in sig_api.hip)
 
 // number of coefficients of levels 1 .. t
 static uint64_t coef_count(uint64_t d, uint64_t t) { return sig_length_u64(d, t) - 1; }
@@ -275,6 +279,115 @@ static void run_tensor_log(const T* sig, T* out, uint64_t batch, uint64_t dimens
     });
 }
 
+// ---------------------------------------------------------------------------
+// a block per row (sig_log_rows.h)
+// ---------------------------------------------------------------------------
+// Rows of up to 65536 coefficients, where the form that launches a kernel per step is not the sooner one.  Whole calls, us, a
+// kernel per step / a block per row, single precision unless noted:
+//  * all coefficients of the logarithm of many rows: the general kernels share the work of several first letters
+//    (16 x d = 4, degree 7: 43 / 38; 257 x 7, 5: 52 / 66; 600 x 6, 6: 161 / 301);
+//  * a recursion of more than 13 steps forward (1 x 2, 14: 106 / 114), or one that leaves a compute unit a single block, many
+//    times over (4000 x 4, 7, double precision: forward 465 / 502; backward, single 1620 / 2045, double 1952 / 2478);
+//  * lower levels that do not fit the LDS: forward never (1000 x 2, 13, double: 259 / 310), backward few rows (64 x 6, 6,
+//    double: 317 / 283; 600: 749 / 1038) or many steps (1000 x 2, 13, double: 2092 / 1667).
+static bool plan_log_rows(LogRowPlan& pl, uint64_t dimension, uint64_t degree, uint64_t n_coef)
+{
+    if (g_chen_adjoint_mode != 0 || g_chen_low_levels != 1 || g_force_wide_index != 0) return false;    // a test asks for the general form
+    if (degree < 2 || degree > uint64_t(kLogRowMaxDegree) || n_coef > 65536) return false;
+    pl.degree = int(degree);
+    pl.d = uint32_t(dimension);
+    pl.n = uint32_t(n_coef);
+    pl.dv = DivBy<uint32_t>(dimension);
+    uint32_t at = 0, size = 1;
+    pl.lo[0] = 0;
+    pl.pw[0] = 1;
+    for (uint64_t t = 1; t <= degree; ++t) {
+        pl.lo[t] = at;
+        size *= pl.d;
+        pl.pw[t] = size;
+        at += size;
+    }
+    pl.lo[degree + 1] = at;
+    pl.low = pl.lo[degree];
+    at = 0;
+    for (uint64_t k = degree; k >= 2; --k) {
+        pl.poff[k] = at;
+        at += pl.lo[degree - k + 2];
+    }
+    pl.p_total = at;
+    return true;
+}
+
+// threads of a block: 4096 x d = 3, degree 4 (128 / 256 / 512 / 1024 threads): backward 63 / 71 / 107 / 220 us; 257 x 7, 5: 256 /
+// 512 / 1024: 111 / 88 / 112; one such row 104 / 78 / 68
+static unsigned log_row_threads(const LogRowPlan& pl, uint64_t batch)
+{
+    if (pl.n < 512) return 128;
+    if (pl.n < 4096) return 256;
+    return batch <= 128 ? 1024 : 512;
+}
+
+// dynamic LDS a block may take beside its static LDS
+constexpr size_t kLogRowLds = size_t(156) << 10, kLogRowBwdLds = size_t(140) << 10;
+static size_t log_row_fwd_entries(const LogRowPlan& pl) { return 2 * size_t(pl.low); }
+static size_t log_row_bwd_entries(const LogRowPlan& pl) { return 4 * size_t(pl.low) + pl.p_total; }
+
+static bool log_rows_forward(const LogRowPlan& pl, uint64_t batch, int method, size_t elem_bytes)
+{
+    const size_t lds = log_row_fwd_entries(pl) * elem_bytes;
+    return lds <= kLogRowLds && pl.degree <= 13 && !(batch > 512 && lds > (size_t(80) << 10)) &&
+           (method != 0 || batch * pl.n <= uint64_t(1) << 20);
+}
+
+static bool log_rows_backward(const LogRowPlan& pl, uint64_t batch, size_t elem_bytes)
+{
+    const size_t lds = log_row_bwd_entries(pl) * elem_bytes;
+    if (lds > kLogRowBwdLds) return batch <= 256 || pl.degree >= 10;
+    return !(batch > 1024 && lds > (size_t(64) << 10) && pl.degree >= 6);
+}
+
+template <typename Kern>
+static void log_row_lds(Kern kern, size_t bytes)
+{
+    if (bytes > size_t(64) << 10)       // above the default limit of dynamic LDS
+        SIG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)));
+}
+
+// P_1 of every row at the positions `index` (null: everywhere), rows of out `out_stride` apart
+template <typename T>
+static void launch_log_rows(const LogRowPlan& pl, const T* sig, T* out, uint64_t batch, const uint64_t* index, uint64_t count,
+                            int64_t out_stride, int out_off, const SigShape& s, hipStream_t stream)
+{
+    const size_t lds = log_row_fwd_entries(pl) * sizeof(T);
+    const unsigned threads = log_row_threads(pl, batch);
+    const uint64_t rows = std::min<uint64_t>(batch, 65535);
+    // few rows: several blocks each, of at least four coefficients a thread
+    const uint64_t parts = std::max<uint64_t>(1, std::min((index ? count : pl.n) / (4 * threads), 512 / rows));
+    log_row_lds(&tensor_log_row_kernel<T>, lds);
+    hipLaunchKernelGGL((tensor_log_row_kernel<T>), dim3(unsigned(parts), unsigned(rows)), dim3(threads), lds, stream, sig, out,
+                       int64_t(batch), pl, index, uint32_t(count), int64_t(s.stride), s.off, out_stride, out_off);
+    SIG_HIP(hipGetLastError());
+}
+
+// ws: (degree + 4) * stride a row
+template <typename T>
+static void launch_log_rows_bwd(const LogRowPlan& pl, const T* sig, T* out, const T* derivs, uint64_t batch, int method,
+                                const DeviceLyndon& lyn, const SigShape& s, T* ws, hipStream_t stream)
+{
+    const size_t lds = log_row_bwd_entries(pl) * sizeof(T);
+    const bool shared = lds <= kLogRowBwdLds;
+    auto go = [&](auto kern) {
+        if (shared) log_row_lds(kern, lds);
+        hipLaunchKernelGGL(kern, dim3(unsigned(std::min<uint64_t>(batch, 1u << 20))), dim3(log_row_threads(pl, batch)), shared ? lds : 0,
+                           stream, sig, out, derivs, int64_t(batch), pl, (const uint64_t*)lyn.index, uint32_t(lyn.count),
+                           (const uint64_t*)(method == 2 ? lyn.t_row_ptr : nullptr), (const uint32_t*)lyn.t_col,
+                           (const int32_t*)lyn.t_val, int64_t(s.stride), s.off, ws, int64_t((pl.degree + 4) * s.stride));
+    };
+    if (shared) go(&tensor_log_row_bwd_kernel<T, true>);
+    else go(&tensor_log_row_bwd_kernel<T, false>);
+    SIG_HIP(hipGetLastError());
+}
+
 template <typename T>
 static void sig_to_log_sig_impl(const T* sig, T* out, uint64_t batch, uint64_t dimension, uint64_t degree, int method,
                                 bool scalar_term)
@@ -297,6 +410,27 @@ static void sig_to_log_sig_impl(const T* sig, T* out, uint64_t batch, uint64_t d
         return;
     }
     T* ws = degree >= 2 ? static_cast<T*>(workspace(7, checked_mul(bytes, 2, "workspace"))) : nullptr;
+    // (the workspaces are asked for before the form is chosen: a call meets the same limit of memory whichever serves it)
+    LogRowPlan rows;
+    if (plan_log_rows(rows, dimension, degree, s.n_coef) && log_rows_forward(rows, batch, method, sizeof(T))) {
+        if (method == 2) {
+            // the logarithm at the Lyndon words, then its coordinates in their basis
+            T* words = static_cast<T*>(workspace(14, bytes));
+            launch_log_rows<T>(rows, sig, words, batch, lyn.index, lyn.count, int64_t(lyn.count), 0, s, stream);
+            launch_indexed(0, lyn.count, batch, [&](auto, dim3 grid) {
+                hipLaunchKernelGGL((lyndon_compress_kernel<T>), grid, dim3(kBlock), 0, stream, (const T*)words, out, int64_t(batch),
+                                   int64_t(lyn.count), int64_t(lyn.count), 0, (const uint64_t*)nullptr, (const uint64_t*)lyn.row_ptr,
+                                   (const uint64_t*)nullptr, (const uint32_t*)lyn.col, (const int32_t*)lyn.val);
+            });
+            SIG_HIP(hipGetLastError());
+        } else if (method == 1) {
+            launch_log_rows<T>(rows, sig, out, batch, lyn.index, lyn.count, int64_t(lyn.count), 0, s, stream);
+        } else {
+            launch_log_rows<T>(rows, sig, out, batch, nullptr, 0, int64_t(s.stride), s.off, s, stream);
+        }
+        SIG_HIP(hipStreamSynchronize(stream));
+        return;
+    }
     const uint64_t elems = batch * s.stride;
     // Lyndon coordinates are read off the expanded logarithm, which then lives in a scratch copy
     T* expanded = method ? static_cast<T*>(workspace(14, bytes)) : out;
@@ -317,7 +451,7 @@ static void sig_to_log_sig_impl(const T* sig, T* out, uint64_t batch, uint64_t d
             hipLaunchKernelGGL((lyndon_compress_kernel<T>), grid, dim3(kBlock), 0, stream, (const T*)expanded, out, int64_t(batch),
                                int64_t(lyn.count), int64_t(s.stride), s.off, (const uint64_t*)lyn.index,
                                (const uint64_t*)(method == 2 ? lyn.row_ptr : nullptr), (const uint64_t*)lyn.col_pos,
-                               (const int32_t*)lyn.val);
+                               (const uint32_t*)nullptr, (const int32_t*)lyn.val);
         });
     }
     SIG_HIP(hipGetLastError());
@@ -342,6 +476,14 @@ static void sig_to_log_sig_backprop_impl(const T* sig, T* out, const T* derivs, 
         SIG_HIP(hipStreamSynchronize(stream));
         return;
     }
+    // -P_2 .. -P_N (the slot of P_1 stays unused), two adjoint buffers, two product-adjoint buffers
+    T* ws = degree >= 2 ? static_cast<T*>(workspace(7, checked_mul(bytes, degree + 4, "workspace"))) : nullptr;
+    LogRowPlan rows;
+    if (plan_log_rows(rows, dimension, degree, s.n_coef) && log_rows_backward(rows, batch, sizeof(T))) {
+        launch_log_rows_bwd<T>(rows, sig, out, derivs, batch, method, lyn, s, ws, stream);
+        SIG_HIP(hipStreamSynchronize(stream));
+        return;
+    }
     const uint64_t elems = batch * s.stride;
     if (method) {
         // gradient w.r.t. the expanded logarithm: the transposed coordinate map, zero off the Lyndon words
@@ -355,8 +497,6 @@ static void sig_to_log_sig_backprop_impl(const T* sig, T* out, const T* derivs, 
         });
         derivs = dexp;
     }
-    // -P_2 .. -P_N (the slot of P_1 stays unused), two adjoint buffers, two product-adjoint buffers
-    T* ws = degree >= 2 ? static_cast<T*>(workspace(7, checked_mul(bytes, degree + 4, "workspace"))) : nullptr;
     if (degree < 2)
         launch_indexed(s.n_coef, s.n_coef, batch, [&](auto ix, dim3 grid) {
             using I = decltype(ix);

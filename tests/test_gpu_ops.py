@@ -765,3 +765,44 @@ def test_sig_to_log_sig_lyndon_vs_oracle(P, oracle, d, deg, batch, dtype, scalar
             assert row_rel_err(gotb[:, off:], wantb[:, off:]) < TOL[dtype] * (1 if dtype == np.float64 else 10)
     finally:
         P.clear_cache()
+
+
+@pytest.mark.parametrize("d,deg,batch", [(8, 3, 3), (63, 2, 2), (64, 2, 2), (65, 2, 3), (9, 4, 130), (7, 5, 257), (3, 9, 2), (2, 13, 1),
+                                         (1, 6, 5), (2, 2, 4), (40, 3, 2), (255, 2, 2)])
+@pytest.mark.parametrize("method", [0, 1, 2])
+def test_log_sig_block_per_row_vs_general_form(P, d, deg, batch, method):
+    """The kernels with a block per row against the ones that launch a kernel per step (which a hook asks for): levels of 63, 64
+    and 65 words, rows that fit the LDS and rows that do not, one and several blocks a row, with and without the scalar
+    term.  Both sum the same up to c(deg) products an entry in another order, c(deg) < 65536 roundings of 1.1e-16 resp. 6e-8."""
+    from pysiglib_amd import _loader as L
+    L.CUSIG.cusig_amd_force_chen_adjoint.argtypes = (ctypes.c_int,)
+    L.CUSIG.cusig_amd_force_chen_adjoint.restype = None
+    rng = np.random.default_rng(17 * d + deg)
+    n = P.sig_length(d, deg)
+    scale = np.concatenate([np.full(d ** k, 0.5 / np.sqrt(float(d) ** k)) for k in range(1, deg + 1)])
+    a = rng.standard_normal((batch, n)) * scale
+    try:
+        if method:
+            P.prepare_log_sig(d, deg, method)
+        g = rng.standard_normal((batch, P.log_sig_length(d, deg) if method else n))
+
+        def both(dtype, scalar):
+            s = np.hstack([np.ones((batch, 1)), a]) if scalar else a
+            w = np.hstack([np.ones((batch, 1)), g]) if scalar and not method else g
+            s, w = dev(s.astype(dtype)), dev(w.astype(dtype))
+            out = P.sig_to_log_sig(s, d, deg, method=method), P.sig_to_log_sig_backprop(s, w, d, deg, method=method)
+            return [v.cpu().numpy() for v in out]
+
+        L.CUSIG.cusig_amd_force_chen_adjoint(2)
+        want = both(np.float64, False)
+        L.CUSIG.cusig_amd_force_chen_adjoint(0)
+        for dtype, tol in ((np.float64, 65536 * 1.2e-16), (np.float32, 65536 * 6e-8 / 16)):
+            for scalar in (False, True):
+                got = both(dtype, scalar)
+                for i, (x, y) in enumerate(zip(got, want)):
+                    x = x if not scalar or (i == 0 and method) else x[:, 1:]
+                    assert x.shape == y.shape and row_rel_err(x, y) < tol
+    finally:
+        L.CUSIG.cusig_amd_force_chen_adjoint(0)
+        if method:
+            P.clear_cache()
