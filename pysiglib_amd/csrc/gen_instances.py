@@ -130,6 +130,70 @@ def fwd_cost(D, N, tail, K):
     return cost
 
 
+def step_cost(D, N, tail, K):
+    """Instruction figure of a forward step of one lane; the dispatch in sig_api.hip (lane_step_cost) uses the same."""
+    m = N - tail
+    cost = m
+    for t in range(1, N + 1):
+        if t == 1:
+            cost += 1
+        elif t <= m:
+            cost += 2 * (t - 1)
+        else:
+            cost += 1 + 2 * (m - 1)
+            nodes = K
+            for e in range(1, t - m + 1):
+                cost += nodes if e == t - m else 2 * nodes + nodes / (K if e == 1 else D)
+                nodes *= D
+    return cost
+
+
+def lone_step_ns(D, N, tail, K, dtype, direction):
+    """Duration of a step of a wave that has its SIMD to itself (sig_api.hip: StepModel).  Backward, every channel beyond four
+    costs a row of the LDS tile of the increment gradient, more in double precision without the half-wave sums (one level)."""
+    c, m = step_cost(D, N, tail, K), N - tail
+    if direction == "fwd":
+        return 40 + 1.65 * c
+    return 200 + 3.2 * c + 6 * m * m + (40 if dtype == "f64" and tail == 1 else 26) * max(0, D - 4)
+
+
+def fine_partition(D, N, dtype, direction):
+    """A second partition of a shape whose default keeps few, heavy lanes busy per path: more and lighter lanes, for launches
+    of few paths.  None where the default needs many waves a path anyway or gains less than 15 % a step.  Among subtrees of up
+    to two levels (two channels: three) and up to four letter groups, the shortest step, where twice the waves have to
+    buy 10 %.  Measured at 4 channels (whole calls, us, default in time pieces / this partition), single precision, degree 6, 256
+    points: backward 1 path 155 / 144, 128 paths 189 / 145, 512 paths 250 / 179 (two groups fewer), forward 128 paths 65 / 50;
+    double, degree 5, 128 points: backward 128 paths 127 / 72, forward 61 / 32, 512 paths 86 / 35."""
+    if N < 3 or D > (64 if direction == "fwd" else 31):
+        return None
+    if direction == "bwd" and rows_sweep_wins(dtype, D, N):
+        return None
+
+    def waves(tail, K, wide):
+        P, groups = D ** (N - tail), -(-D // K)
+        if wide or P >= 48:
+            return groups * -(-P // 64)
+        lanes = groups * P
+        return 1 / (64 // lanes) if lanes <= 64 else -(-lanes // 64)
+
+    tail0, K0 = choose(D, N, dtype, direction)
+    best = None
+    for tail in range(1, min(N - 1, 2 if D > 2 else 3) + 1):
+        for groups in range(1, 5):
+            K = -(-D // groups)
+            if K * (D ** tail - 1) // (D - 1) > 100:
+                continue
+            w, ns = waves(tail, K, True), lone_step_ns(D, N, tail, K, dtype, direction)
+            cand = (ns * w ** 0.14, tail, K, w, ns)
+            if best is None or cand < best:
+                best = cand
+    _, tail, K, w, ns = best
+    w0 = waves(tail0, K0, False)
+    if w0 > 48 or w < 1.5 * w0 or ns > 0.85 * lone_step_ns(D, N, tail0, K0, dtype, direction):
+        return None
+    return tail, K
+
+
 def lead_lag_mode(D, staged):
     """Lead-lag twin of a staged forward instance: 1 (time channel last, D odd), 2 (no time channel, D even), 0 none.
     At least two raw channels, and narrow enough for the skipped half to matter less than the compile time."""
@@ -197,7 +261,7 @@ def main():
     args = ap.parse_args()
     os.makedirs(args.out, exist_ok=True)
 
-    insts = []  # (T, D, N, tail, K, dir)
+    insts = []  # (T, D, N, tail, K, dir, 1 default / 0 further / 2 fine partition, staged)
     shapes = spec_shapes()
     if args.quick:
         shapes = [(2, 2), (2, 3), (2, 4), (3, 2), (3, 3), (3, 4), (4, 3), (5, 3), (10, 5), (5, 7), (3, 12), (17, 4)]
@@ -215,6 +279,9 @@ def main():
                     # wide layout: also the LDS-staged variant (the backward gains nothing from it beyond ~13 channels)
                     if D ** (N - tl) >= 48 and D <= (64 if direction == "fwd" else 31):
                         insts.append((T, D, N, tl, kk, direction, pref, 1))
+                fine = fine_partition(D, N, dtype, direction)
+                if fine:
+                    insts.append((T, D, N, fine[0], fine[1], direction, 2, 1))
         for N in range(2, MAX_GENERIC_N + 1):
             for direction in ("fwd", "bwd"):
                 insts.append((T, 0, N, 1, GENERIC_K, direction, 1, 0))
@@ -272,13 +339,13 @@ def main():
             if direction == "fwd":
                 ll = lead_lag_mode(D, zl)
                 ll_fn = ("&launch_tree_fwd<%s, %d, %d, %d, %d, true, %d>" % (T, D, N, tail, K, ll)) if ll else "nullptr"
-                lines.append('    {%d, %d, %d, %d, %d, %d, &launch_tree_fwd<%s, %d, %d, %d, %d, %s>, nullptr, "%s", %d, &fwd_waves_per_simd<%s, %d, %d, %d, %d, %s>, %d, %s},'
-                             % (is64, D, N, tail, K, zl, T, D, N, tail, K, zs, name, pref, T, D, N, tail, K, zs, pol, ll_fn))
+                lines.append('    {%d, %d, %d, %d, %d, %d, &launch_tree_fwd<%s, %d, %d, %d, %d, %s>, nullptr, "%s", %d, &fwd_waves_per_simd<%s, %d, %d, %d, %d, %s>, %d, %s, nullptr, %d},'
+                             % (is64, D, N, tail, K, zl, T, D, N, tail, K, zs, name, pref == 1, T, D, N, tail, K, zs, pol, ll_fn, pref == 2))
             else:
                 ll = lead_lag_mode_bwd(T, D, tail, zl)
                 ll_fn = ("&launch_tree_bwd<%s, %d, %d, %d, %d, %s, %d>" % (T, D, N, tail, K, zs, ll)) if ll else "nullptr"
-                lines.append('    {%d, %d, %d, %d, %d, %d, nullptr, &launch_tree_bwd<%s, %d, %d, %d, %d, %s>, "%s", %d, &bwd_waves_per_simd<%s, %d, %d, %d, %d, %s>, %d, nullptr, %s},'
-                             % (is64, D, N, tail, K, zl, T, D, N, tail, K, zs, name, pref, T, D, N, tail, K, zs, pol, ll_fn))
+                lines.append('    {%d, %d, %d, %d, %d, %d, nullptr, &launch_tree_bwd<%s, %d, %d, %d, %d, %s>, "%s", %d, &bwd_waves_per_simd<%s, %d, %d, %d, %d, %s>, %d, nullptr, %s, %d},'
+                             % (is64, D, N, tail, K, zl, T, D, N, tail, K, zs, name, pref == 1, T, D, N, tail, K, zs, pol, ll_fn, pref == 2))
         lines.append("};")
         lines.append("extern const EntryList kList_%02d = {kEntries_%02d, %d};" % (fi, fi, len(bucket)))
         lines.append("#endif")
@@ -302,7 +369,7 @@ def main():
     print("wrote %d instances into %d files under %s" % (len(insts), args.files, args.out))
     for (T, D, N, tail, K, direction, pref, zl) in sorted(insts, key=lambda i: (i[0], i[1], i[2], i[5])):
         if (D, N) in ((10, 5), (5, 7), (3, 12), (17, 4)) and not zl:
-            print("  ", T, D, N, direction, "tail", tail, "K", K, "default" if pref else "extra")
+            print("  ", T, D, N, direction, "tail", tail, "K", K, {0: "extra", 1: "default", 2: "fine"}[pref])
 
 
 if __name__ == "__main__":

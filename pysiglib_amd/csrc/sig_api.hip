@@ -42,6 +42,7 @@ thread_local char g_last_error[4096] = {0};
 struct Table {
     // several partitions (tail, k) of one shape may be compiled; the first listed is the default
     std::map<std::tuple<int, int, int>, std::vector<const KernelEntry*>> fwd, bwd;
+    std::map<std::tuple<int, int, int>, const KernelEntry*> fine_fwd, fine_bwd;     // for launches that leave SIMDs without work
     Table()
     {
         int n = 0;
@@ -50,6 +51,10 @@ struct Table {
             for (int j = 0; j < lists[i].count; ++j) {
                 const KernelEntry* e = &lists[i].entries[j];
                 auto key = std::make_tuple(e->is_f64, e->D, e->N);
+                if (e->fine) {
+                    (e->fwd ? fine_fwd : fine_bwd)[key] = e;
+                    continue;
+                }
                 auto& slot = e->fwd ? fwd[key] : bwd[key];
                 if (e->preferred && !e->staged) slot.insert(slot.begin(), e);
                 else slot.push_back(e);
@@ -173,13 +178,15 @@ static double lane_step_cost(int d, int n, int tail, int k)
     return cost;
 }
 
+static TreeGeom geom_of(const KernelEntry* e, int d) { return make_geom(d, e->N - e->tail, e->k, layout_of(e->D, e->staged != 0)); }
+
 // A sweep is a chain of dependent steps: its duration is their number times the longer of one lane-step (latency
 // of a lone wave) and the chip-wide issue time of all waves' steps.  Long paths of an under-filled launch are cut
 // in time (about two waves per SIMD, segments of at least 32 resp. 48 steps), which divides the chain and multiplies
 // the waves.  Returns a relative figure.
 static double sweep_estimate(const KernelEntry* e, int d, int64_t batch, int64_t L, bool backward)
 {
-    const TreeGeom g = make_geom(d, e->N - e->tail, e->k, e->D != 0);
+    const TreeGeom g = geom_of(e, d);
     const double waves = double(total_waves(g, batch));
     const double simds = double(simd_count());
     double cuts = 1.0;
@@ -602,6 +609,97 @@ static bool rows_bwd_mfma_wins(uint64_t d, uint64_t degree, uint64_t batch, uint
 }
 
 // ---------------------------------------------------------------------------
+// a shape's second, finer partition (gen_instances.py: fine_partition)
+// ---------------------------------------------------------------------------
+static Hook g_fine{1};      // test hook: 0 never, 1 by the estimates below, 2 wherever there is one
+
+static const KernelEntry* fine_entry(bool backward, bool f64, uint64_t d, uint64_t degree)
+{
+    if (g_fine == 0 || g_force_tail > 0 || g_force_staged >= 0 || g_ignore_table != 0 || d > 0x7fffffff || degree > 0x7fffffff) return nullptr;
+    const auto& m = backward ? table().fine_bwd : table().fine_fwd;
+    auto it = m.find(std::make_tuple(int(f64), int(d), int(degree)));
+    return it == m.end() ? nullptr : it->second;
+}
+
+// Seconds per step of a launch: a wave alone on its SIMD pays the latency of its step, several share the issue slots; backward,
+// every channel beyond four costs a row of the LDS tile of the increment gradient, more in double precision without the
+// half-wave sums (one subtree level).  Fitted to 110 partitions of 2 .. 24 channels, degrees 3 .. 8, both precisions, at a thousandth to 8
+// waves per SIMD; most within 15 % (ns a step measured / model, one wave per SIMD and eight; single precision: forward d = 4,
+// degree 6, 1 level x 4 letters 106 / 104, 361 / 424, 3 x 4 letters 277 / 309, 1299 / 1416; backward 4, 6, 2 x 2: 443 / 443, 1465 / 1556;
+// 10, 4, 1 x 10: 474 / 490, 2125 / 1898; 17, 4, 2 x 6: 1028 / 984, 4454 / 4855; double, backward 10, 5, 2 x 5: 619 / 685, 4492 / 5128).
+// Scalar-fed forward steps take at least 130 ns, those of the run-time-dimension kernels about 2.2 times as long (one path of 4
+// channels, degree 5, double: 270 / 120 ns).
+struct StepModel {
+    double lone, issue;         // ns: a step of a wave on its own; what each of several waves on a SIMD adds
+    int64_t occ, simds;
+    TreeGeom geom;
+    bool backward;
+    double elem;
+    StepModel(const KernelEntry* e, int d, bool backward_) : occ(std::max(1, resident_waves(e))), simds(simd_count()), geom(geom_of(e, d)), backward(backward_), elem(e->is_f64 ? 8.0 : 4.0)
+    {
+        const double c = lane_step_cost(d, e->N, e->tail, e->k), m = double(e->N - e->tail);
+        const double wide = std::max(0, d - 4), tile = std::max(0, d - 3);
+        const bool f64 = e->is_f64 != 0, no_pairs = f64 && e->tail == 1;
+        if (backward) {
+            lone = 200.0 + 3.2 * c + 6.0 * m * m + (no_pairs ? 40.0 : 26.0) * wide;
+            issue = f64 ? 50.0 + 4.6 * (c + m * m) + (no_pairs ? 40.0 * (d - 1) : 22.0 * tile) : (2.0 + 3.0 / d) * c + 2.9 * m * m + 22.0 * tile;
+            if (!e->staged) lone *= 1.15;
+        } else {
+            lone = 40.0 + 1.65 * c;
+            issue = f64 ? 24.0 + 1.8 * c : 14.0 + c;
+            if (!e->staged) { lone = std::max(130.0, 1.15 * lone); issue += 20.0; }
+        }
+        if (e->D <= 0) { lone *= 2.2; issue *= 1.5; }
+    }
+    double step(int64_t items) const
+    {
+        const int64_t fullest = (total_waves(geom, items) + simds - 1) / simds, rest = fullest % occ;
+        return 1e-9 * (double(fullest / occ) * std::max(lone, issue * double(occ)) + (rest ? std::max(lone, issue * double(rest)) : 0.0));
+    }
+    double sweep(int64_t batch, int64_t L, int g, uint64_t sig_bytes_all_paths) const;
+};
+
+// Whole sweep in g pieces per path, beside what every call pays.  A fold launch takes 6 us (one path of 1024 points, 4 channels,
+// degree 6, 16 pieces: 25 us of folds).  Backward: 10 us, and 4 to 6 us by the length of the rows for each launch of the two
+// scans, beside the forward sweep of the pieces, a third of the backward's, and traffic as in choose_bwd_segments (calls of one
+// path of 1024 points in 32 pieces less their sweeps: 3 channels, degree 5: 56 us; 4, 5: 71; 4, 6: 82).
+double StepModel::sweep(int64_t batch, int64_t L, int g, uint64_t sig_bytes_all_paths) const
+{
+    int lg = 0;
+    while ((1 << lg) < g) ++lg;
+    const double t = double((L + g - 1) / g) * step(batch * g);
+    if (g <= 1) return t;
+    const double bytes = double(g) * double(sig_bytes_all_paths);
+    if (!backward) return t + 2e-6 + 6e-6 * lg + 2.2 * bytes / 4e12;
+    const double launch = 3.8e-6 + 0.55e-6 * std::log2(std::max(1.0, double(sig_bytes_all_paths) / (double(batch) * elem * 363.0)));
+    return 1.31 * t + 10e-6 + launch * (2 * lg + 2) + bytes * (4.2e-12 + 0.64e-12 * lg);
+}
+
+// The finer partition in as many pieces as serve it best (of at least 16 steps; 256 MB of segment signatures forward, 64 MB per
+// buffer backward), if that promises 8 % (backward 12 %) against `now`, the choice made without it.  On return `e` is the kernel to launch.
+static SplitPlan with_fine(const KernelEntry*& e, const KernelEntry* run_now, const SplitPlan& now, bool backward, uint64_t d, uint64_t degree,
+                           uint64_t batch, uint64_t L, uint64_t sig_bytes_all_paths, int forced_pieces, bool whole_only = false)
+{
+    const KernelEntry* f = fine_entry(backward, e->is_f64 != 0, d, degree);
+    if (!f || (forced_pieces > 0 && g_fine != 2)) return now;
+    const int64_t steps = int64_t(L), paths = int64_t(batch);
+    const StepModel model(f, int(d), backward);
+    SplitPlan best{forced_pieces > 0 ? now.pieces : 1, 0.0, 0.0};
+    best.seconds = model.sweep(paths, steps, best.pieces, sig_bytes_all_paths);
+    if (forced_pieces <= 0 && !whole_only) {
+        const uint64_t most = uint64_t(backward ? 64 : 256) << 20;
+        for (int g : {2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128, 192, 256, 384, 512}) {
+            if (steps / g < 16 || uint64_t(g) * sig_bytes_all_paths > most) break;
+            const double t = model.sweep(paths, steps, g, sig_bytes_all_paths);
+            if (t < 0.95 * best.seconds) best = SplitPlan{g, t, 0.0};
+        }
+    }
+    if (g_fine != 2 && best.seconds > (backward ? 0.88 : 0.92) * StepModel(run_now, int(d), backward).sweep(paths, steps, now.pieces, sig_bytes_all_paths)) return now;
+    e = f;
+    return best;
+}
+
+// ---------------------------------------------------------------------------
 // degree 2 in closed form (matrix cores): taken for paths of many channels, where no specialised sweep exists
 // ---------------------------------------------------------------------------
 static Hook g_force_degree2{-1};    // tuning hook: -1 automatic, 0 never, 1 whenever the degree is 2
@@ -905,7 +1003,6 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
                                      ", degree " + std::to_string(degree) + " in this build");
         // Few paths cannot fill the chip with whole-path sweeps: split every path into time segments,
         // sweep all (path, segment) pairs concurrently and fold the pieces with Chen's identity.
-        const TreeGeom geom = make_geom(int(s.d_aug), e->N - e->tail, e->k, e->D != 0);
         // lead-lag sweeps that skip the letters a step cannot move take the step's parity from its position in the
         // segment: segments start on even steps
         const bool sparse_ll = lead_lag && g_lead_lag_sparse != 0;
@@ -919,7 +1016,7 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
         // 48 channels 2.40 -> 2.11, two 4.37 -> 3.48).  Lead-lag paths of that many channels have no instance that skips the
         // letters a step cannot move (those end at 40), so the same holds for them (degree 3, 200 paths of 129 points, 60
         // channels, 120 augmented: 8.72 -> 2.11 ms, 4.42 as library products; 100 x 129 x 64: 2.90 -> 1.14, 2.41).
-        const int64_t instance_waves = total_waves(geom, int64_t(batch));
+        const int64_t instance_waves = total_waves(geom_of(e, int(s.d_aug)), int64_t(batch));
         auto split = [&]() -> SplitPlan {
             if (g_force_segments > 0) return {int(std::min<uint64_t>(uint64_t(g_force_segments), s.L)), 0.0, 0.0};
             return choose_segments(instance_waves, int64_t(s.L), resident_waves(e), batch * (s.full_len - 1) * sizeof(T),
@@ -942,8 +1039,11 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
             const KernelEntry* run = pick_variant(false, e, instance_waves * plan.pieces, sparse_ll);
             by_rows = rows_fwd_seconds(s.d_aug, batch, s.L) < instance_fwd_seconds(run, plan, instance_waves, s.d_aug, s.L);
         }
-        int nseg = by_rows ? 1 : plan.pieces;
         const uint64_t n_coef = s.full_len - 1;
+        if (!by_rows)
+            plan = with_fine(e, pick_variant(false, e, instance_waves * plan.pieces, sparse_ll), plan, false, s.d_aug, degree, batch, s.L,
+                             batch * n_coef * sizeof(T), g_force_segments);
+        int nseg = by_rows ? 1 : plan.pieces;
         FwdParams p;
         p.batch = int64_t(batch) * nseg; p.L = int64_t(s.L); p.d = int(s.d_aug); p.stream = stream;
         p.lseg = (int64_t(s.L) + nseg - 1) / nseg;
@@ -966,7 +1066,7 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
                                                                  sizeof(T), "segment signatures")));
             p.out = segs; p.out_stride = int64_t(n_coef); p.scalar = 0;
         }
-        e = pick_variant(false, e, total_waves(geom, p.batch), sparse_ll);
+        e = pick_variant(false, e, total_waves(geom_of(e, int(s.d_aug)), p.batch), sparse_ll);
         // staged sweeps of plain narrow paths form the increments themselves while staging the points
         if (!by_rows && e->staged && !time_aug && !lead_lag && e->D > 0 && e->D <= kPointFedMaxDim && g_point_fed) {
             p.inc = path;
@@ -1285,7 +1385,6 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
         BwdParams p;
         p.sig = sig; p.gsig = sig_derivs; p.batch = int64_t(batch);
         p.L = int64_t(s.L); p.d = int(s.d_aug); p.sig_stride = int64_t(s.stride); p.scalar = sc; p.stream = stream;
-        const TreeGeom geom = make_geom(int(s.d_aug), e->N - e->tail, e->k, e->D != 0);
         const uint64_t n_coef = s.full_len - 1;
         const KernelEntry* ef = choose_entry(false, sizeof(T) == 8, s.d_aug, degree, batch, s.L);
         // lead-lag sweeps that skip the letters a step cannot move read a step's parity off its position in the
@@ -1298,7 +1397,7 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
         // the matrix form of single precision competes with it, the estimates decide (64 paths of 200 steps, 40 channels
         // 0.328 -> 0.234 ms, 16 x 200, 36: 0.340 -> 0.121); at degree 4 and 40 channels its tiles are 39 % filled: 4.6 -> 6.0
         // ms.  Lead-lag paths are left to the instances that skip their still letters.
-        const int64_t instance_waves = total_waves(geom, int64_t(batch));
+        const int64_t instance_waves = total_waves(geom_of(e, int(s.d_aug)), int64_t(batch));
         auto split = [&]() -> SplitPlan {
             if (arena || !ef || degree > uint64_t(kCombMaxLevels)) return {1, 0.0, 0.0};
             if (g_force_bwd_segments > 0) return {int(std::min<uint64_t>(uint64_t(g_force_bwd_segments), s.L)), 0.0, 0.0};
@@ -1319,6 +1418,9 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
         SplitPlan plan{1, 0.0, 0.0};
         if (!by_rows || compare) plan = split();
         if (compare && by_rows) by_rows = rows_bwd_seconds(s.d_aug, batch, s.L) < instance_bwd_seconds(plan, s.d_aug);
+        if (!by_rows && !arena)
+            plan = with_fine(e, pick_variant(true, e, instance_waves * plan.pieces, sparse_ll), plan, true, s.d_aug, degree, batch, s.L,
+                             batch * n_coef * sizeof(T), g_force_bwd_segments, !ef || degree > uint64_t(kCombMaxLevels));
         int nseg = by_rows ? 1 : plan.pieces;
         int64_t lseg = int64_t(s.L);
         if (nseg > 1) {
@@ -1328,7 +1430,7 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
         }
         // Whole-path staged sweeps of plain narrow paths form the increments themselves while staging the points: no
         // pre-pass launch, so the accumulator comes from the pair that takes turns (cleared by the previous call).
-        const KernelEntry* e_run = pick_variant(true, e, total_waves(geom, int64_t(batch) * nseg), sparse_ll);
+        const KernelEntry* e_run = pick_variant(true, e, total_waves(geom_of(e, int(s.d_aug)), int64_t(batch) * nseg), sparse_ll);
         const bool point_fed = !arena && !by_rows && nseg == 1 && e_run->staged && !time_aug && !lead_lag && e_run->D > 0 &&
                                e_run->D <= kPointFedMaxDim && g_point_fed != 0;
         // by rows in single precision: the increment gradient is summed in double precision, and rounded where the path
@@ -1381,8 +1483,9 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
             FwdParams f;
             f.inc = inc; f.batch = int64_t(rows); f.L = int64_t(s.L); f.d = int(s.d_aug); f.stream = stream;
             f.lseg = lseg; f.nseg = nseg; f.out = segs; f.out_stride = n; f.scalar = 0;
-            const TreeGeom fgeom = make_geom(int(s.d_aug), ef->N - ef->tail, ef->k, ef->D != 0);
-            ef = pick_variant(false, ef, total_waves(fgeom, f.batch), sparse_ll);
+            const KernelEntry* ef_now = pick_variant(false, ef, total_waves(geom_of(ef, int(s.d_aug)), f.batch), sparse_ll);
+            with_fine(ef, ef_now, SplitPlan{1, 0.0, 0.0}, false, s.d_aug, degree, rows, uint64_t(lseg), 0, 0, /*whole_only=*/true);
+            ef = pick_variant(false, ef, total_waves(geom_of(ef, int(s.d_aug)), f.batch), sparse_ll);
             SIG_HIP((sparse_ll && ef->staged && ef->fwd_lead_lag) ? ef->fwd_lead_lag(f) : ef->fwd(f));
             // both scans by doubling: ceil(log2(nseg)) launches, ping-ponging between two scratch copies
             int steps = 0;
@@ -1620,6 +1723,7 @@ CUSIG_AMD_API void cusig_amd_set_lead_lag_sparse(int on) noexcept { if (g_test_h
 
 CUSIG_AMD_API void cusig_amd_force_bwd_segments(int segments) noexcept { if (g_test_hooks) g_force_bwd_segments = segments; }
 
+CUSIG_AMD_API void cusig_amd_set_fine(int mode) noexcept { if (g_test_hooks) g_fine = mode; }
 CUSIG_AMD_API int cusig_amd_last_sweep_on_matrix_units(void) noexcept { return tl_matrix_form; }
 CUSIG_AMD_API void cusig_amd_set_rows_backward(int mode) noexcept { if (g_test_hooks) g_rows_backward = mode; }
 CUSIG_AMD_API void cusig_amd_set_rows_forward(int mode) noexcept { if (g_test_hooks) g_rows_forward = mode; }
@@ -1660,6 +1764,7 @@ CUSIG_AMD_API void cusig_amd_enable_test_hooks(int enabled) noexcept
     g_point_fed = 1;
     g_lead_lag_sparse = 1;
     g_force_bwd_segments = 0;
+    g_fine = 1;
     g_rows_backward = 1;
     g_rows_forward = 1;
     g_force_staged = -1;

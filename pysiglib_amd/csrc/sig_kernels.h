@@ -24,11 +24,11 @@ __device__ __forceinline__ void static_for(F&& f)
 // ---------------------------------------------------------------------------
 // Lane set-up shared by both sweeps.
 // ---------------------------------------------------------------------------
-template <typename T, int D, int N, int TAIL, int K>
+template <typename T, int D, int N, int TAIL, int K, bool ZL>
 struct LaneCtx {
     using Tr = Tree<T, D, N, TAIL, K>;
     static constexpr int M = Tr::M;
-    static constexpr bool WIDE = D > 0 ? ipow64(D > 0 ? D : 1, M) >= 48 : D < 0;
+    static constexpr bool WIDE = ZL ? true : D > 0 ? ipow64(D > 0 ? D : 1, M) >= 48 : D < 0;
     static constexpr bool kWholeGroups = D > 0 && D % K == 0;     // no letter group reaches past the row
     static constexpr bool kRunTimeWide = D < 0;
     int d;
@@ -40,7 +40,7 @@ struct LaneCtx {
     __device__ __forceinline__ void init(int d_rt, int64_t batch, bool xcd = true)
     {
         d = D > 0 ? D : d_rt;
-        G = make_geom(d, M, K, D != 0);
+        G = make_geom(d, M, K, layout_of(D, ZL));
         id = lane_id<WIDE>(G, batch, xcd);
         // idle lanes shadow a valid lane so that every load stays in bounds;
         // they never store and never contribute
@@ -386,9 +386,9 @@ __global__ __launch_bounds__(kBlock) void tree_fwd_kernel(
     // that piece in row vb of `out`.  nseg == 1 is the plain whole-path sweep.
     using Tr = Tree<T, D, N, TAIL, K>;
     constexpr int M = Tr::M;
-    LaneCtx<T, D, N, TAIL, K> cx;
+    LaneCtx<T, D, N, TAIL, K, ZL> cx;
     cx.init(d_rt, batch);
-    if constexpr (LaneCtx<T, D, N, TAIL, K>::WIDE) {
+    if constexpr (LaneCtx<T, D, N, TAIL, K, ZL>::WIDE) {
         if (cx.id.b >= batch) return;   // uniform: the whole wave is past the batch
     }
     const int d = cx.d;
@@ -409,7 +409,7 @@ __global__ __launch_bounds__(kBlock) void tree_fwd_kernel(
         else S.template fwd_step<LeadLagLetters<Tr::DD, decltype(pos)::value, decltype(g0c)::value>>(z);
     };
     if constexpr (ZL) {
-        static_assert(LaneCtx<T, D, N, TAIL, K>::WIDE, "staged increments need the wide layout");
+        static_assert(LaneCtx<T, D, N, TAIL, K, ZL>::WIDE, "staged increments need the wide layout");
         extern __shared__ double lds_raw_f[];
         T* lds_wave = reinterpret_cast<T*>(lds_raw_f) + (threadIdx.x >> 6) * IncRing<T, Tr::DD, 1>::ELEMS;
         constexpr int NG = (Tr::DD + K - 1) / K;
@@ -423,7 +423,7 @@ __global__ __launch_bounds__(kBlock) void tree_fwd_kernel(
             sweep_staged<1, -1, Tr>(cx, row, t0, ns, lds_wave, step, points);
         }
     } else {
-        sweep_direct<1, true, LaneCtx<T, D, N, TAIL, K>, typename Tr::Inc>(cx, row, t0, ns, step);
+        sweep_direct<1, true, LaneCtx<T, D, N, TAIL, K, ZL>, typename Tr::Inc>(cx, row, t0, ns, step);
     }
 
     if (!cx.id.active) return;
@@ -562,7 +562,7 @@ __global__ __launch_bounds__(kBlock) void tree_bwd_kernel(
     // (last) segment, which walk into the previous segment, are dead: their gradient is not emitted.
     using Tr = Tree<T, D, N, TAIL, K>;
     using Ad = TreeAdj<T, D, N, TAIL, K>;
-    using Cx = LaneCtx<T, D, N, TAIL, K>;
+    using Cx = LaneCtx<T, D, N, TAIL, K, ZL>;
     constexpr int M = Tr::M;
     extern __shared__ double lds_raw[];
     T* lds = reinterpret_cast<T*>(lds_raw);

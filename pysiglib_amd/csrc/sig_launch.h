@@ -22,7 +22,7 @@ template <typename T, int D, int N, int TAIL, int K, bool ZL, int LL = 0>
 hipError_t launch_tree_fwd(const FwdParams& p)
 {
     if (LL != 0 && ((p.lseg & 1) || p.from_points)) return hipErrorInvalidConfiguration;    // ranges must start on even steps
-    const TreeGeom g = make_geom(p.d, N - TAIL, K, D != 0);
+    const TreeGeom g = make_geom(p.d, N - TAIL, K, layout_of(D, ZL));
     if (D < 0 && !g.wide) return hipErrorInvalidConfiguration;     // the kernel was compiled for the wide layout
     const int64_t waves = total_waves(g, p.batch);
     const int64_t blocks = (waves + kWavesPerBlock - 1) / kWavesPerBlock;
@@ -55,12 +55,15 @@ int fwd_waves_per_simd()
     return blocks < 1 ? 1 : blocks;
 }
 
-// resident waves per SIMD of the backward kernel (register-limited; its LDS tiles never limit below that)
+// resident waves per SIMD of the backward kernel (registers and, of the staged ones, LDS tile and ring)
 template <typename T, int D, int N, int TAIL, int K, bool ZL>
 int bwd_waves_per_simd()
 {
     int blocks = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, tree_bwd_kernel<T, D, N, TAIL, K, ZL>, kBlock, 0) != hipSuccess) {
+    size_t lds = 0;
+    if constexpr (ZL && D > 0)
+        lds = size_t(kWavesPerBlock) * (size_t(RedPlan<T, D, TAIL, K, ZL>::tile_elems(D)) + IncRing<T, D, -1>::ELEMS) * sizeof(T);
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, tree_bwd_kernel<T, D, N, TAIL, K, ZL>, kBlock, lds) != hipSuccess) {
         (void)hipGetLastError();
         return 1;
     }
@@ -74,7 +77,7 @@ hipError_t launch_tree_bwd(const BwdParams& p)
     // the lead-lag sweep reads a step's parity off its position in the range: ranges must be even and start even
     if (LL != 0 && ((p.L & 1) || (p.nseg > 1 && (p.lseg & 1)) || p.from_points)) return hipErrorInvalidConfiguration;
     if (p.from_points && !(ZL && D > 0 && D <= kPointFedMaxDim)) return hipErrorInvalidConfiguration;
-    const TreeGeom g = make_geom(p.d, N - TAIL, K, D != 0);
+    const TreeGeom g = make_geom(p.d, N - TAIL, K, layout_of(D, ZL));
     if (D < 0 && !g.wide) return hipErrorInvalidConfiguration;     // the kernel was compiled for the wide layout
     const int64_t waves = total_waves(g, p.batch);
     const int64_t blocks = (waves + kWavesPerBlock - 1) / kWavesPerBlock;

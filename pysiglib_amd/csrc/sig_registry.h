@@ -54,6 +54,7 @@ struct KernelEntry {
     // backward instances (staged, and scalar-fed ones with a subtree level below the lane's own letters): likewise; needs
     // an even number of steps per path and an even BwdParams::lseg.
     BwdFn bwd_lead_lag = nullptr;
+    int fine = 0;              // 1: a partition of its shape for launches that leave SIMDs without work (staged, no scalar-fed twin)
 };
 
 // every generated instance file contributes one array

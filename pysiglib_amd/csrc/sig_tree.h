@@ -60,7 +60,8 @@ __device__ __forceinline__ float fmadd<float>(float a, float b, float c) { retur
 // Launch geometry shared by host and device.
 //   wide:   the prefixes of one path fill whole waves; lane order is group-major
 //           with the prefix range padded to a multiple of 64, so path index and
-//           group are wave-uniform (increments become scalar loads).
+//           group are wave-uniform (increments become scalar loads).  Taken from
+//           48 prefixes on, and by every kernel that stages its increments.
 //   packed: lanes of one path are contiguous (prefix-major, group fastest);
 //           if a path needs <= 64 lanes several whole paths share a wave,
 //           otherwise a path takes ceil(lanes/64) waves.
@@ -74,12 +75,15 @@ struct TreeGeom {
     int64_t wpp;        // waves per path when a path spans waves, else 1
 };
 
-__host__ __device__ inline TreeGeom make_geom(int d, int m, int k, bool allow_wide)
+enum Layout { kPackedLayout, kAnyLayout, kWideLayout };      // any: wide from 48 prefixes on
+__host__ __device__ constexpr Layout layout_of(int D, bool staged) { return staged ? kWideLayout : D != 0 ? kAnyLayout : kPackedLayout; }
+
+__host__ __device__ inline TreeGeom make_geom(int d, int m, int k, Layout layout)
 {
     TreeGeom g;
     g.P = ipow64(d, m);
     g.ng = (d + k - 1) / k;
-    g.wide = allow_wide && g.P >= 48;   // must agree with the kernel's compile-time choice
+    g.wide = layout == kWideLayout || (layout == kAnyLayout && g.P >= 48);   // must agree with the kernel's compile-time choice
     if (g.wide) {
         g.p_pad = (g.P + kWave - 1) / kWave * kWave;
         g.lpp = g.ng * g.p_pad;

@@ -1547,3 +1547,44 @@ def test_degrees_beyond_sixteen_at_their_own_dispatch(P, oracle, shape, scalar_t
     off = 1 if scalar_term else 0
     assert level_rel_err(fwd.cpu().numpy()[:, off:], ref[:, off:], d, deg) <= 1e-10, shape
     assert bwd_rel_err(got, want) <= 1e-10, shape
+
+
+@pytest.mark.parametrize("d,deg", [(2, 4), (2, 9), (3, 4), (3, 7), (4, 3), (4, 6), (5, 5), (7, 3), (10, 4), (13, 3), (16, 3), (17, 3)])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_fine_partitions_vs_oracle(P, oracle, d, deg, dtype):
+    """The second partition of a shape (many light lanes a path, wide layout also with a few prefixes), forced wherever one is
+    compiled: one step, both sides of a 16-step chunk of the ring and of the reduction tile, several time pieces, every
+    augmentation."""
+    import ctypes
+    from pysiglib_amd import _loader as L
+    L.CUSIG.cusig_amd_set_fine.argtypes = (ctypes.c_int,)
+    L.CUSIG.cusig_amd_set_fine.restype = None
+    for hook in (L.CUSIG.cusig_amd_force_segments, L.CUSIG.cusig_amd_force_bwd_segments):
+        hook.argtypes = (ctypes.c_int,)
+        hook.restype = None
+    rng = np.random.default_rng(100 * d + deg)
+    tol = TOL[dtype]
+    try:
+        L.CUSIG.cusig_amd_set_fine(2)
+        for aug in ({}, dict(time_aug=True), dict(lead_lag=True), dict(time_aug=True, lead_lag=True)):
+            raw = d - (1 if "time_aug" in aug else 0)
+            if "lead_lag" in aug:
+                raw //= 2
+            if raw < 1:
+                continue
+            for batch, length, pieces in ((1, 2, 0), (3, 16, 0), (2, 17, 0), (2, 34, 0), (2, 70, 4)):
+                x = (np.cumsum(rng.standard_normal((batch, length, raw)), axis=1) / np.sqrt(length * raw)).astype(dtype)
+                L.CUSIG.cusig_amd_force_segments(pieces)
+                L.CUSIG.cusig_amd_force_bwd_segments(pieces)
+                ref = oracle.signature(x.astype(np.float64), deg, n_jobs=-1, **aug)
+                d_aug = (2 * raw if "lead_lag" in aug else raw) + (1 if "time_aug" in aug else 0)
+                got = P.sig(dev(x), deg, **aug).cpu().numpy()
+                assert np.max(level_rel_err(got, ref, d_aug, deg)) < tol
+                g = rng.standard_normal(ref.shape).astype(dtype)
+                want = oracle.sig_backprop(x.astype(np.float64), ref, g.astype(np.float64), deg, n_jobs=-1, **aug)
+                back = P.sig_backprop(dev(x), dev(ref.astype(dtype)), dev(g), deg, **aug).cpu().numpy()
+                assert bwd_rel_err(back, want) < tol
+    finally:
+        L.CUSIG.cusig_amd_set_fine(1)
+        L.CUSIG.cusig_amd_force_segments(0)
+        L.CUSIG.cusig_amd_force_bwd_segments(0)
