@@ -481,10 +481,19 @@ struct RedPlan {
     // wave): without it every lane of a wave would add into the same few LDS words.
     static constexpr int kRowsWide = 2 * kRows + 2;
     __host__ __device__ static constexpr int rows_per_step(int d) { return PAIR ? (d + 1) / 2 : d; }
-    // steps per chunk of the tile; 0: the path is too wide for the tile
+    // Steps per chunk of the tile; 0: the path is too wide for the tile.  A flush sums two halves of every row, one a lane: staged
+    // sweeps fill the 64 lanes once (32 rows), which leaves a small tile and so more blocks to a CU; single precision of 17 .. 21
+    // channels, whose one step would fill two thirds of them, twice.  Against tiles of 16 KB in any case, single precision, ns a step at 1 /
+    // 8 waves per SIMD: 7 channels, degree 5 (2 levels x 7) 648 / 2789 -> 618 / 2381, (2 x 2) 536 / 2352 -> 511 / 1722; 10, degree 6 (2 x 5)
+    // 804 / 3367 -> 756 / 3221; 13, degree 4 (1 x 13) 572 / 2642 -> 528 / 2247; 17, degree 4 (2 x 6) with a single step a chunk 998 / 4390
+    // -> 1165 / 5064.
     __host__ __device__ static constexpr int steps(int d)
     {
         const int r = rows_per_step(d);
+        if (ZL && r <= 32) {
+            const int once = 32 / r;
+            return sizeof(T) == 4 && once * r < 22 && r > 8 ? 64 / r : once > 16 ? 16 : once;
+        }
         return r > kRowsWide ? 0 : r > kRows ? 1 : (kRows / r > 8 ? 8 : kRows / r);
     }
     __host__ __device__ static constexpr int64_t tile_elems(int d) { return int64_t(steps(d)) * rows_per_step(d) * kRedStride; }
