@@ -32,7 +32,12 @@ def check_n_jobs(n_jobs):
         raise ValueError("n_jobs cannot be 0")
 
 
+_TORCH_DTYPES = frozenset((torch.float32, torch.float64))
+
+
 def check_dtype(arr, name):
+    if isinstance(arr, torch.Tensor) and arr.dtype in _TORCH_DTYPES:
+        return
     if arr.dtype not in SUPPORTED:
         raise TypeError(name + ".dtype must be float32 or float64, got " + str(arr.dtype) + " instead")
 
@@ -47,8 +52,7 @@ def own_contiguous(arr):
     """Views, non-contiguous and stride-0 arrays are cloned (one warning per session)."""
     global _warned
     if isinstance(arr, torch.Tensor):
-        needs = arr._base is not None or not arr.is_contiguous() or any(s == 0 for s in arr.stride())
-        if needs:
+        if arr._base is not None or not arr.is_contiguous() or 0 in arr.stride():
             if not _warned:
                 warnings.warn(_MESSAGE, stacklevel=4)
                 _warned = True

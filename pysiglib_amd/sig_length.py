@@ -1,10 +1,18 @@
 """Signature and log-signature sizes (pysiglib/sig_length.py:20-182)."""
+from functools import lru_cache
+
 from ._loader import CUSIG
 from .param_checks import check_non_neg, check_type
 
 
 def aug_dim(dimension, time_aug, lead_lag):
     return (2 * dimension if lead_lag else dimension) + (1 if time_aug else 0)
+
+
+@lru_cache(maxsize=256)
+def _full_length(d, degree):
+    """Coefficients of a signature with its leading 1; 0 where 64 bits do not hold the number."""
+    return int(CUSIG.cusig_amd_sig_length(d, degree))
 
 
 def sig_length(dimension, degree, *, time_aug=False, lead_lag=False, scalar_term=False):
@@ -19,7 +27,7 @@ def sig_length(dimension, degree, *, time_aug=False, lead_lag=False, scalar_term
     check_non_neg(degree, "degree")
     check_type(time_aug, "time_aug", bool)
     check_type(lead_lag, "lead_lag", bool)
-    out = int(CUSIG.cusig_amd_sig_length(aug_dim(dimension, time_aug, lead_lag), degree))
+    out = _full_length(aug_dim(dimension, time_aug, lead_lag), degree)
     if out == 0:
         raise ValueError("Integer overflow encountered in sig_length")
     return out - (0 if scalar_term else 1)
@@ -58,7 +66,11 @@ def log_sig_length(dimension, degree, *, time_aug=False, lead_lag=False):
     check_non_neg(degree, "degree")
     check_type(time_aug, "time_aug", bool)
     check_type(lead_lag, "lead_lag", bool)
-    d = aug_dim(dimension, time_aug, lead_lag)
+    return _lyndon_count(aug_dim(dimension, time_aug, lead_lag), degree)
+
+
+@lru_cache(maxsize=256)
+def _lyndon_count(d, degree):
     total = 0
     for i in range(1, degree + 1):
         total += sum(_mobius(i // x) * d ** x for x in range(1, i + 1) if i % x == 0) // i
