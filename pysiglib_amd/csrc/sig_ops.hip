@@ -11,6 +11,7 @@
 
 #include "../../include/cusig_amd.h"
 #include "sig_host.h"
+#include "sig_join_stream.h"
 #include "sig_kernels.h"
 #include "sig_chen_adjoint.h"
 
@@ -522,6 +523,84 @@ static void linear_sig_impl(const T* disp, T* out, uint64_t batch, uint64_t dime
     SIG_HIP(hipStreamSynchronize(stream));
 }
 
+// ---------------------------------------------------------------------------
+// an appended segment by the words' prefixes (sig_join_stream.h)
+// ---------------------------------------------------------------------------
+extern std::atomic<int> g_chen_adjoint_mode;      // test hook (defined in sig_api.hip): not 0 asks for the general kernels
+
+// Rows of 1024 coefficients and more.  Whole calls, us, general kernels / these, double precision unless noted (20 and 4096
+// rows of 4 letters, degree 4, 340 coefficients: forward 22 / 22 and 30 / 31, backward 39 / 49 and 92 / 100; 4096 x 10, 3: 38 / 33, 129 /
+// 101; 200 x 7, 4: 24 / 23, 66 / 51; 1024 x 10, 5: 526 / 347, 861 / 521; 100 x 90, 3, single: 214 / 133, 1038 / 207; 2 x 12, 6: 50 / 38, 671 /
+// 138; 1 x 2, 16: 26 / 25, 367 / 341).  A launch per level is too many for two letters of many rows: 1000 x 2, 12: backward
+// 312 / 331, but in single precision 376 / 299.
+static bool plan_join_words(JoinPlan& pl, uint64_t dimension, uint64_t degree, uint64_t n_coef, bool prepend)
+{
+    if (prepend || g_chen_adjoint_mode != 0 || g_chen_low_levels != 1 || g_force_wide_index != 0) return false;
+    if (dimension < 2 || dimension > kJoinMaxDim || degree < 2 || degree > uint64_t(kJoinMaxDegree) || n_coef < 1024 || n_coef > (uint64_t(1) << 27)) return false;
+    pl.degree = int(degree);
+    pl.d = uint32_t(dimension);
+    pl.dv = DivBy<uint32_t>(dimension);
+    uint64_t at = 0, size = 1;
+    pl.lo[0] = 0;
+    for (uint64_t t = 1; t <= degree + 1; ++t) {
+        pl.lo[t] = uint32_t(at);
+        if (t <= degree) size *= dimension;
+        at += size;
+    }
+    return true;
+}
+
+// whether entries of `d` to a word can be moved 16 bytes at a time: every row, level and chunk then starts on such a border
+template <typename T>
+static bool join_aligned(uint64_t d, const SigShape& s, std::initializer_list<const void*> rows)
+{
+    constexpr uint64_t V = 16 / sizeof(T);
+    if (d % V != 0 || s.off != 0 || s.stride % V != 0) return false;
+    for (const void* p : rows)
+        if (reinterpret_cast<uintptr_t>(p) % 16 != 0) return false;
+    return true;
+}
+
+template <typename T>
+static void launch_join_words(const JoinPlan& pl, const T* sig, const T* disp, T* out, uint64_t batch, const SigShape& s, hipStream_t stream)
+{
+    const uint32_t total = uint32_t(s.n_coef / pl.d);               // words with children: the empty one and levels below the top
+    const uint32_t words = uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(kBlock, 4096 / pl.d)));
+    const dim3 grid{(total + words - 1) / words, unsigned(std::min<uint64_t>(batch, 65535)), 1};
+    auto go = [&](auto vec) {
+        hipLaunchKernelGGL((join_words_kernel<T, decltype(vec)::value>), grid, dim3(kBlock), 0, stream, sig, disp, out, int64_t(batch), pl,
+                           words, total, int64_t(s.stride), s.off, s.off ? out : (T*)nullptr);
+    };
+    if (join_aligned<T>(pl.d, s, {sig, out})) go(IntC<int(16 / sizeof(T))>{});
+    else go(IntC<1>{});
+}
+
+// w: two arrays of batch * d^(degree-1) entries.  d_disp has been cleared.
+template <typename T>
+static void launch_join_words_bwd(const JoinPlan& pl, const T* d_out, T* d_sig, T* d_disp, const T* sig, const T* disp, uint64_t batch,
+                                  const SigShape& s, T* w0, T* w1, hipStream_t stream)
+{
+    const uint32_t pitch = pl.d | 1u;
+    const bool aligned = join_aligned<T>(pl.d, s, {d_out, d_sig, w0, w1});
+    uint32_t words = kBlock;            // at 256 channels still 8
+    while (words > 4 && size_t(words) * pitch * sizeof(T) > (size_t(24) << 10)) words /= 2;
+    T* from = w1;
+    T* to = w0;
+    for (int l = pl.degree - 1; l >= 0; --l) {
+        const uint32_t count = l ? pl.lo[l + 1] - pl.lo[l] : 1;
+        const int n_in = pl.degree - l - 1;
+        const dim3 grid{(count + words - 1) / words, unsigned(std::min<uint64_t>(batch, 65535)), 1};
+        const size_t lds = size_t(words) * pitch * sizeof(T) * (n_in ? 2 : 1);
+        auto go = [&](auto vec) {
+            hipLaunchKernelGGL((join_words_bwd_kernel<T, decltype(vec)::value>), grid, dim3(kBlock), lds, stream, d_out, sig, disp, d_sig,
+                               d_disp, (const T*)from, to, int64_t(batch), pl, l, n_in, count, words, pitch, int64_t(s.stride), s.off);
+        };
+        if (aligned) go(IntC<int(16 / sizeof(T))>{});
+        else go(IntC<1>{});
+        std::swap(from, to);
+    }
+}
+
 template <typename T>
 static void sig_join_impl(const T* sig, const T* disp, T* out, uint64_t batch, uint64_t dimension, uint64_t degree,
                           bool prepend, bool scalar_term)
@@ -535,6 +614,8 @@ static void sig_join_impl(const T* sig, const T* disp, T* out, uint64_t batch, u
         if (scalar_term)
             hipLaunchKernelGGL((fill_trivial_kernel<T>), dim3(grid_for(batch)), dim3(kBlock), 0, stream, out, int64_t(batch),
                                int64_t(1), 1);
+    } else if (JoinPlan words; plan_join_words(words, dimension, degree, s.n_coef, prepend)) {
+        launch_join_words<T>(words, sig, disp, out, batch, s, stream);
     } else {
         with_chen_fan(dimension, [&](auto fan) {
             constexpr int FAN = decltype(fan)::value;
@@ -576,6 +657,12 @@ static void sig_join_backprop_impl(const T* d_out, T* d_sig, T* d_disp, const T*
     std::lock_guard<std::mutex> lk(g_ws_mutex);
     T* E = static_cast<T*>(workspace(4, bytes));
     T* dE = static_cast<T*>(workspace(5, bytes));
+    if (JoinPlan words; !(dimension == 2 && sizeof(T) == 8 && batch > 256) && plan_join_words(words, dimension, degree, s.n_coef, prepend)) {
+        launch_join_words_bwd<T>(words, d_out, d_sig, d_disp, sig, disp, batch, s, E, dE, stream);
+        SIG_HIP(hipGetLastError());
+        SIG_HIP(hipStreamSynchronize(stream));
+        return;
+    }
     // exp(z) up to level degree - 1: the adjoint never multiplies with a factor's top level
     if (degree >= 2 && !launch_linear_sig_levels<T>(disp, E, batch, dimension, degree - 1, s.n_coef, int64_t(s.stride), s.off, stream))
         with_chen_fan(dimension, [&](auto fan) {

@@ -806,3 +806,30 @@ def test_log_sig_block_per_row_vs_general_form(P, d, deg, batch, method):
         L.CUSIG.cusig_amd_force_chen_adjoint(0)
         if method:
             P.clear_cache()
+
+
+@pytest.mark.parametrize("d,deg,batch", [(2, 10, 3), (3, 7, 2), (5, 5, 3), (10, 3, 2), (11, 3, 2), (16, 3, 2), (33, 2, 3), (64, 2, 2), (255, 2, 2),
+                                         (256, 2, 1), (257, 2, 1), (8, 4, 2)])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("scalar_term", [False, True])
+def test_sig_join_by_words_vs_oracle(P, oracle, d, deg, batch, dtype, scalar_term):
+    """Appended segments of rows of 1024 and more coefficients: channel counts either side of what 16-byte accesses, the odd
+    LDS pitch, the words of a block and the 256 channels of the form by prefixes allow, with and without the scalar slot
+    (which leaves the rows unaligned)."""
+    rng = np.random.default_rng(7 * d + deg)
+    n = oracle.sig_length(d, deg) - 1
+    scale = np.concatenate([np.full(d ** k, 0.5 / np.sqrt(float(d) ** k)) for k in range(1, deg + 1)])
+    a, g = (rng.standard_normal((batch, n)) * scale).astype(dtype), rng.standard_normal((batch, n)).astype(dtype)
+    z = (rng.standard_normal((batch, d)) * 0.5 / np.sqrt(d)).astype(dtype)
+    if scalar_term:
+        a = np.hstack([np.ones((batch, 1), dtype=dtype), a])
+        g = np.hstack([np.full((batch, 1), 3.0, dtype=dtype), g])
+    off = 1 if scalar_term else 0
+    want = oracle.sig_join(a.astype(np.float64), z.astype(np.float64), d, deg)
+    got = P.sig_join(dev(a), dev(z), d, deg).cpu().numpy()
+    assert got.dtype == dtype and row_rel_err(got, want) < TOL[dtype]
+    da, dz = oracle.sig_join_backprop(g.astype(np.float64), a.astype(np.float64), z.astype(np.float64), d, deg)
+    ga, gz = (v.cpu().numpy() for v in P.sig_join_backprop(dev(g), dev(a), dev(z), d, deg))
+    if scalar_term:
+        assert np.all(ga[:, 0] == 0)
+    assert row_rel_err(ga[:, off:], da[:, off:]) < TOL[dtype] and row_rel_err(gz, dz) < TOL[dtype]
