@@ -27,6 +27,7 @@
 #include "sig_deep.h"
 #include "sig_rows.h"
 #include "sig_degree2.h"
+#include "sig_degree2_waves.h"
 #include "sig_degree3.h"
 #include "sig_host.h"
 #include "sig_kernels.h"
@@ -739,6 +740,19 @@ static bool use_degree2(bool backward, uint64_t d_aug, uint64_t degree, uint64_t
     return backward || d_aug >= 12 || batch * 8 <= uint64_t(simd_count());
 }
 
+// The kernels of sig_degree2_waves.h, plain paths only.  Forward at any channel count, but beyond 48 channels not where few paths
+// would have to be cut into slices (their 64 x 64 sums then meet in 16-byte pieces of atomics: 1 x 8192 points x 64 channels
+// 32 -> 52 us, 16 x 4096: 39 -> 65), nor in double precision for fewer than 24 steps (4096 x 16 x 64: 67 -> 74).  Backward up to 48
+// channels: with 64 the registers of A leave too few waves (2048 x 256 x 64: 124 -> 143, double 190 -> 240).
+static bool degree2_by_waves(bool backward, uint64_t d, uint64_t L, uint64_t batch, size_t elem_bytes, bool augmented)
+{
+    if (augmented || g_degree2_staged == 0 || (L + 1) * d >= (uint64_t(1) << 31)) return false;
+    if (d <= 48) return true;
+    const uint64_t groups = (d + 63) / 64;
+    const bool sliced = batch * groups * groups * 4 < uint64_t(simd_count()) && L >= 128;
+    return !backward && !sliced && !(elem_bytes == 8 && L < 24);
+}
+
 // ---------------------------------------------------------------------------
 // degrees beyond the instance table: run-time-degree sweeps (sig_deep.hip)
 // ---------------------------------------------------------------------------
@@ -927,6 +941,43 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
                 hipLaunchKernelGGL((finite_rows_kernel<T>), dim3(grid_for(batch * s.stride)), dim3(kBlock), 0, stream, out,
                                    int64_t(batch * s.stride), flag);
         }
+    } else if (use_degree2(false, s.d_aug, degree, batch) && degree2_by_waves(false, s.d_aug, s.L, batch, sizeof(T), time_aug || lead_lag)) {
+        const int d = int(s.d_aug), groups = (d + 63) / 64, tn = (d + 16 * groups - 1) / (16 * groups);
+        // few paths: two blocks per CU through slices of the steps, at least 64 steps each, that add into the cleared output
+        const int64_t whole = int64_t(batch) * groups * groups;
+        int64_t slices = whole * 4 >= simd_count() ? 1 : std::min<int64_t>(simd_count() / (2 * whole), int64_t(s.L) / 64);
+        slices = std::max<int64_t>(slices, 1);
+        const int64_t slice_len = (int64_t(s.L) + slices - 1) / slices;
+        slices = (int64_t(s.L) + slice_len - 1) / slice_len;
+        const int64_t blocks = whole * slices;
+        if (blocks > 2147483647LL) throw std::runtime_error("signature_cuda: launch too large");
+        if (slices > 1)
+            hipLaunchKernelGGL((zero_kernel<T>), dim3(grid_for(batch * s.stride)), dim3(kBlock), 0, stream, out,
+                               int64_t(batch * s.stride));
+        MainKernelTimer timer(stream, sizeof(T) == 8 ? "degree2_fwd_f64_waves" : "degree2_fwd_f32_waves");
+        auto go = [&](auto tiles, auto same) {
+            constexpr int TN = decltype(tiles)::value;
+            auto run = [&](auto whole_pieces) {
+                hipLaunchKernelGGL((degree2_fwd_waves_kernel<T, TN, decltype(same)::value, decltype(whole_pieces)::value>), dim3(unsigned(blocks)),
+                                   dim3(kBlock), 0, stream, path, out, int64_t(length), d, int64_t(s.stride), sc, groups, int(slices), slice_len,
+                                   slices > 1 ? nullptr : flag);
+            };
+            if (d % TN == 0) run(std::true_type{});
+            else run(std::false_type{});
+        };
+        auto pick = [&](auto same) {
+            if (tn == 1) go(IntC<1>{}, same);
+            else if (tn == 2) go(IntC<2>{}, same);
+            else if (tn == 3) go(IntC<3>{}, same);
+            else go(IntC<4>{}, same);
+        };
+        if (groups == 1) pick(std::true_type{});
+        else if (tn <= 3) go(IntC<3>{}, std::false_type{});
+        else go(IntC<4>{}, std::false_type{});
+        timer.stop();
+        if (slices > 1 && flag)
+            hipLaunchKernelGGL((finite_rows_kernel<T>), dim3(grid_for(batch * s.stride)), dim3(kBlock), 0, stream, out,
+                               int64_t(batch * s.stride), flag);
     } else if (use_degree2(false, s.d_aug, degree, batch)) {
         const int d = int(s.d_aug);
         const int tiles = (d + 15) / 16, col_groups = (tiles + kDeg2Cols - 1) / kDeg2Cols;
@@ -1250,6 +1301,30 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
         SIG_HIP(hipGetLastError());
         finish();
         return;
+    } else if (!arena && use_degree2(true, s.d_aug, degree, batch) &&
+               degree2_by_waves(true, s.d_aug, s.L, batch, sizeof(T), time_aug || lead_lag)) {
+        lock_pool();        // (the timer's events)
+        const int d = int(s.d_aug), tn = (d + 15) / 16;
+        // two blocks per CU at least, of 64 rows (four waves of 16) and more each
+        const int64_t chunks = (int64_t(length) + 63) / 64;
+        int64_t parts = std::min<int64_t>(chunks, std::max<int64_t>(1, (simd_count() / 2 + int64_t(batch) - 1) / int64_t(batch)));
+        const int64_t part_rows = (chunks + parts - 1) / parts * 64;
+        parts = (int64_t(length) + part_rows - 1) / part_rows;
+        const int64_t blocks = int64_t(batch) * parts;
+        if (blocks > 2147483647LL) throw std::runtime_error("sig_backprop_cuda: launch too large");
+        MainKernelTimer timer(stream, sizeof(T) == 8 ? "degree2_bwd_f64_waves" : "degree2_bwd_f32_waves");
+        auto go = [&](auto tiles) {
+            auto run = [&](auto whole_pieces) {
+                hipLaunchKernelGGL((degree2_bwd_waves_kernel<T, decltype(tiles)::value, decltype(whole_pieces)::value>), dim3(unsigned(blocks)),
+                                   dim3(kBlock), 0, stream, path, sig_derivs, out, int64_t(length), d, int64_t(s.stride), sc, int(parts), part_rows);
+            };
+            if (d % 4 == 0) run(std::true_type{});
+            else run(std::false_type{});
+        };
+        if (tn == 1) go(IntC<1>{});
+        else if (tn == 2) go(IntC<2>{});
+        else go(IntC<3>{});
+        timer.stop();
     } else if (use_degree2(true, s.d_aug, degree, batch)) {
         lock_pool();
         const int d = int(s.d_aug);

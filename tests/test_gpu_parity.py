@@ -1588,3 +1588,27 @@ def test_fine_partitions_vs_oracle(P, oracle, d, deg, dtype):
         L.CUSIG.cusig_amd_set_fine(1)
         L.CUSIG.cusig_amd_force_segments(0)
         L.CUSIG.cusig_amd_force_bwd_segments(0)
+
+
+@pytest.mark.parametrize("d", [2, 3, 15, 16, 17, 31, 32, 33, 47, 48, 49, 50, 63, 64, 65, 97, 130])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_degree2_by_waves_vs_oracle(P, oracle, d, dtype):
+    """Degree 2 of plain paths: channel counts either side of the 16-channel tiles, of the 64-channel groups and of what the
+    pieces of a lane divide; one step, quarters of a wave that are empty, partly filled and full, more than one slice."""
+    rng = np.random.default_rng(d)
+    for batch, length in ((1, 2), (3, 3), (2, 6), (300, 17), (5, 18), (2, 66), (1, 131), (300, 40)):
+        x = (np.cumsum(rng.standard_normal((batch, length, d)), axis=1) / np.sqrt(length * d)).astype(dtype)
+        for scalar in (False, True):
+            ref = oracle.signature(x.astype(np.float64), 2, scalar_term=scalar, n_jobs=-1)
+            got = P.sig(dev(x), 2, scalar_term=scalar).cpu().numpy()
+            off = 1 if scalar else 0
+            assert np.max(level_rel_err(got[:, off:], ref[:, off:], d, 2)) < TOL[dtype]
+            assert not scalar or np.all(got[:, 0] == 1)
+            g = rng.standard_normal(ref.shape).astype(dtype)
+            want = oracle.sig_backprop(x.astype(np.float64), ref, g.astype(np.float64), 2, n_jobs=-1)
+            back = P.sig_backprop(dev(x), dev(ref.astype(dtype)), dev(g), 2).cpu().numpy()
+            assert bwd_rel_err(back, want) < TOL[dtype]
+    bad = dev(x).clone()
+    bad[-1, -1, -1] = float("nan")
+    with pytest.warns(RuntimeWarning):
+        assert not bool(torch.isfinite(P.sig(bad, 2)[-1]).all())
