@@ -614,9 +614,28 @@ static bool rows_bwd_mfma_wins(uint64_t d, uint64_t degree, uint64_t batch, uint
 // ---------------------------------------------------------------------------
 static Hook g_fine{1};      // test hook: 0 never, 1 by the estimates below, 2 wherever there is one
 
+// Cutting a path in pieces costs scratch for their signatures.  Where the finer partition cuts more often than the call would
+// be cut without it and the device cannot hold that, the call is served without it: it needs no more memory than it ever did.
+static thread_local bool tl_no_fine = false, tl_fine_more_pieces = false;
+template <typename F>
+static void fine_if_it_fits(F&& run)
+{
+    tl_fine_more_pieces = false;
+    try {
+        run();
+    } catch (const std::bad_alloc&) {
+        if (!tl_fine_more_pieces) throw;
+        struct Off {
+            Off() { tl_no_fine = true; }
+            ~Off() { tl_no_fine = false; }
+        } off;
+        run();
+    }
+}
+
 static const KernelEntry* fine_entry(bool backward, bool f64, uint64_t d, uint64_t degree)
 {
-    if (g_fine == 0 || g_force_tail > 0 || g_force_staged >= 0 || g_ignore_table != 0 || d > 0x7fffffff || degree > 0x7fffffff) return nullptr;
+    if (g_fine == 0 || tl_no_fine || g_force_tail > 0 || g_force_staged >= 0 || g_ignore_table != 0 || d > 0x7fffffff || degree > 0x7fffffff) return nullptr;
     const auto& m = backward ? table().fine_bwd : table().fine_fwd;
     auto it = m.find(std::make_tuple(int(f64), int(d), int(degree)));
     return it == m.end() ? nullptr : it->second;
@@ -696,6 +715,7 @@ static SplitPlan with_fine(const KernelEntry*& e, const KernelEntry* run_now, co
         }
     }
     if (g_fine != 2 && best.seconds > (backward ? 0.88 : 0.92) * StepModel(run_now, int(d), backward).sweep(paths, steps, now.pieces, sig_bytes_all_paths)) return now;
+    tl_fine_more_pieces = tl_fine_more_pieces || best.pieces > now.pieces;
     e = f;
     return best;
 }
@@ -1679,8 +1699,10 @@ static void signature_entry(const T* path, T* out, uint64_t batch, uint64_t dime
     split_on_bad_alloc(batch, "signature", [&](uint64_t first, uint64_t count) {
         uint64_t stride = 0;
         if (first) stride = make_shape(dimension, length, degree, time_aug, lead_lag, scalar_term).stride;
-        signature_impl<T>(path + first * length * dimension, out + first * stride, count, dimension, length, degree, time_aug,
-                          lead_lag, end_time, horner, scalar_term, correction, correction_len);
+        fine_if_it_fits([&] {
+            signature_impl<T>(path + first * length * dimension, out + first * stride, count, dimension, length, degree, time_aug,
+                              lead_lag, end_time, horner, scalar_term, correction, correction_len);
+        });
         const int f = tl_sig_nonfinite;
         nonfinite = (nonfinite < 0 || f < 0) ? -1 : (nonfinite | f);
     });
@@ -1695,9 +1717,11 @@ static void sig_backprop_entry(const T* path, T* out, const T* sig_derivs, const
     split_on_bad_alloc(batch, "sig_backprop", [&](uint64_t first, uint64_t count) {
         uint64_t stride = 0;
         if (first) stride = make_shape(dimension, length, degree, time_aug, lead_lag, scalar_term).stride;
-        sig_backprop_impl<T>(path + first * length * dimension, out + first * length * dimension, sig_derivs + first * stride,
-                             sig + first * stride, count, dimension, length, degree, time_aug, lead_lag, end_time, scalar_term,
-                             correction, correction_len);
+        fine_if_it_fits([&] {
+            sig_backprop_impl<T>(path + first * length * dimension, out + first * length * dimension, sig_derivs + first * stride,
+                                 sig + first * stride, count, dimension, length, degree, time_aug, lead_lag, end_time, scalar_term,
+                                 correction, correction_len);
+        });
     });
 }
 

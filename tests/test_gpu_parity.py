@@ -1590,6 +1590,33 @@ def test_fine_partitions_vs_oracle(P, oracle, d, deg, dtype):
         L.CUSIG.cusig_amd_force_bwd_segments(0)
 
 
+@pytest.mark.parametrize("d,deg,length,dtype", [(3, 7, 129, np.float32), (3, 7, 161, np.float64), (2, 10, 97, np.float64)])
+def test_finer_partitions_ask_for_no_memory_that_is_not_there(P, oracle, d, deg, length, dtype):
+    """One path that the finer partition cuts in pieces and the default sweeps whole: where the signatures of two pieces do not
+    fit, the call is served whole."""
+    L = _alloc_hooks()
+    rng = np.random.default_rng(deg)
+    x = (np.cumsum(rng.standard_normal((1, length, d)), axis=1) / np.sqrt(length * d)).astype(dtype)
+    ref = oracle.signature(x.astype(np.float64), deg, n_jobs=-1)
+    g = rng.standard_normal(ref.shape).astype(dtype)
+    want = oracle.sig_backprop(x.astype(np.float64), ref, g.astype(np.float64), deg, n_jobs=-1)
+    P.sig(dev(x), deg)
+    assert L.CUSIG.cusig_amd_last_segments() > 1        # otherwise the shape shows nothing
+    retries = L.CUSIG.cusig_amd_alloc_retries()
+    try:
+        L.CUSIG.cusig_shutdown()                        # grown workspaces would hide the limit
+        L.CUSIG.cusig_amd_set_alloc_limit(2 * ref.size * np.dtype(dtype).itemsize - 1)
+        got = P.sig(dev(x), deg).cpu().numpy()
+        assert L.CUSIG.cusig_amd_last_segments() == 1
+        back = P.sig_backprop(dev(x), dev(ref.astype(dtype)), dev(g), deg).cpu().numpy()
+    finally:
+        L.CUSIG.cusig_amd_set_alloc_limit(0)
+    assert L.CUSIG.cusig_amd_alloc_retries() == retries
+    assert np.max(level_rel_err(got, ref, d, deg)) < TOL[dtype] and bwd_rel_err(back, want) < TOL[dtype]
+    P.sig(dev(x), deg)
+    assert L.CUSIG.cusig_amd_last_segments() > 1
+
+
 @pytest.mark.parametrize("d", [2, 3, 15, 16, 17, 31, 32, 33, 47, 48, 49, 50, 63, 64, 65, 97, 130])
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 def test_degree2_by_waves_vs_oracle(P, oracle, d, dtype):
