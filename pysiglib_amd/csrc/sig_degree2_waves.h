@@ -54,7 +54,8 @@ __global__ __launch_bounds__(kBlock, TN < 4 ? 1 : sizeof(T) == 8 ? 2 : SAME ? 4 
     const int64_t w_begin = t_begin + wave * quarter < t_end ? t_begin + wave * quarter : t_end;
     const int64_t w_end = w_begin + quarter < t_end ? w_begin + quarter : t_end;
     const uint32_t mine = uint32_t(w_end - w_begin), steps = (mine + 3) / 4;   // of the wave, of a lane group; past the wave's last
-    const uint32_t first = uint32_t(lk) * steps;                               // step points repeat and increments are zero
+    const uint32_t first = uint32_t(lk) * steps;                               // step points repeat and operands are zero (also
+    const uint32_t past = first + steps < mine ? first + steps : mine;         // where the repeated point is infinite)
     const T* xw = x + w_begin * d;
 
     const int ra = rg * W + TN * li, ca = cg * W + TN * li;
@@ -106,11 +107,12 @@ __global__ __launch_bounds__(kBlock, TN < 4 ? 1 : sizeof(T) == 8 ? 2 : SAME ? 4 
 #pragma unroll
         for (int k = 0; k < AHEAD; ++k) {
             const P& cp = SAME ? r1[k] : c1[SAME ? 0 : k];
+            const bool live = first + s + k < past;
             T u[TN], z[TN];
 #pragma unroll
             for (int q = 0; q < TN; ++q) {
-                u[q] = T(0.5) * (r0.v[q] + r1[k].v[q]) - x0.v[q];
-                z[q] = cp.v[q] - c0.v[q];
+                u[q] = live ? T(0.5) * (r0.v[q] + r1[k].v[q]) - x0.v[q] : T(0);
+                z[q] = live ? cp.v[q] - c0.v[q] : T(0);
             }
 #pragma unroll
             for (int i = 0; i < TN; ++i)
@@ -188,7 +190,7 @@ __global__ __launch_bounds__(kBlock, TN < 4 ? 1 : sizeof(T) == 8 ? 2 : SAME ? 4 
 // the channel 16 q + 4 lk + e) and holds four consecutive channels of one row of every result tile.  Nothing but A and h goes
 // through LDS and the four waves of a block run on their own.  Whole calls, us, single / double precision, before -> now: 1000 x 200 x
 // 48: 64 -> 48, 89 -> 65; 1000 x 200 x 32: 113 -> 37, 122 -> 48; 4000 x 100 x 16: 97 -> 33, 115 -> 44.  WHOLE: 4 divides d, pieces are all there or past the last
-// channel (there they repeat the last piece, against zeros of A).
+// channel (there they repeat the last piece and are set to zero).
 template <typename T, int TN, bool WHOLE>
 __global__ __launch_bounds__(kBlock, 2) void degree2_bwd_waves_kernel(
     const T* __restrict__ path, const T* __restrict__ gsig, T* __restrict__ out, int64_t len_raw, int d, int64_t sig_stride, int scalar,
@@ -285,6 +287,9 @@ __global__ __launch_bounds__(kBlock, 2) void degree2_bwd_waves_kernel(
                     u[4 * q + e] = t == last_row ? v : u[4 * q + e];
                 }
         }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)             // channels past the last, all in the last tile
+            u[4 * (TN - 1) + e] = 16 * (TN - 1) + 4 * lk + e < d ? u[4 * (TN - 1) + e] : T(0);
         if (row0 + 64 < end) fetch(row0 + 64, lo, hi);
         typename M::Acc acc[TN];
 #pragma unroll

@@ -1639,3 +1639,27 @@ def test_degree2_by_waves_vs_oracle(P, oracle, d, dtype):
     bad[-1, -1, -1] = float("nan")
     with pytest.warns(RuntimeWarning):
         assert not bool(torch.isfinite(P.sig(bad, 2)[-1]).all())
+
+
+@pytest.mark.parametrize("d", [13, 17, 33, 47])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_degree2_by_waves_infinite_last_point(P, d, dtype):
+    """An infinite coordinate at the end of a path stays infinite in the products it takes part in: the idle steps of a wave
+    and the channels that fill up its last tile add nothing, not even 0 * infinity."""
+    rng = np.random.default_rng(d)
+    for length in (2, 6, 19, 66):
+        x = np.cumsum(rng.standard_normal((300, length, d)), axis=1).astype(dtype)
+        x[:, -1, d - 1] = np.inf
+        z, mid = np.diff(x, axis=1), 0.5 * (x[:, 1:] + x[:, :-1]) - x[:, :1]
+        want = np.concatenate([x[:, -1] - x[:, 0], (mid[:, :, :, None] * z[:, :, None, :]).sum(1).reshape(300, -1)], axis=1)
+        with pytest.warns(RuntimeWarning):
+            got = P.sig(dev(x), 2).cpu().numpy()
+        odd = ~np.isfinite(want)
+        np.testing.assert_array_equal(got[odd], want[odd])
+        np.testing.assert_array_equal(np.isfinite(got), ~odd)
+        g = rng.standard_normal(want.shape).astype(dtype)
+        back = P.sig_backprop(dev(x), dev(want.astype(dtype)), dev(g), 2).cpu().numpy()
+        # rows that neither border the infinite point nor hold an end of the path do not see it
+        assert np.isfinite(back[:, 1:-2]).all()
+        if length > 3:
+            assert np.isinf(back[:, -2, : d - 1]).all()         # X_{t-1} - X_{t+1} times A, whose diagonal is zero
