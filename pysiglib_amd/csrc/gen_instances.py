@@ -59,7 +59,14 @@ STAGE_POLICY = {
 # Partitions and feeds found by a sweep on MI355X (every partition within the register budget whose lane count and
 # letter waste are reasonable, both feeds, at a throughput workload: batch ~3e7 / d^N paths of 128 points): entries
 # that beat the model's choice by at least 12 %.  "staged": 1 always, 3 only when the launch is under-filled.
-# "ms": kernel time of the model's choice and of the entry.  Hand entries above take precedence.
+# "ms": kernel time of the model's choice and of the entry.  Hand entries above take precedence.  "fine": the partition that
+# serves launches of few paths instead (backward of 129 points: 10 channels, degree 6, single precision, 2 levels x 10 letters /
+# 2 x 5: 30 paths 0.45 / 0.60 ms, 3 paths 138 / 119 us; 9 channels, degree 5, double precision, 2 x 5 / 2 x 3: 508 paths 1.02 /
+# 0.97 ms, 50 paths 175 / 126 us).  Backward entries measured with tiles that fill 64 lanes once (sig_kernels.h: RedPlan), which
+# left the staged sweeps ahead of the scalar-fed ones in double precision at degree 6 of 9 to 12 channels; shapes where one
+# augmentation or a range of batches lost with the winner keep what they had (7 channels, degree 5, double precision, 2 x 7 in
+# place of 3 x 1: plain 0.86 of the time, lead-lag with time 1.2).
+FINE = {}
 _TUNED = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuned_partitions.json")
 if os.path.exists(_TUNED):
     import json
@@ -70,6 +77,8 @@ if os.path.exists(_TUNED):
             if _key not in OVERRIDES:
                 OVERRIDES[_key] = tuple(_v["partition"])
                 STAGE_POLICY[_key] = int(_v["staged"])
+                if "fine" in _v:
+                    FINE[_key] = tuple(_v["fine"])
 
 # additional partitions compiled next to the default one (selectable through
 # cusig_amd_force_partition; used for tuning sweeps): (dtype, D, N, dir) -> [(TAIL, K), ...]
@@ -168,6 +177,8 @@ def fine_partition(D, N, dtype, direction):
         return None
     if direction == "bwd" and rows_sweep_wins(dtype, D, N):
         return None
+    if (dtype, D, N, direction) in FINE:
+        return FINE[(dtype, D, N, direction)]
 
     def waves(tail, K, wide):
         P, groups = D ** (N - tail), -(-D // K)

@@ -1549,7 +1549,7 @@ def test_degrees_beyond_sixteen_at_their_own_dispatch(P, oracle, shape, scalar_t
     assert bwd_rel_err(got, want) <= 1e-10, shape
 
 
-@pytest.mark.parametrize("d,deg", [(2, 4), (2, 9), (3, 4), (3, 7), (4, 3), (4, 6), (5, 5), (7, 3), (10, 4), (13, 3), (16, 3), (17, 3)])
+@pytest.mark.parametrize("d,deg", [(2, 4), (2, 9), (3, 4), (3, 7), (4, 3), (4, 6), (5, 5), (7, 3), (9, 5), (10, 4), (13, 3), (16, 3), (17, 3)])
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 def test_fine_partitions_vs_oracle(P, oracle, d, deg, dtype):
     """The second partition of a shape (many light lanes a path, wide layout also with a few prefixes), forced wherever one is
@@ -1663,3 +1663,34 @@ def test_degree2_by_waves_infinite_last_point(P, d, dtype):
         assert np.isfinite(back[:, 1:-2]).all()
         if length > 3:
             assert np.isinf(back[:, -2, : d - 1]).all()         # X_{t-1} - X_{t+1} times A, whose diagonal is zero
+
+
+@pytest.mark.parametrize("dtype,d,deg,tail,k", [
+    (np.float64, 5, 7, 2, 5), (np.float64, 6, 5, 2, 6),
+    (np.float64, 7, 6, 2, 7), (np.float64, 9, 6, 2, 5), (np.float64, 10, 6, 2, 5),
+    (np.float64, 11, 6, 2, 4), (np.float64, 12, 6, 2, 4), (np.float32, 10, 6, 2, 10), (np.float32, 17, 5, 2, 6)])
+def test_staged_backward_partitions_vs_oracle(P, oracle, dtype, d, deg, tail, k):
+    """Shapes whose LDS-staged backward partition is the default on a full chip: one step, both sides of a chunk of the ring
+    and of the reduction tile, lead-lag."""
+    import ctypes
+    from pysiglib_amd import _loader as L
+    L.CUSIG.cusig_amd_force_partition.argtypes = (ctypes.c_int, ctypes.c_int)
+    L.CUSIG.cusig_amd_force_partition.restype = None
+    rng = np.random.default_rng(10 * d + deg)
+    try:
+        L.CUSIG.cusig_amd_set_profiling(1)
+        for batch, length, aug in ((2, 2, {}), (1, 16, {}), (2, 18, {}), (1, 35, dict(time_aug=d % 2 == 1, lead_lag=True))):
+            raw = (d - d % 2) // 2 if aug else d
+            x = (np.cumsum(rng.standard_normal((batch, length, raw)), axis=1) / np.sqrt(length * raw)).astype(dtype)
+            ref = oracle.signature(x.astype(np.float64), deg, n_jobs=-1, **aug)
+            g = rng.standard_normal(ref.shape).astype(dtype)
+            want = oracle.sig_backprop(x.astype(np.float64), ref, g.astype(np.float64), deg, n_jobs=-1, **aug)
+            L.CUSIG.cusig_amd_force_partition(tail, k)
+            back = P.sig_backprop(dev(x), dev(ref.astype(dtype)), dev(g), deg, **aug).cpu().numpy()
+            name = L.CUSIG.cusig_amd_last_kernel_name().decode()
+            L.CUSIG.cusig_amd_force_partition(0, 0)
+            assert "_t%d_k%d_lds" % (tail, k) in name, name
+            assert bwd_rel_err(back, want) < TOL[dtype]
+    finally:
+        L.CUSIG.cusig_amd_force_partition(0, 0)
+        L.CUSIG.cusig_amd_set_profiling(0)
