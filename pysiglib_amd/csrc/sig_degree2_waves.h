@@ -83,8 +83,15 @@ __global__ __launch_bounds__(kBlock, TN < 4 ? 1 : sizeof(T) == 8 ? 2 : SAME ? 4 
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = typename M::Acc{T(0), T(0), T(0), T(0)};
 
+    // U_t is formed from the differences to the first point, (Y_t + Y_{t+1}) / 2 with Y = X - X_0: a sum of the points themselves
+    // would round at the size of the path's offset, which the signature does not depend on (256 points, 64 channels, steps of 1/16,
+    // an offset of 1000, single precision: 2.7e-5 of the result instead of 2.2e-7)
     auto point = [&](uint32_t t) { return t < mine ? t : mine; };
-    P r0 = load(xw, point(first), ro), c0 = SAME ? r0 : load(xw, point(first), co);
+    const P r0 = load(xw, point(first), ro);
+    P c0 = SAME ? r0 : load(xw, point(first), co);
+    T y0[TN];
+#pragma unroll
+    for (int q = 0; q < TN; ++q) y0[q] = r0.v[q] - x0.v[q];
     P rn[AHEAD], cn[SAME ? 1 : AHEAD];
     auto fetch = [&](uint32_t s) {
 #pragma unroll
@@ -111,14 +118,15 @@ __global__ __launch_bounds__(kBlock, TN < 4 ? 1 : sizeof(T) == 8 ? 2 : SAME ? 4 
             T u[TN], z[TN];
 #pragma unroll
             for (int q = 0; q < TN; ++q) {
-                u[q] = live ? T(0.5) * (r0.v[q] + r1[k].v[q]) - x0.v[q] : T(0);
+                const T y1 = r1[k].v[q] - x0.v[q];
+                u[q] = live ? T(0.5) * (y0[q] + y1) : T(0);
                 z[q] = live ? cp.v[q] - c0.v[q] : T(0);
+                y0[q] = y1;
             }
 #pragma unroll
             for (int i = 0; i < TN; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j) acc[i][j] = M::mma(u[i], z[j], acc[i][j]);
-            r0 = r1[k];
             c0 = cp;
         }
     }
@@ -283,7 +291,7 @@ __global__ __launch_bounds__(kBlock, 2) void degree2_bwd_waves_kernel(
             for (int q = 0; q < TN; ++q)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const T v = lo[q].v[e] + (hi[q].v[e] - T(2) * x0[q].v[e]);
+                    const T v = (lo[q].v[e] - x0[q].v[e]) + (hi[q].v[e] - x0[q].v[e]);
                     u[4 * q + e] = t == last_row ? v : u[4 * q + e];
                 }
         }

@@ -1665,6 +1665,40 @@ def test_degree2_by_waves_infinite_last_point(P, d, dtype):
             assert np.isinf(back[:, -2, : d - 1]).all()         # X_{t-1} - X_{t+1} times A, whose diagonal is zero
 
 
+@pytest.mark.parametrize("d", [13, 16, 33, 48, 64, 97, 130])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_degree2_by_waves_of_paths_far_from_the_origin(P, oracle, d, dtype):
+    """Signatures do not depend on where a path starts.  Points that are multiples of the spacing of numbers at the offset have
+    exact differences to the first point, so the results have to be the same to the last bit near the origin and far from
+    it (sums of two such points are not exact)."""
+    import ctypes
+    from pysiglib_amd import _loader as L
+    L.CUSIG.cusig_amd_last_kernel_name.restype = ctypes.c_char_p
+    batch, length = 300, 131
+    rng = np.random.default_rng(d)
+    walk = np.cumsum(rng.standard_normal((batch, length, d)), axis=1) / 16
+    g = dev(rng.standard_normal((batch, d + d * d)).astype(dtype))
+    for offset in (100.0, 1000.0, -3000.0, 300000.0)[:3 if dtype == np.float32 else 4]:
+        unit = float(np.spacing(dtype(abs(offset))))
+        x = np.round(walk / unit) * unit
+        try:
+            L.CUSIG.cusig_amd_set_profiling(1)
+            near = P.sig(dev(x.astype(dtype)), 2)
+            assert L.CUSIG.cusig_amd_last_kernel_name().decode().endswith("_waves")
+            back = P.sig_backprop(dev(x.astype(dtype)), near, g, 2)
+            assert (d > 48) != L.CUSIG.cusig_amd_last_kernel_name().decode().endswith("_waves")
+        finally:
+            L.CUSIG.cusig_amd_set_profiling(0)
+        far = (x + offset).astype(dtype)
+        assert np.array_equal(far - dtype(offset), x)
+        assert torch.equal(P.sig(dev(far), 2), near)
+        assert torch.equal(P.sig_backprop(dev(far), near, g, 2), back)
+        # sums of 130 products of operands that are rounded twice: at most 134 roundings of each product, beside |U| |Z| of a
+        # walk, which exceeds the largest coefficient of its level less than tenfold
+        ref = oracle.signature(x[:3], 2, n_jobs=-1)
+        assert np.max(level_rel_err(near[:3].cpu().numpy(), ref, d, 2)) < 10 * 134 * np.finfo(dtype).eps / 2
+
+
 @pytest.mark.parametrize("dtype,d,deg,tail,k", [
     (np.float64, 5, 7, 2, 5), (np.float64, 6, 5, 2, 6),
     (np.float64, 7, 6, 2, 7), (np.float64, 9, 6, 2, 5), (np.float64, 10, 6, 2, 5),
