@@ -310,7 +310,8 @@ CUSIG_AMD_API void cusig_amd_force_degree3(int mode) CUSIG_AMD_NOEXCEPT;
  * (degree >= 5, 4, 3 respectively) to them; by default they only serve degrees 17 .. 64. */
 CUSIG_AMD_API void cusig_amd_force_deep(int enabled) CUSIG_AMD_NOEXCEPT;
 /* Tuning hook: 0 makes the degree-2 kernels build their operands straight from global memory instead of staging
- * them through LDS (the path taken anyway when a chunk of all channels does not fit). */
+ * them through LDS (the path taken anyway when a chunk of all channels does not fit); 1 (default) takes each form where it
+ * is the sooner one; 2 computes plain paths a wave a block of channels wherever that form applies. */
 CUSIG_AMD_API void cusig_amd_set_degree2_staged(int enabled) CUSIG_AMD_NOEXCEPT;
 /* Tuning hook: with a forced partition, shapes served by a run-time-dimension kernel take its wide-layout variant. */
 /* Tuning hook: nonzero makes every shape run the run-time-dimension kernels (and the by-row reverse sweep where it

@@ -760,17 +760,42 @@ static bool use_degree2(bool backward, uint64_t d_aug, uint64_t degree, uint64_t
     return backward || d_aug >= 12 || batch * 8 <= uint64_t(simd_count());
 }
 
+// Steps from which the forward kernel of sig_degree2_waves.h serves a plain path.  A block of it takes four waves and an exchange
+// through LDS whatever the number of steps, which short paths do not repay, in double precision (two blocks a CU) less than in
+// single; and channel counts that the TN channels of a lane do not divide cost it 2 TN loads a point.  Whole calls of 5000 paths,
+// us, the kernels of sig_degree2.h / this one:
+//  * up to 32 channels, 24: 8 steps 34 / 36, 16: 38 / 36; double 8: 38 / 42, 16: 45 / 42;
+//  * up to 48, 40: 8 steps 44 / 51, 16: 53 / 51; double 8: 50 / 82, 24: 78 / 82, 28: 86 / 82;
+//  * more, TN dividing, single: 96: 4 steps 125 / 128, 8: 136 / 128; double, TN = 3, 96: 20 steps 243 / 242, 24: 269 / 261, 32: 353 / 263,
+//    TN = 4, 112: 24 steps 281 / 340, 40: 359 / 399, 56: 425 / 463, 64: 592 / 475;
+//  * more, not dividing, TN = 3, 95: 24 steps 119 / 154, 48: 196 / 163; double 40 steps 273 / 360, 56: 327 / 369, 64: 446 / 370;
+//  * TN = 4, one group, 61: 16 steps 48 / 58, 64: 74 / 69; double 48 steps 102 / 120, 72: 138 / 150, 80: 152 / 151; several, 111:
+//    4 steps 89 / 211, 64: 290 / 298, 112: 350 / 429, 1500 paths 208 steps 1.04, 256: 0.79 of the time; double 64 steps 481 / 503, 80: 486 / 557,
+//    1500 paths 136: 1.03, 144: 0.90.
+static uint64_t degree2_waves_from(uint64_t d, bool f64)
+{
+    const uint64_t groups = (d + 63) / 64, tn = (d + 16 * groups - 1) / (16 * groups);
+    if (d <= 32) return 16;
+    if (d <= 48) return f64 ? 28 : 16;
+    if (d % tn == 0) return !f64 ? 1 : tn == 3 ? 24 : 64;
+    if (tn == 3) return f64 ? 64 : 48;
+    if (groups == 1) return f64 ? 80 : 64;
+    return f64 ? 140 : 224;
+}
+
 // The kernels of sig_degree2_waves.h, plain paths only.  Forward at any channel count, but beyond 48 channels not where few paths
 // would have to be cut into slices (their 64 x 64 sums then meet in 16-byte pieces of atomics: 1 x 8192 points x 64 channels
-// 32 -> 52 us, 16 x 4096: 39 -> 65), nor in double precision for fewer than 24 steps (4096 x 16 x 64: 67 -> 74).  Backward up to 48
+// 32 -> 52 us, 16 x 4096: 39 -> 65; up to 48 it wins there too: 1 x 8000 x 8: 41 -> 31, 64 x 1000 x 32: 44 -> 32, 1 x 8000 x 48: 45 -> 41; worst of
+// 250 cut shapes 2 x 8000 x 48 in double precision, 50 -> 53), nor for the shortest paths (degree2_waves_from).  Backward up to 48
 // channels: with 64 the registers of A leave too few waves (2048 x 256 x 64: 124 -> 143, double 190 -> 240).
 static bool degree2_by_waves(bool backward, uint64_t d, uint64_t L, uint64_t batch, size_t elem_bytes, bool augmented)
 {
     if (augmented || g_degree2_staged == 0 || (L + 1) * d >= (uint64_t(1) << 31)) return false;
-    if (d <= 48) return true;
+    if (backward) return d <= 48;
+    if (g_degree2_staged == 2) return true;
     const uint64_t groups = (d + 63) / 64;
     const bool sliced = batch * groups * groups * 4 < uint64_t(simd_count()) && L >= 128;
-    return !backward && !sliced && !(elem_bytes == 8 && L < 24);
+    return L >= degree2_waves_from(d, elem_bytes == 8) && !(sliced && d > 48);
 }
 
 // ---------------------------------------------------------------------------

@@ -1665,6 +1665,39 @@ def test_degree2_by_waves_infinite_last_point(P, d, dtype):
             assert np.isinf(back[:, -2, : d - 1]).all()         # X_{t-1} - X_{t+1} times A, whose diagonal is zero
 
 
+@pytest.mark.parametrize("d,steps32,steps64", [(12, 16, 16), (32, 16, 16), (33, 16, 28), (48, 16, 28), (64, 1, 64), (96, 1, 24), (112, 1, 64),
+                                               (95, 48, 64), (61, 64, 80), (111, 224, 140), (189, 224, 140)])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_degree2_form_by_path_length(P, oracle, d, steps32, steps64, dtype):
+    """Which form of the degree-2 forward serves a plain path: either side of each line, by name, and the form by waves below
+    its lines (a hook asks for it), where its quarters of a path are empty or of one step."""
+    import ctypes
+    from pysiglib_amd import _loader as L
+    L.CUSIG.cusig_amd_set_degree2_staged.argtypes = (ctypes.c_int,)
+    L.CUSIG.cusig_amd_last_kernel_name.restype = ctypes.c_char_p
+    first = steps64 if dtype == np.float64 else steps32
+    rng = np.random.default_rng(d)
+
+    def check(steps, by_waves):
+        x = (np.cumsum(rng.standard_normal((300, steps + 1, d)), axis=1) / np.sqrt((steps + 1) * d)).astype(dtype)
+        got = P.sig(dev(x), 2).cpu().numpy()
+        assert L.CUSIG.cusig_amd_last_kernel_name().decode().endswith("_waves") == by_waves, steps
+        ref = oracle.signature(x[::60].astype(np.float64), 2, n_jobs=-1)
+        assert np.max(level_rel_err(got[::60], ref, d, 2)) < TOL[dtype]
+
+    try:
+        L.CUSIG.cusig_amd_set_profiling(1)
+        check(first, True)
+        if first > 1:
+            check(first - 1, False)
+        L.CUSIG.cusig_amd_set_degree2_staged(2)
+        for steps in (1, 2, 5, 17):
+            check(steps, True)
+    finally:
+        L.CUSIG.cusig_amd_set_degree2_staged(1)
+        L.CUSIG.cusig_amd_set_profiling(0)
+
+
 @pytest.mark.parametrize("d", [13, 16, 33, 48, 64, 97, 130])
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 def test_degree2_by_waves_of_paths_far_from_the_origin(P, oracle, d, dtype):
@@ -1674,7 +1707,7 @@ def test_degree2_by_waves_of_paths_far_from_the_origin(P, oracle, d, dtype):
     import ctypes
     from pysiglib_amd import _loader as L
     L.CUSIG.cusig_amd_last_kernel_name.restype = ctypes.c_char_p
-    batch, length = 300, 131
+    batch, length = 300, 231
     rng = np.random.default_rng(d)
     walk = np.cumsum(rng.standard_normal((batch, length, d)), axis=1) / 16
     g = dev(rng.standard_normal((batch, d + d * d)).astype(dtype))
@@ -1693,10 +1726,10 @@ def test_degree2_by_waves_of_paths_far_from_the_origin(P, oracle, d, dtype):
         assert np.array_equal(far - dtype(offset), x)
         assert torch.equal(P.sig(dev(far), 2), near)
         assert torch.equal(P.sig_backprop(dev(far), near, g, 2), back)
-        # sums of 130 products of operands that are rounded twice: at most 134 roundings of each product, beside |U| |Z| of a
+        # sums of 230 products of operands that are rounded twice: at most 234 roundings of each product, beside |U| |Z| of a
         # walk, which exceeds the largest coefficient of its level less than tenfold
         ref = oracle.signature(x[:3], 2, n_jobs=-1)
-        assert np.max(level_rel_err(near[:3].cpu().numpy(), ref, d, 2)) < 10 * 134 * np.finfo(dtype).eps / 2
+        assert np.max(level_rel_err(near[:3].cpu().numpy(), ref, d, 2)) < 10 * 234 * np.finfo(dtype).eps / 2
 
 
 @pytest.mark.parametrize("dtype,d,deg,tail,k", [
