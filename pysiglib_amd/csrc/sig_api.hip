@@ -798,6 +798,10 @@ static bool degree2_by_waves(bool backward, uint64_t d, uint64_t L, uint64_t bat
     return L >= degree2_waves_from(d, elem_bytes == 8) && !(sliced && d > 48);
 }
 
+// Paths that one launch of those kernels takes: HIP numbers the threads of a launch with 32 bits along x, and their blocks serve
+// one path each where the kernels of sig_degree2.h put four short ones into a block.
+static int64_t degree2_paths_per_launch(int64_t blocks_per_path) { return std::max<int64_t>(1, ((int64_t(1) << 32) / kBlock - 1) / blocks_per_path); }
+
 // ---------------------------------------------------------------------------
 // degrees beyond the instance table: run-time-degree sweeps (sig_deep.hip)
 // ---------------------------------------------------------------------------
@@ -994,8 +998,7 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
         slices = std::max<int64_t>(slices, 1);
         const int64_t slice_len = (int64_t(s.L) + slices - 1) / slices;
         slices = (int64_t(s.L) + slice_len - 1) / slice_len;
-        const int64_t blocks = whole * slices;
-        if (blocks > 2147483647LL) throw std::runtime_error("signature_cuda: launch too large");
+        const int64_t per_path = int64_t(groups) * groups * slices, most = degree2_paths_per_launch(per_path);
         if (slices > 1)
             hipLaunchKernelGGL((zero_kernel<T>), dim3(grid_for(batch * s.stride)), dim3(kBlock), 0, stream, out,
                                int64_t(batch * s.stride));
@@ -1003,9 +1006,11 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
         auto go = [&](auto tiles, auto same) {
             constexpr int TN = decltype(tiles)::value;
             auto run = [&](auto whole_pieces) {
-                hipLaunchKernelGGL((degree2_fwd_waves_kernel<T, TN, decltype(same)::value, decltype(whole_pieces)::value>), dim3(unsigned(blocks)),
-                                   dim3(kBlock), 0, stream, path, out, int64_t(length), d, int64_t(s.stride), sc, groups, int(slices), slice_len,
-                                   slices > 1 ? nullptr : flag);
+                for (int64_t first = 0; first < int64_t(batch); first += most)
+                    hipLaunchKernelGGL((degree2_fwd_waves_kernel<T, TN, decltype(same)::value, decltype(whole_pieces)::value>),
+                                       dim3(unsigned(std::min(most, int64_t(batch) - first) * per_path)), dim3(kBlock), 0, stream,
+                                       path + first * int64_t(length) * d, out + first * int64_t(s.stride), int64_t(length), d, int64_t(s.stride),
+                                       sc, groups, int(slices), slice_len, slices > 1 ? nullptr : flag);
             };
             if (d % TN == 0) run(std::true_type{});
             else run(std::false_type{});
@@ -1355,13 +1360,15 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
         int64_t parts = std::min<int64_t>(chunks, std::max<int64_t>(1, (simd_count() / 2 + int64_t(batch) - 1) / int64_t(batch)));
         const int64_t part_rows = (chunks + parts - 1) / parts * 64;
         parts = (int64_t(length) + part_rows - 1) / part_rows;
-        const int64_t blocks = int64_t(batch) * parts;
-        if (blocks > 2147483647LL) throw std::runtime_error("sig_backprop_cuda: launch too large");
+        const int64_t most = degree2_paths_per_launch(parts);
         MainKernelTimer timer(stream, sizeof(T) == 8 ? "degree2_bwd_f64_waves" : "degree2_bwd_f32_waves");
         auto go = [&](auto tiles) {
             auto run = [&](auto whole_pieces) {
-                hipLaunchKernelGGL((degree2_bwd_waves_kernel<T, decltype(tiles)::value, decltype(whole_pieces)::value>), dim3(unsigned(blocks)),
-                                   dim3(kBlock), 0, stream, path, sig_derivs, out, int64_t(length), d, int64_t(s.stride), sc, int(parts), part_rows);
+                for (int64_t first = 0; first < int64_t(batch); first += most)
+                    hipLaunchKernelGGL((degree2_bwd_waves_kernel<T, decltype(tiles)::value, decltype(whole_pieces)::value>),
+                                       dim3(unsigned(std::min(most, int64_t(batch) - first) * parts)), dim3(kBlock), 0, stream,
+                                       path + first * int64_t(length) * d, sig_derivs + first * int64_t(s.stride), out + first * int64_t(length) * d,
+                                       int64_t(length), d, int64_t(s.stride), sc, int(parts), part_rows);
             };
             if (d % 4 == 0) run(std::true_type{});
             else run(std::false_type{});

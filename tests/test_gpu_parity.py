@@ -1698,6 +1698,40 @@ def test_degree2_form_by_path_length(P, oracle, d, steps32, steps64, dtype):
         L.CUSIG.cusig_amd_set_profiling(0)
 
 
+def test_degree2_by_waves_of_more_paths_than_a_launch_has_blocks(P):
+    """2^24 blocks of 256 threads do not fit the 32 bits with which a launch numbers its threads: paths of one step, each with
+    a block of its own, against the closed forms S1 = z, S2 = z (x) z / 2 and dz = G1 + (G2 + G2^T) z / 2."""
+    import ctypes
+    from pysiglib_amd import _loader as L
+    for name in ("cusig_amd_set_degree2_staged", "cusig_amd_force_degree2"):
+        getattr(L.CUSIG, name).argtypes = (ctypes.c_int,)
+    L.CUSIG.cusig_amd_last_kernel_name.restype = ctypes.c_char_p
+    batch, d = 2 ** 24 + 37, 2
+    x = torch.randn((batch, 2, d), device=DEV)
+    g = torch.randn((batch, d + d * d), device=DEV)
+    z = x[:, 1] - x[:, 0]
+    try:
+        L.CUSIG.cusig_amd_set_profiling(1)
+        L.CUSIG.cusig_amd_force_degree2(1)
+        L.CUSIG.cusig_amd_set_degree2_staged(2)
+        s = P.sig(x, 2)
+        assert L.CUSIG.cusig_amd_last_kernel_name() == b"degree2_fwd_f32_waves"
+        L.CUSIG.cusig_amd_force_degree2(-1)
+        L.CUSIG.cusig_amd_set_degree2_staged(1)
+        back = P.sig_backprop(x, s, g, 2)
+        assert L.CUSIG.cusig_amd_last_kernel_name() == b"degree2_bwd_f32_waves"
+    finally:
+        L.CUSIG.cusig_amd_force_degree2(-1)
+        L.CUSIG.cusig_amd_set_degree2_staged(1)
+        L.CUSIG.cusig_amd_set_profiling(0)
+    # four roundings of products of numbers below 2 * 6 (six deviations): at most 4 * 6e-8 * 12^2
+    assert torch.equal(s[:, :d], z)
+    assert float((s[:, d:] - 0.5 * (z[:, :, None] * z[:, None, :]).reshape(batch, -1)).abs().max()) < 4e-5
+    g2 = g[:, d:].reshape(batch, d, d)
+    dz = g[:, :d] + 0.5 * ((g2 + g2.transpose(1, 2)) * z[:, None, :]).sum(2)
+    assert float((back[:, 1] - dz).abs().max()) < 4e-5 and float((back[:, 0] + dz).abs().max()) < 4e-5
+
+
 @pytest.mark.parametrize("d", [13, 16, 33, 48, 64, 97, 130])
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 def test_degree2_by_waves_of_paths_far_from_the_origin(P, oracle, d, dtype):
