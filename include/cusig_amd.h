@@ -240,7 +240,7 @@ CUSIG_AMD_API int cusig_amd_measure_fma_peak(int is_f64, int waves_per_simd, dou
  * scans the result for NaN and Inf) needs no pass of its own over the output.  No counterpart in the reference. */
 CUSIG_AMD_API int cusig_amd_last_sig_nonfinite(void) CUSIG_AMD_NOEXCEPT;
 /* The tuning and test hooks declared from here on (cusig_amd_force_*, cusig_amd_set_point_fed, _set_lead_lag_sparse,
- * _set_chen_low_levels, _set_degree2_staged, _set_alloc_limit) are process-wide switches for offline sweeps and for the
+ * _set_chen_low_levels, _set_row_forms, _set_degree2_staged, _set_alloc_limit) are process-wide switches for offline sweeps and for the
  * test-suite.  They are ignored until cusig_amd_enable_test_hooks(1) has been called; cusig_amd_enable_test_hooks(0)
  * restores every default.  No counterpart in the reference. */
 CUSIG_AMD_API void cusig_amd_enable_test_hooks(int enabled) CUSIG_AMD_NOEXCEPT;
@@ -293,6 +293,11 @@ CUSIG_AMD_API void cusig_amd_force_chen_adjoint(int mode) CUSIG_AMD_NOEXCEPT;
 /* Test hook: the Chen product kernels of sig_combine and of the tensor logarithm can keep the factors' short levels in
  * LDS: 0 = never, 1 (default) = for float64 rows of large launches, 2 = always. */
 CUSIG_AMD_API void cusig_amd_set_chen_low_levels(int enabled) CUSIG_AMD_NOEXCEPT;
+/* Test hook: the forms of sig_join, the tensor logarithm and their adjoints that take a row as a whole (appended segments by
+ * the words' prefixes, a block per row): 0 never, 1 (default) where they are the sooner ones, 2 wherever they apply. */
+CUSIG_AMD_API void cusig_amd_set_row_forms(int mode) CUSIG_AMD_NOEXCEPT;
+/* Whether such a form served the last sig_join* / sig_to_log_sig* call on this thread: 1 or 0. */
+CUSIG_AMD_API int cusig_amd_last_row_form(void) CUSIG_AMD_NOEXCEPT;
 /* Stream-ordered mode (no counterpart in the reference, off by default).  When enabled, signature_cuda_{f,d} and
  * sig_backprop_cuda_{f,d} enqueue their kernels on the null stream and return without waiting, and do not wait for
  * other streams on entry: inputs must be ordered before, and consumers after, the null stream (true for PyTorch's

@@ -219,6 +219,8 @@ struct Workspace {
 std::atomic<int> g_force_wide_index{0};
 std::atomic<int> g_chen_adjoint_mode{0};
 std::atomic<int> g_chen_low_levels{1};
+std::atomic<int> g_row_forms{1};
+thread_local int tl_row_form = 0;
 std::mutex g_ws_mutex;
 static std::map<std::pair<int, int>, Workspace> g_ws;   // (device, slot)
 
@@ -1865,6 +1867,9 @@ CUSIG_AMD_API void cusig_amd_force_wide_index(int enabled) noexcept { if (g_test
 CUSIG_AMD_API void cusig_amd_force_chen_adjoint(int mode) noexcept { if (g_test_hooks) g_chen_adjoint_mode = mode; }
 CUSIG_AMD_API void cusig_amd_set_chen_low_levels(int enabled) noexcept { if (g_test_hooks) g_chen_low_levels = enabled; }
 
+CUSIG_AMD_API void cusig_amd_set_row_forms(int mode) noexcept { if (g_test_hooks) g_row_forms = mode; }
+CUSIG_AMD_API int cusig_amd_last_row_form(void) noexcept { return tl_row_form; }
+
 CUSIG_AMD_API void cusig_amd_set_stream_ordered(int enabled) noexcept { g_stream_ordered = enabled; }
 
 CUSIG_AMD_API int cusig_amd_last_sig_nonfinite(void) noexcept { return tl_sig_nonfinite; }
@@ -1902,6 +1907,7 @@ CUSIG_AMD_API void cusig_amd_enable_test_hooks(int enabled) noexcept
     g_force_wide_index = 0;
     g_chen_adjoint_mode = 0;
     g_chen_low_levels = 1;
+    g_row_forms = 1;
     g_force_degree2 = -1;
     g_force_degree3 = -1;
     g_force_deep = 0;

@@ -3,12 +3,24 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <stdexcept>
 #include <string>
 
 #include "sig_host.h"
+#include "sig_kernels.h"
 
 namespace sigamd {
+
+// Test hooks (defined in sig_api.hip).  g_row_forms: the forms of sig_join_stream.h and sig_log_rows.h never (0), where they are the
+// sooner ones (1), wherever they apply (2); which one served the thread's last call is tl_row_form.  A test that asks for
+// a variant of the general kernels asks for those kernels.
+extern std::atomic<int> g_chen_adjoint_mode, g_row_forms;
+extern thread_local int tl_row_form;
+inline int row_forms()
+{
+    return g_chen_adjoint_mode != 0 || g_chen_low_levels != 1 || g_force_wide_index != 0 ? 0 : g_row_forms.load();
+}
 
 constexpr int kCombMaxLevels = 64;      // highest degree the adjoint of the Chen product takes
 

@@ -244,8 +244,6 @@ __global__ __launch_bounds__(kBlock) void lyndon_expand_kernel(
     }
 }
 
-extern std::atomic<int> g_chen_adjoint_mode;      // test hook (defined in sig_api.hip)
-
 // number of coefficients of levels 1 .. t
 static uint64_t coef_count(uint64_t d, uint64_t t) { return sig_length_u64(d, t) - 1; }
 
@@ -292,7 +290,7 @@ static void run_tensor_log(const T* sig, T* out, uint64_t batch, uint64_t dimens
 //    double: 317 / 283; 600: 749 / 1038) or many steps (1000 x 2, 13, double: 2092 / 1667).
 static bool plan_log_rows(LogRowPlan& pl, uint64_t dimension, uint64_t degree, uint64_t n_coef)
 {
-    if (g_chen_adjoint_mode != 0 || g_chen_low_levels != 1 || g_force_wide_index != 0) return false;    // a test asks for the general form
+    if (row_forms() == 0) return false;
     if (degree < 2 || degree > uint64_t(kLogRowMaxDegree) || n_coef > 65536) return false;
     pl.degree = int(degree);
     pl.d = uint32_t(dimension);
@@ -335,6 +333,7 @@ static size_t log_row_bwd_entries(const LogRowPlan& pl) { return 4 * size_t(pl.l
 static bool log_rows_forward(const LogRowPlan& pl, uint64_t batch, int method, size_t elem_bytes)
 {
     const size_t lds = log_row_fwd_entries(pl) * elem_bytes;
+    if (row_forms() == 2) return lds <= kLogRowLds;
     return lds <= kLogRowLds && pl.degree <= 13 && !(batch > 512 && lds > (size_t(80) << 10)) &&
            (method != 0 || batch * pl.n <= uint64_t(1) << 20);
 }
@@ -342,6 +341,7 @@ static bool log_rows_forward(const LogRowPlan& pl, uint64_t batch, int method, s
 static bool log_rows_backward(const LogRowPlan& pl, uint64_t batch, size_t elem_bytes)
 {
     const size_t lds = log_row_bwd_entries(pl) * elem_bytes;
+    if (row_forms() == 2) return true;
     if (lds > kLogRowBwdLds) return batch <= 256 || pl.degree >= 10;
     return !(batch > 1024 && lds > (size_t(64) << 10) && pl.degree >= 6);
 }
@@ -394,6 +394,7 @@ static void sig_to_log_sig_impl(const T* sig, T* out, uint64_t batch, uint64_t d
 {
     check_method(method, "sig_to_log_sig_cuda");
     const SigShape s = sig_shape(dimension, degree, scalar_term, "sig_to_log_sig_cuda");
+    tl_row_form = 0;
     if (batch == 0) return;
     const uint64_t bytes = checked_mul(checked_mul(batch, s.stride, "signature"), sizeof(T), "signature");
     SIG_HIP(hipDeviceSynchronize());
@@ -413,6 +414,7 @@ static void sig_to_log_sig_impl(const T* sig, T* out, uint64_t batch, uint64_t d
     // (the workspaces are asked for before the form is chosen: a call meets the same limit of memory whichever serves it)
     LogRowPlan rows;
     if (plan_log_rows(rows, dimension, degree, s.n_coef) && log_rows_forward(rows, batch, method, sizeof(T))) {
+        tl_row_form = 1;
         if (method == 2) {
             // the logarithm at the Lyndon words, then its coordinates in their basis
             T* words = static_cast<T*>(workspace(14, bytes));
@@ -464,6 +466,7 @@ static void sig_to_log_sig_backprop_impl(const T* sig, T* out, const T* derivs, 
 {
     check_method(method, "sig_to_log_sig_backprop_cuda");
     const SigShape s = sig_shape(dimension, degree, scalar_term, "sig_to_log_sig_backprop_cuda");
+    tl_row_form = 0;
     if (batch == 0) return;
     const uint64_t bytes = checked_mul(checked_mul(batch, s.stride, "signature"), sizeof(T), "signature");
     SIG_HIP(hipDeviceSynchronize());
@@ -480,6 +483,7 @@ static void sig_to_log_sig_backprop_impl(const T* sig, T* out, const T* derivs, 
     T* ws = degree >= 2 ? static_cast<T*>(workspace(7, checked_mul(bytes, degree + 4, "workspace"))) : nullptr;
     LogRowPlan rows;
     if (plan_log_rows(rows, dimension, degree, s.n_coef) && log_rows_backward(rows, batch, sizeof(T))) {
+        tl_row_form = 1;
         launch_log_rows_bwd<T>(rows, sig, out, derivs, batch, method, lyn, s, ws, stream);
         SIG_HIP(hipStreamSynchronize(stream));
         return;

@@ -526,16 +526,11 @@ static void linear_sig_impl(const T* disp, T* out, uint64_t batch, uint64_t dime
 // ---------------------------------------------------------------------------
 // an appended segment by the words' prefixes (sig_join_stream.h)
 // ---------------------------------------------------------------------------
-extern std::atomic<int> g_chen_adjoint_mode;      // test hook (defined in sig_api.hip): not 0 asks for the general kernels
-
-// Rows of 1024 coefficients and more.  Whole calls, us, general kernels / these, double precision unless noted (20 and 4096
-// rows of 4 letters, degree 4, 340 coefficients: forward 22 / 22 and 30 / 31, backward 39 / 49 and 92 / 100; 4096 x 10, 3: 38 / 33, 129 /
-// 101; 200 x 7, 4: 24 / 23, 66 / 51; 1024 x 10, 5: 526 / 347, 861 / 521; 100 x 90, 3, single: 214 / 133, 1038 / 207; 2 x 12, 6: 50 / 38, 671 /
-// 138; 1 x 2, 16: 26 / 25, 367 / 341).  A launch per level is too many for two letters of many rows: 1000 x 2, 12: backward
-// 312 / 331, but in single precision 376 / 299.
+// Appended segments of rows of 1024 coefficients and more (20 and 4096 rows of 4 letters, degree 4, 340 coefficients: forward 22 / 22 and
+// 30 / 31 us, backward 39 / 49 and 92 / 100).
 static bool plan_join_words(JoinPlan& pl, uint64_t dimension, uint64_t degree, uint64_t n_coef, bool prepend)
 {
-    if (prepend || g_chen_adjoint_mode != 0 || g_chen_low_levels != 1 || g_force_wide_index != 0) return false;
+    if (prepend || row_forms() == 0) return false;
     if (dimension < 2 || dimension > kJoinMaxDim || degree < 2 || degree > uint64_t(kJoinMaxDegree) || n_coef < 1024 || n_coef > (uint64_t(1) << 27)) return false;
     pl.degree = int(degree);
     pl.d = uint32_t(dimension);
@@ -547,6 +542,30 @@ static bool plan_join_words(JoinPlan& pl, uint64_t dimension, uint64_t degree, u
         if (t <= degree) size *= dimension;
         at += size;
     }
+    return true;
+}
+
+// Where that form is the sooner one.  Whole calls, us, general kernels / by prefixes:
+//  * forward, double unless noted: 4096 x d = 10, degree 3: 38 / 33; 200 x 7, 4: 24 / 23; 1024 x 10, 5: 526 / 347; 100 x 90, 3, single: 214 / 133; 2 x 12,
+//    6: 50 / 38; 1 x 2, 16: 26 / 25; two letters of many coefficients in double: 4000 x 2, 10: 76 / 76, 4000 x 2, 11: 124 / 131, 1000 x 2, 13: 146 /
+//    158, 600 x 2, 14: 202 / 216;
+//  * backward, a launch per level, which few coefficients a launch do not repay against the LDS copies of the general kernels.
+//    Single, two letters: 1 / 600 / 1000 x 2, 10: 86 / 145, 156 / 164, 197 / 177, 400 x 2, 11: 192 / 186, 100 / 257 x 2, 12: 190 / 198, 231 / 210, 1 x
+//    2, 13: 341 / 215; three: 1 / 400 / 1000 x 3, 6: 57 / 70, 73 / 77, 97 / 85, 180 / 257 x 3, 7: 94 / 96, 105 / 98, 1 x 3, 8: 138 / 108; four: 1 / 257 x 4, 5:
+//    55 / 59, 67 / 64, 1 x 4, 6: 81 / 72.  Double as single, but two letters: 1 / 180 x 2, 12: 167 / 195, 185 / 215, 1 x 2, 13: 317 / 225, and 1000 x 2, 12:
+//    312 / 331.  More letters always: 1 x 5, 5: 68 / 59; 4096 x 10, 3: 129 / 101; 1024 x 10, 5: 861 / 521; 100 x 90, 3, single: 1038 / 207.
+static bool join_words_forward(uint64_t d, uint64_t n_coef, uint64_t batch, size_t elem_bytes)
+{
+    return row_forms() == 2 || !(d == 2 && elem_bytes == 8 && batch * n_coef > 10u << 20);
+}
+
+static bool join_words_backward(uint64_t d, uint64_t n_coef, uint64_t batch, size_t elem_bytes)
+{
+    if (row_forms() == 2) return true;
+    if (d == 2 && elem_bytes == 8) return n_coef > 8190 && batch <= 256;
+    if (d == 2) return n_coef > 8190 || batch * n_coef >= 3u << 19;
+    if (d == 3) return n_coef > 3279 || batch * n_coef >= 5u << 17;
+    if (d == 4) return n_coef > 1364 || batch * n_coef >= 1u << 18;
     return true;
 }
 
@@ -606,6 +625,7 @@ static void sig_join_impl(const T* sig, const T* disp, T* out, uint64_t batch, u
                           bool prepend, bool scalar_term)
 {
     const SigShape s = sig_shape(dimension, degree, scalar_term, "sig_join_cuda");
+    tl_row_form = 0;
     if (batch == 0) return;
     checked_mul(checked_mul(batch, s.stride, "signature"), sizeof(T), "signature");
     SIG_HIP(hipDeviceSynchronize());
@@ -614,7 +634,9 @@ static void sig_join_impl(const T* sig, const T* disp, T* out, uint64_t batch, u
         if (scalar_term)
             hipLaunchKernelGGL((fill_trivial_kernel<T>), dim3(grid_for(batch)), dim3(kBlock), 0, stream, out, int64_t(batch),
                                int64_t(1), 1);
-    } else if (JoinPlan words; plan_join_words(words, dimension, degree, s.n_coef, prepend)) {
+    } else if (JoinPlan words; plan_join_words(words, dimension, degree, s.n_coef, prepend) &&
+                               join_words_forward(dimension, s.n_coef, batch, sizeof(T))) {
+        tl_row_form = 1;
         launch_join_words<T>(words, sig, disp, out, batch, s, stream);
     } else {
         with_chen_fan(dimension, [&](auto fan) {
@@ -641,6 +663,7 @@ static void sig_join_backprop_impl(const T* d_out, T* d_sig, T* d_disp, const T*
                                    uint64_t dimension, uint64_t degree, bool prepend, bool scalar_term)
 {
     const SigShape s = sig_shape(dimension, degree, scalar_term, "sig_join_backprop_cuda");
+    tl_row_form = 0;
     if (batch == 0) return;
     const uint64_t bytes = checked_mul(checked_mul(batch, s.stride, "signature"), sizeof(T), "signature");
     const uint64_t dz_elems = checked_mul(batch, dimension, "displacement gradient");
@@ -657,7 +680,9 @@ static void sig_join_backprop_impl(const T* d_out, T* d_sig, T* d_disp, const T*
     std::lock_guard<std::mutex> lk(g_ws_mutex);
     T* E = static_cast<T*>(workspace(4, bytes));
     T* dE = static_cast<T*>(workspace(5, bytes));
-    if (JoinPlan words; !(dimension == 2 && sizeof(T) == 8 && batch > 256) && plan_join_words(words, dimension, degree, s.n_coef, prepend)) {
+    if (JoinPlan words; plan_join_words(words, dimension, degree, s.n_coef, prepend) &&
+                        join_words_backward(dimension, s.n_coef, batch, sizeof(T))) {
+        tl_row_form = 1;
         launch_join_words_bwd<T>(words, d_out, d_sig, d_disp, sig, disp, batch, s, E, dE, stream);
         SIG_HIP(hipGetLastError());
         SIG_HIP(hipStreamSynchronize(stream));

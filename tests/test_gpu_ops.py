@@ -833,3 +833,56 @@ def test_sig_join_by_words_vs_oracle(P, oracle, d, deg, batch, dtype, scalar_ter
     if scalar_term:
         assert np.all(ga[:, 0] == 0)
     assert row_rel_err(ga[:, off:], da[:, off:]) < TOL[dtype] and row_rel_err(gz, dz) < TOL[dtype]
+
+
+@pytest.fixture()
+def row_forms():
+    """Chooses between the general kernels of sig_join and the tensor logarithm and those that take a row as a whole (0 never, 1 the
+    rules, 2 wherever they apply) and tells which ran."""
+    from pysiglib_amd import _loader as L
+    L.CUSIG.cusig_amd_set_row_forms.argtypes = (ctypes.c_int,)
+    L.CUSIG.cusig_amd_set_row_forms.restype = None
+    L.CUSIG.cusig_amd_last_row_form.restype = ctypes.c_int
+
+    def choose(mode):
+        L.CUSIG.cusig_amd_set_row_forms(mode)
+
+    choose.last = lambda: L.CUSIG.cusig_amd_last_row_form()
+    yield choose
+    choose(1)
+
+
+@pytest.mark.parametrize("dtype,d,deg,batch,forward,backward", [
+    (np.float32, 2, 10, 600, 1, 0), (np.float32, 2, 10, 1000, 1, 1), (np.float32, 2, 12, 190, 1, 0), (np.float32, 2, 13, 1, 1, 1),
+    (np.float32, 3, 6, 600, 1, 0), (np.float32, 3, 6, 601, 1, 1), (np.float32, 3, 8, 1, 1, 1), (np.float32, 4, 5, 190, 1, 0),
+    (np.float32, 4, 5, 200, 1, 1), (np.float32, 4, 6, 1, 1, 1), (np.float32, 5, 5, 1, 1, 1), (np.float32, 2, 9, 1000, 0, 0),
+    (np.float64, 2, 12, 200, 1, 0), (np.float64, 2, 13, 256, 1, 1), (np.float64, 2, 13, 257, 1, 0), (np.float64, 2, 11, 2562, 0, 0),
+    (np.float64, 3, 7, 190, 1, 0), (np.float64, 3, 7, 200, 1, 1), (np.float64, 257, 2, 2, 0, 0)])
+def test_sig_join_form_by_shape(P, oracle, row_forms, dtype, d, deg, batch, forward, backward):
+    """Either side of the lines that choose between the general kernels of sig_join and those by the words' prefixes, and the
+    latter below their lines, against the oracle."""
+    rng = np.random.default_rng(3 * d + deg)
+    n = oracle.sig_length(d, deg) - 1
+    scale = np.concatenate([np.full(d ** k, 0.5 / np.sqrt(float(d) ** k)) for k in range(1, deg + 1)])
+    a, g = (rng.standard_normal((batch, n)) * scale).astype(dtype), rng.standard_normal((batch, n)).astype(dtype)
+    z = (rng.standard_normal((batch, d)) * 0.5 / np.sqrt(d)).astype(dtype)
+    part = slice(0, None, max(1, batch // 3))
+    want = oracle.sig_join(a[part].astype(np.float64), z[part].astype(np.float64), d, deg)
+    da, dz = oracle.sig_join_backprop(g[part].astype(np.float64), a[part].astype(np.float64), z[part].astype(np.float64), d, deg)
+
+    def check(ran_forward, ran_backward):
+        got = P.sig_join(dev(a), dev(z), d, deg).cpu().numpy()[part]
+        assert row_forms.last() == ran_forward
+        ga, gz = (v.cpu().numpy()[part] for v in P.sig_join_backprop(dev(g), dev(a), dev(z), d, deg))
+        assert row_forms.last() == ran_backward
+        assert row_rel_err(got, want) < TOL[dtype]
+        assert row_rel_err(ga, da) < TOL[dtype] and row_rel_err(gz, dz) < TOL[dtype]
+
+    check(forward, backward)
+    row_forms(0)
+    check(0, 0)
+    if n >= 1024 and d <= 256:
+        row_forms(2)
+        check(1, 1)
+    P.sig_join(dev(a), dev(z), d, deg, prepend=True)
+    assert row_forms.last() == 0
