@@ -886,3 +886,19 @@ def test_sig_join_form_by_shape(P, oracle, row_forms, dtype, d, deg, batch, forw
         check(1, 1)
     P.sig_join(dev(a), dev(z), d, deg, prepend=True)
     assert row_forms.last() == 0
+
+
+@pytest.mark.parametrize("d", [33, 64, 100, 256])
+def test_sig_join_backprop_sums_are_rounded_once(P, row_forms, d):
+    """Degree 2, single precision: dA_1[u] = G_1[u] + sum_x G_2[u x] z[x], whose sum is formed in double precision.  So the only
+    roundings are those of the sum and of the result, 2^-24 of each."""
+    rng = np.random.default_rng(d)
+    n = d + d * d
+    a, g = rng.standard_normal((20, n)).astype(np.float32), rng.standard_normal((20, n)).astype(np.float32)
+    z = rng.standard_normal((20, d)).astype(np.float32)
+    got = P.sig_join_backprop(dev(g), dev(a), dev(z), d, 2)[0].cpu().numpy().astype(np.float64)
+    assert row_forms.last() == 1
+    terms = g[:, d:].reshape(20, d, d).astype(np.float64) @ z[:, :, None].astype(np.float64)
+    want = g[:, :d] + terms[:, :, 0]
+    assert np.all(np.abs(got[:, :d] - want) <= 2.0 ** -24 * (np.abs(terms[:, :, 0]) + np.abs(want)) * (1 + 1e-6))
+    np.testing.assert_array_equal(got[:, d:], g[:, d:])
