@@ -949,11 +949,14 @@ def test_by_row_reverse_sweep_workspace(P, oracle, by_rows, aug):
 @pytest.mark.parametrize("shape", [(2, 10, 48, 3), (3, 11, 64, 3), (2, 12, 33, 4), (1, 4, 33, 6)])
 def test_by_row_sweeps_beside_the_run_time_kernels(P, by_rows, shape):
     """The matrix form of the forward sweep rounds like the run-time-dimension kernels, bit for bit (at degree 6 too, whose
-    chains run level by level), and reports overflow like a scan of its result; the reverse sweep agrees to rounding."""
+    chains run level by level), and reports overflow like a scan of its result; either reverse sweep is as near to double
+    precision as its sums allow."""
     import ctypes
     from pysiglib_amd import _loader as L
     L.CUSIG.cusig_amd_ignore_instance_table.argtypes = (ctypes.c_int,)
+    L.CUSIG.cusig_amd_kernel_choice.argtypes = (ctypes.c_int, ctypes.c_int, ctypes.c_uint64, ctypes.c_uint64) + (ctypes.POINTER(ctypes.c_int),) * 3
     b, length, d, deg = shape
+    tail, k = ctypes.c_int(), ctypes.c_int()
     torch.manual_seed(d + deg)
     x = torch.randn((b, length, d), device=DEV).cumsum(1) / np.sqrt(d * length)
     try:
@@ -967,10 +970,18 @@ def test_by_row_sweeps_beside_the_run_time_kernels(P, by_rows, shape):
         assert torch.equal(fwd, P.sig(x, deg))
         other = P.sig_backprop(x, fwd, g, deg)
         assert not by_rows.last_name().startswith("rows_") and by_rows.last_on_matrix_units() == 0
+        want = P.sig_backprop(x.double(), fwd.double(), g.double(), deg).cpu().numpy()
+        assert L.CUSIG.cusig_amd_kernel_choice(1, 0, d, deg, tail, k, None) == 1
     finally:
         L.CUSIG.cusig_amd_ignore_instance_table(0)
-    # both sides round to 6e-8 of terms that are summed over the d^(deg-1) prefixes, the run-time kernels with atomics
-    assert bwd_rel_err(back.cpu().numpy(), other.cpu().numpy()) <= TOL[np.float32]
+    # By row: gradient rows are sums in double precision of terms that are rounded a few times by 6e-8.
+    assert np.linalg.norm(back.cpu().numpy() - want) <= 6e-7 * np.linalg.norm(want)
+    # Run-time kernels: every wave adds its sum over 64 prefixes and k letters into the single-precision row with an atomic, in
+    # any order.  n such sums of either sign: each addition rounds a partial sum by up to 2^-24 of it, together sqrt(n) of that, and
+    # a point's gradient is the difference of two rows; three deviations of the largest row (2.4e-4 at degree 6, where runs showed 4.9e-5 to
+    # 8.9e-5 and once more than 1e-4).  1e-5: what the steps that recover the states leave where n is small.
+    n = -(-d // k.value) * -(-d ** (deg - tail.value) // 64)
+    assert bwd_rel_err(other.cpu().numpy(), want) <= max(1e-5, 3 * np.sqrt(n) * 2.0 ** -24)
     by_rows(2, 2)
     if deg <= 4:
         for kind in ("overflow", "nan"):
@@ -1549,14 +1560,29 @@ def test_degrees_beyond_sixteen_at_their_own_dispatch(P, oracle, shape, scalar_t
     assert bwd_rel_err(got, want) <= 1e-10, shape
 
 
-@pytest.mark.parametrize("d,deg", [(2, 4), (2, 9), (3, 4), (3, 7), (4, 3), (4, 6), (5, 5), (7, 3), (9, 5), (10, 4), (13, 3), (16, 3), (17, 3)])
+@pytest.mark.parametrize("d,deg", [(2, 4), (2, 9), (3, 4), (3, 7), (4, 3), (4, 6), (5, 5), (7, 3), (9, 5), (10, 4), (13, 3), (16, 3), (17, 3),
+                                   (2, 7), (2, 12), (4, 4), (6, 5), (7, 6)])
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 def test_fine_partitions_vs_oracle(P, oracle, d, deg, dtype):
     """The second partition of a shape (many light lanes a path, wide layout also with a few prefixes), forced wherever one is
     compiled: one step, both sides of a 16-step chunk of the ring and of the reduction tile, several time pieces, every
-    augmentation."""
+    augmentation.  The kernel's name says which partition ran."""
     import ctypes
+    import importlib.util
+    import os
     from pysiglib_amd import _loader as L
+    spec = importlib.util.spec_from_file_location("gen_instances", os.path.join(os.path.dirname(L.__file__), "csrc", "gen_instances.py"))
+    gen = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(gen)
+    compiled, short = set(gen.spec_shapes()), "f64" if dtype == np.float64 else "f32"
+    L.CUSIG.cusig_amd_last_kernel_name.restype = ctypes.c_char_p
+
+    def check_name(d_aug, direction):
+        part = gen.fine_partition(d_aug, deg, short, direction) if (d_aug, deg) in compiled else None
+        name = L.CUSIG.cusig_amd_last_kernel_name().decode()
+        assert part is None or name.startswith("%s_%s_d%d_n%d_t%d_k%d_lds" % ((direction, short, d_aug, deg) + part)), (part, name)
+        return part is not None
+
     L.CUSIG.cusig_amd_set_fine.argtypes = (ctypes.c_int,)
     L.CUSIG.cusig_amd_set_fine.restype = None
     for hook in (L.CUSIG.cusig_amd_force_segments, L.CUSIG.cusig_amd_force_bwd_segments):
@@ -1564,8 +1590,10 @@ def test_fine_partitions_vs_oracle(P, oracle, d, deg, dtype):
         hook.restype = None
     rng = np.random.default_rng(100 * d + deg)
     tol = TOL[dtype]
+    seen = False
     try:
         L.CUSIG.cusig_amd_set_fine(2)
+        L.CUSIG.cusig_amd_set_profiling(1)
         for aug in ({}, dict(time_aug=True), dict(lead_lag=True), dict(time_aug=True, lead_lag=True)):
             raw = d - (1 if "time_aug" in aug else 0)
             if "lead_lag" in aug:
@@ -1579,13 +1607,17 @@ def test_fine_partitions_vs_oracle(P, oracle, d, deg, dtype):
                 ref = oracle.signature(x.astype(np.float64), deg, n_jobs=-1, **aug)
                 d_aug = (2 * raw if "lead_lag" in aug else raw) + (1 if "time_aug" in aug else 0)
                 got = P.sig(dev(x), deg, **aug).cpu().numpy()
+                seen |= check_name(d_aug, "fwd")
                 assert np.max(level_rel_err(got, ref, d_aug, deg)) < tol
                 g = rng.standard_normal(ref.shape).astype(dtype)
                 want = oracle.sig_backprop(x.astype(np.float64), ref, g.astype(np.float64), deg, n_jobs=-1, **aug)
                 back = P.sig_backprop(dev(x), dev(ref.astype(dtype)), dev(g), deg, **aug).cpu().numpy()
+                seen |= check_name(d_aug, "bwd")
                 assert bwd_rel_err(back, want) < tol
+        assert seen
     finally:
         L.CUSIG.cusig_amd_set_fine(1)
+        L.CUSIG.cusig_amd_set_profiling(0)
         L.CUSIG.cusig_amd_force_segments(0)
         L.CUSIG.cusig_amd_force_bwd_segments(0)
 
@@ -1619,21 +1651,43 @@ def test_finer_partitions_ask_for_no_memory_that_is_not_there(P, oracle, d, deg,
 
 @pytest.mark.parametrize("d", [2, 3, 15, 16, 17, 31, 32, 33, 47, 48, 49, 50, 63, 64, 65, 97, 130])
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
-def test_degree2_by_waves_vs_oracle(P, oracle, d, dtype):
+@pytest.mark.parametrize("forced", [False, True])
+def test_degree2_by_waves_vs_oracle(P, oracle, d, dtype, forced):
     """Degree 2 of plain paths: channel counts either side of the 16-channel tiles, of the 64-channel groups and of what the
-    pieces of a lane divide; one step, quarters of a wave that are empty, partly filled and full, more than one slice."""
+    pieces of a lane divide; one step, quarters of a wave that are empty, partly filled and full, more than one slice.  As the dispatch
+    has it, and with the form asked for by hooks, where the kernel's name says that it ran (backward: up to 48 channels)."""
+    import ctypes
+    from pysiglib_amd import _loader as L
+    for name in ("cusig_amd_set_degree2_staged", "cusig_amd_force_degree2"):
+        getattr(L.CUSIG, name).argtypes = (ctypes.c_int,)
+    L.CUSIG.cusig_amd_last_kernel_name.restype = ctypes.c_char_p
+    if forced:
+        L.CUSIG.cusig_amd_set_profiling(1)
+        L.CUSIG.cusig_amd_force_degree2(1)
+        L.CUSIG.cusig_amd_set_degree2_staged(2)
+    try:
+        _degree2_vs_oracle(P, oracle, d, dtype, (lambda: L.CUSIG.cusig_amd_last_kernel_name().decode()) if forced else None)
+    finally:
+        L.CUSIG.cusig_amd_set_profiling(0)
+        L.CUSIG.cusig_amd_force_degree2(-1)
+        L.CUSIG.cusig_amd_set_degree2_staged(1)
+
+
+def _degree2_vs_oracle(P, oracle, d, dtype, last_name):
     rng = np.random.default_rng(d)
     for batch, length in ((1, 2), (3, 3), (2, 6), (300, 17), (5, 18), (2, 66), (1, 131), (300, 40)):
         x = (np.cumsum(rng.standard_normal((batch, length, d)), axis=1) / np.sqrt(length * d)).astype(dtype)
         for scalar in (False, True):
             ref = oracle.signature(x.astype(np.float64), 2, scalar_term=scalar, n_jobs=-1)
             got = P.sig(dev(x), 2, scalar_term=scalar).cpu().numpy()
+            assert last_name is None or last_name().startswith("degree2_fwd_") and last_name().endswith("_waves")
             off = 1 if scalar else 0
             assert np.max(level_rel_err(got[:, off:], ref[:, off:], d, 2)) < TOL[dtype]
             assert not scalar or np.all(got[:, 0] == 1)
             g = rng.standard_normal(ref.shape).astype(dtype)
             want = oracle.sig_backprop(x.astype(np.float64), ref, g.astype(np.float64), 2, n_jobs=-1)
             back = P.sig_backprop(dev(x), dev(ref.astype(dtype)), dev(g), 2).cpu().numpy()
+            assert last_name is None or (d <= 48) == last_name().endswith("_waves")
             assert bwd_rel_err(back, want) < TOL[dtype]
     bad = dev(x).clone()
     bad[-1, -1, -1] = float("nan")
