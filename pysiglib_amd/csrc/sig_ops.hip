@@ -678,16 +678,20 @@ static void sig_join_backprop_impl(const T* d_out, T* d_sig, T* d_disp, const T*
         return;
     }
     std::lock_guard<std::mutex> lk(g_ws_mutex);
-    T* E = static_cast<T*>(workspace(4, bytes));
-    T* dE = static_cast<T*>(workspace(5, bytes));
     if (JoinPlan words; plan_join_words(words, dimension, degree, s.n_coef, prepend) &&
                         join_words_backward(dimension, s.n_coef, batch, sizeof(T))) {
+        // level l has degree - l arrays of d^l words: no more than d^(degree-1) in all, a d-th of a signature
+        const size_t arrays = size_t(batch) * (words.lo[degree] - words.lo[degree - 1]) * sizeof(T);
+        T* w0 = static_cast<T*>(workspace(4, arrays));
+        T* w1 = static_cast<T*>(workspace(5, arrays));
         tl_row_form = 1;
-        launch_join_words_bwd<T>(words, d_out, d_sig, d_disp, sig, disp, batch, s, E, dE, stream);
+        launch_join_words_bwd<T>(words, d_out, d_sig, d_disp, sig, disp, batch, s, w0, w1, stream);
         SIG_HIP(hipGetLastError());
         SIG_HIP(hipStreamSynchronize(stream));
         return;
     }
+    T* E = static_cast<T*>(workspace(4, bytes));
+    T* dE = static_cast<T*>(workspace(5, bytes));
     // exp(z) up to level degree - 1: the adjoint never multiplies with a factor's top level
     if (degree >= 2 && !launch_linear_sig_levels<T>(disp, E, batch, dimension, degree - 1, s.n_coef, int64_t(s.stride), s.off, stream))
         with_chen_fan(dimension, [&](auto fan) {

@@ -902,3 +902,23 @@ def test_sig_join_backprop_sums_are_rounded_once(P, row_forms, d):
     want = g[:, :d] + terms[:, :, 0]
     assert np.all(np.abs(got[:, :d] - want) <= 2.0 ** -24 * (np.abs(terms[:, :, 0]) + np.abs(want)) * (1 + 1e-6))
     np.testing.assert_array_equal(got[:, d:], g[:, d:])
+
+
+@pytest.mark.parametrize("dtype,d,deg,batch", [(np.float32, 10, 4, 12), (np.float64, 5, 6, 7), (np.float64, 2, 13, 3)])
+def test_sig_join_backprop_workspace(P, oracle, row_forms, dtype, d, deg, batch):
+    """The form by the words' prefixes keeps two sets of arrays of d^(degree-1) words a row, a d-th of a signature each; every
+    workspace is an eighth larger than asked for."""
+    from pysiglib_amd import _loader as L
+    L.CUSIG.cusig_amd_workspace_bytes.restype = ctypes.c_uint64
+    rng = np.random.default_rng(d)
+    n = oracle.sig_length(d, deg) - 1
+    scale = np.concatenate([np.full(d ** k, 0.5 / np.sqrt(float(d) ** k)) for k in range(1, deg + 1)])
+    a, g = (rng.standard_normal((batch, n)) * scale).astype(dtype), rng.standard_normal((batch, n)).astype(dtype)
+    z = (rng.standard_normal((batch, d)) * 0.5 / np.sqrt(d)).astype(dtype)
+    L.CUSIG.cusig_shutdown()                     # the pool only grows
+    ga, gz = (v.cpu().numpy() for v in P.sig_join_backprop(dev(g), dev(a), dev(z), d, deg))
+    assert row_forms.last() == 1
+    asked = 2 * batch * d ** (deg - 1) * np.dtype(dtype).itemsize
+    assert asked <= L.CUSIG.cusig_amd_workspace_bytes() <= asked + asked // 8 + 1024
+    da, dz = oracle.sig_join_backprop(g.astype(np.float64), a.astype(np.float64), z.astype(np.float64), d, deg)
+    assert row_rel_err(ga, da) < TOL[dtype] and row_rel_err(gz, dz) < TOL[dtype]
