@@ -280,14 +280,7 @@ static void run_tensor_log(const T* sig, T* out, uint64_t batch, uint64_t dimens
 // ---------------------------------------------------------------------------
 // a block per row (sig_log_rows.h)
 // ---------------------------------------------------------------------------
-// Rows of up to 65536 coefficients, where the form that launches a kernel per step is not the sooner one.  Whole calls, us, a
-// kernel per step / a block per row, single precision unless noted:
-//  * all coefficients of the logarithm of many rows: the general kernels share the work of several first letters
-//    (16 x d = 4, degree 7: 43 / 38; 257 x 7, 5: 52 / 66; 600 x 6, 6: 161 / 301);
-//  * a recursion of more than 13 steps forward (1 x 2, 14: 106 / 114), or one that leaves a compute unit a single block, many
-//    times over (4000 x 4, 7, double precision: forward 465 / 502; backward, single 1620 / 2045, double 1952 / 2478);
-//  * lower levels that do not fit the LDS: forward never (1000 x 2, 13, double: 259 / 310), backward few rows (64 x 6, 6,
-//    double: 317 / 283; 600: 749 / 1038) or many steps (1000 x 2, 13, double: 2092 / 1667).
+// Rows of up to 65536 coefficients; where this form is the sooner one: log_rows_forward, log_rows_backward.
 static bool plan_log_rows(LogRowPlan& pl, uint64_t dimension, uint64_t degree, uint64_t n_coef)
 {
     if (row_forms() == 0) return false;
@@ -330,19 +323,47 @@ constexpr size_t kLogRowLds = size_t(156) << 10, kLogRowBwdLds = size_t(140) << 
 static size_t log_row_fwd_entries(const LogRowPlan& pl) { return 2 * size_t(pl.low); }
 static size_t log_row_bwd_entries(const LogRowPlan& pl) { return 4 * size_t(pl.low) + pl.p_total; }
 
+// Where that form is the sooner one.  Whole calls, us, a kernel per step / a block per row, single precision unless noted; what loses:
+//  * all coefficients of the logarithm of many rows: the general kernels share the work of several first letters
+//    (16 x d = 4, degree 7: 43 / 38; 257 x 7, 5: 52 / 66; 600 x 6, 6: 161 / 301);
+//  * a recursion of more than 13 steps forward (1 x 2, 14: 106 / 114), lower levels that do not fit the LDS (1000 x 2, 13, double: 259 /
+//    310), and those that leave a compute unit a single block, many times over (4000 x 4, 7, double: 465 / 502), words alone at more
+//    than 120 KB already beyond one round of blocks (double, 257 x 2, 13: 126 / 150, x 3, 9: 99 / 124, x 6, 6: 86 / 108; in the Lyndon basis
+//    400 rows: 0.98, 0.95, 0.92).
 static bool log_rows_forward(const LogRowPlan& pl, uint64_t batch, int method, size_t elem_bytes)
 {
     const size_t lds = log_row_fwd_entries(pl) * elem_bytes;
     if (row_forms() == 2) return lds <= kLogRowLds;
-    return lds <= kLogRowLds && pl.degree <= 13 && !(batch > 512 && lds > (size_t(80) << 10)) &&
-           (method != 0 || batch * pl.n <= uint64_t(1) << 20);
+    if (lds > kLogRowLds || pl.degree > 13) return false;
+    if (lds > (size_t(80) << 10) && batch > (method == 1 && lds > (size_t(120) << 10) ? 256 : 512)) return false;
+    return method != 0 || batch * pl.n <= uint64_t(1) << 20;
 }
 
-static bool log_rows_backward(const LogRowPlan& pl, uint64_t batch, size_t elem_bytes)
+// The adjoint:
+//  * one letter: a lane sums a whole row of the one matrix (1 x 1, degree 4, double: 62 / 49, 5: 64 / 67, 8: 88 / 152, 20: 276 / 1061;
+//    4000 x 1, 3, double 50 / 65);
+//  * a compute unit left a single block, many times over (4000 x 4, 7: 1620 / 2045); where the general kernels move 16 bytes at a time also
+//    beyond one round of blocks (8, 5: 200 rows 0.73 of the time, 257: 185 / 245, 600: 267 / 363), all coefficients of degree 4 beyond two (12,
+//    4, double, 400 rows 0.79, 600: 202 / 212, 1025: 328 / 403);
+//  * lower levels that do not fit the LDS, and so lie in the workspace: many rows of up to 9 levels (600 x 6, 6, double: 749 / 1038;
+//    1000 x 2, 13: 2092 / 1667) and more than a megabyte of them (2, 15, double, 1 / 115 / 257 rows: 1252 / 1369, 1935 /
+//    1650, 2690 / 3161).  Double, 6, 6 by rows,
+//    all / words / basis: 1: 0.90 / 0.86 / 1.12 of the time, 128: - / - / 0.91, 200: 1.07 / 0.90 / 0.98; 15, 4: 1: 1.35 / 1.19 / 1.33, 64: 1.11 / 0.91 / 1.05, 128:
+//    0.86 / 0.72 / 0.81; 8, 5: 1.05 / 0.95 / 1.11, 200: 1.23 / 1.05 / 1.17.
+static bool log_rows_backward(const LogRowPlan& pl, uint64_t batch, int method, size_t elem_bytes)
 {
     const size_t lds = log_row_bwd_entries(pl) * elem_bytes;
     if (row_forms() == 2) return true;
-    if (lds > kLogRowBwdLds) return batch <= 256 || pl.degree >= 10;
+    if (pl.d == 1) return pl.degree <= 5 && batch <= 1024;
+    const bool by_16_bytes = pl.d >= 8 && pl.d % 4 == 0;
+    if (lds > kLogRowBwdLds) {
+        if (pl.degree >= 10) return lds <= size_t(1) << 20 || (batch >= 100 && batch <= 200);
+        if (batch > 256 || by_16_bytes) return false;
+        if (pl.d >= 8) return batch >= 100;
+        if (pl.d >= 6 && lds > (size_t(256) << 10)) return method == 1 || (method == 2 ? batch >= 100 : batch <= 128);
+        return true;
+    }
+    if (by_16_bytes && lds > (size_t(70) << 10)) return batch <= (pl.degree >= 5 ? 256 : method == 0 ? 512 : ~uint64_t(0));
     return !(batch > 1024 && lds > (size_t(64) << 10) && pl.degree >= 6);
 }
 
@@ -361,8 +382,10 @@ static void launch_log_rows(const LogRowPlan& pl, const T* sig, T* out, uint64_t
     const size_t lds = log_row_fwd_entries(pl) * sizeof(T);
     const unsigned threads = log_row_threads(pl, batch);
     const uint64_t rows = std::min<uint64_t>(batch, 65535);
-    // few rows: several blocks each, of at least four coefficients a thread
-    const uint64_t parts = std::max<uint64_t>(1, std::min((index ? count : pl.n) / (4 * threads), 512 / rows));
+    // few rows: several blocks each, of at least four coefficients a thread, no more than the compute units hold at once (double, 200 x d = 6,
+    // degree 6, 145 KB a block: two blocks a row 77 -> 90 us of the general kernels)
+    const uint64_t resident = lds > (size_t(80) << 10) ? 256 : 512;
+    const uint64_t parts = std::max<uint64_t>(1, std::min((index ? count : pl.n) / (4 * threads), resident / rows));
     log_row_lds(&tensor_log_row_kernel<T>, lds);
     hipLaunchKernelGGL((tensor_log_row_kernel<T>), dim3(unsigned(parts), unsigned(rows)), dim3(threads), lds, stream, sig, out,
                        int64_t(batch), pl, index, uint32_t(count), int64_t(s.stride), s.off, out_stride, out_off);
@@ -482,7 +505,7 @@ static void sig_to_log_sig_backprop_impl(const T* sig, T* out, const T* derivs, 
     // -P_2 .. -P_N (the slot of P_1 stays unused), two adjoint buffers, two product-adjoint buffers
     T* ws = degree >= 2 ? static_cast<T*>(workspace(7, checked_mul(bytes, degree + 4, "workspace"))) : nullptr;
     LogRowPlan rows;
-    if (plan_log_rows(rows, dimension, degree, s.n_coef) && log_rows_backward(rows, batch, sizeof(T))) {
+    if (plan_log_rows(rows, dimension, degree, s.n_coef) && log_rows_backward(rows, batch, method, sizeof(T))) {
         tl_row_form = 1;
         launch_log_rows_bwd<T>(rows, sig, out, derivs, batch, method, lyn, s, ws, stream);
         SIG_HIP(hipStreamSynchronize(stream));

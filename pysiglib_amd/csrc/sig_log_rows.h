@@ -6,8 +6,8 @@
 // in LDS (the adjoint of a few rows that need more: in a workspace that stays in the L2) and runs the whole recursion between
 // barriers; the top level, most of the row, stays where it is.  The form that launches a kernel per step instead is bound by
 // the number of its launches: six forward and some thirty backward, 5 us each for a few us of work.  257 rows of 7 letters,
-// degree 5, single precision, Lyndon words, whole calls: forward 59 -> 40 us, backward 220 -> 85; one row 41 -> 32, 162 -> 67;
-// 2048 rows 150 -> 69, 790 -> 295.  What bounds them now: the reads of the top level, 2 (N - 1) times from the L2, by a block
+// degree 5, single precision, Lyndon words, whole calls: forward 54 -> 34 us, backward 211 -> 77; one row 36 -> 27, 147 -> 60;
+// 2048 rows 144 -> 63, 784 -> 290.  What bounds them now: the reads of the top level, 2 (N - 1) times from the L2, by a block
 // that has its compute unit to itself.  With the whole row in LDS the adjoint of one row takes 67 instead of 74 us, that of
 // 257 rows 99 instead of 84 (one block a unit instead of two): left out.
 //
@@ -68,10 +68,9 @@ __device__ __forceinline__ void log_row_levels(const LogRowPlan& pl, LogRowLevel
     }
 }
 
-// Forward.  Block (part, row): every part of a row runs the recursion of the lower levels for itself and evaluates its share
-// of P_1 (`index`: at the listed positions, the Lyndon words; null: everywhere).  With `col` (the Lyndon basis; one part) the
-// coordinates are then combined within the block: `lw` holds them in between.
-// ws (SHARED = false): per block, low entries of x are read in place and P lives there, followed by the coordinates.
+// Forward.  Block (part, row): every part of a row runs the recursion of the lower levels for itself, on copies of x and P in LDS (the
+// host takes this form only where they fit), and evaluates its share of P_1: `index`: at the listed positions, the Lyndon words, one
+// after the other; null: everywhere.  Coordinates in the Lyndon basis are combined by a launch of their own.
 template <typename T>
 __global__ __launch_bounds__(kLogRowBlock) void tensor_log_row_kernel(
     const T* __restrict__ X, T* __restrict__ out, int64_t batch, LogRowPlan pl, const uint64_t* __restrict__ index, uint32_t count,

@@ -767,10 +767,27 @@ def test_sig_to_log_sig_lyndon_vs_oracle(P, oracle, d, deg, batch, dtype, scalar
         P.clear_cache()
 
 
+@pytest.fixture()
+def row_forms():
+    """Chooses between the general kernels of sig_join and the tensor logarithm and those that take a row as a whole (0 never, 1 the
+    rules, 2 wherever they apply) and tells which ran."""
+    from pysiglib_amd import _loader as L
+    L.CUSIG.cusig_amd_set_row_forms.argtypes = (ctypes.c_int,)
+    L.CUSIG.cusig_amd_set_row_forms.restype = None
+    L.CUSIG.cusig_amd_last_row_form.restype = ctypes.c_int
+
+    def choose(mode):
+        L.CUSIG.cusig_amd_set_row_forms(mode)
+
+    choose.last = lambda: L.CUSIG.cusig_amd_last_row_form()
+    yield choose
+    choose(1)
+
+
 @pytest.mark.parametrize("d,deg,batch", [(8, 3, 3), (63, 2, 2), (64, 2, 2), (65, 2, 3), (9, 4, 130), (7, 5, 257), (3, 9, 2), (2, 13, 1),
-                                         (1, 6, 5), (2, 2, 4), (40, 3, 2), (255, 2, 2)])
+                                         (1, 6, 5), (2, 2, 4), (39, 3, 2), (40, 3, 2), (255, 2, 2)])
 @pytest.mark.parametrize("method", [0, 1, 2])
-def test_log_sig_block_per_row_vs_general_form(P, d, deg, batch, method):
+def test_log_sig_block_per_row_vs_general_form(P, row_forms, d, deg, batch, method):
     """The kernels with a block per row against the ones that launch a kernel per step (which a hook asks for): levels of 63, 64
     and 65 words, rows that fit the LDS and rows that do not, one and several blocks a row, with and without the scalar
     term.  Both sum the same up to c(deg) products an entry in another order, c(deg) < 65536 roundings of 1.1e-16 resp. 6e-8."""
@@ -786,24 +803,60 @@ def test_log_sig_block_per_row_vs_general_form(P, d, deg, batch, method):
             P.prepare_log_sig(d, deg, method)
         g = rng.standard_normal((batch, P.log_sig_length(d, deg) if method else n))
 
-        def both(dtype, scalar):
+        def both(dtype, scalar, form):
             s = np.hstack([np.ones((batch, 1)), a]) if scalar else a
             w = np.hstack([np.ones((batch, 1)), g]) if scalar and not method else g
             s, w = dev(s.astype(dtype)), dev(w.astype(dtype))
-            out = P.sig_to_log_sig(s, d, deg, method=method), P.sig_to_log_sig_backprop(s, w, d, deg, method=method)
-            return [v.cpu().numpy() for v in out]
+            out = []
+            for call in (lambda: P.sig_to_log_sig(s, d, deg, method=method), lambda: P.sig_to_log_sig_backprop(s, w, d, deg, method=method)):
+                out.append(call().cpu().numpy())
+                assert row_forms.last() == form
+            return out
 
         L.CUSIG.cusig_amd_force_chen_adjoint(2)
-        want = both(np.float64, False)
+        want = both(np.float64, False, 0)
         L.CUSIG.cusig_amd_force_chen_adjoint(0)
+        row_forms(2)
         for dtype, tol in ((np.float64, 65536 * 1.2e-16), (np.float32, 65536 * 6e-8 / 16)):
             for scalar in (False, True):
-                got = both(dtype, scalar)
+                got = both(dtype, scalar, int(n <= 65536))      # of 40 letters, degree 3: the general form again
                 for i, (x, y) in enumerate(zip(got, want)):
                     x = x if not scalar or (i == 0 and method) else x[:, 1:]
                     assert x.shape == y.shape and row_rel_err(x, y) < tol
     finally:
         L.CUSIG.cusig_amd_force_chen_adjoint(0)
+        if method:
+            P.clear_cache()
+
+
+@pytest.mark.parametrize("dtype,d,deg,batch,method,forward,backward", [
+    (np.float32, 1, 5, 1024, 0, 1, 1), (np.float32, 1, 3, 1025, 0, 1, 0), (np.float64, 1, 6, 3, 0, 1, 0), (np.float64, 1, 20, 2, 0, 0, 0),
+    (np.float32, 8, 5, 256, 1, 1, 1), (np.float32, 8, 5, 257, 1, 1, 0), (np.float64, 8, 5, 3, 1, 1, 0),
+    (np.float64, 12, 4, 512, 0, 0, 1), (np.float64, 12, 4, 513, 0, 0, 0), (np.float64, 12, 4, 513, 1, 1, 1),
+    (np.float64, 15, 4, 99, 1, 1, 0), (np.float64, 15, 4, 100, 1, 1, 1), (np.float32, 15, 4, 2, 2, 1, 1),
+    (np.float64, 6, 6, 99, 2, 1, 0), (np.float64, 6, 6, 100, 2, 1, 1), (np.float64, 6, 6, 128, 0, 0, 1), (np.float64, 6, 6, 129, 0, 0, 0),
+    (np.float64, 6, 6, 256, 1, 1, 1), (np.float64, 6, 6, 257, 1, 0, 0), (np.float64, 6, 6, 257, 2, 1, 0),
+    (np.float64, 2, 14, 3, 1, 0, 1), (np.float64, 2, 15, 3, 1, 0, 0), (np.float64, 2, 15, 100, 1, 0, 1), (np.float32, 2, 15, 3, 1, 0, 1)])
+def test_log_sig_form_by_shape(P, row_forms, dtype, d, deg, batch, method, forward, backward):
+    """Either side of the lines that choose between a block per row and a kernel per step, against the latter.  Both sum up to
+    c(deg) products an entry in another order, as above."""
+    rng = np.random.default_rng(19 * d + deg)
+    scale = np.concatenate([np.full(d ** k, 0.5 / np.sqrt(float(d) ** k)) for k in range(1, deg + 1)])
+    s = dev((rng.standard_normal((batch, scale.size)) * scale).astype(dtype))
+    try:
+        if method:
+            P.prepare_log_sig(d, deg, method)
+        g = dev(rng.standard_normal((batch, P.log_sig_length(d, deg) if method else scale.size)).astype(dtype))
+        tol = 65536 * (1.2e-16 if dtype == np.float64 else 6e-8 / 16)
+        for call, form in ((lambda: P.sig_to_log_sig(s, d, deg, method=method), forward),
+                           (lambda: P.sig_to_log_sig_backprop(s, g, d, deg, method=method), backward)):
+            row_forms(1)
+            got = call().cpu().numpy()
+            assert row_forms.last() == form
+            row_forms(0)
+            want = call().cpu().numpy()
+            assert row_forms.last() == 0 and row_rel_err(got, want) < tol
+    finally:
         if method:
             P.clear_cache()
 
@@ -833,23 +886,6 @@ def test_sig_join_by_words_vs_oracle(P, oracle, d, deg, batch, dtype, scalar_ter
     if scalar_term:
         assert np.all(ga[:, 0] == 0)
     assert row_rel_err(ga[:, off:], da[:, off:]) < TOL[dtype] and row_rel_err(gz, dz) < TOL[dtype]
-
-
-@pytest.fixture()
-def row_forms():
-    """Chooses between the general kernels of sig_join and the tensor logarithm and those that take a row as a whole (0 never, 1 the
-    rules, 2 wherever they apply) and tells which ran."""
-    from pysiglib_amd import _loader as L
-    L.CUSIG.cusig_amd_set_row_forms.argtypes = (ctypes.c_int,)
-    L.CUSIG.cusig_amd_set_row_forms.restype = None
-    L.CUSIG.cusig_amd_last_row_form.restype = ctypes.c_int
-
-    def choose(mode):
-        L.CUSIG.cusig_amd_set_row_forms(mode)
-
-    choose.last = lambda: L.CUSIG.cusig_amd_last_row_form()
-    yield choose
-    choose(1)
 
 
 @pytest.mark.parametrize("dtype,d,deg,batch,forward,backward", [
