@@ -487,16 +487,31 @@ struct RedPlan {
     // 8 waves per SIMD: 7 channels, degree 5 (2 levels x 7) 648 / 2789 -> 618 / 2381, (2 x 2) 536 / 2352 -> 511 / 1722; 10, degree 6 (2 x 5)
     // 804 / 3367 -> 756 / 3221; 13, degree 4 (1 x 13) 572 / 2642 -> 528 / 2247; 17, degree 4 (2 x 6) with a single step a chunk 998 / 4390
     // -> 1165 / 5064.
+    // One number, written in two ways: the compiler folds the first (EARLY) sooner, which changes what it keeps in registers around a
+    // flush by up to 90 of them either way.  kernel_folds_early: which of them leaves an instance fewer (12 channels, degree 4, double,
+    // 2 levels x 4 letters: 276 / 254 registers, one or two waves a SIMD, 140 to 220 paths of 540 points 0.63 / 0.54 ms; 7,
+    // 6, 2 x 7: 306 / 396, 11 paths of 1003 points 0.61 / 0.70 ms).
+    template <bool EARLY = false>
     __host__ __device__ static constexpr int steps(int d)
     {
         const int r = rows_per_step(d);
-        if (ZL && r <= 32) {
+        if (EARLY && ZL && r <= 32) {
             const int once = 32 / r;
             return sizeof(T) == 4 && once * r < 22 && r > 8 ? 64 / r : once > 16 ? 16 : once;
         }
-        return r > kRowsWide ? 0 : r > kRows ? 1 : (kRows / r > 8 ? 8 : kRows / r);
+        constexpr int room = !ZL ? kRows : sizeof(T) == 4 && D >= 17 && D <= 21 ? 64 : 32, most = ZL ? 16 : 8;
+        return r > kRowsWide ? 0 : r > room ? 1 : (room / r > most ? most : room / r);
     }
-    __host__ __device__ static constexpr int64_t tile_elems(int d) { return int64_t(steps(d)) * rows_per_step(d) * kRedStride; }
+    template <bool EARLY = false>
+    __host__ __device__ static constexpr int64_t tile_elems(int d) { return int64_t(steps<EARLY>(d)) * rows_per_step(d) * kRedStride; }
+    static constexpr int kSub = D > 0 ? (TAIL == 1 ? K : K + K * D) : 0;      // nodes of a subtree of up to two levels
+    static constexpr bool kernel_folds_early(int m, int lead_lag)
+    {
+        if (!ZL || TAIL >= 3) return ZL;
+        if (sizeof(T) == 4 || TAIL < 2 || lead_lag != 0) return false;
+        if (PAIR) return m >= 4 && (kSub >= 55 || m >= 6);
+        return m >= 3 ? kSub >= 50 : K >= 3 && kSub >= 60;
+    }
 };
 
 // lanes 0-31: lo[lane] + lo[lane + 32];  lanes 32-63: hi[lane - 32] + hi[lane]
@@ -629,11 +644,12 @@ __global__ __launch_bounds__(kBlock) void tree_bwd_kernel(
     constexpr bool WIDE = Cx::WIDE;
     using Plan = RedPlan<T, D, TAIL, K, ZL>;
     constexpr bool PAIR = Plan::PAIR;
-    const int CH = Plan::steps(d);
+    constexpr bool EARLY = Plan::kernel_folds_early(M, LL);
+    const int CH = Plan::template steps<EARLY>(d);
     const int RS = Plan::rows_per_step(d);      // tile rows per step
     const bool tiled = CH > 0;
     const int slots = WIDE ? 1 : cx.G.ppw;
-    T* wbuf = lds + int64_t(wave_in_block) * (tiled ? Plan::tile_elems(d) : use_lds == 2 ? int64_t(Plan::kRows) * kRedStride : int64_t(slots) * d);
+    T* wbuf = lds + int64_t(wave_in_block) * (tiled ? Plan::template tile_elems<EARLY>(d) : use_lds == 2 ? int64_t(Plan::kRows) * kRedStride : int64_t(slots) * d);
     T* acc = wbuf + int64_t(cx.id.slot) * d;
     const int nsg = slots > 1 ? slots : 2;                    // column segments per row
     const int seg_cnt = slots > 1 ? int(cx.G.lpp) : kWave / 2; // lanes per segment

@@ -180,3 +180,34 @@ def test_wrapper_argument_errors():
         P.sig(np.zeros((4, 2)), 2)
     with pytest.raises(RuntimeError):
         P.sig(x, 2)
+
+
+def test_staged_reverse_sweeps_fit_a_simd_twice():
+    """Registers of this library's own sweeps, from the notes of its code objects: staged reverse sweeps of two subtree levels
+    around 256 registers run two waves on a SIMD (512 registers a lane), which a few more would halve."""
+    import shutil
+    import struct
+    import subprocess
+    import tempfile
+    readelf = shutil.which("llvm-readelf", path=os.pathsep.join(["/opt/rocm/llvm/bin", os.environ.get("PATH", "")]))
+    if readelf is None:
+        pytest.skip("needs llvm-readelf")
+    wanted = {"d%s" % s: 256 for s in ("Li12ELi4ELi2ELi4ELb1ELi0", "Li16ELi4ELi2ELi2ELb1ELi0", "Li8ELi7ELi2ELi4ELb1ELi0", "Li17ELi4ELi2ELi3ELb1ELi1",
+                                      "Li18ELi4ELi2ELi3ELb1ELi2", "Li25ELi4ELi2ELi2ELb1ELi1", "Li24ELi5ELi2ELi2ELb1ELi2")}
+    wanted.update({"f%s" % s: 168 for s in ("Li24ELi4ELi2ELi3ELb1ELi2", "Li16ELi4ELi2ELi4ELb1ELi2", "Li18ELi5ELi2ELi3ELb1ELi0", "Li21ELi5ELi2ELi3ELb1ELi1")})
+    data, at, seen = open(LIB, "rb").read(), 0, {}
+    while True:
+        at = data.find(b"\x7fELF\x02\x01\x01", at + 1)
+        if at < 0:
+            break
+        if struct.unpack_from("<H", data, at + 18)[0] != 224:        # EM_AMDGPU
+            continue
+        sections, (size, count) = struct.unpack_from("<Q", data, at + 40)[0], struct.unpack_from("<HH", data, at + 58)
+        with tempfile.NamedTemporaryFile() as f:
+            f.write(data[at:at + sections + size * count])
+            f.flush()
+            notes = subprocess.run([readelf, "--notes", f.name], capture_output=True, text=True).stdout
+        for m in re.finditer(r"\.symbol:\s+\S*tree_bwd_kernelI(\w+?)E+vP\S*\.kd.*?\.vgpr_count:\s+(\d+)", notes, re.S):
+            seen[m[1]] = int(m[2])
+    assert all(key in seen for key in wanted)
+    assert {key: seen[key] for key in wanted if seen[key] > wanted[key]} == {}
