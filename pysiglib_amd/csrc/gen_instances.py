@@ -158,8 +158,9 @@ def step_cost(D, N, tail, K):
 
 
 def lone_step_ns(D, N, tail, K, dtype, direction):
-    """Duration of a step of a wave that has its SIMD to itself (sig_api.hip: StepModel).  Backward, every channel beyond four
-    costs a row of the LDS tile of the increment gradient, more in double precision without the half-wave sums (one level)."""
+    """Duration of a step of a wave that has its SIMD to itself (sig_api.hip: StepModel, which forward adds the reads of the
+    letters from 17 channels on).  Backward, every channel beyond four costs a row of the LDS tile of the increment gradient, more in
+    double precision without the half-wave sums (one level)."""
     c, m = step_cost(D, N, tail, K), N - tail
     if direction == "fwd":
         return 40 + 1.65 * c

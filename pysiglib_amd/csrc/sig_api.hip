@@ -650,25 +650,42 @@ static const KernelEntry* fine_entry(bool backward, bool f64, uint64_t d, uint64
 // degree 6, 1 level x 4 letters 106 / 104, 361 / 424, 3 x 4 letters 277 / 309, 1299 / 1416; backward 4, 6, 2 x 2: 443 / 443, 1465 / 1556;
 // 10, 4, 1 x 10: 474 / 490, 2125 / 1898; 17, 4, 2 x 6: 1028 / 984, 4454 / 4855; double, backward 10, 5, 2 x 5: 619 / 685, 4492 / 5128).
 // Scalar-fed forward steps take at least 130 ns, those of the run-time-dimension kernels about 2.2 times as long (one path of 4
-// channels, degree 5, double: 270 / 120 ns).
+// channels, degree 5, double: 270 / 120 ns).  Forward, from 17 channels on: the letters of a staged step come from LDS, and every one
+// beyond four that a lane reads costs that again; groups of which the last is not whole guard each read (staged: from four groups
+// on); lead-lag sweeps take half of the top level and its letters, unless there are four and more groups of a single level.  Degree 3, ns a step measured / model, one wave
+// per SIMD and six: single precision, 27 channels, 27 letters 150 / 141, 678 / 667; 7 letters 134 / 125, 271 / 223; lead-lag 27 letters 108 / 94, 406 /
+// 367; 34 channels, lead-lag, 34 letters 122 / 106, 491 / 445; 9 letters 147 / 133, 333 / 267; double, 32 channels, 32 letters 279 / 263, 1451 / 1450; 8
+// letters 102 / 89, 462 / 442 (the measured ones with 20 ns of the launch).
 struct StepModel {
     double lone, issue;         // ns: a step of a wave on its own; what each of several waves on a SIMD adds
     int64_t occ, simds;
     TreeGeom geom;
     bool backward;
     double elem;
-    StepModel(const KernelEntry* e, int d, bool backward_) : occ(std::max(1, resident_waves(e))), simds(simd_count()), geom(geom_of(e, d)), backward(backward_), elem(e->is_f64 ? 8.0 : 4.0)
+    StepModel(const KernelEntry* e, int d, bool backward_, bool sparse_ll = false)
+        : occ(std::max(1, resident_waves(e))), simds(simd_count()), geom(geom_of(e, d)), backward(backward_), elem(e->is_f64 ? 8.0 : 4.0)
     {
-        const double c = lane_step_cost(d, e->N, e->tail, e->k), m = double(e->N - e->tail);
-        const double wide = std::max(0, d - 4), tile = std::max(0, d - 3);
+        double c = lane_step_cost(d, e->N, e->tail, e->k);
+        const double m = double(e->N - e->tail), wide = std::max(0, d - 4), tile = std::max(0, d - 3);
         const bool f64 = e->is_f64 != 0, no_pairs = f64 && e->tail == 1;
         if (backward) {
             lone = 200.0 + 3.2 * c + 6.0 * m * m + (no_pairs ? 40.0 : 26.0) * wide;
             issue = f64 ? 50.0 + 4.6 * (c + m * m) + (no_pairs ? 40.0 * (d - 1) : 22.0 * tile) : (2.0 + 3.0 / d) * c + 2.9 * m * m + 22.0 * tile;
             if (!e->staged) lone *= 1.15;
         } else {
-            lone = 40.0 + 1.65 * c;
-            issue = f64 ? 24.0 + 1.8 * c : 14.0 + c;
+            const int groups = (d + e->k - 1) / e->k;
+            double beyond = 0.0, guards = 0.0;
+            if (d > kPointFedMaxDim && e->D > 0) {
+                double letters = e->tail == 1 ? e->k : groups <= 3 ? d : d + e->k;
+                if (sparse_ll && e->staged && e->fwd_lead_lag && (groups <= 3 || e->tail > 1)) {
+                    c -= 0.5 * e->k * std::pow(double(d), e->tail - 1);
+                    letters *= 0.5;
+                }
+                if (e->staged) beyond = std::max(0.0, letters - 4.0);
+                if (d % e->k && groups > (e->staged ? 3 : 1)) guards = e->staged ? 55.0 : 190.0;
+            }
+            lone = 40.0 + 1.65 * c + (f64 ? 5.6 : 1.9) * beyond + guards;
+            issue = f64 ? 24.0 + 1.8 * c + 5.2 * beyond : 14.0 + c + 2.7 * beyond;
             if (!e->staged) { lone = std::max(130.0, 1.15 * lone); issue += 20.0; }
         }
         if (e->D <= 0) { lone *= 2.2; issue *= 1.5; }
@@ -700,12 +717,12 @@ double StepModel::sweep(int64_t batch, int64_t L, int g, uint64_t sig_bytes_all_
 // The finer partition in as many pieces as serve it best (of at least 16 steps; 256 MB of segment signatures forward, 64 MB per
 // buffer backward), if that promises 8 % (backward 12 %) against `now`, the choice made without it.  On return `e` is the kernel to launch.
 static SplitPlan with_fine(const KernelEntry*& e, const KernelEntry* run_now, const SplitPlan& now, bool backward, uint64_t d, uint64_t degree,
-                           uint64_t batch, uint64_t L, uint64_t sig_bytes_all_paths, int forced_pieces, bool whole_only = false)
+                           uint64_t batch, uint64_t L, uint64_t sig_bytes_all_paths, bool sparse_ll, int forced_pieces, bool whole_only = false)
 {
     const KernelEntry* f = fine_entry(backward, e->is_f64 != 0, d, degree);
     if (!f || (forced_pieces > 0 && g_fine != 2)) return now;
     const int64_t steps = int64_t(L), paths = int64_t(batch);
-    const StepModel model(f, int(d), backward);
+    const StepModel model(f, int(d), backward, sparse_ll);
     SplitPlan best{forced_pieces > 0 ? now.pieces : 1, 0.0, 0.0};
     best.seconds = model.sweep(paths, steps, best.pieces, sig_bytes_all_paths);
     if (forced_pieces <= 0 && !whole_only) {
@@ -716,7 +733,7 @@ static SplitPlan with_fine(const KernelEntry*& e, const KernelEntry* run_now, co
             if (t < 0.95 * best.seconds) best = SplitPlan{g, t, 0.0};
         }
     }
-    if (g_fine != 2 && best.seconds > (backward ? 0.88 : 0.92) * StepModel(run_now, int(d), backward).sweep(paths, steps, now.pieces, sig_bytes_all_paths)) return now;
+    if (g_fine != 2 && best.seconds > (backward ? 0.88 : 0.92) * StepModel(run_now, int(d), backward, sparse_ll).sweep(paths, steps, now.pieces, sig_bytes_all_paths)) return now;
     tl_fine_more_pieces = tl_fine_more_pieces || best.pieces > now.pieces;
     e = f;
     return best;
@@ -1145,7 +1162,7 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
         const uint64_t n_coef = s.full_len - 1;
         if (!by_rows)
             plan = with_fine(e, pick_variant(false, e, instance_waves * plan.pieces, sparse_ll), plan, false, s.d_aug, degree, batch, s.L,
-                             batch * n_coef * sizeof(T), g_force_segments);
+                             batch * n_coef * sizeof(T), sparse_ll, g_force_segments);
         int nseg = by_rows ? 1 : plan.pieces;
         FwdParams p;
         p.batch = int64_t(batch) * nseg; p.L = int64_t(s.L); p.d = int(s.d_aug); p.stream = stream;
@@ -1549,7 +1566,7 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
         if (compare && by_rows) by_rows = rows_bwd_seconds(s.d_aug, batch, s.L) < instance_bwd_seconds(plan, s.d_aug);
         if (!by_rows && !arena)
             plan = with_fine(e, pick_variant(true, e, instance_waves * plan.pieces, sparse_ll), plan, true, s.d_aug, degree, batch, s.L,
-                             batch * n_coef * sizeof(T), g_force_bwd_segments, !ef || degree > uint64_t(kCombMaxLevels));
+                             batch * n_coef * sizeof(T), sparse_ll, g_force_bwd_segments, !ef || degree > uint64_t(kCombMaxLevels));
         int nseg = by_rows ? 1 : plan.pieces;
         int64_t lseg = int64_t(s.L);
         if (nseg > 1) {
@@ -1613,7 +1630,7 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
             f.inc = inc; f.batch = int64_t(rows); f.L = int64_t(s.L); f.d = int(s.d_aug); f.stream = stream;
             f.lseg = lseg; f.nseg = nseg; f.out = segs; f.out_stride = n; f.scalar = 0;
             const KernelEntry* ef_now = pick_variant(false, ef, total_waves(geom_of(ef, int(s.d_aug)), f.batch), sparse_ll);
-            with_fine(ef, ef_now, SplitPlan{1, 0.0, 0.0}, false, s.d_aug, degree, rows, uint64_t(lseg), 0, 0, /*whole_only=*/true);
+            with_fine(ef, ef_now, SplitPlan{1, 0.0, 0.0}, false, s.d_aug, degree, rows, uint64_t(lseg), 0, sparse_ll, 0, /*whole_only=*/true);
             ef = pick_variant(false, ef, total_waves(geom_of(ef, int(s.d_aug)), f.batch), sparse_ll);
             SIG_HIP((sparse_ll && ef->staged && ef->fwd_lead_lag) ? ef->fwd_lead_lag(f) : ef->fwd(f));
             // both scans by doubling: ceil(log2(nseg)) launches, ping-ponging between two scratch copies

@@ -43,12 +43,14 @@ hipError_t launch_tree_fwd(const FwdParams& p)
     return hipGetLastError();
 }
 
-// resident waves per SIMD of the forward kernel (register-limited)
+// resident waves per SIMD of the forward kernel (registers and, of the staged ones, the LDS ring)
 template <typename T, int D, int N, int TAIL, int K, bool ZL>
 int fwd_waves_per_simd()
 {
     int blocks = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, tree_fwd_kernel<T, D, N, TAIL, K, ZL>, kBlock, 0) != hipSuccess) {
+    size_t lds = 0;
+    if constexpr (ZL && D > 0) lds = size_t(kWavesPerBlock) * IncRing<T, D, 1>::ELEMS * sizeof(T);
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, tree_fwd_kernel<T, D, N, TAIL, K, ZL>, kBlock, lds) != hipSuccess) {
         (void)hipGetLastError();
         return 1;
     }

@@ -1622,6 +1622,29 @@ def test_fine_partitions_vs_oracle(P, oracle, d, deg, dtype):
         L.CUSIG.cusig_amd_force_bwd_segments(0)
 
 
+@pytest.mark.parametrize("d,deg,batch,length,aug,dtype,k", [
+    (17, 3, 38, 474, dict(lead_lag=True), np.float32, 34), (19, 3, 14, 284, dict(lead_lag=True, time_aug=True), np.float32, 39),
+    (14, 3, 24, 213, dict(lead_lag=True, time_aug=True), np.float32, 29), (13, 3, 46, 141, dict(lead_lag=True, time_aug=True), np.float32, 27),
+    (20, 3, 62, 102, {}, np.float32, 5), (16, 3, 2, 56, dict(lead_lag=True), np.float32, 8), (24, 3, 13, 403, {}, np.float64, 6)])
+def test_finer_partitions_of_many_channels(P, oracle, d, deg, batch, length, aug, dtype, k):
+    """Degree 3 of 17 and more channels: a wave that holds a whole row takes half of a lead-lag step and is left alone where the
+    finer partition's four waves would each read the letters and the guards of a group; elsewhere the latter serves."""
+    import ctypes
+    from pysiglib_amd import _loader as L
+    L.CUSIG.cusig_amd_last_kernel_name.restype = ctypes.c_char_p
+    rng = np.random.default_rng(d)
+    x = (np.cumsum(rng.standard_normal((batch, length, d)), axis=1) / np.sqrt(length * d)).astype(dtype)
+    try:
+        L.CUSIG.cusig_amd_set_profiling(1)
+        got = P.sig(dev(x), deg, **aug).cpu().numpy()
+        name = L.CUSIG.cusig_amd_last_kernel_name().decode()
+    finally:
+        L.CUSIG.cusig_amd_set_profiling(0)
+    assert "_t1_k%d_lds" % k in name, name
+    ref = oracle.signature(x[:3].astype(np.float64), deg, n_jobs=-1, **aug)
+    assert np.max(level_rel_err(got[:3], ref, (2 * d if "lead_lag" in aug else d) + int("time_aug" in aug), deg)) < TOL[dtype]
+
+
 @pytest.mark.parametrize("d,deg,length,dtype", [(3, 7, 129, np.float32), (3, 7, 161, np.float64), (2, 10, 97, np.float64)])
 def test_finer_partitions_ask_for_no_memory_that_is_not_there(P, oracle, d, deg, length, dtype):
     """One path that the finer partition cuts in pieces and the default sweeps whole: where the signatures of two pieces do not
