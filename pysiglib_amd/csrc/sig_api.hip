@@ -652,9 +652,7 @@ static const KernelEntry* fine_entry(bool backward, bool f64, uint64_t d, uint64
 // Scalar-fed forward steps take at least 130 ns, those of the run-time-dimension kernels about 2.2 times as long (one path of 4
 // channels, degree 5, double: 270 / 120 ns).  Forward, from 17 channels on: the letters of a staged step come from LDS, and every one
 // beyond four that a lane reads costs that again; groups of which the last is not whole guard each read (staged: from four groups
-// on); lead-lag sweeps take half of the top level and its letters, unless there are four and more groups of a single level.  Backward
-// they take half of the top level of two and more (10 channels, degree 4, single, 147 lead-lag paths of 105 points, 2 x 10 / 1 x 10: 151 /
-// 174 us; 11, 4, 130 of 26, 2 x 6 / 2 x 3: 62 / 71).  Degree 3, ns a step measured / model, one wave
+// on); lead-lag sweeps take half of the top level and its letters, unless there are four and more groups of a single level.  Degree 3, ns a step measured / model, one wave
 // per SIMD and six: single precision, 27 channels, 27 letters 150 / 141, 678 / 667; 7 letters 134 / 125, 271 / 223; lead-lag 27 letters 108 / 94, 406 /
 // 367; 34 channels, lead-lag, 34 letters 122 / 106, 491 / 445; 9 letters 147 / 133, 333 / 267; double, 32 channels, 32 letters 279 / 263, 1451 / 1450; 8
 // letters 102 / 89, 462 / 442 (the measured ones with 20 ns of the launch).
@@ -671,7 +669,6 @@ struct StepModel {
         const double m = double(e->N - e->tail), wide = std::max(0, d - 4), tile = std::max(0, d - 3);
         const bool f64 = e->is_f64 != 0, no_pairs = f64 && e->tail == 1;
         if (backward) {
-            if (sparse_ll && e->bwd_lead_lag && e->tail > 1) c -= 0.5 * e->k * std::pow(double(d), e->tail - 1);
             lone = 200.0 + 3.2 * c + 6.0 * m * m + (no_pairs ? 40.0 : 26.0) * wide;
             issue = f64 ? 50.0 + 4.6 * (c + m * m) + (no_pairs ? 40.0 * (d - 1) : 22.0 * tile) : (2.0 + 3.0 / d) * c + 2.9 * m * m + 22.0 * tile;
             if (!e->staged) lone *= 1.15;

@@ -1645,30 +1645,6 @@ def test_finer_partitions_of_many_channels(P, oracle, d, deg, batch, length, aug
     assert np.max(level_rel_err(got[:3], ref, (2 * d if "lead_lag" in aug else d) + int("time_aug" in aug), deg)) < TOL[dtype]
 
 
-@pytest.mark.parametrize("d,deg,batch,length,aug,part", [
-    (5, 4, 147, 105, dict(lead_lag=True), (2, 10)), (5, 4, 130, 26, dict(lead_lag=True, time_aug=True), (2, 6)),
-    (5, 4, 40, 105, dict(lead_lag=True), (1, 10))])
-def test_finer_backward_partitions_of_lead_lag_paths(P, oracle, d, deg, batch, length, aug, part):
-    """A lead-lag step takes half of a two-level partition's top level: the finer one is left to launches that gain from it all the
-    same."""
-    import ctypes
-    from pysiglib_amd import _loader as L
-    L.CUSIG.cusig_amd_last_kernel_name.restype = ctypes.c_char_p
-    rng = np.random.default_rng(batch)
-    x = (np.cumsum(rng.standard_normal((batch, length, d)), axis=1) / np.sqrt(length * d)).astype(np.float32)
-    ref = oracle.signature(x.astype(np.float64), deg, n_jobs=-1, **aug)
-    g = rng.standard_normal(ref.shape).astype(np.float32)
-    want = oracle.sig_backprop(x.astype(np.float64), ref, g.astype(np.float64), deg, n_jobs=-1, **aug)
-    try:
-        L.CUSIG.cusig_amd_set_profiling(1)
-        back = P.sig_backprop(dev(x), dev(ref.astype(np.float32)), dev(g), deg, **aug).cpu().numpy()
-        name = L.CUSIG.cusig_amd_last_kernel_name().decode()
-    finally:
-        L.CUSIG.cusig_amd_set_profiling(0)
-    assert "_t%d_k%d_lds" % part in name, name
-    assert bwd_rel_err(back, want) < TOL[np.float32]
-
-
 @pytest.mark.parametrize("d,deg,length,dtype", [(3, 7, 129, np.float32), (3, 7, 161, np.float64), (2, 10, 97, np.float64)])
 def test_finer_partitions_ask_for_no_memory_that_is_not_there(P, oracle, d, deg, length, dtype):
     """One path that the finer partition cuts in pieces and the default sweeps whole: where the signatures of two pieces do not
