@@ -649,12 +649,12 @@ static const KernelEntry* fine_entry(bool backward, bool f64, uint64_t d, uint64
 // waves per SIMD; most within 15 % (ns a step measured / model, one wave per SIMD and eight; single precision: forward d = 4,
 // degree 6, 1 level x 4 letters 106 / 104, 361 / 424, 3 x 4 letters 277 / 309, 1299 / 1416; backward 4, 6, 2 x 2: 443 / 443, 1465 / 1556;
 // 10, 4, 1 x 10: 474 / 490, 2125 / 1898; 17, 4, 2 x 6: 1028 / 984, 4454 / 4855; double, backward 10, 5, 2 x 5: 619 / 685, 4492 / 5128).
-// Scalar-fed forward steps take at least 130 ns, those of the run-time-dimension kernels about 2.2 times as long (one path of 4
-// channels, degree 5, double: 270 / 120 ns).  Forward, from 17 channels on: the letters of a staged step come from LDS, and every one
+// Scalar-fed forward steps take at least 130 ns (of four and more levels no longer than staged ones: 1325 paths of 2 channels, degree 9, 5 x 1: 285 /
+// 288), those of the run-time-dimension kernels about 2.2 times as long (one path of 4 channels, degree 5, double: 270 / 120 ns).  Forward, from 17 channels on: the letters of a staged step come from LDS, and every one
 // beyond four that a lane reads costs that again; groups of which the last is not whole guard each read (staged: from four groups
 // on); lead-lag sweeps take half of the top level and its letters, unless there are four and more groups of a single level.  Degree 3, ns a step measured / model, one wave
-// per SIMD and six: single precision, 27 channels, 27 letters 150 / 141, 678 / 667; 7 letters 134 / 125, 271 / 223; lead-lag 27 letters 108 / 94, 406 /
-// 367; 34 channels, lead-lag, 34 letters 122 / 106, 491 / 445; 9 letters 147 / 133, 333 / 267; double, 32 channels, 32 letters 279 / 263, 1451 / 1450; 8
+// per SIMD and six: single precision, 27 channels, 27 letters 150 / 141, 678 / 667; 7 letters 134 / 125, 271 / 283; lead-lag 27 letters 108 / 94, 406 /
+// 367; 34 channels, lead-lag, 34 letters 122 / 106, 491 / 445; 9 letters 147 / 133, 333 / 327; double, 32 channels, 32 letters 279 / 263, 1451 / 1450; 8
 // letters 102 / 89, 462 / 442 (the measured ones with 20 ns of the launch).
 struct StepModel {
     double lone, issue;         // ns: a step of a wave on its own; what each of several waves on a SIMD adds
@@ -686,7 +686,8 @@ struct StepModel {
             }
             lone = 40.0 + 1.65 * c + (f64 ? 5.6 : 1.9) * beyond + guards;
             issue = f64 ? 24.0 + 1.8 * c + 5.2 * beyond : 14.0 + c + 2.7 * beyond;
-            if (!e->staged) { lone = std::max(130.0, 1.15 * lone); issue += 20.0; }
+            if (!e->staged) { lone = std::max(130.0, (e->tail >= 4 ? 1.0 : 1.15) * lone); issue += 20.0; }
+            else if (guards > 0.0) issue += 10.0;
         }
         if (e->D <= 0) { lone *= 2.2; issue *= 1.5; }
     }
@@ -715,7 +716,9 @@ double StepModel::sweep(int64_t batch, int64_t L, int g, uint64_t sig_bytes_all_
 }
 
 // The finer partition in as many pieces as serve it best (of at least 16 steps; 256 MB of segment signatures forward, 64 MB per
-// buffer backward), if that promises 8 % (backward 12 %) against `now`, the choice made without it.  On return `e` is the kernel to launch.
+// buffer backward), if that promises 8 % (backward 12 %, of whole lead-lag paths, whose steps skip half of what the estimates count, 16 %: single
+// precision, 10 channels, degree 4, 147 paths of 105 points, promised 15 %: 151 -> 174 us; 11, 4, 130 of 26, 13 %: 62 -> 71) against `now`, the
+// choice made without it.  On return `e` is the kernel to launch.
 static SplitPlan with_fine(const KernelEntry*& e, const KernelEntry* run_now, const SplitPlan& now, bool backward, uint64_t d, uint64_t degree,
                            uint64_t batch, uint64_t L, uint64_t sig_bytes_all_paths, bool sparse_ll, int forced_pieces, bool whole_only = false)
 {
@@ -733,7 +736,7 @@ static SplitPlan with_fine(const KernelEntry*& e, const KernelEntry* run_now, co
             if (t < 0.95 * best.seconds) best = SplitPlan{g, t, 0.0};
         }
     }
-    if (g_fine != 2 && best.seconds > (backward ? 0.88 : 0.92) * StepModel(run_now, int(d), backward, sparse_ll).sweep(paths, steps, now.pieces, sig_bytes_all_paths)) return now;
+    if (g_fine != 2 && best.seconds > (!backward ? 0.92 : sparse_ll && best.pieces == 1 ? 0.84 : 0.88) * StepModel(run_now, int(d), backward, sparse_ll).sweep(paths, steps, now.pieces, sig_bytes_all_paths)) return now;
     tl_fine_more_pieces = tl_fine_more_pieces || best.pieces > now.pieces;
     e = f;
     return best;

@@ -1625,9 +1625,10 @@ def test_fine_partitions_vs_oracle(P, oracle, d, deg, dtype):
 @pytest.mark.parametrize("d,deg,batch,length,aug,dtype,k", [
     (17, 3, 38, 474, dict(lead_lag=True), np.float32, 34), (19, 3, 14, 284, dict(lead_lag=True, time_aug=True), np.float32, 39),
     (14, 3, 24, 213, dict(lead_lag=True, time_aug=True), np.float32, 29), (13, 3, 46, 141, dict(lead_lag=True, time_aug=True), np.float32, 27),
-    (20, 3, 62, 102, {}, np.float32, 5), (16, 3, 2, 56, dict(lead_lag=True), np.float32, 8), (24, 3, 13, 403, {}, np.float64, 6)])
+    (20, 3, 62, 102, {}, np.float32, 5), (16, 3, 2, 56, dict(lead_lag=True), np.float32, 8), (24, 3, 13, 403, {}, np.float64, 6),
+    (29, 3, 47, 796, {}, np.float32, 29), (10, 3, 2315, 20, {}, np.float32, 5)])
 def test_finer_partitions_of_many_channels(P, oracle, d, deg, batch, length, aug, dtype, k):
-    """Degree 3 of 17 and more channels: a wave that holds a whole row takes half of a lead-lag step and is left alone where the
+    """Degree 3, mostly of 17 and more channels: a wave that holds a whole row takes half of a lead-lag step and is left alone where the
     finer partition's four waves would each read the letters and the guards of a group; elsewhere the latter serves."""
     import ctypes
     from pysiglib_amd import _loader as L
@@ -1643,6 +1644,29 @@ def test_finer_partitions_of_many_channels(P, oracle, d, deg, batch, length, aug
     assert "_t1_k%d_lds" % k in name, name
     ref = oracle.signature(x[:3].astype(np.float64), deg, n_jobs=-1, **aug)
     assert np.max(level_rel_err(got[:3], ref, (2 * d if "lead_lag" in aug else d) + int("time_aug" in aug), deg)) < TOL[dtype]
+
+
+@pytest.mark.parametrize("d,deg,batch,length,aug,part", [
+    (5, 4, 147, 105, dict(lead_lag=True), (2, 10)), (5, 4, 130, 26, dict(lead_lag=True, time_aug=True), (2, 6)),
+    (7, 4, 32, 11, dict(lead_lag=True), (1, 14)), (11, 4, 3, 53, dict(lead_lag=True), (1, 22)), (7, 4, 4, 340, dict(lead_lag=True), (1, 14))])
+def test_finer_backward_partitions_of_lead_lag_paths(P, oracle, d, deg, batch, length, aug, part):
+    """Either side of what the finer partition has to promise lead-lag paths, whose steps take half of the default's top level."""
+    import ctypes
+    from pysiglib_amd import _loader as L
+    L.CUSIG.cusig_amd_last_kernel_name.restype = ctypes.c_char_p
+    rng = np.random.default_rng(batch)
+    x = (np.cumsum(rng.standard_normal((batch, length, d)), axis=1) / np.sqrt(length * d)).astype(np.float32)
+    ref = oracle.signature(x.astype(np.float64), deg, n_jobs=-1, **aug)
+    g = rng.standard_normal(ref.shape).astype(np.float32)
+    want = oracle.sig_backprop(x.astype(np.float64), ref, g.astype(np.float64), deg, n_jobs=-1, **aug)
+    try:
+        L.CUSIG.cusig_amd_set_profiling(1)
+        back = P.sig_backprop(dev(x), dev(ref.astype(np.float32)), dev(g), deg, **aug).cpu().numpy()
+        name = L.CUSIG.cusig_amd_last_kernel_name().decode()
+    finally:
+        L.CUSIG.cusig_amd_set_profiling(0)
+    assert "_t%d_k%d_lds" % part in name, name
+    assert bwd_rel_err(back, want) < TOL[np.float32]
 
 
 @pytest.mark.parametrize("d,deg,length,dtype", [(3, 7, 129, np.float32), (3, 7, 161, np.float64), (2, 10, 97, np.float64)])
