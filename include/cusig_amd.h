@@ -278,6 +278,9 @@ CUSIG_AMD_API void cusig_amd_set_rows_backward(int mode) CUSIG_AMD_NOEXCEPT;
 /* Test hook: the same switch for the forward sweep of such shapes: 0 never, 1 (default) where it is expected to be the
  * fastest form, 2 wherever it applies. */
 CUSIG_AMD_API void cusig_amd_set_rows_forward(int mode) CUSIG_AMD_NOEXCEPT;
+/* Test hook: the forward sweep that shares the prefix chains of few channels at high degrees: 0 never, 1 (default) where it is
+ * expected to be the fastest form, 2 wherever there is one. */
+CUSIG_AMD_API void cusig_amd_set_heads_forward(int mode) CUSIG_AMD_NOEXCEPT;
 /* Test hook: the second, finer partition that shapes have for launches of few paths: 0 never, 1 (default) where it is expected
  * to be the sooner one, 2 wherever there is one (forced pieces included). */
 CUSIG_AMD_API void cusig_amd_set_fine(int mode) CUSIG_AMD_NOEXCEPT;

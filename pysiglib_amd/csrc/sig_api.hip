@@ -25,6 +25,7 @@
 #include "../../include/cusig_amd.h"
 #include "sig_chen_adjoint.h"
 #include "sig_deep.h"
+#include "sig_heads.h"
 #include "sig_rows.h"
 #include "sig_degree2.h"
 #include "sig_degree2_waves.h"
@@ -617,7 +618,8 @@ static bool rows_bwd_mfma_wins(uint64_t d, uint64_t degree, uint64_t batch, uint
 static Hook g_fine{1};      // test hook: 0 never, 1 by the estimates below, 2 wherever there is one
 
 // Cutting a path in pieces costs scratch for their signatures.  Where the finer partition cuts more often than the call would
-// be cut without it and the device cannot hold that, the call is served without it: it needs no more memory than it ever did.
+// be cut without it (or the sweep with shared prefix chains is taken, which has a table of its own) and the device cannot hold
+// that, the call is served without it: it needs no more memory than it ever did.
 static thread_local bool tl_no_fine = false, tl_fine_more_pieces = false;
 template <typename F>
 static void fine_if_it_fits(F&& run)
@@ -936,6 +938,45 @@ struct Degree3Buffers {
 };
 
 // ---------------------------------------------------------------------------
+// few channels to high degrees in double precision: shared prefix chains (sig_heads.hip)
+// ---------------------------------------------------------------------------
+static Hook g_heads{1};     // test hook: 0 never, 1 by the estimates below, 2 wherever there is such a sweep
+constexpr uint64_t kHeadsTableBytes = uint64_t(1) << 30;     // the table of fractions; paths are taken in chunks that fit
+
+// Pieces per path of such a sweep if that promises 10 % against `now`, the sweep of `run` chosen without it; 0 if not.  Blocks run in rounds of
+// what the compute units hold; beside the sweep a call lays out the table, and its lanes store runs of a few values each.
+// Lead-lag twins of the tree kernels skip half of what the estimate of theirs counts.
+static int heads_pieces(const HeadsEntry* e, const KernelEntry* run, const SplitPlan& now, uint64_t d, uint64_t batch, uint64_t L, uint64_t sig_bytes_all_paths,
+                        bool sparse_ll)
+{
+    const int mode = g_heads, forced = g_force_segments;
+    if (!e || mode == 0 || tl_no_fine || g_force_tail > 0 || g_force_staged >= 0 || g_ignore_table != 0 || L >= (uint64_t(1) << 30) ||
+        checked_mul(L + 1, uint64_t(e->row) * sizeof(double), "table") > kHeadsTableBytes || batch > (uint64_t(1) << 40) / uint64_t(e->blocks))
+        return 0;
+    if (forced > 0) return mode == 2 ? int(std::min<uint64_t>(uint64_t(forced), L)) : 0;
+    const int64_t cus = simd_count() / 4;
+    auto seconds = [&](int g) {
+        const int64_t fullest = (int64_t(batch) * g * e->blocks + cus - 1) / cus, rest = fullest % e->resident;
+        const double step = double(fullest / e->resident) * e->step_ns + (rest ? std::max(double(e->lone_ns), double(e->step_ns) * double(rest) / e->resident) : 0.0);
+        int lg = 0;
+        while ((1 << lg) < g) ++lg;
+        const double folds = g > 1 ? 2e-6 + 6e-6 * lg + 2.2 * g * double(sig_bytes_all_paths) / 4e12 : 0.0;
+        return 12e-6 + double((L + g - 1) / g) * step * 1e-9 + double(batch * L) * e->row * 8.0 / 3e12 + double(sig_bytes_all_paths) * g / 4e12 + folds;
+    };
+    int best = 1;
+    double best_t = seconds(1);
+    for (int g : {2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64}) {
+        if (L / uint64_t(g) < 48 || uint64_t(g) * sig_bytes_all_paths > (uint64_t(256) << 20)) break;
+        const double t = seconds(g);
+        if (t < 0.95 * best_t) { best = g; best_t = t; }
+    }
+    if (mode == 2) return best;
+    double old = StepModel(run, int(d), false, sparse_ll).sweep(int64_t(batch), int64_t(L), now.pieces, sig_bytes_all_paths);
+    if (sparse_ll && run->staged && run->fwd_lead_lag) old *= 0.6;
+    return best_t < 0.9 * old ? best : 0;
+}
+
+// ---------------------------------------------------------------------------
 // forward  (dispatch mirrors siglib/cpsig/cp_signature.h:740-851 and
 // siglib/cusig/cu_signature.cu:2592-2657)
 // ---------------------------------------------------------------------------
@@ -1166,6 +1207,17 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
         if (!by_rows)
             plan = with_fine(e, pick_variant(false, e, instance_waves * plan.pieces, sparse_ll), plan, false, s.d_aug, degree, batch, s.L,
                              batch * n_coef * sizeof(T), sparse_ll, g_force_segments);
+        const HeadsEntry* heads = sizeof(T) == 8 && !by_rows ? heads_entry(s.d_aug, degree) : nullptr;
+        if (heads) {
+            const KernelEntry* run = pick_variant(false, e, total_waves(geom_of(e, int(s.d_aug)), int64_t(batch) * plan.pieces), sparse_ll);
+            const int pieces = heads_pieces(heads, run, plan, s.d_aug, batch, s.L, batch * n_coef * sizeof(T), sparse_ll);
+            if (pieces > 0) {
+                plan = SplitPlan{pieces, 0.0, 0.0};
+                tl_fine_more_pieces = true;         // needs memory that the tree kernels do not
+            } else {
+                heads = nullptr;
+            }
+        }
         int nseg = by_rows ? 1 : plan.pieces;
         FwdParams p;
         p.batch = int64_t(batch) * nseg; p.L = int64_t(s.L); p.d = int(s.d_aug); p.stream = stream;
@@ -1191,7 +1243,7 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
         }
         e = pick_variant(false, e, total_waves(geom_of(e, int(s.d_aug)), p.batch), sparse_ll);
         // staged sweeps of plain narrow paths form the increments themselves while staging the points
-        if (!by_rows && e->staged && !time_aug && !lead_lag && e->D > 0 && e->D <= kPointFedMaxDim && g_point_fed) {
+        if (!by_rows && !heads && e->staged && !time_aug && !lead_lag && e->D > 0 && e->D <= kPointFedMaxDim && g_point_fed) {
             p.inc = path;
             p.from_points = 1;
         } else {
@@ -1201,12 +1253,26 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
             compute_increments(path, inc, batch, dimension, length, time_aug, lead_lag, end_time, s, stream);
             p.inc = inc;
         }
-        const bool use_ll = !by_rows && sparse_ll && e->staged && e->fwd_lead_lag && !p.from_points;
-        const std::string shown = by_rows ? std::string(sizeof(T) == 8 ? "rows_fwd_f64_n" : "rows_fwd_f32_n") + std::to_string(degree)
+        const bool use_ll = !by_rows && !heads && sparse_ll && e->staged && e->fwd_lead_lag && !p.from_points;
+        const std::string shown = heads ? "heads_fwd_f64_d" + std::to_string(heads->D) + "_n" + std::to_string(degree)
+                                  : by_rows ? std::string(sizeof(T) == 8 ? "rows_fwd_f64_n" : "rows_fwd_f32_n") + std::to_string(degree)
                                   : use_ll ? std::string(e->name) + "_ll" : std::string(e->name);
         MainKernelTimer timer(stream, shown.c_str());
         tl_matrix_form = by_rows && sizeof(T) == 4;
-        if (by_rows) SIG_HIP(sizeof(T) == 4 ? launch_rows_fwd_mfma(p, int(degree)) : launch_rows_fwd_f64(p, int(degree)));
+        if (heads) {
+            const uint64_t path_bytes = s.L * uint64_t(heads->row) * sizeof(T);
+            const uint64_t chunk = std::min<uint64_t>(batch, kHeadsTableBytes / path_bytes);
+            HeadsParams hp;
+            hp.table = workspace(20, chunk * path_bytes + uint64_t(heads->row) * sizeof(T));
+            hp.L = p.L; hp.out_stride = p.out_stride; hp.scalar = p.scalar; hp.nseg = p.nseg; hp.lseg = p.lseg; hp.nonfinite = p.nonfinite;
+            hp.stream = stream;
+            for (uint64_t first = 0; first < batch; first += chunk) {
+                hp.inc = static_cast<const T*>(p.inc) + first * (s.L + 2) * s.d_aug;
+                hp.out = static_cast<T*>(p.out) + first * uint64_t(p.nseg) * uint64_t(p.out_stride);
+                hp.paths = int64_t(std::min<uint64_t>(chunk, batch - first));
+                SIG_HIP(heads->launch(hp));
+            }
+        } else if (by_rows) SIG_HIP(sizeof(T) == 4 ? launch_rows_fwd_mfma(p, int(degree)) : launch_rows_fwd_f64(p, int(degree)));
         else SIG_HIP(use_ll ? e->fwd_lead_lag(p) : e->fwd(p));
         timer.stop(/*defer=*/true);
         if (nseg > 1) {
@@ -1879,6 +1945,7 @@ CUSIG_AMD_API void cusig_amd_force_bwd_segments(int segments) noexcept { if (g_t
 CUSIG_AMD_API void cusig_amd_set_fine(int mode) noexcept { if (g_test_hooks) g_fine = mode; }
 CUSIG_AMD_API int cusig_amd_last_sweep_on_matrix_units(void) noexcept { return tl_matrix_form; }
 CUSIG_AMD_API void cusig_amd_set_rows_backward(int mode) noexcept { if (g_test_hooks) g_rows_backward = mode; }
+CUSIG_AMD_API void cusig_amd_set_heads_forward(int mode) noexcept { if (g_test_hooks) g_heads = mode; }
 CUSIG_AMD_API void cusig_amd_set_rows_forward(int mode) noexcept { if (g_test_hooks) g_rows_forward = mode; }
 
 CUSIG_AMD_API void cusig_amd_force_staged(int mode) noexcept { if (g_test_hooks) g_force_staged = mode; }
@@ -1923,6 +1990,7 @@ CUSIG_AMD_API void cusig_amd_enable_test_hooks(int enabled) noexcept
     g_fine = 1;
     g_rows_backward = 1;
     g_rows_forward = 1;
+    g_heads = 1;
     g_force_staged = -1;
     g_force_wide_index = 0;
     g_chen_adjoint_mode = 0;

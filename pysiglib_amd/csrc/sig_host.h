@@ -14,7 +14,7 @@ namespace sigamd {
 extern thread_local char g_last_error[4096];
 
 // Grow-only device buffers, one per (current device, slot), released by cusig_shutdown(); hold g_ws_mutex while a
-// buffer is in use (defined in sig_api.hip).  Slots 0-3: signature sweeps; 4-5: sig_join_backprop; 6: word tables of sig_coef; 7, 14, 15: tensor logarithm; 8-11: time-split backward; 12-13: degree-2 backward.
+// buffer is in use (defined in sig_api.hip).  Slots 0-3: signature sweeps; 4-5: sig_join_backprop; 6: word tables of sig_coef; 7, 14, 15: tensor logarithm; 8-11: time-split backward; 12-13: degree-2 backward; 18-19: degree 3 as products; 20: table of the sweeps with shared prefix chains.
 extern std::mutex g_ws_mutex;
 void* workspace(int slot, size_t bytes);
 

@@ -1896,3 +1896,54 @@ def test_staged_backward_partitions_vs_oracle(P, oracle, dtype, d, deg, tail, k)
     finally:
         L.CUSIG.cusig_amd_force_partition(0, 0)
         L.CUSIG.cusig_amd_set_profiling(0)
+
+
+@pytest.mark.parametrize("d,deg", [
+    (3, 9), (3, 10), (3, 11), (3, 12), (3, 13), (3, 14), (3, 15), (3, 16), (4, 9), (4, 10), (4, 11), (4, 12), (5, 8), (5, 9), (5, 10),
+    (5, 11), (6, 7), (6, 8), (6, 9), (7, 8), (7, 9), (8, 7), (8, 8), (9, 7), (9, 8), (10, 7), (11, 6), (11, 7), (12, 7)])
+def test_shared_prefix_chains_vs_oracle(P, oracle, d, deg):
+    """Forward sweeps of sig_heads.hip: a single step, both sides of one and of two chunks of head values (8 or 16 steps), paths in
+    pieces, the scalar term, an augmented path, the report of values that are not finite, and a device that cannot hold the table."""
+    import ctypes
+    from pysiglib_amd import _loader as L
+    lib = L.CUSIG
+    for hook in (lib.cusig_amd_set_heads_forward, lib.cusig_amd_force_segments):
+        hook.argtypes = (ctypes.c_int,)
+        hook.restype = None
+    lib.cusig_amd_set_alloc_limit.argtypes = (ctypes.c_uint64,)
+    lib.cusig_amd_set_alloc_limit.restype = None
+    lib.cusig_amd_last_kernel_name.restype = ctypes.c_char_p
+    rng = np.random.default_rng(100 * d + deg)
+    large = d ** deg > 2000000
+    cases = [(1, 18, 0, {})] if large else [(1, 2, 0, {}), (2, 9, 0, {}), (1, 10, 0, {}), (2, 17, 0, {}), (1, 18, 0, {}), (1, 34, 0, {}), (2, 36, 3, {}),
+                                            (1, 101, 0, dict(time_aug=True))]
+    try:
+        lib.cusig_amd_set_heads_forward(2)
+        lib.cusig_amd_set_profiling(1)
+        for batch, length, pieces, aug in cases:
+            x = np.cumsum(rng.standard_normal((batch, length, d - len(aug))), axis=1) / np.sqrt(length * d)
+            ref = oracle.signature(x, deg, scalar_term=True, n_jobs=-1, **aug)
+            lib.cusig_amd_force_segments(pieces)
+            got = P.sig(dev(x), deg, scalar_term=True, **aug)
+            assert lib.cusig_amd_last_kernel_name().decode() == "heads_fwd_f64_d%d_n%d" % (d, deg)
+            assert lib.cusig_amd_last_sig_nonfinite() == 0
+            assert torch.all(got[:, 0] == 1)
+            assert np.max(level_rel_err(got.cpu().numpy()[:, 1:], ref[:, 1:], d, deg)) < TOL[np.float64], (batch, length, pieces)
+            assert torch.equal(P.sig(dev(x), deg, **aug), got[:, 1:])
+        if not large:
+            lib.cusig_amd_force_segments(1)
+            # room for the increments and their slack (36 rows), not for the table, whose rows are at least twice as long
+            lib.cusig_shutdown()
+            lib.cusig_amd_set_alloc_limit((batch * (length + 1) + 36) * d * 9 + 256)
+            without = P.sig(dev(x), deg, **aug)
+            lib.cusig_amd_set_alloc_limit(0)
+            assert not lib.cusig_amd_last_kernel_name().decode().startswith("heads")
+            assert np.max(level_rel_err(without.cpu().numpy(), ref[:, 1:], d, deg)) < TOL[np.float64]
+            x[-1, -1, 0] = np.inf
+            P.sig(dev(x), deg, **aug)
+            assert lib.cusig_amd_last_sig_nonfinite() == 1
+    finally:
+        lib.cusig_amd_set_heads_forward(1)
+        lib.cusig_amd_force_segments(0)
+        lib.cusig_amd_set_alloc_limit(0)
+        lib.cusig_amd_set_profiling(0)
