@@ -301,6 +301,9 @@ CUSIG_AMD_API void cusig_amd_set_chen_low_levels(int enabled) CUSIG_AMD_NOEXCEPT
 CUSIG_AMD_API void cusig_amd_set_row_forms(int mode) CUSIG_AMD_NOEXCEPT;
 /* Whether such a form served the last sig_join* / sig_to_log_sig* call on this thread: 1 or 0. */
 CUSIG_AMD_API int cusig_amd_last_row_form(void) CUSIG_AMD_NOEXCEPT;
+/* Whether the last adjoint of a Chen product on this thread (sig_combine_backprop and what else calls it) took both factors in
+ * one pass over the gradient: 1 or 0.  cusig_amd_set_row_forms chooses that form too. */
+CUSIG_AMD_API int cusig_amd_last_chen_both(void) CUSIG_AMD_NOEXCEPT;
 /* Stream-ordered mode (no counterpart in the reference, off by default).  When enabled, signature_cuda_{f,d} and
  * sig_backprop_cuda_{f,d} enqueue their kernels on the null stream and return without waiting, and do not wait for
  * other streams on entry: inputs must be ordered before, and consumers after, the null stream (true for PyTorch's

@@ -221,7 +221,7 @@ std::atomic<int> g_force_wide_index{0};
 std::atomic<int> g_chen_adjoint_mode{0};
 std::atomic<int> g_chen_low_levels{1};
 std::atomic<int> g_row_forms{1};
-thread_local int tl_row_form = 0;
+thread_local int tl_row_form = 0, tl_chen_both = 0;
 std::mutex g_ws_mutex;
 static std::map<std::pair<int, int>, Workspace> g_ws;   // (device, slot)
 
@@ -1956,6 +1956,7 @@ CUSIG_AMD_API void cusig_amd_set_chen_low_levels(int enabled) noexcept { if (g_t
 
 CUSIG_AMD_API void cusig_amd_set_row_forms(int mode) noexcept { if (g_test_hooks) g_row_forms = mode; }
 CUSIG_AMD_API int cusig_amd_last_row_form(void) noexcept { return tl_row_form; }
+CUSIG_AMD_API int cusig_amd_last_chen_both(void) noexcept { return tl_chen_both; }
 
 CUSIG_AMD_API void cusig_amd_set_stream_ordered(int enabled) noexcept { g_stream_ordered = enabled; }
 

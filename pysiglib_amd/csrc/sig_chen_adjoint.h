@@ -12,11 +12,12 @@
 
 namespace sigamd {
 
-// Test hooks (defined in sig_api.hip).  g_row_forms: the forms of sig_join_stream.h and sig_log_rows.h never (0), where they are the
+// Test hooks (defined in sig_api.hip).  g_row_forms: the forms of sig_join_stream.h, sig_log_rows.h and sig_chen_both.h never (0), where they are the
 // sooner ones (1), wherever they apply (2); which one served the thread's last call is tl_row_form.  A test that asks for
 // a variant of the general kernels asks for those kernels.
 extern std::atomic<int> g_chen_adjoint_mode, g_row_forms;
 extern thread_local int tl_row_form;
+extern thread_local int tl_chen_both;       // 1: the thread's last adjoint of a Chen product took both factors in one pass
 inline int row_forms()
 {
     return g_chen_adjoint_mode != 0 || g_chen_low_levels != 1 || g_force_wide_index != 0 ? 0 : g_row_forms.load();

@@ -6,6 +6,7 @@
 #include <type_traits>
 
 #include "sig_kernels.h"
+#include "sig_chen_both.h"
 #include "sig_chen_stream.h"
 
 namespace sigamd {
@@ -200,6 +201,54 @@ static void launch_right_stream(const RightPlan& rp, const T* dC, T* dB, const T
     }
 }
 
+template <typename T, typename P>
+static void launch_both(const T* dC, T* dA, T* dB, const T* A, const T* B, uint64_t batch, const SigShape& s, hipStream_t stream)
+{
+    constexpr size_t lds = P::lds_entries() * sizeof(T);
+    static_assert(lds <= size_t(160) * 1024, "a row's pieces fit a compute unit");
+    if (lds > 64 * 1024)
+        SIG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(chen_adjoint_both_kernel<T, P>), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+    const uint64_t most = ((uint64_t(1) << 32) - 1) / P::THREADS;      // a launch numbers its threads with 32 bits; further items in the same blocks
+    hipLaunchKernelGGL((chen_adjoint_both_kernel<T, P>), dim3(unsigned(std::min<uint64_t>(batch * P::PARTS, most))), dim3(P::THREADS), lds, stream, dC, dA,
+                       dB, A, B, int64_t(batch) * P::PARTS, int64_t(s.stride), s.off);
+}
+
+template <typename... P>
+struct BothPlans {};
+template <typename Go, typename... P>
+static bool any_of_plans(Go&& go, BothPlans<P...>)
+{
+    return (go(P()) || ...);
+}
+
+// Both factors in one pass over dC, where there is such a kernel.  Blocks of a row (D / R), registers (waves a SIMD) and the rows from which
+// it takes over were measured for each (ms before / with, double precision): 1080 rows of 10 channels, degree 5: 1.05 / 0.85; 1806 of 9, 5: 1.30 /
+// 0.81; 4096 of 6, 5: 0.67 / 0.32, of 5, 6: 1.03 / 0.68, of 3, 7: 0.62 / 0.22; 298 of 13, 5: 2.99 / 0.93; 488 of 22, 4: 1.50 / 0.74; single row of 6,
+// 6: 0.167 / 0.072; of 8, 4: 0.053 / 0.057 (at 400 rows 0.065 / 0.063).  Slower: 2 channels, degree 11 (0.84 / 1.16), 8, 6 (1.28 / 1.33).
+template <typename T>
+static bool launch_both_factors(const T* dC, T* dA, T* dB, const T* A, const T* B, uint64_t batch, uint64_t dimension, uint64_t degree,
+                                const SigShape& s, hipStream_t stream, const SharedRows& dc)
+{
+    auto go = [&](auto plan) {
+        using P = decltype(plan);
+        if (dimension != uint64_t(P::D) || degree != uint64_t(P::N) || (row_forms() != 2 && batch < uint64_t(P::FROM))) return false;
+        launch_combine_bwd_items<T>(dC, dA, dB, A, B, batch, dimension, uint64_t(P::Q), s, stream, 3, dc, 2, 0);
+        launch_both<T, P>(dC, dA, dB, A, B, batch, s, stream);
+        tl_chen_both = 1;
+        return true;
+    };
+    return any_of_plans(go, BothPlans<BothPlan<4, 3, 4, 4, 192>, BothPlan<5, 3, 5, 4, 96>, BothPlan<6, 2, 6, 4, 256>, BothPlan<8, 2, 8, 4, 400>,
+                        BothPlan<9, 2, 9, 4, 48>, BothPlan<10, 2, 10, 3, 96>, BothPlan<11, 2, 11, 3, 1>, BothPlan<12, 2, 12, 3, 1>,
+                        BothPlan<13, 2, 13, 3, 1>, BothPlan<14, 2, 14, 3, 160>, BothPlan<15, 2, 15, 2, 128>, BothPlan<16, 2, 16, 2, 128>,
+                        BothPlan<17, 2, 17, 2, 1>, BothPlan<18, 2, 9, 2, 1>, BothPlan<19, 2, 19, 2, 1>, BothPlan<20, 2, 10, 2, 1>,
+                        BothPlan<21, 2, 7, 2, 1>, BothPlan<22, 2, 11, 2, 1>, BothPlan<24, 2, 8, 2, 1>, BothPlan<6, 3, 6, 4, 1>,
+                        BothPlan<7, 3, 1, 4, 1>, BothPlan<8, 3, 4, 3, 1>, BothPlan<9, 3, 3, 3, 1>, BothPlan<10, 3, 2, 3, 1>,
+                        BothPlan<11, 3, 1, 3, 1>, BothPlan<12, 3, 1, 3, 1>, BothPlan<13, 3, 1, 2, 1>, BothPlan<14, 3, 1, 2, 1>,
+                        BothPlan<16, 3, 1, 2, 1>, BothPlan<4, 4, 2, 4, 1>, BothPlan<5, 4, 1, 3, 1>, BothPlan<6, 4, 1, 3, 1>,
+                        BothPlan<7, 4, 1, 3, 1>, BothPlan<3, 5, 3, 4, 64>, BothPlan<4, 5, 1, 3, 1>, BothPlan<3, 6, 1, 3, 1>,
+                        BothPlan<2, 8, 1, 3, 1>>());
+}
+
 // launches the adjoint of the Chen product on `stream`
 template <typename T>
 void launch_combine_bwd(const T* dC, T* dA, T* dB, const T* A, const T* B, uint64_t batch, uint64_t dimension,
@@ -214,6 +263,10 @@ void launch_combine_bwd(const T* dC, T* dA, T* dB, const T* A, const T* B, uint6
     const bool streaming = mode != 2 && (mode == 1 || s.n_coef >= kStreamMinCoef) && dimension >= 2 && degree >= 2 &&
                            degree <= uint64_t(kStreamMaxLevels) && s.n_coef < (uint64_t(1) << 28) &&
                            !g_force_wide_index;
+    tl_chen_both = 0;
+    if (families == 2 && identity == 3 && !fold && row_forms() != 0 && dc.share == 1 && dc.stride == int64_t(s.stride) && dc.off == s.off &&
+        launch_both_factors<T>(dC, dA, dB, A, B, batch, dimension, degree, s, stream, dc))
+        return;
     LeftPlan lp;
     RowsPlan wp;
     RightPlan rp;

@@ -18,6 +18,7 @@
 // for scalar operands and for the other waves of a block at the end of a chunk.
 #include <algorithm>
 
+#include "sig_barrier.h"
 #include "sig_heads.h"
 #include "sig_kernels.h"
 
@@ -79,16 +80,6 @@ __global__ __launch_bounds__(kBlock) void head_table_kernel(const T* __restrict_
         const T z = letter < Plan::D ? inc[((r / L) * (L + 2) + 1 + r % L) * Plan::D + letter] : T(0);
         table[i] = z / by;
     }
-}
-
-__device__ __forceinline__ void lds_barrier()
-{
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0xc07f);     // own LDS operations have completed
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
 }
 
 // values read through the scalar cache: wave-uniform address, never written by the kernel that reads them

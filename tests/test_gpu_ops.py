@@ -958,3 +958,34 @@ def test_sig_join_backprop_workspace(P, oracle, row_forms, dtype, d, deg, batch)
     assert asked <= L.CUSIG.cusig_amd_workspace_bytes() <= asked + asked // 8 + 1024
     da, dz = oracle.sig_join_backprop(g.astype(np.float64), a.astype(np.float64), z.astype(np.float64), d, deg)
     assert row_rel_err(ga, da) < TOL[dtype] and row_rel_err(gz, dz) < TOL[dtype]
+
+
+@pytest.mark.parametrize("d,deg", [(4, 5), (5, 5), (6, 4), (8, 4), (9, 4), (10, 4), (11, 4), (12, 4), (13, 4), (14, 4), (15, 4), (16, 4), (17, 4), (18, 4),
+                                   (19, 4), (20, 4), (21, 4), (22, 4), (24, 4), (6, 5), (7, 5), (8, 5), (9, 5), (10, 5), (11, 5), (12, 5), (13, 5), (14, 5),
+                                   (16, 5), (4, 6), (5, 6), (6, 6), (7, 6), (3, 7), (4, 7), (3, 8), (2, 10)])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_combine_backprop_in_one_pass(P, oracle, row_forms, d, deg, dtype):
+    """The adjoint of the Chen product that takes both factors in one pass over dC, against the oracle; an entry of dC that is not finite
+    reaches the same gradients as in the general kernels."""
+    from pysiglib_amd import _loader as L
+    L.CUSIG.cusig_amd_last_chen_both.restype = ctypes.c_int
+    rng = np.random.default_rng(13 * d + deg)
+    scale = np.concatenate([np.full(d ** k, 1.0 / np.sqrt(float(d) ** k)) for k in range(deg + 1)])
+    a, b, g = ((rng.standard_normal((3, scale.size)) * scale).astype(dtype) for _ in range(3))
+    a[:, 0] = 1
+    b[:, 0] = 1
+    want = oracle.sig_combine_backprop(g, a, b, d, deg)
+    row_forms(2)
+    with_scalar = [v.cpu().numpy() for v in P.sig_combine_backprop(dev(g), dev(a), dev(b), d, deg)]
+    assert L.CUSIG.cusig_amd_last_chen_both() == 1
+    without = [v.cpu().numpy() for v in P.sig_combine_backprop(*(dev(np.ascontiguousarray(v[:, 1:])) for v in (g, a, b)), d, deg)]
+    for got, more, ref in zip(without, with_scalar, want):
+        assert row_rel_err(got, ref[:, 1:]) < TOL[dtype]
+        assert row_rel_err(more[:, 1:], ref[:, 1:]) < TOL[dtype] and np.all(more[:, 0] == 0)
+    g[1, -1 - d * d], g[2, scale.size - d ** deg - 1] = np.inf, np.nan
+    bad = [v.cpu().numpy() for v in P.sig_combine_backprop(dev(g), dev(a), dev(b), d, deg)]
+    row_forms(0)
+    general = [v.cpu().numpy() for v in P.sig_combine_backprop(dev(g), dev(a), dev(b), d, deg)]
+    assert L.CUSIG.cusig_amd_last_chen_both() == 0
+    for got, ref in zip(bad, general):
+        np.testing.assert_array_equal(np.isfinite(got), np.isfinite(ref))
