@@ -102,11 +102,15 @@ def rows_sweep_wins(dtype, D, N):
 
 def spec_shapes():
     """(D, N) pairs that get specialised kernels."""
-    caps = {2: 16, 3: 14, 4: 10, 5: 9, 6: 8, 7: 7, 8: 7}
-    caps.update({d: 5 for d in range(9, 21)})
-    caps.update({d: 6 for d in range(9, 13)})
-    caps.update({d: 4 for d in range(21, 49)})
-    caps.update({d: 5 for d in range(21, 25)})
+    # The last degree of each of 4 to 16 and all of 25 to 28 channels at degree 5 (4e6 to 2e7 coefficients), against the run-time
+    # kernels, ms: 4 channels, degree 11, double, 14 paths of 65 points, forward 5.67 / 0.63, backward 22.5 / 2.93; 7, 8, single, 10 paths
+    # 1.01 / 0.30, 6.79 / 0.87; 13, 6, double, 12 paths 0.94 / 0.50, 4.57 / 1.92; 28, 5, double, one path of 100 points
+    # 0.39 / 0.31, 2.47 / 1.34 (the least gains).
+    caps = {2: 16, 3: 14, 4: 12, 5: 10, 6: 9, 7: 8, 8: 8}
+    caps.update({d: 7 for d in range(9, 13)})
+    caps.update({d: 6 for d in range(13, 17)})
+    caps.update({d: 5 for d in range(17, 29)})
+    caps.update({d: 4 for d in range(29, 49)})
     caps.update({d: 3 for d in range(49, 129)})
     out = []
     for d, nmax in sorted(caps.items()):
@@ -176,6 +180,8 @@ def fine_partition(D, N, dtype, direction):
     double, degree 5, 128 points: backward 128 paths 127 / 72, forward 61 / 32, 512 paths 86 / 35."""
     if N < 3 or D > (64 if direction == "fwd" else 31):
         return None
+    if D >= 4 and N > 4 and D ** N >= 4000000 and not 17 <= D <= 24:
+        return None         # a path fills the chip by itself: 11 000 random calls 0.999 (forward) and 0.994 of the time, up to 1.12
     if direction == "bwd" and rows_sweep_wins(dtype, D, N):
         return None
     if (dtype, D, N, direction) in FINE:

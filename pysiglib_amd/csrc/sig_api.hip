@@ -144,13 +144,20 @@ static const KernelEntry* find_entry(bool backward, bool f64, uint64_t d, uint64
         if (run_time) it = m.find(std::make_tuple(int(f64), 0, int(degree)));
         if (it != m.end() && !it->second.empty()) {
             if (g_force_tail > 0) {
-                auto from = it;
-                if (run_time && g_force_run_time_wide && ipow64(int64_t(d), int(degree) - 1) >= 48) {
-                    auto w = m.find(std::make_tuple(int(f64), -1, int(degree)));
-                    if (w != m.end()) from = w;
+                auto forced = [](const std::vector<const KernelEntry*>& from) -> const KernelEntry* {
+                    for (const KernelEntry* e : from)
+                        if (e->tail == g_force_tail && e->k == g_force_k && !e->staged) return e;
+                    return nullptr;
+                };
+                // a partition that an instance does not have: the run-time kernels' one
+                const KernelEntry* e = run_time ? nullptr : forced(it->second);
+                if (!e) {
+                    const bool wide = g_force_run_time_wide && ipow64(int64_t(d), int(degree) - 1) >= 48;
+                    auto rt = m.find(std::make_tuple(int(f64), wide ? -1 : 0, int(degree)));
+                    if (wide && rt == m.end()) rt = m.find(std::make_tuple(int(f64), 0, int(degree)));
+                    if (rt != m.end()) e = forced(rt->second);
                 }
-                for (const KernelEntry* e : from->second)
-                    if (e->tail == g_force_tail && e->k == g_force_k && !e->staged) return e;
+                if (e) return e;
             }
             if (run_time) return pick_run_time_entry(backward, f64, int(d), int(degree));
             return it->second.front();

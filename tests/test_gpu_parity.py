@@ -1947,3 +1947,35 @@ def test_shared_prefix_chains_vs_oracle(P, oracle, d, deg):
         lib.cusig_amd_force_segments(0)
         lib.cusig_amd_set_alloc_limit(0)
         lib.cusig_amd_set_profiling(0)
+
+
+@pytest.mark.parametrize("d,deg", [(4, 11), (4, 12), (5, 10), (6, 9), (7, 8), (8, 8), (9, 7), (10, 7), (11, 7), (12, 7), (13, 6), (14, 6), (15, 6), (16, 6),
+                                   (25, 5), (26, 5), (27, 5), (28, 5)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_instances_of_the_largest_shapes(P, oracle, d, deg, dtype):
+    """The compiled instances of 4e6 to 2e7 coefficients, forward and backward: one step, both sides of a chunk of the ring, and the steps of
+    a lead-lag path."""
+    import ctypes
+    from pysiglib_amd import _loader as L
+    L.CUSIG.cusig_amd_set_heads_forward.argtypes = (ctypes.c_int,)
+    L.CUSIG.cusig_amd_set_heads_forward.restype = None
+    L.CUSIG.cusig_amd_last_kernel_name.restype = ctypes.c_char_p
+    rng = np.random.default_rng(100 * d + deg)
+    try:
+        L.CUSIG.cusig_amd_set_heads_forward(0)
+        L.CUSIG.cusig_amd_set_profiling(1)
+        for length, aug in ((2, {}), (18, {}), (5, dict(lead_lag=True, time_aug=d % 2 == 1))):
+            raw = d // 2 if aug else d
+            x = (np.cumsum(rng.standard_normal((1, length, raw)), axis=1) / np.sqrt(length * raw)).astype(dtype)
+            ref = oracle.signature(x.astype(np.float64), deg, n_jobs=-1, **aug)
+            got = P.sig(dev(x), deg, **aug)
+            assert L.CUSIG.cusig_amd_last_kernel_name().decode().startswith("fwd_%s_d%d_n%d_" % ("f32" if dtype == np.float32 else "f64", d, deg))
+            assert np.max(level_rel_err(got.cpu().numpy(), ref, d, deg)) < TOL[dtype]
+            g = rng.standard_normal(ref.shape).astype(dtype)
+            want = oracle.sig_backprop(x.astype(np.float64), ref, g.astype(np.float64), deg, n_jobs=-1, **aug)
+            back = P.sig_backprop(dev(x), dev(ref.astype(dtype)), dev(g), deg, **aug).cpu().numpy()
+            assert L.CUSIG.cusig_amd_last_kernel_name().decode().startswith("bwd_%s_d%d_n%d_" % ("f32" if dtype == np.float32 else "f64", d, deg))
+            assert bwd_rel_err(back, want) < TOL[dtype]
+    finally:
+        L.CUSIG.cusig_amd_set_heads_forward(1)
+        L.CUSIG.cusig_amd_set_profiling(0)
