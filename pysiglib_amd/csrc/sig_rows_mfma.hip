@@ -199,13 +199,20 @@ __global__ __launch_bounds__(kBlock, 4) void rows_fwd_mfma_kernel(
 //   1. red for all of them, 16x16x4 products (steps x letters) (letters x prefixes), through LDS to lane = prefix;
 //   2. the steps themselves: chain back, pullback; U_t[p] takes red's place in LDS;
 //   3. dz for all of them, (steps x prefixes) (prefixes x letters).
+// To degree 4 the products of 1. stand between the pieces of 2. of the sixteen steps before, one by one: the matrix and the
+// vector unit of a SIMD, 35 % of the time each when a wave used one at a time, then work side by side in one wave too
+// (degree 4, single precision, ms: 64 paths x 128 steps x 64 channels 10.9 -> 10.1, 1 x 399 x 65 2.30 -> 2.02, 8 x 33 x 96
+// 5.29 -> 5.01; degree 3: 300 x 49 x 64 0.477 -> 0.440).  At degrees 5 and 6 the steps are most of the work and the next
+// steps' operands would not fit the registers (1 x 399 x 34, degree 5: 4.85 -> 4.93), so 1. comes first there.  3. in the
+// same manner, as products of four steps (4x4x1), gained nothing more (10.02 -> 10.08).
 // The wave holds its tile of G in both operand layouts (128 registers); each product is summed in two halves of K.
 // The pieces of a step's gradient row stay in the waves' own LDS until the block adds them up and onto the row.  Thousands
 // of blocks add to a row: it is kept in double precision, so that their number costs no accuracy.
 // ---------------------------------------------------------------------------
 constexpr int kMxSteps = 16;
 constexpr int kMxStride = 68;       // words per step: writes of four rows apart and 16-byte reads of 16 rows both spread over all banks
-constexpr int kMxWaveWords = 2 * kMxSteps * kMxStride;
+constexpr int kMxBuf = kMxSteps * kMxStride;
+constexpr int kMxWaveWords = 3 * kMxBuf;      // red / U of these and of the next steps, pieces
 constexpr int kMxGroup = 4;        // steps in a straight line: their red values and increments are loaded together
 // Waves per block: two blocks share a CU and drift apart, so that one's products run beside the other's chains (16 paths of
 // 200 steps, 64 channels, degree 4, with elements dealt out one by one at the
@@ -224,6 +231,7 @@ __global__ __launch_bounds__((kMxWaves * kWave), 2) void rows_bwd_mfma_kernel(
     using Ad = TreeAdj<T, -1, N, 1, 1>;
     constexpr int M = N - 1;
     constexpr int W = kMxWaves;
+    constexpr bool kAhead = N <= 4;                     // red of the next steps between the pieces of these
     static_assert(M >= 2, "degree 3 and up");
     const int lane = threadIdx.x & (kWave - 1);
     const int wib = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
@@ -298,7 +306,8 @@ __global__ __launch_bounds__((kMxWaves * kWave), 2) void rows_bwd_mfma_kernel(
     T* mx_lds = reinterpret_cast<T*>(mx_lds_raw);
     __shared__ int wave_a0[W], wave_l0[W];
     T* mine = mx_lds + wib * kMxWaveWords;              // [step][kMxStride]: red, then U, then the by-letter sums
-    T* mine_c = mine + kMxSteps * kMxStride;            // pieces of the last prefix letter
+    T* mine_next = mine + kMxBuf;                       // red of the steps after these
+    T* mine_c = mine + 2 * kMxBuf;                      // pieces of the last prefix letter
     T* tile = mx_lds + W * kMxWaveWords;                // [step][d]: pieces of the shared prefix letters
     for (int e = threadIdx.x; e < kMxSteps * d; e += W * kWave) tile[e] = T(0);
     if (lane == 0) {
@@ -323,34 +332,69 @@ __global__ __launch_bounds__((kMxWaves * kWave), 2) void rows_bwd_mfma_kernel(
     };
     fetch_last();
     struct alignas(4) Quad { T v[4]; };                 // the rows have the alignment of an element
-    for (int64_t t_first = L - 1; t_first >= 0; t_first -= kMxSteps) {
-        const int n = t_first + 1 < kMxSteps ? int(t_first + 1) : kMxSteps;
-        T pz_shared[M - 1];                             // the shared prefix letters: lane s holds those of step t_first - s
-        {
-            // rows in front of the path read its zero row; letters beyond the row meet adjoints that are zero
-            const int64_t t = t_first - x16 < 0 ? int64_t(-1) : t_first - x16;
-            const T* zt = zbase + t * d;
+    // the rows of the steps from t_first on: rows in front of the path read its zero row; letters beyond the row meet adjoints
+    // that are zero
+    auto step_row = [&](int64_t t_first) {
+        const int64_t t = t_first - x16 < 0 ? int64_t(-1) : t_first - x16;
+        return zbase + t * d;
+    };
+    T pz_shared[M - 1], pz_ahead[M - 1];                // the shared prefix letters: lane s holds those of step t_first - s
+    auto all_red = [&](int64_t t_first) {
+        const T* zt = step_row(t_first);
 #pragma unroll
-            for (int l = 0; l < M - 1; ++l) pz_shared[l] = zt[tl.pu[l]];
-            const Quad* zp = reinterpret_cast<const Quad*>(zt + a0 + 16 * g16);
-            f32x4 c[4][2];
+        for (int l = 0; l < M - 1; ++l) pz_ahead[l] = zt[tl.pu[l]];
+        const Quad* zp = reinterpret_cast<const Quad*>(zt + a0 + 16 * g16);
+        f32x4 c[4][2];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) c[i >> 1][i & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
-            Quad zq[4];
+        for (int i = 0; i < 8; ++i) c[i >> 1][i & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+        Quad zq[4];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) zq[k] = zp[k];
+        for (int k = 0; k < 4; ++k) zq[k] = zp[k];
 #pragma unroll
-            for (int k = 0; k < 16; ++k)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    c[i][k >> 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(zq[k >> 2].v[k & 3], gp[i][k], c[i][k >> 3], 0, 0, 0);
+        for (int k = 0; k < 16; ++k)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
+                c[i][k >> 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(zq[k >> 2].v[k & 3], gp[i][k], c[i][k >> 3], 0, 0, 0);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) mine[(4 * g16 + r) * kMxStride + 16 * i + x16] = c[i][0][r] + c[i][1][r];
-        }
-        for (int s0 = 0; s0 < n; s0 += kMxGroup) {
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) mine[(4 * g16 + r) * kMxStride + 16 * i + x16] = c[i][0][r] + c[i][1][r];
+    };
+    if constexpr (kAhead) all_red(L - 1);
+    int turn = 0;                                       // which of the two buffers is `mine`
+    [[maybe_unused]] Quad zq[4];                        // the next steps' increments, left operand of red
+    [[maybe_unused]] auto fetch_rows = [&](int64_t t_first) {
+        const Quad* zp = reinterpret_cast<const Quad*>(step_row(t_first) + a0 + 16 * g16);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) zq[k] = zp[k];
+    };
+    if constexpr (kAhead)
+        if (L > kMxSteps) fetch_rows(L - 1 - kMxSteps);
+    for (int64_t t_first = L - 1; t_first >= 0; t_first -= kMxSteps) {
+        const int n = t_first + 1 < kMxSteps ? int(t_first + 1) : kMxSteps;
+        if constexpr (!kAhead) all_red(t_first);
+#pragma unroll
+        for (int l = 0; l < M - 1; ++l) pz_shared[l] = pz_ahead[l];
+        [[maybe_unused]] const T* zt_ahead = step_row(t_first - kMxSteps);
+        // four steps; PART >= 0: sixteen prefixes' part of the next steps' red, a product between the pieces of a step
+        auto group = [&](int s0, auto part) {
+            constexpr int PART = decltype(part)::value;
+            constexpr bool AHEAD = PART >= 0;
+            constexpr int I = AHEAD ? PART : 0;
             T zl[kMxGroup], red[kMxGroup], dcs[M - 1][kMxGroup];
+            [[maybe_unused]] f32x4 c0 = f32x4{0.f, 0.f, 0.f, 0.f}, c1 = c0;
+            if constexpr (PART == 3) {
+#pragma unroll
+                for (int l = 0; l < M - 1; ++l) pz_ahead[l] = zt_ahead[tl.pu[l]];
+            }
+            auto product = [&](int k) {
+                if constexpr (AHEAD) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (k < 8) c0 = __builtin_amdgcn_mfma_f32_16x16x4f32(zq[k >> 2].v[k & 3], gp[I][k], c0, 0, 0, 0);
+                    else c1 = __builtin_amdgcn_mfma_f32_16x16x4f32(zq[k >> 2].v[k & 3], gp[I][k], c1, 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            };
 #pragma unroll
             for (int k = 0; k < kMxGroup; ++k) {
                 zl[k] = zl_next[k];
@@ -364,7 +408,9 @@ __global__ __launch_bounds__((kMxWaves * kWave), 2) void rows_bwd_mfma_kernel(
                 in.pz[M - 1] = zl[k];
                 in.zs[0] = red[k];
                 typename Tr::Chain unmul;
+                product(4 * k);
                 S.template fwd_step<AllLetters, true>(in, &unmul);
+                product(4 * k + 1);
                 T u;
                 if constexpr (Tr::kLockstep) {
                     typename Tr::Chain ch;
@@ -381,7 +427,9 @@ __global__ __launch_bounds__((kMxWaves * kWave), 2) void rows_bwd_mfma_kernel(
                 dz.da[0] = T(0);
 #pragma unroll
                 for (int l = 0; l < M; ++l) dz.dc[l] = T(0);
+                product(4 * k + 2);
                 A.template pullback<-1, AllLetters>(S, in, dz, Tr::kLockstep ? &unmul : nullptr);
+                product(4 * k + 3);
                 mine_c[(s0 + k) * kMxStride + lane] = dz.dc[M - 1];
 #pragma unroll
                 for (int l = 0; l < M - 1; ++l) dcs[l][k] = dz.dc[l];
@@ -396,7 +444,21 @@ __global__ __launch_bounds__((kMxWaves * kWave), 2) void rows_bwd_mfma_kernel(
                 letter = x16 == l ? tl.pu[l] : letter;
             }
             if (x16 < M - 1) lds_add_shared(&tile[(s0 + g16) * d + letter], piece);
+            if constexpr (AHEAD) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) mine_next[(4 * g16 + r) * kMxStride + 16 * I + x16] = c0[r] + c1[r];
+            }
+        };
+        bool ahead = false;
+        if constexpr (kAhead) {
+            ahead = t_first >= kMxSteps;
+            if (ahead) {
+                static_for<0, 3>([&](auto part) { group(decltype(part)::value * kMxGroup, part); });
+                if (t_first >= 2 * kMxSteps) fetch_rows(t_first - 2 * kMxSteps);
+            }
         }
+        if (!ahead)
+            for (int s0 = 0; s0 < n; s0 += kMxGroup) group(s0, IntC<-1>{});
         {
             f32x4 c[4][2];
 #pragma unroll
@@ -428,13 +490,19 @@ __global__ __launch_bounds__((kMxWaves * kWave), 2) void rows_bwd_mfma_kernel(
                 for (int k = 0; k < W; ++k) {
                     const T* wr = mx_lds + k * kMxWaveWords + s * kMxStride;
                     const unsigned ia = unsigned(a - wave_a0[k]), il = unsigned(a - wave_l0[k]);
-                    if (ia < unsigned(kWave)) v += wr[ia];
-                    if (il < unsigned(kWave)) v += wr[kMxSteps * kMxStride + il];
+                    if (ia < unsigned(kWave)) v += wr[turn * kMxBuf + ia];
+                    if (il < unsigned(kWave)) v += wr[2 * kMxBuf + il];
                 }
                 dev_add(&out[a - int64_t(s) * d], double(v));       // step s lies s gradient rows before t_first
             }
         }
         __syncthreads();
+        if constexpr (kAhead) {
+            T* const other = mine;
+            mine = mine_next;
+            mine_next = other;
+            turn ^= 1;
+        }
     }
 }
 

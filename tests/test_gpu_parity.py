@@ -814,6 +814,21 @@ def test_by_row_sweeps_on_the_matrix_units(P, oracle, by_rows, shape, aug, scala
     assert bwd_rel_err(got, want) <= 1e-5
 
 
+@pytest.mark.parametrize("steps", [15, 16, 17, 31, 32, 33, 36, 48, 65])
+@pytest.mark.parametrize("channels,deg", [(65, 3), (49, 4), (33, 5)])
+def test_chunks_of_the_reverse_sweep_on_the_matrix_units(P, oracle, by_rows, channels, deg, steps):
+    """Chunks of sixteen steps that prepare the next one, the last one in part or whole; degree 5 prepares each chunk for itself.
+    The same bound as above."""
+    rng = np.random.default_rng(steps * 100 + channels)
+    x = (np.cumsum(rng.standard_normal((2, steps + 1, channels)), axis=1) / np.sqrt(channels * steps)).astype(np.float32)
+    ref = oracle.signature(x.astype(np.float64), deg, n_jobs=-1)
+    g = rng.standard_normal(ref.shape).astype(np.float32)
+    got = P.sig_backprop(dev(x), dev(ref.astype(np.float32)), dev(g), deg).cpu().numpy()
+    assert by_rows.last_name() == "rows_bwd_f32_n%d" % deg and by_rows.last_on_matrix_units() == 1
+    want = oracle.sig_backprop(x.astype(np.float64), ref, g.astype(np.float64), deg, n_jobs=-1)
+    assert bwd_rel_err(got, want) <= 1e-5
+
+
 @pytest.mark.parametrize("shape,aug,scalar_term", [
     ((1, 5, 64, 4), {}, False), ((2, 6, 49, 4), {}, True), ((2, 5, 70, 4), {}, False),
     ((2, 4, 52, 4), dict(time_aug=True), False), ((1, 4, 130, 3), {}, True),
