@@ -272,7 +272,7 @@ void launch_combine_bwd(const T* dC, T* dA, T* dB, const T* A, const T* B, uint6
     RightPlan rp;
     const bool rows = streaming && make_rows_plan(wp, dimension, degree, kStreamLdsEntries);
     const bool left = rows || (streaming && make_left_plan(lp, dimension, degree, kStreamLdsEntries));
-    const bool right = streaming && families > 1 && make_right_plan(rp, dimension, degree);
+    const bool right = streaming && families > 1 && make_right_plan(rp, dimension, degree, batch);
     if (!left && !right) {
         launch_combine_bwd_items<T>(dC, dA, dB, A, B, batch, dimension, degree, s, stream, identity, dc, families, 0);
         return;

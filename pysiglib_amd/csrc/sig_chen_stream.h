@@ -718,7 +718,29 @@ static inline bool fill_stream_levels(StreamLevels& lv, uint64_t d, uint64_t deg
 }
 
 // the lanes' word length: enough words for four waves per row, and a walk of at most kRightMaxRel levels
-static inline bool make_right_plan(RightPlan& P, uint64_t d, uint64_t degree)
+// Length of the lanes' words.  A short one leaves few lanes with long walks, d + .. + d^rel loads one after the other (one row of 16 channels,
+// degree 6: 256 lanes, 69904 each); a long one makes every lane add to the words below its own, d words for all of them in the first level.  Both
+// factors' gradients, us, by length (single precision): 1 row of 16, 6: 23462 (2), 1487 (3), 735 (4), 3237 (5); 16 rows of 26, 5: 7964 (2),
+// 1622 (3), 2231 (4); 16 of 9, 7: 3328 (3), 1192 (4), 1469 (5); 64 of 16, 5: 1877 (2), 459 (3), 1520 (4); 256 of 4, 9: 1055 (5), 1203 (6).
+// The estimate, us: 0.35 a load of the walk while a SIMD has no second wave of them; 0.03 an addition to one address, 2e-5 any; a longer
+// word has to save 15.
+static inline int right_word_length(uint64_t d, int degree, uint64_t batch, int shortest)
+{
+    auto estimate = [&](int qe) {
+        double words = 1.0, walk = 0.0;
+        for (int i = 0; i < qe; ++i) words *= double(d);
+        for (int i = qe; i < degree; ++i) walk = (walk + 1.0) * double(d);
+        const double waves = double(batch) * words / kWave;
+        const double adds = qe > 1 ? std::max(0.03 * words / double(d), 2e-5 * words * double(batch) * (qe - 1)) : 0.0;
+        return 0.35 * walk * std::max(1.0, waves / 1024.0) + adds;
+    };
+    int best = shortest;
+    for (int qe = shortest + 1; qe <= degree - 1 && qe - 1 <= kRightMaxLow; ++qe)
+        if (estimate(qe) + 15.0 * (qe - best) < estimate(best)) best = qe;
+    return best;
+}
+
+static inline bool make_right_plan(RightPlan& P, uint64_t d, uint64_t degree, uint64_t batch)
 {
     if (d < 2 || degree < 2 || !fill_stream_levels(P.lv, d, degree)) return false;
     int qmin = 1;
@@ -726,6 +748,7 @@ static inline bool make_right_plan(RightPlan& P, uint64_t d, uint64_t degree)
     while (words < 256 && qmin < int(degree) - 1) { ++qmin; words *= d; }
     int qe = std::max(qmin, int(degree) - kRightMaxRel);
     if (qe > int(degree) - 1 || qe - 1 > kRightMaxLow) return false;
+    qe = right_word_length(d, int(degree), batch, qe);
     P.degree = int(degree);
     P.qe = qe;
     P.rel = int(degree) - qe;

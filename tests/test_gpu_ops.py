@@ -989,3 +989,25 @@ def test_combine_backprop_in_one_pass(P, oracle, row_forms, d, deg, dtype):
     assert L.CUSIG.cusig_amd_last_chen_both() == 0
     for got, ref in zip(bad, general):
         np.testing.assert_array_equal(np.isfinite(got), np.isfinite(ref))
+
+
+@pytest.mark.parametrize("batch,d,deg", [(1, 4, 7), (1, 5, 8), (3, 7, 6), (1, 8, 6), (2, 16, 4), (1, 16, 5), (2, 20, 4), (1, 34, 4)])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_few_rows_of_the_chen_adjoint(P, oracle, row_forms, batch, d, deg, dtype):
+    """Few rows, where the right factor's lanes own longer words and walk in front of them less: both gradients against the oracle, the adjoint
+    that folds the exponential into the walk, and the logarithm's, which reads a row of dC for several products."""
+    rng = np.random.default_rng(17 * d + deg)
+    scale = np.concatenate([np.full(d ** k, 1.0 / np.sqrt(float(d) ** k)) for k in range(deg + 1)])
+    a, b, g = ((rng.standard_normal((batch, scale.size)) * scale).astype(dtype) for _ in range(3))
+    a[:, 0] = b[:, 0] = 1
+    z = (rng.standard_normal((batch, d)) / np.sqrt(d)).astype(dtype)
+    row_forms(0)
+    for got, ref in zip(P.sig_combine_backprop(dev(g), dev(a), dev(b), d, deg), oracle.sig_combine_backprop(g, a, b, d, deg)):
+        got = got.cpu().numpy()
+        assert row_rel_err(got[:, 1:], ref[:, 1:]) < TOL[dtype] and np.all(got[:, 0] == 0)
+        assert row_rel_err(got[:, 1:d + 1], ref[:, 1:d + 1]) < TOL[dtype]       # the level that every lane adds to
+    for got, ref in zip(P.sig_join_backprop(dev(g), dev(a), dev(z), d, deg), oracle.sig_join_backprop(g, a, z, d, deg)):
+        assert row_rel_err(got.cpu().numpy(), ref) < TOL[dtype]
+    if scale.size < 100000:
+        got = P.sig_to_log_sig_backprop(dev(a), dev(g), d, deg, method=0).cpu().numpy()
+        assert row_rel_err(got[:, 1:], oracle.sig_to_log_sig_backprop(a, g, d, deg)[:, 1:]) < TOL[dtype]
