@@ -102,6 +102,27 @@ static const KernelEntry* choose_entry(bool backward, bool f64, uint64_t d, uint
                : spec;
 }
 
+// Where choose_entry's estimate asks for the run-time kernel and no finer partition takes its place, the instance after all (else null): time pieces and
+// the staged twin make it the sooner one of 16548 random calls in that state, but where this rule says (9700 calls with the instance now: 0.81 of their time,
+// 25 of them 1.03 to 1.08 times as long; 571 paths x 6136 steps x 12 channels, degree 3, double, backward 14.6 -> 4.0 ms; 1 x 15 x 29, degree 4, single
+// 0.26 -> 0.06):
+// - forward, lanes that hold one level, or few steps: 0.92 on average, but up to 1.47 (3 x 731 x 13, degree 3);
+// - backward, lanes that hold four levels and more: 135 x 80 x 2, degree 9, single 0.19 -> 0.34;
+// - backward, few steps: 40 us -> 47 (5 x 4 x 32, degree 3); many steps in all of few coefficients: 116 x 13224 x 2, degree 4, 0.39 -> 0.59;
+//   few paths of 128 to 511 steps, which instances do not cut yet: 2 x 345 x 8, degree 4, double 0.13 -> 0.19.
+static const KernelEntry* instance_after_all(const KernelEntry* e, bool backward, uint64_t d, uint64_t degree, uint64_t batch, uint64_t L)
+{
+    if (e->D != 0 || g_force_tail > 0) return nullptr;
+    const KernelEntry* spec = find_entry(backward, e->is_f64 != 0, d, degree);
+    if (!spec || spec->D <= 0) return nullptr;
+    if (!backward) return L >= 256 && spec->tail >= 2 ? spec : nullptr;
+    if (L < 8 || spec->tail >= 4) return nullptr;
+    const int64_t top = ipow64(int64_t(d), int(degree));
+    if (top <= 32 && batch * L > 100000) return nullptr;
+    if (top >= 4096 && batch <= 8 && L >= 128 && L < 512) return nullptr;
+    return spec;
+}
+
 // Shapes without a specialised instance run a run-time-dimension kernel.  Its default carries few depth-1 letters
 // per lane in the packed layout, which suits the few lanes of small shapes.  Up to degree 10 there are variants with
 // more letters per lane (the chain work of a lane is shared by more top-level updates), most of them in the wide
@@ -1187,7 +1208,7 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
         // 48 channels 2.40 -> 2.11, two 4.37 -> 3.48).  Lead-lag paths of that many channels have no instance that skips the
         // letters a step cannot move (those end at 40), so the same holds for them (degree 3, 200 paths of 129 points, 60
         // channels, 120 augmented: 8.72 -> 2.11 ms, 4.42 as library products; 100 x 129 x 64: 2.90 -> 1.14, 2.41).
-        const int64_t instance_waves = total_waves(geom_of(e, int(s.d_aug)), int64_t(batch));
+        int64_t instance_waves = total_waves(geom_of(e, int(s.d_aug)), int64_t(batch));
         auto split = [&]() -> SplitPlan {
             if (g_force_segments > 0) return {int(std::min<uint64_t>(uint64_t(g_force_segments), s.L)), 0.0, 0.0};
             return choose_segments(instance_waves, int64_t(s.L), resident_waves(e), batch * (s.full_len - 1) * sizeof(T),
@@ -1211,9 +1232,19 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
             by_rows = rows_fwd_seconds(s.d_aug, batch, s.L) < instance_fwd_seconds(run, plan, instance_waves, s.d_aug, s.L);
         }
         const uint64_t n_coef = s.full_len - 1;
-        if (!by_rows)
-            plan = with_fine(e, pick_variant(false, e, instance_waves * plan.pieces, sparse_ll), plan, false, s.d_aug, degree, batch, s.L,
+        auto finer = [&]() {
+            return with_fine(e, pick_variant(false, e, instance_waves * plan.pieces, sparse_ll), plan, false, s.d_aug, degree, batch, s.L,
                              batch * n_coef * sizeof(T), sparse_ll, g_force_segments);
+        };
+        if (!by_rows) {
+            plan = finer();
+            if (const KernelEntry* spec = instance_after_all(e, false, s.d_aug, degree, batch, s.L)) {
+                e = spec;
+                instance_waves = total_waves(geom_of(e, int(s.d_aug)), int64_t(batch));
+                plan = split();
+                plan = finer();
+            }
+        }
         const HeadsEntry* heads = sizeof(T) == 8 && !by_rows ? heads_entry(s.d_aug, degree) : nullptr;
         if (heads) {
             const KernelEntry* run = pick_variant(false, e, total_waves(geom_of(e, int(s.d_aug)), int64_t(batch) * plan.pieces), sparse_ll);
@@ -1619,7 +1650,7 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
         // the matrix form of single precision competes with it, the estimates decide (64 paths of 200 steps, 40 channels
         // 0.328 -> 0.234 ms, 16 x 200, 36: 0.340 -> 0.121); at degree 4 and 40 channels its tiles are 39 % filled: 4.6 -> 6.0
         // ms.  Lead-lag paths are left to the instances that skip their still letters.
-        const int64_t instance_waves = total_waves(geom_of(e, int(s.d_aug)), int64_t(batch));
+        int64_t instance_waves = total_waves(geom_of(e, int(s.d_aug)), int64_t(batch));
         auto split = [&]() -> SplitPlan {
             if (arena || !ef || degree > uint64_t(kCombMaxLevels)) return {1, 0.0, 0.0};
             if (g_force_bwd_segments > 0) return {int(std::min<uint64_t>(uint64_t(g_force_bwd_segments), s.L)), 0.0, 0.0};
@@ -1640,9 +1671,19 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
         SplitPlan plan{1, 0.0, 0.0};
         if (!by_rows || compare) plan = split();
         if (compare && by_rows) by_rows = rows_bwd_seconds(s.d_aug, batch, s.L) < instance_bwd_seconds(plan, s.d_aug);
-        if (!by_rows && !arena)
-            plan = with_fine(e, pick_variant(true, e, instance_waves * plan.pieces, sparse_ll), plan, true, s.d_aug, degree, batch, s.L,
+        auto finer = [&]() {
+            return with_fine(e, pick_variant(true, e, instance_waves * plan.pieces, sparse_ll), plan, true, s.d_aug, degree, batch, s.L,
                              batch * n_coef * sizeof(T), sparse_ll, g_force_bwd_segments, !ef || degree > uint64_t(kCombMaxLevels));
+        };
+        if (!by_rows && !arena) {
+            plan = finer();
+            if (const KernelEntry* spec = instance_after_all(e, true, s.d_aug, degree, batch, s.L)) {
+                e = spec;
+                instance_waves = total_waves(geom_of(e, int(s.d_aug)), int64_t(batch));
+                plan = split();
+                plan = finer();
+            }
+        }
         int nseg = by_rows ? 1 : plan.pieces;
         int64_t lseg = int64_t(s.L);
         if (nseg > 1) {

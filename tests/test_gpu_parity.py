@@ -1994,3 +1994,26 @@ def test_instances_of_the_largest_shapes(P, oracle, d, deg, dtype):
     finally:
         L.CUSIG.cusig_amd_set_heads_forward(1)
         L.CUSIG.cusig_amd_set_profiling(0)
+
+
+@pytest.mark.parametrize("batch,length,d,deg,instance", [
+    (1, 9, 29, 4, True), (1, 8, 29, 4, False), (14, 42, 2, 4, True), (14, 42, 2, 9, False), (2, 128, 8, 4, True), (2, 129, 8, 4, False),
+    (2, 512, 8, 4, False), (2, 513, 8, 4, True), (100, 1000, 2, 4, True), (101, 1002, 2, 4, False), (65, 70, 12, 3, True)])
+def test_instances_where_lanes_are_few(P, oracle, batch, length, d, deg, instance):
+    """Backward, double precision (degree 9: single), launches that leave the chip without work: either side of the lines between the compiled
+    instances and the run-time kernels, whichever of them the shape's partition puts there."""
+    from pysiglib_amd import _loader as L
+    dtype = np.float32 if deg == 9 else np.float64
+    rng = np.random.default_rng(100 * d + length)
+    x = (np.cumsum(rng.standard_normal((batch, length, d)), axis=1) / np.sqrt(length * d)).astype(dtype)
+    ref = oracle.signature(x, deg, n_jobs=-1)
+    g = rng.standard_normal(ref.shape).astype(dtype)
+    want = oracle.sig_backprop(x, ref, g, deg, n_jobs=-1)
+    L.CUSIG.cusig_amd_set_profiling(1)
+    try:
+        got = P.sig_backprop(dev(x), dev(ref), dev(g), deg).cpu().numpy()
+        name = L.CUSIG.cusig_amd_last_kernel_name().decode()
+    finally:
+        L.CUSIG.cusig_amd_set_profiling(0)
+    assert not (instance and "_d0_" in name), name
+    assert bwd_rel_err(got, want) <= TOL[dtype]
