@@ -461,8 +461,9 @@ static constexpr HeadsEntry entry(int step_ns, int lone_ns)
 // tree kernels.  ms before / with: 3 channels, degree 9 .. 14: 2.80 / 1.98, 7.14 / 4.84, 7.58 / 4.92, 6.53 / 4.71, 8.83 / 4.65, 9.61 / 4.66;
 // 4, 9 and 10: 4.25 / 3.81, 4.46 / 3.72; 5, 8 and 9: 4.09 / 3.46, 4.55 / 3.38; 6, 7 and 8: 3.14 / 2.77, 3.53 / 2.56; 8, 7: 3.25 / 2.47; 11, 6:
 // 3.64 / 2.78; 4, 11 and 12: 5.02 / 4.22, 5.09 / 3.62; 5, 10: 5.33 / 3.51; 6, 9: 3.70 / 2.52; 7, 8: 3.68 / 2.97; 8, 8: 3.25 / 2.31; 10, 7:
-// 3.26 / 2.45.  3, 15 and 16, 5, 11, 7, 9 and 9, 8 have no compiled tree kernel (3, 15: 94.0 / 4.89).  2 channels, and fewer levels
-// than these, are faster in the tree kernels (2, 14: 3.9 / 4.3; 7, 6: 2.8 / 3.6).
+// 3.26 / 2.45.  3, 15 and 16, 5, 11, 7, 9 and 9, 8 have no compiled tree kernel (3, 15: 94.0 / 4.89).  12, 7 gains only in
+// calls that leave the tree kernel a last round of few waves (2 x 400: 1.84 / 1.70).  2 channels, 9 and 11 at degree 7, and fewer levels than these,
+// are faster in the tree kernels (2, 14: 3.9 / 4.3; 7, 6: 2.8 / 3.6).
 static const HeadsEntry kHeads[] = {
     entry<HeadPlan<3, 9, 5, 4, 1, 3, 4, 8, 1>>(545, 305),
     entry<HeadPlan<3, 10, 6, 3, 3, 3, 4, 8, 1>>(620, 309),
@@ -487,11 +488,9 @@ static const HeadsEntry kHeads[] = {
     entry<HeadPlan<7, 9, 4, 2, 7, 11, 3, 16, 1>>(470, 440),
     entry<HeadPlan<8, 7, 3, 2, 4, 15, 4, 16, 1>>(380, 380),
     entry<HeadPlan<8, 8, 4, 2, 4, 15, 4, 16, 1>>(390, 380),
-    entry<HeadPlan<9, 7, 4, 2, 3, 14, 4, 16, 16>>(330, 320),
     entry<HeadPlan<9, 8, 4, 2, 3, 14, 4, 16, 16>>(360, 340),
     entry<HeadPlan<10, 7, 3, 2, 5, 11, 3, 16, 1>>(410, 400),
     entry<HeadPlan<11, 6, 4, 2, 1, 11, 8, 16, 1>>(240, 230),
-    entry<HeadPlan<11, 7, 5, 2, 1, 11, 8, 16, 1>>(260, 240),
     entry<HeadPlan<12, 7, 3, 2, 3, 14, 4, 16, 16>>(400, 390),
 };
 

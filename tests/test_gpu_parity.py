@@ -1915,7 +1915,7 @@ def test_staged_backward_partitions_vs_oracle(P, oracle, dtype, d, deg, tail, k)
 
 @pytest.mark.parametrize("d,deg", [
     (3, 9), (3, 10), (3, 11), (3, 12), (3, 13), (3, 14), (3, 15), (3, 16), (4, 9), (4, 10), (4, 11), (4, 12), (5, 8), (5, 9), (5, 10),
-    (5, 11), (6, 7), (6, 8), (6, 9), (7, 8), (7, 9), (8, 7), (8, 8), (9, 7), (9, 8), (10, 7), (11, 6), (11, 7), (12, 7)])
+    (5, 11), (6, 7), (6, 8), (6, 9), (7, 8), (7, 9), (8, 7), (8, 8), (9, 8), (10, 7), (11, 6), (12, 7)])
 def test_shared_prefix_chains_vs_oracle(P, oracle, d, deg):
     """Forward sweeps of sig_heads.hip: a single step, both sides of one and of two chunks of head values (8 or 16 steps), paths in
     pieces, the scalar term, an augmented path, the report of values that are not finite, and a device that cannot hold the table."""
