@@ -102,6 +102,12 @@ static const KernelEntry* choose_entry(bool backward, bool f64, uint64_t d, uint
                : spec;
 }
 
+// Cutting a path in pieces costs scratch for their signatures.  Where the finer partition cuts more often than the call would
+// be cut without it (or an instance more often than the run-time kernel in its place, or the sweep with shared prefix chains is taken, which has a
+// table of its own) and the device cannot hold
+// that, the call is served without it: it needs no more memory than it ever did.
+static thread_local bool tl_no_fine = false, tl_fine_more_pieces = false;
+
 // Where choose_entry's estimate asks for the run-time kernel and no finer partition takes its place, the instance after all (else null): time pieces and
 // the staged twin make it the sooner one of 16548 random calls in that state, but where this rule says (9700 calls with the instance now: 0.81 of their time,
 // 25 of them 1.03 to 1.08 times as long; 571 paths x 6136 steps x 12 channels, degree 3, double, backward 14.6 -> 4.0 ms; 1 x 15 x 29, degree 4, single
@@ -112,7 +118,7 @@ static const KernelEntry* choose_entry(bool backward, bool f64, uint64_t d, uint
 //   few paths of 128 to 511 steps, which instances do not cut yet: 2 x 345 x 8, degree 4, double 0.13 -> 0.19.
 static const KernelEntry* instance_after_all(const KernelEntry* e, bool backward, uint64_t d, uint64_t degree, uint64_t batch, uint64_t L)
 {
-    if (e->D != 0 || g_force_tail > 0) return nullptr;
+    if (e->D != 0 || g_force_tail > 0 || tl_no_fine) return nullptr;
     const KernelEntry* spec = find_entry(backward, e->is_f64 != 0, d, degree);
     if (!spec || spec->D <= 0) return nullptr;
     if (!backward) return L >= 256 && spec->tail >= 2 ? spec : nullptr;
@@ -645,10 +651,6 @@ static bool rows_bwd_mfma_wins(uint64_t d, uint64_t degree, uint64_t batch, uint
 // ---------------------------------------------------------------------------
 static Hook g_fine{1};      // test hook: 0 never, 1 by the estimates below, 2 wherever there is one
 
-// Cutting a path in pieces costs scratch for their signatures.  Where the finer partition cuts more often than the call would
-// be cut without it (or the sweep with shared prefix chains is taken, which has a table of its own) and the device cannot hold
-// that, the call is served without it: it needs no more memory than it ever did.
-static thread_local bool tl_no_fine = false, tl_fine_more_pieces = false;
 template <typename F>
 static void fine_if_it_fits(F&& run)
 {
@@ -1241,8 +1243,10 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
             if (const KernelEntry* spec = instance_after_all(e, false, s.d_aug, degree, batch, s.L)) {
                 e = spec;
                 instance_waves = total_waves(geom_of(e, int(s.d_aug)), int64_t(batch));
+                const int before = plan.pieces;
                 plan = split();
                 plan = finer();
+                tl_fine_more_pieces = tl_fine_more_pieces || plan.pieces > before;
             }
         }
         const HeadsEntry* heads = sizeof(T) == 8 && !by_rows ? heads_entry(s.d_aug, degree) : nullptr;
@@ -1680,8 +1684,10 @@ static void sig_backprop_impl(const T* path, T* out, const T* sig_derivs, const 
             if (const KernelEntry* spec = instance_after_all(e, true, s.d_aug, degree, batch, s.L)) {
                 e = spec;
                 instance_waves = total_waves(geom_of(e, int(s.d_aug)), int64_t(batch));
+                const int before = plan.pieces;
                 plan = split();
                 plan = finer();
+                tl_fine_more_pieces = tl_fine_more_pieces || plan.pieces > before;
             }
         }
         int nseg = by_rows ? 1 : plan.pieces;
