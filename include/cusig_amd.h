@@ -281,6 +281,8 @@ CUSIG_AMD_API void cusig_amd_set_rows_forward(int mode) CUSIG_AMD_NOEXCEPT;
 /* Test hook: the forward sweep that shares the prefix chains of few channels at high degrees: 0 never, 1 (default) where it is
  * expected to be the fastest form, 2 wherever there is one. */
 CUSIG_AMD_API void cusig_amd_set_heads_forward(int mode) CUSIG_AMD_NOEXCEPT;
+/* Test hook: bytes that the table of that sweep may take (paths go in chunks that fit); 0 the default, 1 GiB. */
+CUSIG_AMD_API void cusig_amd_set_heads_table_limit(uint64_t bytes) CUSIG_AMD_NOEXCEPT;
 /* Test hook: the second, finer partition that shapes have for launches of few paths: 0 never, 1 (default) where it is expected
  * to be the sooner one, 2 wherever there is one (forced pieces included). */
 CUSIG_AMD_API void cusig_amd_set_fine(int mode) CUSIG_AMD_NOEXCEPT;

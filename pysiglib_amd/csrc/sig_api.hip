@@ -971,23 +971,43 @@ struct Degree3Buffers {
 // few channels to high degrees in double precision: shared prefix chains (sig_heads.hip)
 // ---------------------------------------------------------------------------
 static Hook g_heads{1};     // test hook: 0 never, 1 by the estimates below, 2 wherever there is such a sweep
-constexpr uint64_t kHeadsTableBytes = uint64_t(1) << 30;     // the table of fractions; paths are taken in chunks that fit
+// the table of fractions; paths are taken in chunks that fit (test hook: cusig_amd_set_heads_table_limit)
+constexpr uint64_t kHeadsTableBytes = uint64_t(1) << 30;
+static std::atomic<uint64_t> g_heads_table{kHeadsTableBytes};
+
+// Paths whose table fits, 0 if not even one's does.  A row beyond the paths' own ends the table.
+static uint64_t heads_chunk(const HeadsEntry* e, uint64_t L)
+{
+    const uint64_t rows = g_heads_table / (uint64_t(e->row) * sizeof(double));
+    return rows > 1 ? (rows - 1) / L : 0;
+}
 
 // Pieces per path of such a sweep if that promises 10 % against `now`, the sweep of `run` chosen without it; 0 if not.  Blocks run in rounds of
-// what the compute units hold; beside the sweep a call lays out the table, and its lanes store runs of a few values each.
-// Lead-lag twins of the tree kernels skip half of what the estimate of theirs counts.
+// what the compute units hold, chunk of paths by chunk: where a chunk is a few long paths, each of its launches leaves most of the chip idle
+// (186 x 155309 x 3, degree 9, in chunks of 53: 279 ms, tree kernels 86).  A step that is shorter than a row of the table takes from memory waits for
+// it once the table is too large for the last cache (tables of 120 / 500 MB, ns a step: 3 channels, degree 9, one block a compute unit 324 / 453, four 635 /
+// 736; 3, 10: 311 / 438, 697 / 753; 4, 9: 462 / 533; 5, 8: 377 / 444; 11, 6: 326 / 426; 3, 12: 583 / 586).  With both counted, of 1155 random calls up
+// to 300000 steps 489 take this form, 0.75 of the tree kernels' time on average.  Beside the sweep a call
+// lays out the table, and its lanes store runs of a few values each.  Lead-lag twins of the tree kernels skip half of what the estimate of theirs counts.
 static int heads_pieces(const HeadsEntry* e, const KernelEntry* run, const SplitPlan& now, uint64_t d, uint64_t batch, uint64_t L, uint64_t sig_bytes_all_paths,
                         bool sparse_ll)
 {
     const int mode = g_heads, forced = g_force_segments;
     if (!e || mode == 0 || tl_no_fine || g_force_tail > 0 || g_force_staged >= 0 || g_ignore_table != 0 || L >= (uint64_t(1) << 30) ||
-        checked_mul(L + 1, uint64_t(e->row) * sizeof(double), "table") > kHeadsTableBytes || batch > (uint64_t(1) << 40) / uint64_t(e->blocks))
+        batch > (uint64_t(1) << 40) / uint64_t(e->blocks))
         return 0;
+    const uint64_t chunk = std::min(batch, heads_chunk(e, L));
+    if (chunk == 0) return 0;
     if (forced > 0) return mode == 2 ? int(std::min<uint64_t>(uint64_t(forced), L)) : 0;
     const int64_t cus = simd_count() / 4;
+    const double wait = e->lone_ns < 500 && double(chunk) * double(L) * e->row * sizeof(double) > 140e6 ? 100.0 : 0.0;
+    auto step_of = [&](uint64_t paths, int g) {      // ns of a step of one launch
+        const int64_t fullest = (int64_t(paths) * g * e->blocks + cus - 1) / cus, rest = fullest % e->resident;
+        return double(fullest / e->resident) * (e->step_ns + (e->resident > 2 ? 0.6 : 1.0) * wait) +
+               (rest ? wait + std::max(double(e->lone_ns), double(e->step_ns) * double(rest) / e->resident) : 0.0);
+    };
     auto seconds = [&](int g) {
-        const int64_t fullest = (int64_t(batch) * g * e->blocks + cus - 1) / cus, rest = fullest % e->resident;
-        const double step = double(fullest / e->resident) * e->step_ns + (rest ? std::max(double(e->lone_ns), double(e->step_ns) * double(rest) / e->resident) : 0.0);
+        const double step = double(batch / chunk) * step_of(chunk, g) + step_of(batch % chunk, g);
         int lg = 0;
         while ((1 << lg) < g) ++lg;
         const double folds = g > 1 ? 2e-6 + 6e-6 * lg + 2.2 * g * double(sig_bytes_all_paths) / 4e12 : 0.0;
@@ -1303,7 +1323,7 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
         tl_matrix_form = by_rows && sizeof(T) == 4;
         if (heads) {
             const uint64_t path_bytes = s.L * uint64_t(heads->row) * sizeof(T);
-            const uint64_t chunk = std::min<uint64_t>(batch, kHeadsTableBytes / path_bytes);
+            const uint64_t chunk = std::min(batch, heads_chunk(heads, s.L));
             HeadsParams hp;
             hp.table = workspace(20, chunk * path_bytes + uint64_t(heads->row) * sizeof(T));
             hp.L = p.L; hp.out_stride = p.out_stride; hp.scalar = p.scalar; hp.nseg = p.nseg; hp.lseg = p.lseg; hp.nonfinite = p.nonfinite;
@@ -2000,6 +2020,7 @@ CUSIG_AMD_API void cusig_amd_set_fine(int mode) noexcept { if (g_test_hooks) g_f
 CUSIG_AMD_API int cusig_amd_last_sweep_on_matrix_units(void) noexcept { return tl_matrix_form; }
 CUSIG_AMD_API void cusig_amd_set_rows_backward(int mode) noexcept { if (g_test_hooks) g_rows_backward = mode; }
 CUSIG_AMD_API void cusig_amd_set_heads_forward(int mode) noexcept { if (g_test_hooks) g_heads = mode; }
+CUSIG_AMD_API void cusig_amd_set_heads_table_limit(uint64_t bytes) noexcept { if (g_test_hooks) g_heads_table = bytes ? bytes : kHeadsTableBytes; }
 CUSIG_AMD_API void cusig_amd_set_rows_forward(int mode) noexcept { if (g_test_hooks) g_rows_forward = mode; }
 
 CUSIG_AMD_API void cusig_amd_force_staged(int mode) noexcept { if (g_test_hooks) g_force_staged = mode; }
@@ -2046,6 +2067,7 @@ CUSIG_AMD_API void cusig_amd_enable_test_hooks(int enabled) noexcept
     g_rows_backward = 1;
     g_rows_forward = 1;
     g_heads = 1;
+    g_heads_table = kHeadsTableBytes;
     g_force_staged = -1;
     g_force_wide_index = 0;
     g_chen_adjoint_mode = 0;

@@ -2017,3 +2017,68 @@ def test_instances_where_lanes_are_few(P, oracle, batch, length, d, deg, instanc
         L.CUSIG.cusig_amd_set_profiling(0)
     assert not (instance and "_d0_" in name), name
     assert bwd_rel_err(got, want) <= TOL[dtype]
+
+
+@pytest.fixture
+def heads():
+    """Hooks of the forward sweep with shared prefix chains; the defaults again afterwards."""
+    import ctypes
+    import types
+    from pysiglib_amd import _loader as L
+    lib = L.CUSIG
+    for hook, arg in ((lib.cusig_amd_set_heads_forward, ctypes.c_int), (lib.cusig_amd_force_segments, ctypes.c_int),
+                      (lib.cusig_amd_set_heads_table_limit, ctypes.c_uint64)):
+        hook.argtypes, hook.restype = (arg,), None
+    lib.cusig_amd_last_kernel_name.restype = ctypes.c_char_p
+    lib.cusig_amd_set_profiling(1)
+    yield types.SimpleNamespace(mode=lib.cusig_amd_set_heads_forward, pieces=lib.cusig_amd_force_segments, table=lib.cusig_amd_set_heads_table_limit,
+                                name=lambda: lib.cusig_amd_last_kernel_name().decode())
+    lib.cusig_amd_set_heads_forward(1)
+    lib.cusig_amd_force_segments(0)
+    lib.cusig_amd_set_heads_table_limit(0)
+    lib.cusig_amd_set_profiling(0)
+
+
+# elements of a step's row in the table, by plan
+HEADS_ROW = {(3, 9): 16, (3, 11): 40, (3, 13): 40, (4, 9): 48, (5, 8): 48, (5, 10): 56, (6, 7): 32, (7, 8): 40, (8, 7): 56, (9, 8): 64, (10, 7): 72, (11, 6): 40}
+
+
+@pytest.mark.parametrize("d,deg", sorted(HEADS_ROW))
+def test_shared_prefix_chains_by_chunks_of_paths(P, oracle, heads, d, deg):
+    """Three chunks of two paths, two and one, whole and in pieces, plain and lead-lag (whose pieces start on even steps): the same values as in one
+    chunk, and the oracle's.  A table that not even one path fits leaves the call to the tree kernels."""
+    rng = np.random.default_rng(1000 * d + deg)
+    large = d ** deg > 2000000
+    heads.mode(2)
+    for batch, length, pieces, aug in ((3, 18, 2, {}),) if large else ((5, 21, 1, {}), (5, 21, 3, {}), (5, 11, 3, dict(lead_lag=True, time_aug=d % 2 == 1))):
+        raw = d // 2 if aug else d
+        x = np.cumsum(rng.standard_normal((batch, length, raw)), axis=1) / np.sqrt(length * d)
+        steps = 2 * (length - 1) if aug else length - 1
+        one = HEADS_ROW[d, deg] * 8 * steps
+        heads.pieces(pieces)
+        heads.table(0)
+        whole = P.sig(dev(x), deg, scalar_term=True, **aug)
+        for paths in (1, 2):
+            heads.table((paths * steps + 1) * HEADS_ROW[d, deg] * 8)
+            got = P.sig(dev(x), deg, scalar_term=True, **aug)
+            assert heads.name().startswith("heads_fwd")
+            assert torch.equal(got, whole), (batch, length, pieces, paths)
+        ref = oracle.signature(x, deg, scalar_term=True, n_jobs=-1, **aug)
+        assert np.max(level_rel_err(whole.cpu().numpy()[:, 1:], ref[:, 1:], d, deg)) < TOL[np.float64]
+        heads.table(one)        # a row short
+        P.sig(dev(x), deg, **aug)
+        assert not heads.name().startswith("heads")
+
+
+@pytest.mark.parametrize("batch,length,d,deg", [(60, 2000, 4, 9), (200, 1500, 3, 9)])
+def test_shared_prefix_chains_that_leave_the_chip_idle(P, heads, batch, length, d, deg):
+    """By the estimates: the sweep is taken where all paths go in one launch, and left to the tree kernels where the table holds a few of them, whose launches
+    one after the other would leave most of the chip without work."""
+    rng = np.random.default_rng(d)
+    x = dev(np.cumsum(rng.standard_normal((batch, length, d)), axis=1) / np.sqrt(length * d))
+    whole = P.sig(x, deg)
+    assert heads.name().startswith("heads_fwd")
+    heads.table((2 * (length - 1) + 1) * HEADS_ROW[d, deg] * 8)
+    few = P.sig(x, deg)
+    assert heads.name().startswith("fwd_f64_")
+    assert np.max(level_rel_err(few.cpu().numpy(), whole.cpu().numpy(), d, deg)) < TOL[np.float64]
