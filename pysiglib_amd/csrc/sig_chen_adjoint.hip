@@ -173,12 +173,12 @@ static bool right_fold_fits(uint64_t dimension)
 }
 
 template <typename T, int QL = 0, int REL = 1>
-static void launch_right_stream(const RightPlan& rp, const T* dC, T* dB, const T* A, uint64_t batch, const SigShape& s,
+static void launch_right_stream(const RightPlan& rp, const T* dC, T* dB, const T* A, T* sum_rows, uint64_t batch, const SigShape& s,
                                 hipStream_t stream, int identity, const SharedRows& dc, const ExpFold<T>* fold)
 {
     if constexpr (QL <= kRightMaxLow && REL <= kRightMaxRel) {
-        if (rp.qe - 1 != QL) return launch_right_stream<T, QL + 1, REL>(rp, dC, dB, A, batch, s, stream, identity, dc, fold);
-        if (rp.rel != REL) return launch_right_stream<T, QL, REL + 1>(rp, dC, dB, A, batch, s, stream, identity, dc, fold);
+        if (rp.qe - 1 != QL) return launch_right_stream<T, QL + 1, REL>(rp, dC, dB, A, sum_rows, batch, s, stream, identity, dc, fold);
+        if (rp.rel != REL) return launch_right_stream<T, QL, REL + 1>(rp, dC, dB, A, sum_rows, batch, s, stream, identity, dc, fold);
         const uint64_t waves = (uint64_t(rp.words) + kWave - 1) / kWave;
         const dim3 grid{unsigned((waves + kWavesPerBlock - 1) / kWavesPerBlock), unsigned(std::min<uint64_t>(batch, 65535)), 1};
         FoldScale<T> fs{};
@@ -192,11 +192,11 @@ static void launch_right_stream(const RightPlan& rp, const T* dC, T* dB, const T
             }
             hipLaunchKernelGGL((chen_adjoint_right_kernel<T, QL, REL, true>), grid, dim3(kBlock),
                                size_t(rp.d) * kBlock * sizeof(T), stream, dC, dB, A, int64_t(batch), rp, int64_t(s.stride), s.off,
-                               identity, dc.share, dc.stride, dc.off, fold->z, fold->dz, fs);
+                               identity, dc.share, dc.stride, dc.off, fold->z, fold->dz, fs, sum_rows);
         } else {
             hipLaunchKernelGGL((chen_adjoint_right_kernel<T, QL, REL, false>), grid, dim3(kBlock), 0, stream, dC, dB, A,
                                int64_t(batch), rp, int64_t(s.stride), s.off, identity, dc.share, dc.stride, dc.off,
-                               (const T*)nullptr, (T*)nullptr, fs);
+                               (const T*)nullptr, (T*)nullptr, fs, sum_rows);
         }
     }
 }
@@ -272,73 +272,90 @@ void launch_combine_bwd(const T* dC, T* dA, T* dB, const T* A, const T* B, uint6
     RightPlan rp;
     const bool rows = streaming && make_rows_plan(wp, dimension, degree, kStreamLdsEntries);
     const bool left = rows || (streaming && make_left_plan(lp, dimension, degree, kStreamLdsEntries));
-    const bool right = streaming && families > 1 && make_right_plan(rp, dimension, degree, batch);
+    const bool right = streaming && families > 1 && make_right_plan(rp, dimension, degree, batch, sizeof(T));
     if (!left && !right) {
         launch_combine_bwd_items<T>(dC, dA, dB, A, B, batch, dimension, degree, s, stream, identity, dc, families, 0);
         return;
     }
-    // left factor: words shorter than the blocks' own take their low-level terms from the truncated problem first
-    if (!left) {
-        launch_combine_bwd_items<T>(dC, dA, dB, A, B, batch, dimension, degree, s, stream, identity, dc, 1, 0);
-    } else if (rows) {
-        if (wp.np >= 2)
-            launch_combine_bwd_items<T>(dC, dA, dB, A, B, batch, dimension, uint64_t(wp.np), s, stream, identity, dc, 1, 0);
-        const uint64_t groups = (uint64_t(wp.units) + uint64_t(wp.upb) - 1) / uint64_t(wp.upb);
-        const dim3 grid{unsigned(groups), unsigned(std::min<uint64_t>(batch, 65535)), 1};
-        const size_t lds = (size_t(wp.bs) + 2 * size_t(wp.targets) + size_t(wp.img)) * sizeof(T);
-        const int kt = int((wp.top + kBlock - 1) / kBlock), ks = int((wp.targets + kBlock - 1) / kBlock);
-        auto go3 = [&](auto dc_, auto kt_, auto ks_) {
-            hipLaunchKernelGGL((chen_adjoint_left_rows_kernel<T, decltype(dc_)::value, decltype(kt_)::value, decltype(ks_)::value>),
-                               grid, dim3(kBlock), lds, stream, dC, dA, B, int64_t(batch), wp, int64_t(s.stride), s.off, ida,
-                               dc.share, dc.stride, dc.off);
-        };
-        auto go2 = [&](auto dc_, auto ks_) {
-            if (kt <= 2) go3(dc_, std::integral_constant<int, 2>(), ks_);
-            else if (kt <= 4) go3(dc_, std::integral_constant<int, 4>(), ks_);
-            else go3(dc_, std::integral_constant<int, kRowsMaxTop>(), ks_);
-        };
-        // owned entries per thread: more than one only for few channels (targets ~ top / (d - 1))
-        auto go = [&](auto dc_) {
-            constexpr int DC = decltype(dc_)::value;
-            if (ks <= 1) go2(dc_, std::integral_constant<int, 1>());
-            else if constexpr (DC <= 8) {
-                if (ks <= 2) go2(dc_, std::integral_constant<int, 2>());
-                else if constexpr (DC <= 4) go2(dc_, std::integral_constant<int, kRowsMaxLow>());
-                else throw std::logic_error("sig_combine_backprop_cuda: kernel plan");
-            } else throw std::logic_error("sig_combine_backprop_cuda: kernel plan");
-        };
-        const uint64_t d = dimension;
-        if (d <= 4) go(std::integral_constant<int, 4>());
-        else if (d <= 8) go(std::integral_constant<int, 8>());
-        else if (d <= 12) go(std::integral_constant<int, 12>());
-        else if (d <= 16) go(std::integral_constant<int, 16>());
-        else go(std::integral_constant<int, 32>());
-    } else {
-        if (lp.np >= 2)
-            launch_combine_bwd_items<T>(dC, dA, dB, A, B, batch, dimension, uint64_t(lp.np), s, stream, identity, dc, 1, 0);
-        const uint64_t groups = (uint64_t(lp.units) + uint64_t(lp.upb) - 1) / uint64_t(lp.upb);
-        const dim3 grid{unsigned(groups), unsigned(std::min<uint64_t>(batch, 65535)), 1};
-        const size_t lds = (size_t(lp.xs) + size_t(lp.bs)) * sizeof(T);
-        auto go = [&](auto kx) {
-            hipLaunchKernelGGL((chen_adjoint_left_kernel<T, decltype(kx)::value>), grid, dim3(kBlock), lds, stream, dC, dA, B,
-                               int64_t(batch), lp, int64_t(s.stride), s.off, ida, dc.share, dc.stride, dc.off);
-        };
-        const uint32_t per = (lp.xs + kBlock - 1) / kBlock;      // entries of a unit per thread
-        if (per <= 4) go(std::integral_constant<int, 4>());
-        else if (per <= 8) go(std::integral_constant<int, 8>());
-        else if (per <= 12) go(std::integral_constant<int, 12>());
-        else if (per <= 16) go(std::integral_constant<int, 16>());
-        else go(std::integral_constant<int, 24>());
-    }
-    if (families < 2) return;
-    if (!right) {
-        launch_combine_bwd_items<T>(dC, dA, dB, A, B, batch, dimension, degree, s, stream, identity, dc, 1, 1);
-    } else {
+    // words shorter than the blocks' own take their low-level terms from the truncated problem first
+    auto left_factor = [&] {
+        if (!left) {
+            launch_combine_bwd_items<T>(dC, dA, dB, A, B, batch, dimension, degree, s, stream, identity, dc, 1, 0);
+        } else if (rows) {
+            if (wp.np >= 2)
+                launch_combine_bwd_items<T>(dC, dA, dB, A, B, batch, dimension, uint64_t(wp.np), s, stream, identity, dc, 1, 0);
+            const uint64_t groups = (uint64_t(wp.units) + uint64_t(wp.upb) - 1) / uint64_t(wp.upb);
+            const dim3 grid{unsigned(groups), unsigned(std::min<uint64_t>(batch, 65535)), 1};
+            const size_t lds = (size_t(wp.bs) + 2 * size_t(wp.targets) + size_t(wp.img)) * sizeof(T);
+            const int kt = int((wp.top + kBlock - 1) / kBlock), ks = int((wp.targets + kBlock - 1) / kBlock);
+            auto go3 = [&](auto dc_, auto kt_, auto ks_) {
+                hipLaunchKernelGGL((chen_adjoint_left_rows_kernel<T, decltype(dc_)::value, decltype(kt_)::value, decltype(ks_)::value>),
+                                   grid, dim3(kBlock), lds, stream, dC, dA, B, int64_t(batch), wp, int64_t(s.stride), s.off, ida,
+                                   dc.share, dc.stride, dc.off);
+            };
+            auto go2 = [&](auto dc_, auto ks_) {
+                if (kt <= 2) go3(dc_, std::integral_constant<int, 2>(), ks_);
+                else if (kt <= 4) go3(dc_, std::integral_constant<int, 4>(), ks_);
+                else go3(dc_, std::integral_constant<int, kRowsMaxTop>(), ks_);
+            };
+            // owned entries per thread: more than one only for few channels (targets ~ top / (d - 1))
+            auto go = [&](auto dc_) {
+                constexpr int DC = decltype(dc_)::value;
+                if (ks <= 1) go2(dc_, std::integral_constant<int, 1>());
+                else if constexpr (DC <= 8) {
+                    if (ks <= 2) go2(dc_, std::integral_constant<int, 2>());
+                    else if constexpr (DC <= 4) go2(dc_, std::integral_constant<int, kRowsMaxLow>());
+                    else throw std::logic_error("sig_combine_backprop_cuda: kernel plan");
+                } else throw std::logic_error("sig_combine_backprop_cuda: kernel plan");
+            };
+            const uint64_t d = dimension;
+            if (d <= 4) go(std::integral_constant<int, 4>());
+            else if (d <= 8) go(std::integral_constant<int, 8>());
+            else if (d <= 12) go(std::integral_constant<int, 12>());
+            else if (d <= 16) go(std::integral_constant<int, 16>());
+            else go(std::integral_constant<int, 32>());
+        } else {
+            if (lp.np >= 2)
+                launch_combine_bwd_items<T>(dC, dA, dB, A, B, batch, dimension, uint64_t(lp.np), s, stream, identity, dc, 1, 0);
+            const uint64_t groups = (uint64_t(lp.units) + uint64_t(lp.upb) - 1) / uint64_t(lp.upb);
+            const dim3 grid{unsigned(groups), unsigned(std::min<uint64_t>(batch, 65535)), 1};
+            const size_t lds = (size_t(lp.xs) + size_t(lp.bs)) * sizeof(T);
+            auto go = [&](auto kx) {
+                hipLaunchKernelGGL((chen_adjoint_left_kernel<T, decltype(kx)::value>), grid, dim3(kBlock), lds, stream, dC, dA, B,
+                                   int64_t(batch), lp, int64_t(s.stride), s.off, ida, dc.share, dc.stride, dc.off);
+            };
+            const uint32_t per = (lp.xs + kBlock - 1) / kBlock;      // entries of a unit per thread
+            if (per <= 4) go(std::integral_constant<int, 4>());
+            else if (per <= 8) go(std::integral_constant<int, 8>());
+            else if (per <= 12) go(std::integral_constant<int, 12>());
+            else if (per <= 16) go(std::integral_constant<int, 16>());
+            else go(std::integral_constant<int, 24>());
+        }
+    };
+    auto right_factor = [&] {
+        if (!right) {
+            launch_combine_bwd_items<T>(dC, dA, dB, A, B, batch, dimension, degree, s, stream, identity, dc, 1, 1);
+            return;
+        }
         if (rp.qe >= 2)
             launch_combine_bwd_items<T>(dC, dA, dB, A, B, batch, dimension, uint64_t(rp.qe - 1), s, stream, identity, dc, 1, 1);
         const bool folding = fold && idb == 1 && rp.rel >= 1 && right_fold_fits<T>(dimension);
         if (folding) fold->level = rp.qe;
-        launch_right_stream<T>(rp, dC, dB, A, batch, s, stream, idb, dc, folding ? fold : nullptr);
+        const dim3 grid{unsigned((rp.lv.lo[rp.qe] + rp.d + kBlock - 1) / kBlock), unsigned(std::min<uint64_t>(batch, 65535)), 1};
+        if (rp.longer)
+            hipLaunchKernelGGL((right_sums_zero_kernel<T>), grid, dim3(kBlock), 0, stream, dA, int64_t(batch), rp, int64_t(s.stride), s.off);
+        launch_right_stream<T>(rp, dC, dB, A, rp.longer ? dA : nullptr, batch, s, stream, idb, dc, folding ? fold : nullptr);
+        if (rp.longer)
+            hipLaunchKernelGGL((right_sums_add_kernel<T>), grid, dim3(kBlock), 0, stream, dA, dB, folding ? fold->dz : nullptr, int64_t(batch), rp,
+                               int64_t(s.stride), s.off);
+    };
+    if (families < 2) return left_factor();
+    if (right && rp.longer) {       // keeps sums in dA
+        right_factor();
+        left_factor();
+    } else {
+        left_factor();
+        right_factor();
     }
 }
 

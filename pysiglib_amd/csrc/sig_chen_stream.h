@@ -42,6 +42,7 @@ static inline bool fill_stream_levels(StreamLevels& lv, uint64_t d, uint64_t deg
 struct RightPlan {
     int degree, qe, rel;        // rel = degree - qe
     uint32_t d, words;          // words = d^qe
+    bool longer;                // than the shortest: right_sums
     StreamLevels lv;
 };
 
@@ -184,6 +185,39 @@ __device__ __forceinline__ void right_descend(RightLane<T, QL>& L, const RightPl
     }
 }
 
+// Lanes of longer words than the shortest (right_word_length) add to the words below theirs many at a time: d^(qe-1) lanes to a word of
+// level 1.  Each such addition in T rounds the whole sum (single precision, factors as signatures are, level 1, relative to 64 bits, shortest / longer
+// words: 8 channels, degree 7 2.9e-7 / 1.7e-6; 5, 7: 2.7e-7 / 6.2e-7).  They are summed from zero in double precision instead, where the left factor's
+// gradient will have its top level (its kernels run afterwards): levels 1 .. qe - 1, then d values of dz.
+template <typename T>
+__device__ __forceinline__ double* right_sums(T* row, const RightPlan& P)
+{
+    return reinterpret_cast<double*>((reinterpret_cast<uintptr_t>(row + P.lv.lo[P.degree]) + 7) & ~uintptr_t(7));
+}
+
+template <typename T>
+__global__ __launch_bounds__(kBlock) void right_sums_zero_kernel(T* __restrict__ sum_rows, int64_t batch, RightPlan P, int64_t stride, int off)
+{
+    const uint32_t n = P.lv.lo[P.qe] + P.d;
+    for (int64_t b = blockIdx.y; b < batch; b += gridDim.y)
+        for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) right_sums(sum_rows + b * stride + off, P)[i] = 0.0;
+}
+
+// adds them to what dB's low levels, and dz (may be null), hold
+template <typename T>
+__global__ __launch_bounds__(kBlock) void right_sums_add_kernel(T* __restrict__ sum_rows, T* __restrict__ dB, T* __restrict__ dz, int64_t batch, RightPlan P,
+                                                                int64_t stride, int off)
+{
+    const uint32_t low = P.lv.lo[P.qe], n = low + (dz ? P.d : 0u);
+    for (int64_t b = blockIdx.y; b < batch; b += gridDim.y) {
+        const double* sums = right_sums(sum_rows + b * stride + off, P);
+        for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+            T* at = i < low ? dB + b * stride + off + i : dz + b * int64_t(P.d) + (i - low);
+            *at = T(double(*at) + sums[i]);
+        }
+    }
+}
+
 // grid: x over the waves of a row (4 per block), y over the rows
 //
 // FOLD: B = exp(z) and the caller wants dz, not dB (sig_join_backprop, siglib/cpsig/cp_sig_join.h:36-238).  With
@@ -197,7 +231,7 @@ template <typename T, int QL, int REL, bool FOLD>
 __global__ __launch_bounds__(kBlock) void chen_adjoint_right_kernel(
     const T* __restrict__ dC, T* __restrict__ dB, const T* __restrict__ A, int64_t batch, RightPlan P, int64_t stride,
     int off, int identity, int64_t dc_share, int64_t dc_stride, int dc_off, const T* __restrict__ Z, T* __restrict__ dz,
-    FoldScale<T> F)
+    FoldScale<T> F, T* __restrict__ sum_rows)
 {
     extern __shared__ double right_lds_raw[];
     const Block2 blk = xcd_block_2d();
@@ -248,13 +282,22 @@ __global__ __launch_bounds__(kBlock) void chen_adjoint_right_kernel(
             for (uint32_t x = 0; x < P.d; ++x) {
                 const T v = wave_sum(slot[x * kBlock]);
                 slot[x * kBlock] = T(0);
-                if ((threadIdx.x & (kWave - 1)) == 0) dev_add(dz + b * int64_t(P.d) + x, v);
+                if ((threadIdx.x & (kWave - 1)) == 0) {
+                    if (sum_rows) dev_add(right_sums(sum_rows + b * stride + off, P) + P.lv.lo[P.qe] + x, double(v));
+                    else dev_add(dz + b * int64_t(P.d) + x, v);
+                }
             }
         }
         if (L.live) {
             L.out[pos] = L.acc[0];
+            if (sum_rows) {
+                double* sums = right_sums(sum_rows + b * stride + off, P);
 #pragma unroll
-            for (int t = 1; t <= QL; ++t) dev_add(L.out + P.lv.lo[t] + (L.f - L.cq[t - 1] * P.lv.pw[t]), L.low[t - 1]);
+                for (int t = 1; t <= QL; ++t) dev_add(sums + P.lv.lo[t] + (L.f - L.cq[t - 1] * P.lv.pw[t]), double(L.low[t - 1]));
+            } else {
+#pragma unroll
+                for (int t = 1; t <= QL; ++t) dev_add(L.out + P.lv.lo[t] + (L.f - L.cq[t - 1] * P.lv.pw[t]), L.low[t - 1]);
+            }
         }
     }
 }
@@ -717,38 +760,53 @@ static inline bool fill_stream_levels(StreamLevels& lv, uint64_t d, uint64_t deg
     return true;
 }
 
-// the lanes' word length: enough words for four waves per row, and a walk of at most kRightMaxRel levels
-// Length of the lanes' words.  A short one leaves few lanes with long walks, d + .. + d^rel loads one after the other (one row of 16 channels,
-// degree 6: 256 lanes, 69904 each); a long one makes every lane add to the words below its own, d words for all of them in the first level.  Both
-// factors' gradients, us, by length (single precision): 1 row of 16, 6: 23462 (2), 1487 (3), 735 (4), 3237 (5); 16 rows of 26, 5: 7964 (2),
-// 1622 (3), 2231 (4); 16 of 9, 7: 3328 (3), 1192 (4), 1469 (5); 64 of 16, 5: 1877 (2), 459 (3), 1520 (4); 256 of 4, 9: 1055 (5), 1203 (6).
+// Length of the lanes' words, `shortest` and longer.  A short one leaves few lanes with long walks, d + .. + d^rel loads one after the other (one row of 16
+// channels, degree 6: 256 lanes, 69904 each); a long one makes every lane add to the words below its own, d words for all of them in the first level.  Both
+// factors' gradients, us, shortest / the length taken (single precision): 1 row of 16, 6: 23259 (2) / 667 (4); 4 rows of 20, 5: 2070 (2) / 239 (3); 5 of 8, 7:
+// 1327 (3) / 318 (5); 3 of 7, 7: 965 (3) / 358 (5); 1 of 33, 4: 224 (2) / 117 (3); 2 of 5, 9: 527 (5) / 428 (6); 4 of 4, 8: 215 (4) / 175 (5); 3 of 5, 7: 139 (4) /
+// 137 (5), which is left at 4.
 // The estimate, us: 0.35 a load of the walk while a SIMD has no second wave of them; 0.03 an addition to one address, 2e-5 any; a longer
-// word has to save 15.
-static inline int right_word_length(uint64_t d, int degree, uint64_t batch, int shortest)
+// word has to save 15, and 20 more for the two launches that longer words than the shortest take.
+// The sums of longer words are kept in double precision (right_sums; `elem_bytes` of T: they have to fit a row's top level).  For T = double that is no
+// better than T, so there the additions to one address may not grow by more than the walk, whose products a lane sums, gets shorter: errors as of that many
+// roundings.
+static inline int right_word_length(const StreamLevels& lv, uint64_t d, int degree, uint64_t batch, int shortest, size_t elem_bytes)
 {
-    auto estimate = [&](int qe) {
+    struct Cost { double time, roundings; };
+    auto cost = [&](int qe) {
         double words = 1.0, walk = 0.0;
         for (int i = 0; i < qe; ++i) words *= double(d);
         for (int i = qe; i < degree; ++i) walk = (walk + 1.0) * double(d);
         const double waves = double(batch) * words / kWave;
         const double adds = qe > 1 ? std::max(0.03 * words / double(d), 2e-5 * words * double(batch) * (qe - 1)) : 0.0;
-        return 0.35 * walk * std::max(1.0, waves / 1024.0) + adds;
+        return Cost{0.35 * walk * std::max(1.0, waves / 1024.0) + adds, std::sqrt(walk) + (qe > 1 ? std::sqrt(words / double(d)) : 0.0)};
     };
+    const Cost first = cost(shortest);
+    double top = 1.0;
+    for (int i = 0; i < degree; ++i) top *= double(d);
     int best = shortest;
-    for (int qe = shortest + 1; qe <= degree - 1 && qe - 1 <= kRightMaxLow; ++qe)
-        if (estimate(qe) + 15.0 * (qe - best) < estimate(best)) best = qe;
+    double best_time = first.time;
+    for (int qe = shortest + 1; qe <= degree - 1 && qe - 1 <= kRightMaxLow; ++qe) {
+        const Cost c = cost(qe);
+        if (c.time + 15.0 * (qe - best) + (best == shortest ? 20.0 : 0.0) >= best_time || 8.0 * (double(lv.lo[qe]) + double(d) + 1.0) > top * double(elem_bytes)) continue;
+        if (elem_bytes == 8 && c.roundings > first.roundings) continue;
+        best = qe;
+        best_time = c.time;
+    }
     return best;
 }
 
-static inline bool make_right_plan(RightPlan& P, uint64_t d, uint64_t degree, uint64_t batch)
+// the shortest words: enough of them for four waves per row, and a walk of at most kRightMaxRel levels
+static inline bool make_right_plan(RightPlan& P, uint64_t d, uint64_t degree, uint64_t batch, size_t elem_bytes)
 {
     if (d < 2 || degree < 2 || !fill_stream_levels(P.lv, d, degree)) return false;
     int qmin = 1;
     uint64_t words = d;
     while (words < 256 && qmin < int(degree) - 1) { ++qmin; words *= d; }
-    int qe = std::max(qmin, int(degree) - kRightMaxRel);
-    if (qe > int(degree) - 1 || qe - 1 > kRightMaxLow) return false;
-    qe = right_word_length(d, int(degree), batch, qe);
+    const int shortest = std::max(qmin, int(degree) - kRightMaxRel);
+    if (shortest > int(degree) - 1 || shortest - 1 > kRightMaxLow) return false;
+    const int qe = right_word_length(P.lv, d, int(degree), batch, shortest, elem_bytes);
+    P.longer = qe > shortest;
     P.degree = int(degree);
     P.qe = qe;
     P.rel = int(degree) - qe;

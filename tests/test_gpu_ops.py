@@ -1011,3 +1011,21 @@ def test_few_rows_of_the_chen_adjoint(P, oracle, row_forms, batch, d, deg, dtype
     if scale.size < 100000:
         got = P.sig_to_log_sig_backprop(dev(a), dev(g), d, deg, method=0).cpu().numpy()
         assert row_rel_err(got[:, 1:], oracle.sig_to_log_sig_backprop(a, g, d, deg)[:, 1:]) < TOL[dtype]
+
+
+@pytest.mark.parametrize("batch,d,deg", [(2, 8, 7), (3, 7, 7), (3, 12, 6), (1, 16, 6)])
+@pytest.mark.parametrize("scalar_term", [False, True])
+def test_level_one_of_the_right_factor_in_single_precision(P, row_forms, batch, d, deg, scalar_term):
+    """Few rows, where thousands of lanes add to a word of level 1 of the right factor's gradient: their sum does not lose what one rounding each would (2 rows
+    of 8 channels, degree 7: 1.7e-6).  Bound: the sum is rounded to single precision a handful of times, 2^-24 each, 8 of them one way."""
+    gen = torch.Generator(device=DEV).manual_seed(100 * d + deg)
+    path = (torch.randn(batch, 24, d, device=DEV, dtype=torch.float64, generator=gen) / 24 ** 0.5).cumsum(1)
+    sig = P.sig(path, deg, scalar_term=scalar_term).float()
+    g = torch.randn(sig.shape, device=DEV, dtype=torch.float32, generator=gen)
+    z = torch.randn(batch, d, device=DEV, dtype=torch.float32, generator=gen) * 0.2
+    row_forms(0)
+    got = P.sig_join_backprop(g, sig, z, d, deg, prepend=True)[0].double()
+    want = P.sig_join_backprop(g.double(), sig.double(), z.double(), d, deg, prepend=True)[0]
+    one = slice(1, d + 1) if scalar_term else slice(0, d)
+    assert float((got - want)[:, one].norm() / want[:, one].norm()) < 2.0 ** -21
+    assert float((got - want).norm() / want.norm()) < 2.0 ** -21
