@@ -67,7 +67,8 @@ __global__ __launch_bounds__(kBlock) void sig_combine_bwd_init_kernel(
     }
 }
 
-template <typename T, typename I>
+// Acc: what an item sums in
+template <typename T, typename I, typename Acc>
 __global__ __launch_bounds__(kBlock) void sig_combine_bwd_kernel(
     const T* __restrict__ dC, T* __restrict__ dA, T* __restrict__ dB, const T* __restrict__ A,
     const T* __restrict__ B, int64_t batch, CombBwdPlan<I> plan, int64_t stride, int off, int identity,
@@ -89,7 +90,7 @@ __global__ __launch_bounds__(kBlock) void sig_combine_bwd_kernel(
             const I x0 = q * kCombChunk;
             const I x1 = x0 + kCombChunk < s_t ? x0 + kCombChunk : s_t;
             const T* other = (fam_b ? A : B) + b * stride + off;      // the factor the sum runs over
-            T s0 = T(0), s1 = T(0), s2 = T(0), s3 = T(0);
+            Acc s0 = Acc(0), s1 = Acc(0), s2 = Acc(0), s3 = Acc(0);
             for (int m = 1; m <= N - t; ++m) {
                 const I seg0 = plan.lo[m] > x0 ? plan.lo[m] : x0;
                 const I seg1 = plan.lo[m + 1] < x1 ? plan.lo[m + 1] : x1;
@@ -103,12 +104,12 @@ __global__ __launch_bounds__(kBlock) void sig_combine_bwd_kernel(
                         // four consecutive entries in wide loads (element alignment is all that is known)
                         const Quad<T> gq = *reinterpret_cast<const Quad<T>*>(blockp + x);
                         const Quad<T> oq = *reinterpret_cast<const Quad<T>*>(other + x);
-                        s0 = fmadd(gq.v[0], oq.v[0], s0);
-                        s1 = fmadd(gq.v[1], oq.v[1], s1);
-                        s2 = fmadd(gq.v[2], oq.v[2], s2);
-                        s3 = fmadd(gq.v[3], oq.v[3], s3);
+                        s0 = fmadd(Acc(gq.v[0]), Acc(oq.v[0]), s0);
+                        s1 = fmadd(Acc(gq.v[1]), Acc(oq.v[1]), s1);
+                        s2 = fmadd(Acc(gq.v[2]), Acc(oq.v[2]), s2);
+                        s3 = fmadd(Acc(gq.v[3]), Acc(oq.v[3]), s3);
                     }
-                    for (; x < seg1; ++x) s0 = fmadd(blockp[x], other[x], s0);
+                    for (; x < seg1; ++x) s0 = fmadd(Acc(blockp[x]), Acc(other[x]), s0);
                 } else {
                     const T* strided = up + w;                         // words u w: index u * d^t + w
                     I x = seg0;
@@ -116,19 +117,19 @@ __global__ __launch_bounds__(kBlock) void sig_combine_bwd_kernel(
                         const T* sp = strided + (x - plan.lo[m]) * sz_t;
                         const T g0 = sp[0], g1 = sp[sz_t], g2 = sp[2 * sz_t], g3 = sp[3 * sz_t];
                         const Quad<T> oq = *reinterpret_cast<const Quad<T>*>(other + x);      // the same four for the whole wave
-                        s0 = fmadd(g0, oq.v[0], s0);
-                        s1 = fmadd(g1, oq.v[1], s1);
-                        s2 = fmadd(g2, oq.v[2], s2);
-                        s3 = fmadd(g3, oq.v[3], s3);
+                        s0 = fmadd(Acc(g0), Acc(oq.v[0]), s0);
+                        s1 = fmadd(Acc(g1), Acc(oq.v[1]), s1);
+                        s2 = fmadd(Acc(g2), Acc(oq.v[2]), s2);
+                        s3 = fmadd(Acc(g3), Acc(oq.v[3]), s3);
                     }
-                    for (; x < seg1; ++x) s0 = fmadd(strided[(x - plan.lo[m]) * sz_t], other[x], s0);
+                    for (; x < seg1; ++x) s0 = fmadd(Acc(strided[(x - plan.lo[m]) * sz_t]), Acc(other[x]), s0);
                 }
             }
             const I r = plan.lo[t] + w;
             T* dst = (fam_b ? dB : dA) + b * stride + off + r;
-            const T sum = (s0 + s1) + (s2 + s3);
-            if (plan.parts[t] == 1) *dst = ((identity >> int(fam_b)) & 1 ? g[r] : T(0)) + sum;
-            else dev_add(dst, sum);
+            const Acc sum = (s0 + s1) + (s2 + s3);
+            if (plan.parts[t] == 1) *dst = T(((identity >> int(fam_b)) & 1 ? Acc(g[r]) : Acc(0)) + sum);
+            else dev_add(dst, T(sum));
             if (off && it == 0) {
                 if (!only_b) dA[b * stride] = T(0);
                 if (families > 1 || only_b) dB[b * stride] = T(0);
@@ -144,7 +145,7 @@ constexpr uint64_t kStreamMinCoef = 4096;
 constexpr uint64_t kStreamLdsEntries = 6144;      // 48 KB of float64
 
 // the item-per-word kernels on the signature truncated at `degree` (rows keep their stride): both factors, or one
-template <typename T>
+template <typename T, typename Acc = T>
 static void launch_combine_bwd_items(const T* dC, T* dA, T* dB, const T* A, const T* B, uint64_t batch, uint64_t dimension,
                                      uint64_t degree, const SigShape& s, hipStream_t stream, int identity,
                                      const SharedRows& dc, int families, int only_b)
@@ -159,7 +160,7 @@ static void launch_combine_bwd_items(const T* dC, T* dA, T* dB, const T* A, cons
                                    dc.off, families, only_b);
             });
         launch_indexed(0, uint64_t(families) * uint64_t(plan.items), batch, [&](auto, dim3 grid) {
-            hipLaunchKernelGGL((sig_combine_bwd_kernel<T, I>), grid, dim3(kBlock), 0, stream, dC, dA, dB, A, B, int64_t(batch),
+            hipLaunchKernelGGL((sig_combine_bwd_kernel<T, I, Acc>), grid, dim3(kBlock), 0, stream, dC, dA, dB, A, B, int64_t(batch),
                                plan, int64_t(s.stride), s.off, identity, dc.share, dc.stride, dc.off, families, only_b);
         });
     });
@@ -205,7 +206,7 @@ template <typename T, typename P>
 static void launch_both(const T* dC, T* dA, T* dB, const T* A, const T* B, uint64_t batch, const SigShape& s, hipStream_t stream)
 {
     constexpr size_t lds = P::lds_entries() * sizeof(T);
-    static_assert(lds <= size_t(160) * 1024, "a row's pieces fit a compute unit");
+    static_assert(lds + P::THREADS / kWave * sizeof(double) <= size_t(160) * 1024, "a row's pieces fit a compute unit");
     if (lds > 64 * 1024)
         SIG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(chen_adjoint_both_kernel<T, P>), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
     const uint64_t most = ((uint64_t(1) << 32) - 1) / P::THREADS;      // a launch numbers its threads with 32 bits; further items in the same blocks
@@ -232,7 +233,7 @@ static bool launch_both_factors(const T* dC, T* dA, T* dB, const T* A, const T* 
     auto go = [&](auto plan) {
         using P = decltype(plan);
         if (dimension != uint64_t(P::D) || degree != uint64_t(P::N) || (row_forms() != 2 && batch < uint64_t(P::FROM))) return false;
-        launch_combine_bwd_items<T>(dC, dA, dB, A, B, batch, dimension, uint64_t(P::Q), s, stream, 3, dc, 2, 0);
+        launch_combine_bwd_items<T, double>(dC, dA, dB, A, B, batch, dimension, uint64_t(P::Q), s, stream, 3, dc, 2, 0);
         launch_both<T, P>(dC, dA, dB, A, B, batch, s, stream);
         tl_chen_both = 1;
         return true;

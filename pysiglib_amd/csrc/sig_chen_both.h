@@ -14,6 +14,11 @@
 // Level degree - 1 goes along: a thread's word x y s' is one of its entries.  The levels below come from the item-per-word
 // kernels on the signature truncated at Q, launched first; this kernel adds to them at the end, atomically, since the blocks of a
 // row meet there.
+//
+// Partial sums that meet are added up in double precision, and a thread sums the words of an x by themselves: in single precision, one after the other,
+// the sums of D * D words cost accuracy (relative to 64 bits, general kernels / one chain / now: 13 channels, degree 4, dB_2 1.0e-7 / 2.2e-7 / 1.0e-7; 16, 5,
+// dA_2 1.0e-7 / 1.4e-7 / 1.1e-7; with the items of the truncated problem 3, 8, dA_1 1.0e-7 / 1.8e-7 / 1.0e-7), which takes no time that could be
+// measured (74 calls of all plans: 1.006, two runs of the same 1.005).
 #pragma once
 #include "sig_barrier.h"
 #include "sig_chen_stream.h"
@@ -36,7 +41,7 @@ struct BothPlan {
     static constexpr int CHILDREN = OWNP * (D + PAD);
     static constexpr int TILE = D * CHILDREN > lo(Q) ? D * CHILDREN : lo(Q);
     static constexpr int SUMS = (Q - 1) * OWN;                              // ancestors' sums of one x, and once summed over a letter
-    static constexpr size_t lds_entries() { return size_t(TILE) + 2 * LOW + SUMS + SUMS / R + THREADS / kWave; }
+    static constexpr size_t lds_entries() { return size_t(TILE) + 2 * LOW + SUMS + SUMS / R; }      // beside a sum per wave
 };
 
 template <typename T, typename P>
@@ -51,7 +56,7 @@ __global__ __launch_bounds__(P::THREADS) __attribute__((amdgpu_waves_per_eu(P::P
     T* Ra = Bl + P::LOW;                            // sums for dA, the block's words of a level end to end
     T* sums = Ra + P::LOW;                          // [m - 2][y][own s']
     T* next = sums + P::SUMS;                       // the same with one letter summed over
-    T* part_sum = next + P::SUMS / R;               // one value a wave
+    __shared__ double part_sum[P::THREADS / kWave];
     const int own_tid = threadIdx.x, lane = own_tid & (kWave - 1);
     const bool live = own_tid < OWN;
     const int mine = live ? own_tid : OWN - 1;      // idle threads do the last one's work again, but for its sums
@@ -87,7 +92,7 @@ __global__ __launch_bounds__(P::THREADS) __attribute__((amdgpu_waves_per_eu(P::P
             const int yi = own / OWNP, sp = part * OWNP + own % OWNP;       // the thread's word x y s'
             const uint32_t io = uint32_t(yi * SP + sp) * uint32_t(sizeof(T));
             const T a1 = fa[x];
-            T k1 = T(0), e[D], by[D];
+            T k1 = T(0), xy = T(0), e[D], by[D];
 #pragma unroll
             for (int y = 0; y < D; ++y) {
                 e[y] = load_at(g + P::lo(N) + x * (D * rs) + y * rs, so);
@@ -101,9 +106,10 @@ __global__ __launch_bounds__(P::THREADS) __attribute__((amdgpu_waves_per_eu(P::P
                 store_at(ta + y * rs, so, e[y]);
                 store_at(tb + y * rs, so, e[y]);
                 sum_x[y] = fmadd(a1, e[y], sum_x[y]);
-                sum_xy = fmadd(fa[D + x * D + y], e[y], sum_xy);
+                xy = fmadd(fa[D + x * D + y], e[y], xy);
                 k1 = fmadd(e[y], by[y], k1);
             }
+            sum_xy += xy;
             const T g1 = load_at(g + P::lo(N - 1) + x * rs, io);
             T w[Q];
             w[0] = load_at(fa + D + x * D, uint32_t(yi) * uint32_t(sizeof(T)));
@@ -139,13 +145,13 @@ __global__ __launch_bounds__(P::THREADS) __attribute__((amdgpu_waves_per_eu(P::P
 #pragma unroll
             for (int j = 0; j + 1 < Q; ++j) item_low[j] = fmadd(w[j], g1, item_low[j]);
             k1 = fmadd(g1, Bx[P::lo(Q) + yi * SP + sp], k1);
-            k1 = wave_sum(live ? k1 : T(0));
-            if (lane == 0) part_sum[own_tid / kWave] = k1;
+            const double block_k1 = wave_sum(live ? double(k1) : 0.0);
+            if (lane == 0) part_sum[own_tid / kWave] = block_k1;
             lds_barrier();
             if (own_tid == 0) {
-                T v = part_sum[0];
+                double v = part_sum[0];
                 for (int i = 1; i < P::THREADS / kWave; ++i) v += part_sum[i];
-                Ra[x] = v;
+                Ra[x] = T(v);
             }
             // the sums over the last letter, the last two, ...: level N - m takes m - 1 of these steps
             static_for<2, Q>([&](auto kc) {
@@ -157,11 +163,11 @@ __global__ __launch_bounds__(P::THREADS) __attribute__((amdgpu_waves_per_eu(P::P
                 for (int i = tid; i < (Q - k + 1) * out; i += P::THREADS) {
                     const int m = k + i / out, o = i % out;
                     const T* v = from + (m - (k == 2 ? 2 : k - 1)) * in + o * fan;
-                    T t = v[0];
+                    double t = double(v[0]);
 #pragma unroll
-                    for (int z = 1; z < fan; ++z) t += v[z];
-                    if (m == k) Ra[P::lo(N - k) + x * out + o] = t;     // level N - k is complete
-                    else to[(m - k) * out + o] = t;
+                    for (int z = 1; z < fan; ++z) t += double(v[z]);
+                    if (m == k) Ra[P::lo(N - k) + x * out + o] = T(t);     // level N - k is complete
+                    else to[(m - k) * out + o] = T(t);
                 }
                 lds_barrier();
             });

@@ -1029,3 +1029,21 @@ def test_level_one_of_the_right_factor_in_single_precision(P, row_forms, batch, 
     one = slice(1, d + 1) if scalar_term else slice(0, d)
     assert float((got - want)[:, one].norm() / want[:, one].norm()) < 2.0 ** -21
     assert float((got - want).norm() / want.norm()) < 2.0 ** -21
+
+
+@pytest.mark.parametrize("batch,d,deg,factor,level", [(8, 11, 4, 1, 2), (8, 12, 4, 1, 2), (8, 13, 4, 1, 2), (64, 6, 5, 1, 3), (200, 3, 8, 0, 1), (200, 4, 7, 0, 1)])
+def test_short_words_of_the_chen_adjoint_in_one_pass(P, row_forms, batch, d, deg, factor, level):
+    """Single precision, factors as signatures are: the levels that the one pass over dC sums from the most terms, both of its parts.  Bound: a value is
+    rounded where the pass keeps its part and where that is added to the truncated problem's, 2^-24 each (13 channels, degree 4, level 2, a thread's 169
+    terms one after the other in single precision: 2.2e-7)."""
+    from pysiglib_amd import _loader as L
+    L.CUSIG.cusig_amd_last_chen_both.restype = ctypes.c_int
+    gen = torch.Generator(device=DEV).manual_seed(100 * d + deg)
+    a, b = (P.sig((torch.randn(batch, 24, d, device=DEV, dtype=torch.float64, generator=gen) / 24 ** 0.5).cumsum(1), deg).float() for _ in range(2))
+    g = torch.randn(a.shape, device=DEV, dtype=torch.float32, generator=gen)
+    row_forms(2)
+    got = P.sig_combine_backprop(g, a, b, d, deg)[factor].double()
+    assert L.CUSIG.cusig_amd_last_chen_both() == 1
+    want = P.sig_combine_backprop(g.double(), a.double(), b.double(), d, deg)[factor]
+    at = slice(sum(d ** k for k in range(1, level)), sum(d ** k for k in range(1, level + 1)))
+    assert float((got - want)[:, at].norm() / want[:, at].norm()) < 2.0 ** -23
