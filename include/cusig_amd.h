@@ -240,7 +240,7 @@ CUSIG_AMD_API int cusig_amd_measure_fma_peak(int is_f64, int waves_per_simd, dou
  * scans the result for NaN and Inf) needs no pass of its own over the output.  No counterpart in the reference. */
 CUSIG_AMD_API int cusig_amd_last_sig_nonfinite(void) CUSIG_AMD_NOEXCEPT;
 /* The tuning and test hooks declared from here on (cusig_amd_force_*, cusig_amd_set_point_fed, _set_lead_lag_sparse,
- * _set_chen_low_levels, _set_row_forms, _set_degree2_staged, _set_alloc_limit) are process-wide switches for offline sweeps and for the
+ * _set_chen_low_levels, _set_row_forms, _set_degree2_staged, _set_alloc_limit, _set_pool_limit) are process-wide switches for offline sweeps and for the
  * test-suite.  They are ignored until cusig_amd_enable_test_hooks(1) has been called; cusig_amd_enable_test_hooks(0)
  * restores every default.  No counterpart in the reference. */
 CUSIG_AMD_API void cusig_amd_enable_test_hooks(int enabled) CUSIG_AMD_NOEXCEPT;
@@ -248,6 +248,9 @@ CUSIG_AMD_API void cusig_amd_enable_test_hooks(int enabled) CUSIG_AMD_NOEXCEPT;
  * exercises the retry on halves of the batch (siglib/cusig/cu_runtime_utils.h:103-105,212-235) and the fall-back of the
  * degree-3 matrix form to the sweeps.  cusig_amd_alloc_retries counts the splits since the library was loaded. */
 CUSIG_AMD_API void cusig_amd_set_alloc_limit(uint64_t bytes) CUSIG_AMD_NOEXCEPT;
+/* Test hook: the same for requests that would make the device's pool (cusig_amd_workspace_bytes) larger than `bytes` bytes (0: no
+ * limit). */
+CUSIG_AMD_API void cusig_amd_set_pool_limit(uint64_t bytes) CUSIG_AMD_NOEXCEPT;
 CUSIG_AMD_API int cusig_amd_alloc_retries(void) CUSIG_AMD_NOEXCEPT;
 /* Bytes the library's grow-only workspace pool holds on the current device (released by cusig_shutdown).  A host-side
  * query; no counterpart in the reference. */

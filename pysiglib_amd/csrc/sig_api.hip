@@ -259,9 +259,30 @@ thread_local int tl_row_form = 0, tl_chen_both = 0;
 std::mutex g_ws_mutex;
 static std::map<std::pair<int, int>, Workspace> g_ws;   // (device, slot)
 
-// test hook: workspace requests above this many bytes fail as if the device were out of memory (0: no limit)
-static std::atomic<uint64_t> g_alloc_limit{0};
+// test hooks: workspace requests above this many bytes, and those that would make the device's pool larger than this, fail as if
+// the device were out of memory (0: no limit)
+static std::atomic<uint64_t> g_alloc_limit{0}, g_pool_limit{0};
 static std::atomic<int> g_alloc_retries{0};     // calls split in two after a failed workspace allocation
+
+static uint64_t pool_bytes(int dev)
+{
+    uint64_t total = 0;
+    for (const auto& kv : g_ws)
+        if (kv.first.first == dev) total += kv.second.bytes;
+    return total;
+}
+
+static void give_back(Workspace& w)     // hipFree waits for the device, and so for whatever still uses the buffer
+{
+    if (!w.ptr) return;
+    void* const ptr = w.ptr;
+    w.ptr = nullptr;
+    w.bytes = 0;
+    SIG_HIP(hipFree(ptr));
+}
+
+static thread_local uint64_t tl_grown = 0;      // slots that grew since fine_if_it_fits began this thread's call
+constexpr int kHeadsSlot = 20;
 
 void* workspace(int slot, size_t bytes)
 {
@@ -269,19 +290,27 @@ void* workspace(int slot, size_t bytes)
     SIG_HIP(hipGetDevice(&dev));
     Workspace& w = g_ws[{dev, slot}];
     if (w.bytes < bytes) {
-        if (w.ptr) {
-            SIG_HIP(hipFree(w.ptr));
-            w.ptr = nullptr;
-            w.bytes = 0;
-        }
+        give_back(w);
         const size_t want = (bytes + bytes / 8 + 255) & ~size_t(255);
-        const uint64_t limit = g_alloc_limit;
-        if ((limit && want > limit) || hipMalloc(&w.ptr, want) != hipSuccess) {
-            (void)hipGetLastError();
-            w.ptr = nullptr;
-            throw std::bad_alloc();
+        auto allocate = [&] {
+            const uint64_t limit = g_alloc_limit, pool = g_pool_limit;
+            if ((limit && want > limit) || (pool && pool_bytes(dev) + want > pool) || hipMalloc(&w.ptr, want) != hipSuccess) {
+                (void)hipGetLastError();
+                w.ptr = nullptr;
+                return false;
+            }
+            w.bytes = want;
+            return true;
+        };
+        if (!allocate()) {
+            // the table of the sweeps with shared prefix chains, up to 1.1 GiB, was the last thing its call asked for, so no call that is under
+            // way here holds it: a call that fits without it gets that room
+            Workspace& table = g_ws[{dev, kHeadsSlot}];
+            if (slot == kHeadsSlot || !table.ptr) throw std::bad_alloc();
+            give_back(table);
+            if (!allocate()) throw std::bad_alloc();
         }
-        w.bytes = want;
+        tl_grown |= uint64_t(1) << slot;
     }
     return w.ptr;
 }
@@ -312,6 +341,21 @@ static void* dz_pair_buffer(DzPair& st, int which, size_t bytes)
         st.dirty[which] = capacity;
     }
     return p;
+}
+
+// what the thread's call has grown since fine_if_it_fits began it goes back to the device
+static void give_back_grown()
+{
+    std::lock_guard<std::mutex> lk(g_ws_mutex);
+    int dev = 0;
+    SIG_HIP(hipGetDevice(&dev));
+    for (int slot = 0; slot < 64; ++slot) {
+        if (!(tl_grown >> slot & 1)) continue;
+        auto it = g_ws.find({dev, slot});
+        if (it != g_ws.end()) give_back(it->second);
+        if (slot == kDzSlot[0] || slot == kDzSlot[1]) g_dz.erase(dev);      // what it knows of their contents
+    }
+    tl_grown = 0;
 }
 
 static int* g_flag_host = nullptr;     // pinned word the forward kernels report NaN / infinity through
@@ -655,10 +699,12 @@ template <typename F>
 static void fine_if_it_fits(F&& run)
 {
     tl_fine_more_pieces = false;
+    tl_grown = 0;
     try {
         run();
     } catch (const std::bad_alloc&) {
         if (!tl_fine_more_pieces) throw;
+        give_back_grown();          // the retry has the memory that it would have had without the attempt
         struct Off {
             Off() { tl_no_fine = true; }
             ~Off() { tl_no_fine = false; }
@@ -1325,7 +1371,7 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
             const uint64_t path_bytes = s.L * uint64_t(heads->row) * sizeof(T);
             const uint64_t chunk = std::min(batch, heads_chunk(heads, s.L));
             HeadsParams hp;
-            hp.table = workspace(20, chunk * path_bytes + uint64_t(heads->row) * sizeof(T));
+            hp.table = workspace(kHeadsSlot, chunk * path_bytes + uint64_t(heads->row) * sizeof(T));
             hp.L = p.L; hp.out_stride = p.out_stride; hp.scalar = p.scalar; hp.nseg = p.nseg; hp.lseg = p.lseg; hp.nonfinite = p.nonfinite;
             hp.stream = stream;
             for (uint64_t first = 0; first < batch; first += chunk) {
@@ -2082,6 +2128,7 @@ CUSIG_AMD_API void cusig_amd_enable_test_hooks(int enabled) noexcept
     g_force_tail = 0;
     g_force_k = 0;
     g_alloc_limit = 0;
+    g_pool_limit = 0;
 }
 
 CUSIG_AMD_API uint64_t cusig_amd_workspace_bytes(void) noexcept
@@ -2089,13 +2136,11 @@ CUSIG_AMD_API uint64_t cusig_amd_workspace_bytes(void) noexcept
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 0;
     std::lock_guard<std::mutex> lk(g_ws_mutex);
-    uint64_t total = 0;
-    for (const auto& kv : g_ws)
-        if (kv.first.first == dev) total += kv.second.bytes;
-    return total;
+    return pool_bytes(dev);
 }
 
 CUSIG_AMD_API void cusig_amd_set_alloc_limit(uint64_t bytes) noexcept { if (g_test_hooks) g_alloc_limit = bytes; }
+CUSIG_AMD_API void cusig_amd_set_pool_limit(uint64_t bytes) noexcept { if (g_test_hooks) g_pool_limit = bytes; }
 CUSIG_AMD_API int cusig_amd_alloc_retries(void) noexcept { return g_alloc_retries; }
 
 CUSIG_AMD_API int cusig_amd_kernel_choice(int backward, int is_f64, uint64_t dimension, uint64_t degree,

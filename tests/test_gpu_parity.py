@@ -1483,8 +1483,10 @@ def test_stream_ordered_mode(P, oracle):
 def _alloc_hooks():
     import ctypes
     from pysiglib_amd import _loader as L
-    L.CUSIG.cusig_amd_set_alloc_limit.argtypes = (ctypes.c_uint64,)
-    L.CUSIG.cusig_amd_set_alloc_limit.restype = None
+    for hook in (L.CUSIG.cusig_amd_set_alloc_limit, L.CUSIG.cusig_amd_set_pool_limit):
+        hook.argtypes, hook.restype = (ctypes.c_uint64,), None
+    L.CUSIG.cusig_amd_workspace_bytes.argtypes = ()
+    L.CUSIG.cusig_amd_workspace_bytes.restype = ctypes.c_uint64
     L.CUSIG.cusig_amd_alloc_retries.argtypes = ()
     L.CUSIG.cusig_amd_alloc_retries.restype = ctypes.c_int
     return L
@@ -2082,3 +2084,64 @@ def test_shared_prefix_chains_that_leave_the_chip_idle(P, heads, batch, length, 
     few = P.sig(x, deg)
     assert heads.name().startswith("fwd_f64_")
     assert np.max(level_rel_err(few.cpu().numpy(), whole.cpu().numpy(), d, deg)) < TOL[np.float64]
+
+
+def test_table_of_shared_prefix_chains_makes_room(P, heads):
+    """The table of an earlier call goes back to the device where a later call does not fit beside it: that call is neither halved nor refused."""
+    L = _alloc_hooks()
+    lib = L.CUSIG
+    rng = np.random.default_rng(5)
+    x = dev(np.cumsum(rng.standard_normal((64, 1000, 3)), axis=1) / 50)
+    z = dev((np.cumsum(rng.standard_normal((8, 4000, 20)), axis=1) / 300).astype(np.float32))
+    heads.pieces(1)
+    want = P.sig(z, 3)
+    heads.mode(2)
+    try:
+        lib.cusig_shutdown()
+        P.sig(x, 9)
+        assert heads.name().startswith("heads_fwd")
+        held, table = lib.cusig_amd_workspace_bytes(), 64 * 999 * HEADS_ROW[3, 9] * 8
+        retries = lib.cusig_amd_alloc_retries()
+        lib.cusig_amd_set_pool_limit(held)
+        got = P.sig(z, 3)
+        assert lib.cusig_amd_alloc_retries() == retries
+        assert lib.cusig_amd_workspace_bytes() < held - table // 2      # its increments are larger than the first call's
+        assert torch.equal(got, want)
+    finally:
+        lib.cusig_amd_set_pool_limit(0)
+
+
+def test_retry_without_extra_pieces_has_the_memory_of_the_attempt(P, heads):
+    """Paths that the compiled instance cuts in more pieces than the run-time kernel would: where their signatures do not fit, the run-time kernel serves
+    the call, whole, in the memory that it needs by itself: what the attempt had obtained is given back first."""
+    L = _alloc_hooks()
+    lib = L.CUSIG
+    rng = np.random.default_rng(6)
+    batch, length, d, deg = 217, 5392, 2, 6
+    x = dev(np.cumsum(rng.standard_normal((batch, length, d)), axis=1) / 100)
+    want = P.sig(x, deg)
+    name, pieces = heads.name(), lib.cusig_amd_last_segments()
+    assert name.startswith("fwd_f64_d2_")
+    retries = lib.cusig_amd_alloc_retries()
+    try:
+        lib.cusig_shutdown()
+        # room for the increments, the largest thing that the run-time kernel asks for, not for the products of the instance's pieces
+        increments = (batch * (length + 1) + 100) * d * 8 * 9 // 8 + 256
+        assert increments < (pieces + 32) * batch * want.shape[1] * 9
+        lib.cusig_amd_set_alloc_limit(increments)
+        P.sig(x, deg)
+        assert heads.name().startswith("fwd_f64_d0_")
+        few = lib.cusig_amd_last_segments()
+        row = batch * want.shape[1] * 8
+        need = lib.cusig_amd_workspace_bytes()
+        assert few < pieces and need <= (few + few + 32) * row * 9 // 8 + 512 + increments
+        lib.cusig_shutdown()
+        lib.cusig_amd_set_alloc_limit(0)
+        lib.cusig_amd_set_pool_limit(need)
+        got = P.sig(x, deg)
+        assert heads.name().startswith("fwd_f64_d0_") and lib.cusig_amd_last_segments() == few
+    finally:
+        lib.cusig_amd_set_alloc_limit(0)
+        lib.cusig_amd_set_pool_limit(0)
+    assert lib.cusig_amd_alloc_retries() == retries
+    assert np.max(level_rel_err(got.cpu().numpy(), want.cpu().numpy(), d, deg)) < TOL[np.float64]
