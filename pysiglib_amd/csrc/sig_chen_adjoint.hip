@@ -222,32 +222,36 @@ static bool any_of_plans(Go&& go, BothPlans<P...>)
     return (go(P()) || ...);
 }
 
-// Both factors in one pass over dC, where there is such a kernel.  Blocks of a row (D / R), registers (waves a SIMD) and the rows from which
-// it takes over were measured for each (ms before / with, double precision): 1080 rows of 10 channels, degree 5: 1.05 / 0.85; 1806 of 9, 5: 1.30 /
-// 0.81; 4096 of 6, 5: 0.67 / 0.32, of 5, 6: 1.03 / 0.68, of 3, 7: 0.62 / 0.22; 298 of 13, 5: 2.99 / 0.93; 488 of 22, 4: 1.50 / 0.74; single row of 6,
-// 6: 0.167 / 0.072; of 8, 4: 0.053 / 0.057 (at 400 rows 0.065 / 0.063).  Slower: 2 channels, degree 11 (0.84 / 1.16), 8, 6 (1.28 / 1.33).
+// Both factors in one pass over dC, where there is such a kernel.  Blocks of a row (D / R), registers (waves a SIMD) and, per precision, the rows from
+// which it takes over were measured for each against the general kernels with the longer words that those take where rows are few
+// (right_word_length).  us, general / one pass, double: 1080 rows of 10 channels, degree 5: 1050 / 850; 1806 of 9, 5: 1300 / 810; 4096 of 6, 5: 670 / 320, of
+// 5, 6: 1030 / 680, of 3, 7: 620 / 220; 298 of 13, 5: 2990 / 930; 512 of 22, 4: 1542 / 748; single row of 6, 6: 155 / 54.  Where a row's few blocks leave
+// the chip idle: 1 row of 20, 4: 63 / 141, 32: 94 / 147, 80: 188 / 200, 96: 213 / 204; 24 of 22, 4: 132 / 167, 28: 179 / 167; 1 of 8, 4: 35 / 43, 512:
+// 51 / 50; of 14, 5: 94 / 101, 3: 109 / 106.  Single precision moves half as much and gains sooner: 1 row of 17, 4: 110 / 118 and 106 / 84; 48 of
+// 20, 4: 134 / 148 and 101 / 100.  16 channels, degree 5, has one word a thread in 16 blocks of a row, each with 113 KB of LDS in double precision: 123 / 183,
+// 128 rows 1289 / 1567.  Without a plan: 2 channels, degree 11 (0.84 / 1.16 ms), 8, 6 (1.28 / 1.33).
 template <typename T>
 static bool launch_both_factors(const T* dC, T* dA, T* dB, const T* A, const T* B, uint64_t batch, uint64_t dimension, uint64_t degree,
                                 const SigShape& s, hipStream_t stream, const SharedRows& dc)
 {
     auto go = [&](auto plan) {
         using P = decltype(plan);
-        if (dimension != uint64_t(P::D) || degree != uint64_t(P::N) || (row_forms() != 2 && batch < uint64_t(P::FROM))) return false;
+        if (dimension != uint64_t(P::D) || degree != uint64_t(P::N) || (row_forms() != 2 && batch < uint64_t(sizeof(T) == 8 ? P::FROM64 : P::FROM32))) return false;
         launch_combine_bwd_items<T, double>(dC, dA, dB, A, B, batch, dimension, uint64_t(P::Q), s, stream, 3, dc, 2, 0);
         launch_both<T, P>(dC, dA, dB, A, B, batch, s, stream);
         tl_chen_both = 1;
         return true;
     };
-    return any_of_plans(go, BothPlans<BothPlan<4, 3, 4, 4, 192>, BothPlan<5, 3, 5, 4, 96>, BothPlan<6, 2, 6, 4, 256>, BothPlan<8, 2, 8, 4, 400>,
-                        BothPlan<9, 2, 9, 4, 48>, BothPlan<10, 2, 10, 3, 96>, BothPlan<11, 2, 11, 3, 1>, BothPlan<12, 2, 12, 3, 1>,
-                        BothPlan<13, 2, 13, 3, 1>, BothPlan<14, 2, 14, 3, 160>, BothPlan<15, 2, 15, 2, 128>, BothPlan<16, 2, 16, 2, 128>,
-                        BothPlan<17, 2, 17, 2, 1>, BothPlan<18, 2, 9, 2, 1>, BothPlan<19, 2, 19, 2, 1>, BothPlan<20, 2, 10, 2, 1>,
-                        BothPlan<21, 2, 7, 2, 1>, BothPlan<22, 2, 11, 2, 1>, BothPlan<24, 2, 8, 2, 1>, BothPlan<6, 3, 6, 4, 1>,
-                        BothPlan<7, 3, 1, 4, 1>, BothPlan<8, 3, 4, 3, 1>, BothPlan<9, 3, 3, 3, 1>, BothPlan<10, 3, 2, 3, 1>,
-                        BothPlan<11, 3, 1, 3, 1>, BothPlan<12, 3, 1, 3, 1>, BothPlan<13, 3, 1, 2, 1>, BothPlan<14, 3, 1, 2, 1>,
-                        BothPlan<16, 3, 1, 2, 1>, BothPlan<4, 4, 2, 4, 1>, BothPlan<5, 4, 1, 3, 1>, BothPlan<6, 4, 1, 3, 1>,
-                        BothPlan<7, 4, 1, 3, 1>, BothPlan<3, 5, 3, 4, 64>, BothPlan<4, 5, 1, 3, 1>, BothPlan<3, 6, 1, 3, 1>,
-                        BothPlan<2, 8, 1, 3, 1>>());
+    return any_of_plans(go, BothPlans<BothPlan<4, 3, 4, 4, 192, 256>, BothPlan<5, 3, 5, 4, 96, 96>, BothPlan<6, 2, 6, 4, 256, 256>,
+                        BothPlan<8, 2, 8, 4, 512, 400>, BothPlan<9, 2, 9, 4, 48, 48>, BothPlan<10, 2, 10, 3, 96, 96>, BothPlan<11, 2, 11, 3, 1, 1>,
+                        BothPlan<12, 2, 12, 3, 1, 1>, BothPlan<13, 2, 13, 3, 1, 1>, BothPlan<14, 2, 14, 3, 160, 160>,
+                        BothPlan<15, 2, 15, 2, 128, 128>, BothPlan<16, 2, 16, 2, 128, 128>, BothPlan<17, 2, 17, 2, 12, 1>,
+                        BothPlan<18, 2, 9, 2, 64, 48>, BothPlan<19, 2, 19, 2, 32, 1>, BothPlan<20, 2, 10, 2, 96, 48>, BothPlan<21, 2, 7, 2, 48, 32>,
+                        BothPlan<22, 2, 11, 2, 28, 20>, BothPlan<24, 2, 8, 2, 56, 28>, BothPlan<6, 3, 6, 4, 1, 1>, BothPlan<7, 3, 1, 4, 1, 1>,
+                        BothPlan<8, 3, 4, 3, 1, 1>, BothPlan<9, 3, 3, 3, 1, 1>, BothPlan<10, 3, 2, 3, 1, 1>, BothPlan<11, 3, 1, 3, 1, 1>,
+                        BothPlan<12, 3, 1, 3, 1, 1>, BothPlan<13, 3, 1, 2, 1, 1>, BothPlan<14, 3, 1, 2, 3, 1>, BothPlan<16, 3, 1, 2, kBothNever, 1>,
+                        BothPlan<4, 4, 2, 4, 1, 1>, BothPlan<5, 4, 1, 3, 1, 1>, BothPlan<6, 4, 1, 3, 1, 1>, BothPlan<7, 4, 1, 3, 1, 1>,
+                        BothPlan<3, 5, 3, 4, 64, 64>, BothPlan<4, 5, 1, 3, 1, 1>, BothPlan<3, 6, 1, 3, 1, 1>, BothPlan<2, 8, 1, 3, 1, 1>>());
 }
 
 // launches the adjoint of the Chen product on `stream`

@@ -26,10 +26,12 @@
 
 namespace sigamd {
 
-// FROM: rows of a call from which the kernel is the sooner one
-template <int D_, int Q_, int R_, int PER_SIMD_, int FROM_>
+constexpr int kBothNever = 0x7fffffff;
+
+// FROM64, FROM32: rows of a call from which the kernel is the sooner one, in double and in single precision
+template <int D_, int Q_, int R_, int PER_SIMD_, int FROM64_, int FROM32_>
 struct BothPlan {
-    static constexpr int D = D_, Q = Q_, R = R_, N = Q + 2, PER_SIMD = PER_SIMD_, FROM = FROM_;
+    static constexpr int D = D_, Q = Q_, R = R_, N = Q + 2, PER_SIMD = PER_SIMD_, FROM64 = FROM64_, FROM32 = FROM32_;
     static constexpr int PARTS = D / R;                                     // blocks of a row
     static constexpr int S = int(ipow64(D, Q)), SP = S / D;                 // words s, s'
     static constexpr int OWN = S / PARTS, OWNP = SP / PARTS;                // a block's

@@ -1047,3 +1047,23 @@ def test_short_words_of_the_chen_adjoint_in_one_pass(P, row_forms, batch, d, deg
     want = P.sig_combine_backprop(g.double(), a.double(), b.double(), d, deg)[factor]
     at = slice(sum(d ** k for k in range(1, level)), sum(d ** k for k in range(1, level + 1)))
     assert float((got - want)[:, at].norm() / want[:, at].norm()) < 2.0 ** -23
+
+
+@pytest.mark.parametrize("d,deg,dtype,line", [
+    (8, 4, np.float64, 512), (17, 4, np.float64, 12), (18, 4, np.float64, 64), (18, 4, np.float32, 48), (19, 4, np.float64, 32), (20, 4, np.float64, 96),
+    (20, 4, np.float32, 48), (21, 4, np.float64, 48), (22, 4, np.float64, 28), (22, 4, np.float32, 20), (24, 4, np.float64, 56), (14, 5, np.float64, 3),
+    (16, 5, np.float64, None), (16, 5, np.float32, 1), (17, 4, np.float32, 1), (6, 6, np.float64, 1)])
+def test_rows_from_which_the_chen_adjoint_takes_one_pass(P, oracle, d, deg, dtype, line):
+    """The line between the general kernels of the Chen product's adjoint and the pass that takes both factors: either side of it, as measured for each
+    precision, and single rows, which the general kernels' longer words serve sooner; both sides against the oracle."""
+    from pysiglib_amd import _loader as L
+    L.CUSIG.cusig_amd_last_chen_both.restype = ctypes.c_int
+    rng = np.random.default_rng(19 * d + deg)
+    scale = np.concatenate([np.full(d ** k, 1.0 / np.sqrt(float(d) ** k)) for k in range(1, deg + 1)])
+    for batch in (1, 16) if line is None else sorted({1, max(1, line - 1), line}):
+        g, a, b = (dev((rng.standard_normal((batch, scale.size)) * scale).astype(dtype)) for _ in range(3))
+        got = P.sig_combine_backprop(g, a, b, d, deg)
+        assert L.CUSIG.cusig_amd_last_chen_both() == (0 if line is None else batch >= line), batch
+        want = oracle.sig_combine_backprop(*(v[-1:].cpu().numpy().astype(np.float64) for v in (g, a, b)), d, deg)
+        for v, ref in zip(got, want):
+            assert row_rel_err(v[-1:].cpu().numpy(), ref) < TOL[dtype]
