@@ -109,13 +109,17 @@ static const KernelEntry* choose_entry(bool backward, bool f64, uint64_t d, uint
 static thread_local bool tl_no_fine = false, tl_fine_more_pieces = false;
 
 // Where choose_entry's estimate asks for the run-time kernel and no finer partition takes its place, the instance after all (else null): time pieces and
-// the staged twin make it the sooner one of 16548 random calls in that state, but where this rule says (9700 calls with the instance now: 0.81 of their time,
-// 25 of them 1.03 to 1.08 times as long; 571 paths x 6136 steps x 12 channels, degree 3, double, backward 14.6 -> 4.0 ms; 1 x 15 x 29, degree 4, single
-// 0.26 -> 0.06):
+// the staged twin make it the sooner one of 28000 random calls in that state, but where this rule says (0.80 of the run-time kernel's time on average, four calls
+// 1.03 to 1.05 times as long, 59 x 6384 x 4, degree 3, the longest; 571 paths x 6136 steps x 12 channels, degree 3, double, backward 14.6 -> 4.0 ms;
+// 1 x 15 x 29, degree 4, single 0.26 -> 0.06):
 // - forward, lanes that hold one level, or few steps: 0.92 on average, but up to 1.47 (3 x 731 x 13, degree 3);
 // - backward, lanes that hold four levels and more: 135 x 80 x 2, degree 9, single 0.19 -> 0.34;
-// - backward, few steps: 40 us -> 47 (5 x 4 x 32, degree 3); many steps in all of few coefficients: 116 x 13224 x 2, degree 4, 0.39 -> 0.59;
-//   few paths of 128 to 511 steps, which instances do not cut yet: 2 x 345 x 8, degree 4, double 0.13 -> 0.19.
+// - backward, few steps: 40 us -> 47 (5 x 4 x 32, degree 3), in single precision where a prefix's last lane lacks letters up to 15 (3 x 14 x 32, degree 3:
+//   44 -> 48);
+// - many steps in all of few coefficients: 116 x 13224 x 2, degree 4, 0.39 -> 0.59; a few times ten paths of the longest, 3 channels, degree 4: 1.02 on average of
+//   13, up to 1.16 (64 x 8480: 255 us -> 296);
+// - few paths of 128 to 511 steps, which instances do not cut yet: 2 x 345 x 8, degree 4, double 0.13 -> 0.19; up to 16 paths at 8 channels, degree 4, from 256
+//   steps, where the run-time kernel cuts them, to 399 (10 x 348: 140 us -> 168; 10 x 224: 207 -> 116, 9 x 508: 164 -> 120).
 static const KernelEntry* instance_after_all(const KernelEntry* e, bool backward, uint64_t d, uint64_t degree, uint64_t batch, uint64_t L)
 {
     if (e->D != 0 || g_force_tail > 0 || tl_no_fine) return nullptr;
@@ -123,9 +127,12 @@ static const KernelEntry* instance_after_all(const KernelEntry* e, bool backward
     if (!spec || spec->D <= 0) return nullptr;
     if (!backward) return L >= 256 && spec->tail >= 2 ? spec : nullptr;
     if (L < 8 || spec->tail >= 4) return nullptr;
+    if (L < 16 && batch < 16 && !spec->is_f64 && d % uint64_t(spec->k) != 0) return nullptr;
     const int64_t top = ipow64(int64_t(d), int(degree));
     if (top <= 32 && batch * L > 100000) return nullptr;
+    if (top == 81 && L >= 6900 && batch < 84) return nullptr;
     if (top >= 4096 && batch <= 8 && L >= 128 && L < 512) return nullptr;
+    if (top >= 4096 && degree == 4 && d <= 8 && batch <= 16 && L >= 256 && L < 400) return nullptr;
     return spec;
 }
 

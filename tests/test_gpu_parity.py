@@ -2145,3 +2145,50 @@ def test_retry_without_extra_pieces_has_the_memory_of_the_attempt(P, heads):
         lib.cusig_amd_set_pool_limit(0)
     assert lib.cusig_amd_alloc_retries() == retries
     assert np.max(level_rel_err(got.cpu().numpy(), want.cpu().numpy(), d, deg)) < TOL[np.float64]
+
+
+@pytest.fixture
+def no_finer_partitions():
+    import ctypes
+    from pysiglib_amd import _loader as L
+    L.CUSIG.cusig_amd_set_fine.argtypes, L.CUSIG.cusig_amd_set_fine.restype = (ctypes.c_int,), None
+    L.CUSIG.cusig_amd_set_fine(0)
+    L.CUSIG.cusig_amd_set_profiling(1)
+    yield lambda: L.CUSIG.cusig_amd_last_kernel_name().decode()
+    L.CUSIG.cusig_amd_set_fine(1)
+    L.CUSIG.cusig_amd_set_profiling(0)
+
+
+@pytest.mark.parametrize("batch,steps,d,deg,dtype,instance", [
+    (1, 7, 29, 4, np.float64, False), (1, 8, 29, 4, np.float64, True), (4, 7, 12, 3, np.float32, False), (4, 8, 12, 3, np.float32, True),
+    (14, 41, 2, 4, np.float64, True), (14, 41, 2, 9, np.float32, False),
+    (2, 127, 8, 4, np.float64, True), (2, 128, 8, 4, np.float64, False), (2, 511, 8, 4, np.float64, False), (2, 512, 8, 4, np.float64, True),
+    (10, 255, 8, 4, np.float64, True), (10, 256, 8, 4, np.float64, False), (10, 399, 8, 4, np.float64, False), (10, 400, 8, 4, np.float64, True),
+    (14, 300, 8, 4, np.float64, False), (17, 300, 8, 4, np.float64, True),
+    (100, 1000, 2, 4, np.float64, True), (100, 1001, 2, 4, np.float64, False),
+    (60, 6899, 3, 4, np.float64, True), (60, 6900, 3, 4, np.float64, False), (83, 7000, 3, 4, np.float64, False), (84, 7000, 3, 4, np.float64, True),
+    (3, 15, 32, 3, np.float32, False), (3, 16, 32, 3, np.float32, True), (15, 12, 32, 3, np.float32, False), (16, 12, 32, 3, np.float32, True)])
+def test_lines_between_instances_and_run_time_kernels_backward(P, oracle, no_finer_partitions, batch, steps, d, deg, dtype, instance):
+    """Launches that leave the chip without work: the kernel either side of each line, and the gradient."""
+    rng = np.random.default_rng(100 * d + steps)
+    x = (np.cumsum(rng.standard_normal((batch, steps + 1, d)), axis=1) / np.sqrt(steps * d)).astype(dtype)
+    ref = oracle.signature(x.astype(np.float64), deg, n_jobs=-1)
+    g = rng.standard_normal(ref.shape).astype(dtype)
+    want = oracle.sig_backprop(x.astype(np.float64), ref, g.astype(np.float64), deg, n_jobs=-1)
+    got = P.sig_backprop(dev(x), dev(ref.astype(dtype)), dev(g), deg).cpu().numpy()
+    name = no_finer_partitions()
+    assert ("_d%d_" % d if instance else "_d0_") in name, name
+    assert bwd_rel_err(got, want) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("batch,steps,d,deg,dtype,instance", [
+    (4, 255, 2, 4, np.float64, False), (4, 256, 2, 4, np.float64, True), (1, 255, 8, 4, np.float32, False), (1, 256, 8, 4, np.float32, True),
+    (256, 255, 6, 3, np.float64, False), (256, 256, 6, 3, np.float64, True), (16, 256, 10, 3, np.float64, True),
+    (3, 730, 13, 3, np.float64, False), (1, 730, 29, 3, np.float32, False)])        # the last two: lanes that hold one level
+def test_lines_between_instances_and_run_time_kernels_forward(P, oracle, no_finer_partitions, batch, steps, d, deg, dtype, instance):
+    rng = np.random.default_rng(100 * d + steps)
+    x = (np.cumsum(rng.standard_normal((batch, steps + 1, d)), axis=1) / np.sqrt(steps * d)).astype(dtype)
+    got = P.sig(dev(x), deg).cpu().numpy()
+    name = no_finer_partitions()
+    assert ("_d%d_" % d if instance else "_d0_") in name, name
+    assert np.max(level_rel_err(got, oracle.signature(x.astype(np.float64), deg, n_jobs=-1), d, deg)) < TOL[dtype]
