@@ -1051,7 +1051,7 @@ static int heads_pieces(const HeadsEntry* e, const KernelEntry* run, const Split
         return 0;
     const uint64_t chunk = std::min(batch, heads_chunk(e, L));
     if (chunk == 0) return 0;
-    if (forced > 0) return mode == 2 ? int(std::min<uint64_t>(uint64_t(forced), L)) : 0;
+    if (forced > 0) return mode == 2 ? int(std::min<uint64_t>(std::min<uint64_t>(uint64_t(forced), L), uint64_t(e->most_blocks / e->blocks))) : 0;
     const int64_t cus = simd_count() / 4;
     const double wait = e->lone_ns < 500 && double(chunk) * double(L) * e->row * sizeof(double) > 140e6 ? 100.0 : 0.0;
     auto step_of = [&](uint64_t paths, int g) {      // ns of a step of one launch
@@ -1376,7 +1376,8 @@ static void signature_impl(const T* path, T* out, uint64_t batch, uint64_t dimen
         tl_matrix_form = by_rows && sizeof(T) == 4;
         if (heads) {
             const uint64_t path_bytes = s.L * uint64_t(heads->row) * sizeof(T);
-            const uint64_t chunk = std::min(batch, heads_chunk(heads, s.L));
+            const uint64_t launch = uint64_t(heads->most_blocks) / (uint64_t(heads->blocks) * uint64_t(p.nseg));      // the memory ends sooner
+            const uint64_t chunk = std::min({batch, heads_chunk(heads, s.L), launch});
             HeadsParams hp;
             hp.table = workspace(kHeadsSlot, chunk * path_bytes + uint64_t(heads->row) * sizeof(T));
             hp.L = p.L; hp.out_stride = p.out_stride; hp.scalar = p.scalar; hp.nseg = p.nseg; hp.lseg = p.lseg; hp.nonfinite = p.nonfinite;

@@ -22,6 +22,7 @@ struct HeadsEntry {
     int D, N;
     int row;                // elements of the table per step
     int blocks;             // blocks per (path, segment)
+    int64_t most_blocks;    // of a launch, which numbers its threads with 32 bits
     int resident;           // blocks of a compute unit
     int step_ns, lone_ns;   // duration of a step: so many blocks on every compute unit; a block or less
     hipError_t (*launch)(const HeadsParams&);

@@ -430,11 +430,14 @@ __global__ __launch_bounds__(Plan::WAVES * kWave) __attribute__((amdgpu_waves_pe
 }
 
 template <typename Plan>
+constexpr int64_t kMostBlocks = ((int64_t(1) << 32) - 1) / (Plan::WAVES * kWave);
+
+template <typename Plan>
 static hipError_t launch_plan(const HeadsParams& p)
 {
     const int64_t rows = p.paths * p.L;
     const int64_t blocks = p.paths * p.nseg * Plan::GROUPS * Plan::PARTS;
-    if (blocks < 1 || blocks > 2147483647LL) return hipErrorInvalidConfiguration;
+    if (blocks < 1 || blocks > kMostBlocks<Plan>) return hipErrorInvalidConfiguration;
     hipLaunchKernelGGL((head_table_kernel<Plan>), dim3(unsigned(std::min<int64_t>((rows * Plan::ROW + kBlock - 1) / kBlock, 8192))), dim3(kBlock), 0,
                        p.stream, static_cast<const T*>(p.inc), static_cast<T*>(p.table), rows, p.L);
     hipError_t e = hipGetLastError();
@@ -454,7 +457,9 @@ static constexpr HeadsEntry entry(int step_ns, int lone_ns)
 {
     constexpr int by_waves = 4 * Plan::PER_SIMD / Plan::WAVES, by_lds = int(160 * 1024 / Plan::kLds);
     static_assert(by_waves >= 1 && by_lds >= 1, "a block fits a compute unit");
-    return HeadsEntry{Plan::D, Plan::N, Plan::ROW, Plan::GROUPS * Plan::PARTS, by_waves < by_lds ? by_waves : by_lds, step_ns, lone_ns, launch_plan<Plan>};
+    static_assert(Plan::GROUPS * Plan::PARTS <= kMostBlocks<Plan> / 64, "a path in as many pieces as the dispatch cuts fits a launch");
+    return HeadsEntry{Plan::D, Plan::N, Plan::ROW, Plan::GROUPS * Plan::PARTS, kMostBlocks<Plan>, by_waves < by_lds ? by_waves : by_lds, step_ns, lone_ns,
+                      launch_plan<Plan>};
 }
 
 // Plans found by a sweep over heads, tails and blocks at full launches (3e7 / D^N x 5 paths of 257 points), kept where at least 12 % faster than the
