@@ -227,9 +227,10 @@ static bool any_of_plans(Go&& go, BothPlans<P...>)
 // (right_word_length).  us, general / one pass, double: 1080 rows of 10 channels, degree 5: 1050 / 850; 1806 of 9, 5: 1300 / 810; 4096 of 6, 5: 670 / 320, of
 // 5, 6: 1030 / 680, of 3, 7: 620 / 220; 298 of 13, 5: 2990 / 930; 512 of 22, 4: 1542 / 748; single row of 6, 6: 155 / 54.  Where a row's few blocks leave
 // the chip idle: 1 row of 20, 4: 63 / 141, 32: 94 / 147, 80: 188 / 200, 96: 213 / 204; 24 of 22, 4: 132 / 167, 28: 179 / 167; 1 of 8, 4: 35 / 43, 512:
-// 51 / 50; of 14, 5: 94 / 101, 3: 109 / 106.  Single precision moves half as much and gains sooner: 1 row of 17, 4: 110 / 118 and 106 / 84; 48 of
-// 20, 4: 134 / 148 and 101 / 100.  16 channels, degree 5, has one word a thread in 16 blocks of a row, each with 113 KB of LDS in double precision: 123 / 183,
-// 128 rows 1289 / 1567.  No line was raised for less than 4 % at the cost of accuracy (256 rows of 4, 5, single: 31 / 30).  Without a plan: 2 channels, degree 11 (0.84 / 1.16 ms), 8, 6 (1.28 / 1.33).
+// 51 / 50.  Single precision moves half as much and gains sooner: 1 row of 17, 4: 110 / 118 and 106 / 84; 48 of 20, 4: 134 / 148 and 101 / 100.
+// 16 channels, degree 5, has one word a thread in 16 blocks of a row, each with 113 KB of LDS in double precision: 123 / 183, 128 rows 1289 / 1567.
+// The one pass rounds less at degree 5 (1 row, double, right factor: 14, 5: 3.0e-16 / 1.6e-16; 16, 5: 3.6 / 1.6; degree 4 1.6-2.5 / 1.3-1.7), so no line was
+// raised for less than a tenth (1 row of 14, 5: 94 / 101; 256 rows of 4, 5, single: 31 / 30).  Without a plan: 2 channels, degree 11 (0.84 / 1.16 ms), 8, 6 (1.28 / 1.33).
 template <typename T>
 static bool launch_both_factors(const T* dC, T* dA, T* dB, const T* A, const T* B, uint64_t batch, uint64_t dimension, uint64_t degree,
                                 const SigShape& s, hipStream_t stream, const SharedRows& dc)
@@ -249,7 +250,7 @@ static bool launch_both_factors(const T* dC, T* dA, T* dB, const T* A, const T* 
                         BothPlan<18, 2, 9, 2, 64, 48>, BothPlan<19, 2, 19, 2, 32, 1>, BothPlan<20, 2, 10, 2, 96, 48>, BothPlan<21, 2, 7, 2, 48, 32>,
                         BothPlan<22, 2, 11, 2, 28, 20>, BothPlan<24, 2, 8, 2, 56, 28>, BothPlan<6, 3, 6, 4, 1, 1>, BothPlan<7, 3, 1, 4, 1, 1>,
                         BothPlan<8, 3, 4, 3, 1, 1>, BothPlan<9, 3, 3, 3, 1, 1>, BothPlan<10, 3, 2, 3, 1, 1>, BothPlan<11, 3, 1, 3, 1, 1>,
-                        BothPlan<12, 3, 1, 3, 1, 1>, BothPlan<13, 3, 1, 2, 1, 1>, BothPlan<14, 3, 1, 2, 3, 1>, BothPlan<16, 3, 1, 2, kBothNever, 1>,
+                        BothPlan<12, 3, 1, 3, 1, 1>, BothPlan<13, 3, 1, 2, 1, 1>, BothPlan<14, 3, 1, 2, 1, 1>, BothPlan<16, 3, 1, 2, kBothNever, 1>,
                         BothPlan<4, 4, 2, 4, 1, 1>, BothPlan<5, 4, 1, 3, 1, 1>, BothPlan<6, 4, 1, 3, 1, 1>, BothPlan<7, 4, 1, 3, 1, 1>,
                         BothPlan<3, 5, 3, 4, 64, 64>, BothPlan<4, 5, 1, 3, 1, 1>, BothPlan<3, 6, 1, 3, 1, 1>, BothPlan<2, 8, 1, 3, 1, 1>>());
 }

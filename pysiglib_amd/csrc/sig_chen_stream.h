@@ -765,13 +765,14 @@ static inline bool fill_stream_levels(StreamLevels& lv, uint64_t d, uint64_t deg
 // factors' gradients, us, shortest / the length taken (single precision): 1 row of 16, 6: 23259 (2) / 667 (4); 4 rows of 20, 5: 2070 (2) / 239 (3); 5 of 8, 7:
 // 1327 (3) / 318 (5); 3 of 7, 7: 965 (3) / 358 (5); 1 of 33, 4: 224 (2) / 117 (3); 2 of 5, 9: 527 (5) / 428 (6); 4 of 4, 8: 215 (4) / 175 (5); 3 of 5, 7: 139 (4) /
 // 137 (5), which is left at 4.
-// The estimate, us: 0.35 a load of the walk while a SIMD has no second wave of them; 0.03 an addition to one address, 2e-5 any; a longer
+// The estimate, us, as measured on 1024 SIMDs: 0.35 a load of the walk while a SIMD has no second wave of them; 0.03 an addition to one address, 2e-5 any; a longer
 // word has to save 15, and 20 more for the two launches that longer words than the shortest take.
 // The sums of longer words are kept in double precision (right_sums; `elem_bytes` of T: they have to fit a row's top level).  For T = double that is no
 // better than T, so there the additions to one address may not grow by more than the walk, whose products a lane sums, gets shorter: errors as of that many
 // roundings.
 static inline int right_word_length(const StreamLevels& lv, uint64_t d, int degree, uint64_t batch, int shortest, size_t elem_bytes)
 {
+    constexpr double kMeasuredSimds = 1024.0;
     struct Cost { double time, roundings; };
     auto cost = [&](int qe) {
         double words = 1.0, walk = 0.0;
@@ -779,7 +780,7 @@ static inline int right_word_length(const StreamLevels& lv, uint64_t d, int degr
         for (int i = qe; i < degree; ++i) walk = (walk + 1.0) * double(d);
         const double waves = double(batch) * words / kWave;
         const double adds = qe > 1 ? std::max(0.03 * words / double(d), 2e-5 * words * double(batch) * (qe - 1)) : 0.0;
-        return Cost{0.35 * walk * std::max(1.0, waves / 1024.0) + adds, std::sqrt(walk) + (qe > 1 ? std::sqrt(words / double(d)) : 0.0)};
+        return Cost{0.35 * walk * std::max(1.0, waves / kMeasuredSimds) + adds, std::sqrt(walk) + (qe > 1 ? std::sqrt(words / double(d)) : 0.0)};
     };
     const Cost first = cost(shortest);
     double top = 1.0;

@@ -13,9 +13,10 @@
 //
 // Double precision only: single precision has the registers for larger subtrees in the tree kernels, whose all-vector
 // operands it issues faster (3 channels, degree 12, 282 paths of 257 points: tree 3.1 ms, this form 4.9).
-// Measured at 3 channels, degree 12, 64 paths of 4096 points: 23.3 -> 14.5-15.5 ms; 74 vector instructions a step and wave for
-// 27 top-level values (tree: 455 for 81), four waves a SIMD.  Bound: vector FP64 issue, 86 % of it at the clock of 2.3 GHz; the rest are waits
-// for scalar operands and for the other waves of a block at the end of a chunk.
+// Measured at 3 channels, degree 12, 64 paths of 4096 points: 23.3 -> 14.4-15.3 ms; 74 vector instructions a step and wave for
+// 27 top-level values (tree: 455 for 81), four waves a SIMD.  Bound: vector FP64 issue, 80 % of a SIMD's cycles (6.9e6 instructions of four
+// cycles in 34.4e6, at 2.3 GHz; counters), beside the scalar cache, whose 36 dwords a step and wave take as long; the rest are waits for scalar operands and
+// for the other waves of a block at the end of a chunk.
 #include <algorithm>
 
 #include "sig_barrier.h"
@@ -462,8 +463,8 @@ static constexpr HeadsEntry entry(int step_ns, int lone_ns)
                       launch_plan<Plan>};
 }
 
-// Plans found by a sweep over heads, tails and blocks at full launches (3e7 / D^N x 5 paths of 257 points), kept where at least 12 % faster than the
-// tree kernels.  ms before / with: 3 channels, degree 9 .. 14: 2.80 / 1.98, 7.14 / 4.84, 7.58 / 4.92, 6.53 / 4.71, 8.83 / 4.65, 9.61 / 4.66;
+// Plans found by a sweep over heads, tails and blocks at full launches (3e7 / D^N x 5 paths of 257 points), kept where they take at most 0.9 of the
+// tree kernels' time.  ms before / with: 3 channels, degree 9 .. 14: 2.80 / 1.98, 7.14 / 4.84, 7.58 / 4.92, 6.53 / 4.71, 8.83 / 4.65, 9.61 / 4.66;
 // 4, 9 and 10: 4.25 / 3.81, 4.46 / 3.72; 5, 8 and 9: 4.09 / 3.46, 4.55 / 3.38; 6, 7 and 8: 3.14 / 2.77, 3.53 / 2.56; 8, 7: 3.25 / 2.47; 11, 6:
 // 3.64 / 2.78; 4, 11 and 12: 5.02 / 4.22, 5.09 / 3.62; 5, 10: 5.33 / 3.51; 6, 9: 3.70 / 2.52; 7, 8: 3.68 / 2.97; 8, 8: 3.25 / 2.31; 10, 7:
 // 3.26 / 2.45.  3, 15 and 16, 5, 11, 7, 9 and 9, 8 have no compiled tree kernel (3, 15: 94.0 / 4.89).  12, 7 gains only in

@@ -1051,7 +1051,7 @@ def test_short_words_of_the_chen_adjoint_in_one_pass(P, row_forms, batch, d, deg
 
 @pytest.mark.parametrize("d,deg,dtype,line", [
     (8, 4, np.float64, 512), (17, 4, np.float64, 12), (18, 4, np.float64, 64), (18, 4, np.float32, 48), (19, 4, np.float64, 32), (20, 4, np.float64, 96),
-    (20, 4, np.float32, 48), (21, 4, np.float64, 48), (22, 4, np.float64, 28), (22, 4, np.float32, 20), (24, 4, np.float64, 56), (14, 5, np.float64, 3),
+    (20, 4, np.float32, 48), (21, 4, np.float64, 48), (22, 4, np.float64, 28), (22, 4, np.float32, 20), (24, 4, np.float64, 56), (14, 5, np.float64, 1),
     (16, 5, np.float64, None), (16, 5, np.float32, 1), (17, 4, np.float32, 1), (6, 6, np.float64, 1)])
 def test_rows_from_which_the_chen_adjoint_takes_one_pass(P, oracle, d, deg, dtype, line):
     """The line between the general kernels of the Chen product's adjoint and the pass that takes both factors: either side of it, as measured for each
