@@ -767,6 +767,8 @@ static inline bool fill_stream_levels(StreamLevels& lv, uint64_t d, uint64_t deg
 // 137 (5), which is left at 4.
 // The estimate, us, as measured on 1024 SIMDs: 0.35 a load of the walk while a SIMD has no second wave of them; 0.03 an addition to one address, 2e-5 any; a longer
 // word has to save 15, and 20 more for the two launches that longer words than the shortest take.
+// What it does not see is the alignment of a wave's loads, a level of words apart from each other: at 29 to 31 channels, degree 4, single precision, 32 to 52 rows
+// the longer words are the slower ones by up to 12 % (36 rows of 31: 459 / 515; of 32: 514 / 420), as they are the sooner ones at 25 to 28 and 33 to 48.
 // The sums of longer words are kept in double precision (right_sums; `elem_bytes` of T: they have to fit a row's top level).  For T = double that is no
 // better than T, so there the additions to one address may not grow by more than the walk, whose products a lane sums, gets shorter: errors as of that many
 // roundings.
